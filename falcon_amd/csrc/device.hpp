@@ -151,6 +151,11 @@ void launch_diffusion(const Dims &d, const DevTables &t, const TIN *in, const do
 // workgroups of the stage (kernel 0) or diffusion (1) march of a precision that
 // the device holds resident at once: the persistent grid
 int march_resident_wgs(int kernel, int precision, int tile);
+// radial segments that a one-workgroup-per-tile launch of the stage or
+// diffusion march cuts each tile's column into; 1 for a persistent launch
+// (wgs > 0).  Results do not depend on it; the dt partial minima are
+// one per tile and segment.
+int march_segments(const Dims &d, int tile, int wgs);
 // every ghost entry of g
 template <typename TS>
 void launch_exchange(const Dims &d, const DevGhosts &g, TS *state, hipStream_t s);
@@ -161,8 +166,11 @@ template <typename TS>
 void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull = nullptr);
 template <typename TS>
 void launch_copy_radial(const Dims &d, const DevBoundary &b, const TS *src, TS *dst, hipStream_t s);
-void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile);
-void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile);
+// nseg: the radial segments of the diffusion's tiles (march_segments): one
+// partial minimum per tile and segment
+void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile,
+                       int nseg);
+void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile, int nseg);
 void launch_to_f32(const double *src, float *dst, long long n, hipStream_t s);
 void launch_set_scalar(double *p, double v, hipStream_t s);
 // NaN scan of a padded state (see k_nan_scan): w[0] counts, w[1] first position;

@@ -490,10 +490,13 @@ void alloc_state(falcon_handle *h) {
         }
     }
     if (!h->dtp.p) { h->dtp.alloc(sizeof(double)); HIPCHECK(hipMemset(h->dtp.p, 0, sizeof(double))); }
-    // one partial minimum per workgroup of the diffusion / k_dt_tile; the 8-edge
-    // tiling has the most
-    const long long nt8 = (long long)h->dims.nblocks * ((h->dims.nj + 7) / 8) * ((h->dims.nk + 7) / 8);
-    if (!h->partial.p) h->partial.alloc(sizeof(double) * std::max(1LL, nt8));
+    // one partial minimum per workgroup of the diffusion / k_dt_tile (tile and
+    // radial segment); the larger of the two tilings
+    long long np = 1;
+    for (int e : {8, 16})
+        np = std::max(np, (long long)h->dims.nblocks * ((h->dims.nj + e - 1) / e) * ((h->dims.nk + e - 1) / e) *
+                              march_segments(h->dims, e, 0));
+    if (!h->partial.p) h->partial.alloc(sizeof(double) * np);
 }
 
 void alloc_stage(falcon_handle *h) {
@@ -549,7 +552,7 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
     const int ws = h->wgs_stage[h->precision], wd = h->wgs_diff[h->precision];
     timed(h, K_DT, [&] {
         if (h->fixed_dt > 0) launch_set_scalar(dtp, h->fixed_dt, s);
-        else launch_dt_final(d, part, dtp, cfl, s, td);
+        else launch_dt_final(d, part, dtp, cfl, s, td, march_segments(d, td, wd));
     });
     if (h->precision == 0) {
         double *S0 = h->S64[0].as<double>(), *S1 = h->S64[1].as<double>();
@@ -643,8 +646,9 @@ void prepare_steps(falcon_handle *h) {
         h->u_ghosts_valid = true;
     }
     if (!h->partials_valid) {
-        launch_dt_partial(d, h->dt, h->U[h->cur].as<double>(), h->partial.as<double>(), h->stream,
-                          h->tile_diff[h->precision]);
+        const int td = h->tile_diff[h->precision];
+        launch_dt_partial(d, h->dt, h->U[h->cur].as<double>(), h->partial.as<double>(), h->stream, td,
+                          march_segments(d, td, h->wgs_diff[h->precision]));
         h->partials_valid = true;
     }
 }
@@ -1140,8 +1144,9 @@ int falcon_set_precision(falcon_handle_t h, int mode) {
             refresh_u_ghosts(h);
             h->shadow_valid = false;
         }
-        // the partial minima are laid out per tile of the diffusion's edge
-        if (h->tile_diff[mode] != h->tile_diff[h->precision]) h->partials_valid = false;
+        // the partial minima are laid out per tile and radial segment of the diffusion
+        if (h->tile_diff[mode] != h->tile_diff[h->precision] || h->wgs_diff[mode] != h->wgs_diff[h->precision])
+            h->partials_valid = false;
         h->precision = mode;
     });
 }
@@ -1157,7 +1162,7 @@ static void apply_shape(falcon_handle *h, int p, int ts, int ws, int td, int wd)
         HIPCHECK(hipGraphExecDestroy(h->graph));
         h->graph = nullptr;
     }
-    if (p == h->precision && td != h->tile_diff[p]) h->partials_valid = false;
+    if (p == h->precision && (td != h->tile_diff[p] || wd != h->wgs_diff[p])) h->partials_valid = false;
     h->tile_stage[p] = ts;
     h->tile_diff[p] = td;
     h->wgs_stage[p] = ws;
@@ -1212,7 +1217,7 @@ int falcon_autotune(falcon_handle_t h, int reps, int *shape_out, double *ms_out)
         const int32_t *pull = (p == 1 && h->ghost_pull) ? h->gh32.pull : nullptr;
         // a time step for the timed launches to scale by; the diffusion launches
         // then overwrite the partial minima
-        launch_dt_final(d, part, dtp, 0.5, s, h->tile_diff[p]);
+        launch_dt_final(d, part, dtp, 0.5, s, h->tile_diff[p], march_segments(d, h->tile_diff[p], h->wgs_diff[p]));
         h->partials_valid = false;
         // destroyed on every exit, an error included
         struct Ev {
@@ -1338,8 +1343,9 @@ int falcon_compute_dt(falcon_handle_t h, double cfl, double *dt) {
         h->need_tables();
         ensure_device_tables(h);
         const int td = h->tile_diff[h->precision];
-        launch_dt_partial(h->dims, h->dt, h->U[h->cur].as<double>(), h->partial.as<double>(), h->stream, td);
-        launch_dt_final(h->dims, h->partial.as<double>(), h->dtp.as<double>(), cfl, h->stream, td);
+        const int ns = march_segments(h->dims, td, h->wgs_diff[h->precision]);
+        launch_dt_partial(h->dims, h->dt, h->U[h->cur].as<double>(), h->partial.as<double>(), h->stream, td, ns);
+        launch_dt_final(h->dims, h->partial.as<double>(), h->dtp.as<double>(), cfl, h->stream, td, ns);
         h->partials_valid = true;
         check_launch();
         HIPCHECK(hipMemcpyAsync(dt, h->dtp.p, sizeof(double), hipMemcpyDeviceToHost, h->stream));
@@ -1408,8 +1414,8 @@ int falcon_compute_dt_noalloc(falcon_handle_t h, double cfl, double *dt) {
                         std::to_string(DT_NOALLOC_MAX_PARTIALS) + " (falcon_compute_dt has none)");
         // every partial is written by the tile pass before the final pass reads it
         double *part = base, *dtp = base + DT_NOALLOC_MAX_PARTIALS;
-        launch_dt_partial(d, h->dt, h->U[h->cur].as<double>(), part, h->stream, td);
-        launch_dt_final(d, part, dtp, cfl, h->stream, td);
+        launch_dt_partial(d, h->dt, h->U[h->cur].as<double>(), part, h->stream, td, 1);
+        launch_dt_final(d, part, dtp, cfl, h->stream, td, 1);
         check_launch();
         HIPCHECK(hipMemcpyAsync(dt, dtp, sizeof(double), hipMemcpyDeviceToHost, h->stream));
         HIPCHECK(hipStreamSynchronize(h->stream));

@@ -357,7 +357,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                                                const TB *__restrict__ U, TOUT *__restrict__ out,
                                                float *__restrict__ shadow, const double *__restrict__ dtp,
                                                double div, const int32_t *__restrict__ pull,
-                                               const double *__restrict__ glm) {
+                                               const double *__restrict__ glm, int nseg) {
     constexpr int PL = tile_pl<TL>();
     __shared__ T lds[2][8][PL][PL];
     // LEAN (FP32 storage): the block's radial coefficient rows (xi, rho0, gp,
@@ -372,13 +372,16 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
     constexpr bool LEAN = sizeof(T) == 4;
     __shared__ double crow[kStageRows][kMaxNI];
     const int ntk = (d.nk + TL - 1) / TL, tpb = ((d.nj + TL - 1) / TL) * ntk;
-    const int ntot = d.nblocks * tpb;
+    const int ntot = d.nblocks * tpb * nseg;
     // PERSIST: a grid smaller than the tile count (a persistent launch) takes
     // the next tile at a stride of the grid size; otherwise one pass, tile =
-    // the workgroup
+    // the workgroup.  A tile's march is cut into nseg radial segments
+    // (march_segments), the segments of a tile consecutive.
     for (int tile = PERSIST ? (int)blockIdx.x : xcd_tile(blockIdx.x, ntot); tile < ntot; tile += gridDim.x) {
-        const int b = tile / tpb;
-        const int trem = tile - b * tpb;
+        const int tcol = tile / nseg, seg = tile - tcol * nseg;
+        const int iA = seg * d.ni / nseg, iB = (seg + 1) * d.ni / nseg;
+        const int b = tcol / tpb;
+        const int trem = tcol - b * tpb;
         const int tj = trem / ntk, tk = trem - tj * ntk;
         const int j0 = tj * TL, k0 = tk * TL;
         const int TJa = min(TL, d.nj - j0), TKa = min(TL, d.nk - k0);
@@ -420,15 +423,15 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
     #pragma unroll
         for (int v = 0; v < 8; v++) {
     #pragma unroll
-            for (int q = 0; q < 5; q++) win[v][q] = m.col(v, q);
-            hn[v] = m.halo(v, d.ng);
+            for (int q = 0; q < 5; q++) win[v][q] = m.col(v, iA + q);
+            hn[v] = m.halo(v, iA + d.ng);
         }
         const long long ubase = (long long)b * 8 * d.P + m.coff;
         // G ([block][3][interior cells]) at this lane's column; plane i at + i nj nk
         const long long gnn = (long long)d.ni * d.nj * d.nk;
         const double *gcol = GLM ? glm + (b * 3 * gnn + ((long long)(j0 + ty) * d.nk + (k0 + tx))) : nullptr;
 
-        for (int i = 0; i < d.ni; i++) {
+        for (int i = iA; i < iB; i++) {
             const int I = i + d.ng;
             const int buf = i & 1;
             // U of this plane, issued first: the plane's arithmetic covers its latency
@@ -446,7 +449,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
             // prefetch the next window plane and the next halo (on the last plane
             // the clamped loads are discarded)
             const int In = min(I + 3, d.NI - 1), Ih = min(I + 1, d.NI - 1);
-            const bool more = i + 1 < d.ni;
+            const bool more = i + 1 < iB;
     #pragma unroll
             for (int v = 0; v < 8; v++) {
                 nxt[v] = (LEAN || (m.act && more)) ? m.col(v, In) : T(0);
@@ -515,8 +518,8 @@ __global__ void __launch_bounds__(TL * TL) k_stage(Dims d, DevTables t, const TI
                                                const TB *__restrict__ U, TOUT *__restrict__ out,
                                                float *__restrict__ shadow, const double *__restrict__ dtp,
                                                double div, const int32_t *__restrict__ pull,
-                                               const double *__restrict__ glm) {
-    stage_body<T, TIN, TOUT, TB, MODE, SHADOW, TL, PERSIST, GLM>(d, t, in, U, out, shadow, dtp, div, pull, glm);
+                                               const double *__restrict__ glm, int nseg) {
+    stage_body<T, TIN, TOUT, TB, MODE, SHADOW, TL, PERSIST, GLM>(d, t, in, U, out, shadow, dtp, div, pull, glm, nseg);
 }
 
 // The FP64 step's stage (16-edge tiles, one workgroup per tile) held to two
@@ -530,8 +533,8 @@ template <typename T, typename TIN, typename TOUT, typename TB, int MODE, bool S
 __global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2)))
 k_stage_w2(Dims d, DevTables t, const TIN *__restrict__ in, const TB *__restrict__ U, TOUT *__restrict__ out,
            float *__restrict__ shadow, const double *__restrict__ dtp, double div,
-           const int32_t *__restrict__ pull, const double *__restrict__ glm) {
-    stage_body<T, TIN, TOUT, TB, MODE, SHADOW, TL, PERSIST, GLM>(d, t, in, U, out, shadow, dtp, div, pull, glm);
+           const int32_t *__restrict__ pull, const double *__restrict__ glm, int nseg) {
+    stage_body<T, TIN, TOUT, TB, MODE, SHADOW, TL, PERSIST, GLM>(d, t, in, U, out, shadow, dtp, div, pull, glm, nseg);
 }
 
 // ---------------------------------------------------------------- diffusion
@@ -567,7 +570,8 @@ template <typename T, typename TIN, int MODE, int TL, bool PERSIST>
 __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, const TIN *__restrict__ in,
                                                    const double *U, double *out, float *__restrict__ shadow,
                                                    double *__restrict__ partial, const double *__restrict__ dtp,
-                                                   const int32_t *__restrict__ pull, const double *__restrict__ Uold) {
+                                                   const int32_t *__restrict__ pull, const double *__restrict__ Uold,
+                                                   int nseg) {
     // one r-plane with its theta/phi halo; the second barrier of each plane
     // orders its reuse, so it is not double-buffered
     constexpr int PL = tile_pl<TL>();
@@ -595,14 +599,18 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
     __shared__ T sj[LEAN ? 8 : 1][TL + 2][TL];
     __shared__ T sk[LEAN ? 8 : 1][TL][TL + 2];
     const int ntk = (d.nk + TL - 1) / TL, tpb = ((d.nj + TL - 1) / TL) * ntk;
-    const int ntot = d.nblocks * tpb;
+    const int ntot = d.nblocks * tpb * nseg;
     // PERSIST: a grid smaller than the tile count (a persistent launch) takes
     // the next tile at a stride of the grid size; otherwise one pass, tile =
-    // the workgroup
+    // the workgroup.  nseg: radial segments per tile, as in stage_body; a
+    // segment forms its first plane's lower r-face itself and has at least two
+    // planes (march_segments), which the FP32 path's boundary faces need.
     for (int tile = PERSIST ? (int)blockIdx.x : xcd_tile(blockIdx.x, ntot); tile < ntot; tile += gridDim.x) {
-        const int b = tile / tpb;
+        const int tcol = tile / nseg, seg = tile - tcol * nseg;
+        const int iA = seg * d.ni / nseg, iB = (seg + 1) * d.ni / nseg;
+        const int b = tcol / tpb;
         if (sizeof(T) == 4 && MODE == 0 && threadIdx.x < 27) pdir[threadIdx.x] = pull ? pull[b * 27 + threadIdx.x] : -1;
-        const int trem = tile - b * tpb;
+        const int trem = tcol - b * tpb;
         const int tj = trem / ntk, tk = trem - tj * ntk;
         const int j0 = tj * TL, k0 = tk * TL;
         const int TJa = min(TL, d.nj - j0), TKa = min(TL, d.nk - k0);
@@ -648,8 +656,8 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
     #pragma unroll
         for (int v = 0; v < 8; v++) {
     #pragma unroll
-            for (int q = 0; q < 5; q++) win[v][q] = (LEAN || m.act) ? m.col(v, q) : T(0);
-            hn[v] = (LEAN || m.hv) ? m.halo(v, d.ng) : T(0);
+            for (int q = 0; q < 5; q++) win[v][q] = (LEAN || m.act) ? m.col(v, iA + q) : T(0);
+            hn[v] = (LEAN || m.hv) ? m.halo(v, iA + d.ng) : T(0);
             fr[v] = T(0);
         }
         // a ghost in a direction listed in the pull table is the same-level
@@ -682,7 +690,7 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
         const int bJ0 = bj ? j0 + d.ng : j0 + by + d.ng - 2, bK0 = bj ? k0 + bx + d.ng - 2 : k0 + d.ng;
         const int bJ1 = bj ? bJ0 - 1 : bJ0, bK1 = bj ? bK0 : bK0 - 1;
 
-        for (int i = 0; i < d.ni; i++) {
+        for (int i = iA; i < iB; i++) {
             const int I = i + d.ng;
             // LEAN: U^n of the plane and |v_d| at the shifted speed cells, issued
             // before the prefetch (inactive lanes read at the tile's first column)
@@ -711,7 +719,7 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
                 if (m.act) lds[v][ty + 2][tx + 2] = win[v][2];
                 if (m.hv) lds[v][m.hly][m.hlx] = hn[v];
             }
-            const bool more = i + 1 < d.ni;
+            const bool more = i + 1 < iB;
             const int In = min(I + 3, d.NI - 1), Ih = min(I + 1, d.NI - 1);
     #pragma unroll
             for (int v = 0; v < 8; v++) {
@@ -1121,11 +1129,13 @@ __global__ void __launch_bounds__(256) k_boundary(Dims d, DevBoundary bl, TS *__
 // stepping the diffusion kernel produces the same partials.
 template <int TL>
 __global__ void __launch_bounds__(TL * TL) k_dt_tile(Dims d, DevTables t, const double *__restrict__ U,
-                                                     double *__restrict__ partial) {
+                                                     double *__restrict__ partial, int nseg) {
     __shared__ double red[4];
     const int ntk = (d.nk + TL - 1) / TL, tpb = ((d.nj + TL - 1) / TL) * ntk;
-    const int b = blockIdx.x / tpb;
-    const int trem = blockIdx.x - b * tpb;
+    const int tcol = blockIdx.x / nseg, seg = blockIdx.x - tcol * nseg;
+    const int iA = seg * d.ni / nseg, iB = (seg + 1) * d.ni / nseg;
+    const int b = tcol / tpb;
+    const int trem = tcol - b * tpb;
     const int tj = trem / ntk, tk = trem - tj * ntk;
     const int tx = threadIdx.x & (TL - 1), ty = threadIdx.x / TL;
     const int j = tj * TL + ty, k = tk * TL + tx;
@@ -1136,7 +1146,7 @@ __global__ void __launch_bounds__(TL * TL) k_dt_tile(Dims d, DevTables t, const 
     if (j < d.nj && k < d.nk) {
         const int J = j + d.ng, K = k + d.ng;
         const double st = t.sint[tb + J];
-        for (int i = 0; i < d.ni; i++) {
+        for (int i = iA; i < iB; i++) {
             const int I = i + d.ng;
             const long long q = cell_off(d, I, J, K);
             const double vr = Ub[q + d.P], vt = Ub[q + 2 * d.P], vp = Ub[q + 3 * d.P];
@@ -1315,15 +1325,61 @@ static void check_tile(int tile) {
     if (tile != 8 && tile != 16) throw std::runtime_error("tile edge must be 8 or 16");
 }
 
+// Blocks whose faces fit an 8-edge tile run the 8-edge march also where 16 is
+// asked for (one tile per block either way).
+static inline int march_edge(const Dims &d, int tile, int wgs) {
+    return tile == 16 && wgs == 0 && d.nj <= 8 && d.nk <= 8 ? 8 : tile;
+}
+
+// Radial segments per tile.  A march is a serial chain of planes, so a layout
+// with few tiles leaves compute units idle or with an uneven last round; cut
+// in segments the tiles fill the chip, at the price of the extra planes each
+// segment loads.  The rule minimises the time of the busiest of the 256
+// compute units: it runs n workgroups (4 of the 64-lane ones count as one), a
+// pair of resident workgroups takes 2 x kPair of one alone, and a segment of
+// len planes costs len + kFill (its first window and face).  Both constants
+// are fits to the stage and diffusion at 1 .. 8 segments over twelve layouts
+// of 40 to 12288 blocks (us per launch, one against the chosen number of
+// segments; FP64 stage / FP64 diffusion / FP32 stage / FP32 diffusion):
+//    40 blocks of  8x6x12    33.0->13.8   82.0->26.7   25.4->12.7   71.8->26.2
+//    60 blocks of 16x16x16   68.6->20.2  154.3->39.2   46.7->17.1  141.1->34.0
+//   192 blocks of 16x16x16   79.9->56.9  161.4->103.8  49.2->38.8  137.9->91.6
+//   528 blocks of 16x16x16  196.1->155.2 358.9->274.2 107.8->98.7  283.2->216.6
+//   128 blocks of 64x16x48  521.5->423.8 929.7->705.4 301.0->259.7 608.8->512.0
+// From about 768 16^3 blocks on one segment is best (1536 blocks: 399 against
+// 406 us for two, FP32 diffusion 490 against 529), and the rule keeps it
+// unless more segments are predicted to save 3%.  A segment has at least two
+// planes: the FP32 diffusion's radial boundary faces read the neighbouring
+// plane of their own segment.
+int march_segments(const Dims &d, int tile, int wgs) {
+    if (wgs != 0) return 1;
+    constexpr double kPair = 0.75, kFill = 1.5;
+    const int TL = march_edge(d, tile, wgs);
+    const long long cus = TL == 16 ? 256 : 4 * 256, nt = tiles(d, TL);
+    int best = 1;
+    double cost = 0.0;
+    for (int ns = 1; ns <= 8 && (ns == 1 || 2 * ns <= d.ni); ns *= 2) {
+        const long long n = (nt * ns + cus - 1) / cus;
+        const double rounds = n > 6 ? kPair * (double)(nt * ns) / (double)cus
+                                    : (n & 1) ? (double)(n - 1) * kPair + 1.0 : (double)n * kPair;
+        const double c = ((d.ni + ns - 1) / ns + kFill) * rounds;
+        if (ns == 1 || c < 0.97 * cost) {
+            best = ns;
+            cost = c;
+        }
+    }
+    return best;
+}
+
 static void check_stage_ni(const Dims &d) {
     if (d.NI > kMaxNI) throw std::runtime_error("stage march: more than 128 radial cells per block");
 }
 
 // grid of a march: one workgroup per tile (wgs = 0) or wgs workgroups that
 // loop over the tiles (a persistent launch), never more than the tiles
-static inline dim3 march_grid(const Dims &d, int TL, int wgs) {
+static inline dim3 march_grid(const Dims &d, int TL, int wgs, int nseg) {
     if (wgs < 0) throw std::runtime_error("workgroup count < 0");
-    const unsigned n = tiles(d, TL);
+    const unsigned n = tiles(d, TL) * (unsigned)nseg;
     return dim3(wgs == 0 ? n : std::min<unsigned>(n, (unsigned)wgs));
 }
 
@@ -1361,39 +1417,40 @@ int march_resident_wgs(int kernel, int precision, int tile) {
 template <int TL, typename T, typename TIN, typename TOUT, typename TB>
 static void stage_tl(const Dims &d, const DevTables &t, const TIN *in, const TB *U, TOUT *out, float *shadow,
                      const double *dtp, double div, hipStream_t s, const int32_t *pull, int wgs, const double *glm) {
-    const dim3 g = march_grid(d, TL, wgs), b(TL * TL);
+    const int nseg = march_segments(d, TL, wgs);
+    const dim3 g = march_grid(d, TL, wgs, nseg), b(TL * TL);
     if constexpr (sizeof(T) == 8) {
         if (glm) {
             if (shadow) throw std::runtime_error("GLM stage: no FP32 copy");
             if (wgs)
                 hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, false, TL, true, true>), g, b, 0, s, d, t, in, U, out,
-                                   (float *)nullptr, dtp, div, pull, glm);
+                                   (float *)nullptr, dtp, div, pull, glm, nseg);
             else if (TL == 16)
                 hipLaunchKernelGGL((k_stage_w2<T, TIN, TOUT, TB, 0, false, TL, false, true>), g, b, 0, s, d, t, in, U,
-                                   out, (float *)nullptr, dtp, div, pull, glm);
+                                   out, (float *)nullptr, dtp, div, pull, glm, nseg);
             else
                 hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, false, TL, false, true>), g, b, 0, s, d, t, in, U, out,
-                                   (float *)nullptr, dtp, div, pull, glm);
+                                   (float *)nullptr, dtp, div, pull, glm, nseg);
             return;
         }
         if (!shadow && !wgs && TL == 16) {
             hipLaunchKernelGGL((k_stage_w2<T, TIN, TOUT, TB, 0, false, TL, false>), g, b, 0, s, d, t, in, U, out,
-                               (float *)nullptr, dtp, div, pull, glm);
+                               (float *)nullptr, dtp, div, pull, glm, nseg);
             return;
         }
     }
     if (shadow && wgs)
         hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, true, TL, true>), g, b, 0, s, d, t, in, U, out, shadow, dtp, div,
-                           pull, glm);
+                           pull, glm, nseg);
     else if (shadow)
         hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, true, TL, false>), g, b, 0, s, d, t, in, U, out, shadow, dtp, div,
-                           pull, glm);
+                           pull, glm, nseg);
     else if (wgs)
         hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, false, TL, true>), g, b, 0, s, d, t, in, U, out,
-                           (float *)nullptr, dtp, div, pull, glm);
+                           (float *)nullptr, dtp, div, pull, glm, nseg);
     else
         hipLaunchKernelGGL((k_stage<T, TIN, TOUT, TB, 0, false, TL, false>), g, b, 0, s, d, t, in, U, out,
-                           (float *)nullptr, dtp, div, pull, glm);
+                           (float *)nullptr, dtp, div, pull, glm, nseg);
 }
 
 template <typename T, typename TIN, typename TOUT, typename TB>
@@ -1403,15 +1460,15 @@ void launch_stage(const Dims &d, const DevTables &t, const TIN *in, const TB *U,
     check_tile(tile);
     check_stage_ni(d);
     if (glm && sizeof(T) != 8) throw std::runtime_error("GLM divergence cleaning runs on the FP64 path only");
-    if (tile == 16) stage_tl<16, T>(d, t, in, U, out, shadow, dtp, div, s, pull, wgs, glm);
+    if (march_edge(d, tile, wgs) == 16) stage_tl<16, T>(d, t, in, U, out, shadow, dtp, div, s, pull, wgs, glm);
     else stage_tl<8, T>(d, t, in, U, out, shadow, dtp, div, s, pull, wgs, glm);
 }
 
 template <int TL, bool PERSIST, typename T, typename TIN>
 static void rhs_tl(const Dims &d, const DevTables &t, const TIN *in, double *R, hipStream_t s, int wgs) {
-    hipLaunchKernelGGL((k_stage<T, TIN, double, double, 1, false, TL, PERSIST>), march_grid(d, TL, wgs), dim3(TL * TL), 0,
-                       s, d, t, in, (const double *)nullptr, R, (float *)nullptr, (const double *)nullptr, 1.0,
-                       (const int32_t *)nullptr, (const double *)nullptr);
+    hipLaunchKernelGGL((k_stage<T, TIN, double, double, 1, false, TL, PERSIST>), march_grid(d, TL, wgs, 1),
+                       dim3(TL * TL), 0, s, d, t, in, (const double *)nullptr, R, (float *)nullptr,
+                       (const double *)nullptr, 1.0, (const int32_t *)nullptr, (const double *)nullptr, 1);
 }
 
 template <typename T, typename TIN>
@@ -1431,8 +1488,9 @@ template <int TL, bool PERSIST, int MODE, typename T, typename TIN>
 static void diffusion_tl(const Dims &d, const DevTables &t, const TIN *in, const double *U, double *out,
                          float *shadow, double *partial, const double *dtp, hipStream_t s, const int32_t *pull,
                          int wgs, const double *Uold) {
-    hipLaunchKernelGGL((k_diffusion<T, TIN, MODE, TL, PERSIST>), march_grid(d, TL, wgs), dim3(TL * TL), 0, s, d, t, in,
-                       U, out, shadow, partial, dtp, pull, Uold);
+    const int nseg = MODE == 0 ? march_segments(d, TL, wgs) : 1;
+    hipLaunchKernelGGL((k_diffusion<T, TIN, MODE, TL, PERSIST>), march_grid(d, TL, wgs, nseg), dim3(TL * TL), 0, s, d,
+                       t, in, U, out, shadow, partial, dtp, pull, Uold, nseg);
 }
 
 template <int MODE, typename T, typename TIN>
@@ -1440,7 +1498,7 @@ static void diffusion_any(const Dims &d, const DevTables &t, const TIN *in, cons
                           float *shadow, double *partial, const double *dtp, hipStream_t s, const int32_t *pull,
                           int tile, int wgs, const double *Uold) {
     check_tile(tile);
-    if (tile == 16) {
+    if (march_edge(d, tile, wgs) == 16) {
         if (wgs) diffusion_tl<16, true, MODE, T>(d, t, in, U, out, shadow, partial, dtp, s, pull, wgs, Uold);
         else diffusion_tl<16, false, MODE, T>(d, t, in, U, out, shadow, partial, dtp, s, pull, wgs, Uold);
     } else {
@@ -1504,15 +1562,18 @@ void launch_copy_radial(const Dims &d, const DevBoundary &b, const TS *src, TS *
 
 // the partial minima are laid out as the diffusion with the same tile edge
 // leaves them, one per workgroup
-void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile) {
+void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile,
+                       int nseg) {
     check_tile(tile);
-    if (tile == 16) hipLaunchKernelGGL(k_dt_tile<16>, dim3(tiles(d, 16)), dim3(256), 0, s, d, t, U, partial);
-    else hipLaunchKernelGGL(k_dt_tile<8>, dim3(tiles(d, 8)), dim3(64), 0, s, d, t, U, partial);
+    const dim3 g(tiles(d, tile) * (unsigned)nseg);
+    if (march_edge(d, tile, 0) == 16) hipLaunchKernelGGL(k_dt_tile<16>, g, dim3(256), 0, s, d, t, U, partial, nseg);
+    else hipLaunchKernelGGL(k_dt_tile<8>, g, dim3(64), 0, s, d, t, U, partial, nseg);
 }
 
-void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile) {
+void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile,
+                     int nseg) {
     check_tile(tile);
-    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, s, partial, (int)tiles(d, tile), cfl, dtp);
+    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, s, partial, (int)(tiles(d, tile) * (unsigned)nseg), cfl, dtp);
 }
 
 void launch_set_scalar(double *p, double v, hipStream_t s) {

@@ -462,3 +462,32 @@ def test_synthetic_state_on_device_matches_the_restatement(name):
         assert np.all(got[ib][0:4] == 0.0)
         assert np.array_equal(got[ib][7], want[ib][7]), ib
         assert np.max(np.abs(got[ib][4:7] - want[ib][4:7])) <= 1e-12 * bmax, ib
+
+
+# radial extents whose segments are uneven or as short as two planes, on faces
+# within one 8-edge tile, on partial 16-edge tiles and on several tiles
+@pytest.mark.parametrize("block,split", [((4, 8, 8), (2, 2, 6)), ((5, 6, 8), (2, 3, 4)), ((7, 9, 17), (1, 2, 3)),
+                                         ((16, 16, 16), (1, 2, 4))])
+def test_radial_segments_bit_identical(block, split):
+    """Few blocks: the marches run in radial segments.  FP64 steps equal the
+    oracle's; both precisions equal looping workgroups, which march whole columns."""
+    print(f"[segments] block={block} split={split}", flush=True)
+    lay = {"ni": block[0], "nj": block[1], "nk": block[2], "ng": 2, "r_rsun": (0.7, 1.0), "ops": [("split", split)]}
+    s, o = _pair(lay, seed=23)
+    s.sendrecv_gc(0); o.exchange(0)
+    assert s.compute_dt(0.5) == o.dt(0.5)
+    for step in range(2):
+        assert s.advance_rk4(0.5) == o.step(0.5), step
+    assert np.array_equal(_states(s, o.nblocks), _states(o, o.nblocks))
+    for prec in ("fp64", "fp32"):
+        runs = []
+        for wgs in (0, 3):
+            s = Shell(lay)
+            s.set_gc_all()
+            s.background_polytrope(20.0)
+            s.init_synthetic(seed=29)
+            s.set_precision(prec)
+            s.set_tiles(1 if prec == "fp32" else 0, 16, 16, wgs, wgs)
+            s.advance(5, 0.5, graph=True)
+            runs.append(_states(s, s.nblocks))
+        assert np.array_equal(runs[0], runs[1]), prec
