@@ -68,9 +68,27 @@ constexpr int kMaxNI = 132;
 
 // ModDerivative_1st_O4_3D (3_6/ModDerivative.f90:16-19):
 // (1./12./dx)*( -f(+2) + 8.*f(+1) - 8.*f(-1) + f(-2) )
-template <typename T>
-__device__ __forceinline__ T d4(T fm2, T fm1, T fp1, T fp2, T c) {
-    return c * ((((-fp2) + T(8) * fp1) - T(8) * fm1) + fm2);
+// The products with 8 are exact, so each fused multiply-add rounds as the
+// reference's product and sum do.
+__device__ __forceinline__ double d4(double fm2, double fm1, double fp1, double fp2, double c) {
+    return c * (__builtin_fma(-8.0, fm1, __builtin_fma(8.0, fp1, -fp2)) + fm2);
+}
+
+// x / b for many x and one b: y = 1/b by two Newton steps on the hardware
+// reciprocal, then Markstein's correction of x*y by its exact remainder: the
+// correctly rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990) in 3
+// operations per x, where the general division takes 11 (the same steps with
+// a rescaling of operands near the ends of the exponent range, which neither
+// the background's and metric's divisors nor values above 1e-290 reach).  The
+// fix-up gives zeros, infinities and NaN as the division does.
+__device__ __forceinline__ double div_rcp(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+}
+__device__ __forceinline__ double div_by(double x, double b, double y) {
+    const double q = x * y;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, x), y, q), b, x);
 }
 
 // ModLinReconstruct_minmod (3_6/ModLinReconstruct.f90:37-48) for one triple
@@ -136,10 +154,13 @@ struct Marcher {
     int SI, SJ;             // main-part plane and row pitch (cell_off)
     int ilo, ihi;           // first interior plane, first plane above the interior
     int J, K;           // padded column of this lane
-    long long coff;     // J*SJ + K, clamped into the block for lanes outside a partial tile
+    // addresses are a base that is the same for the whole workgroup (scalar
+    // registers) plus this 32-bit lane offset: J*SJ + K, clamped into the block
+    // for lanes outside a partial tile
+    unsigned coff;
     bool act;
     bool hv;
-    long long hoff;     // cell_off of the halo point at plane 0 (a valid cell for lanes without one)
+    unsigned hoff;      // cell_off of the halo point at plane 0 (a valid cell for lanes without one)
     int hsi;            // plane pitch of the halo point's part (main or side)
     int hly, hlx;
 
@@ -164,7 +185,7 @@ struct Marcher {
         K = k0 + tx + d.ng;
         // loads of inactive lanes read the tile's first cell, so every load can be
         // issued without a branch; their values are never used
-        coff = act ? (long long)J * SJ + (K - d.ng) : (long long)(j0 + d.ng) * SJ + k0;
+        coff = (unsigned)(act ? J * SJ + (K - d.ng) : (j0 + d.ng) * SJ + k0);
         const int h = threadIdx.x;
         hv = false; hly = 0; hlx = 0;
         if (h < 4 * TL) {
@@ -181,7 +202,7 @@ struct Marcher {
         }
         const int HJ = j0 + hly, HK = k0 + hlx;   // padded halo cell
         const bool hmain = HK >= d.ng && HK < d.ng + d.nk;
-        hoff = hv ? cell_off(d, 0, HJ, HK) : coff;
+        hoff = hv ? (unsigned)cell_off(d, 0, HJ, HK) : coff;
         hsi = (!hv || hmain) ? SI : d.NJ * 2 * d.ng;
         if (PULL && pull && hv) {
             const int dj = HJ < d.ng ? -1 : (HJ >= d.ng + d.nj ? 1 : 0);
@@ -191,7 +212,7 @@ struct Marcher {
                 if (D >= 0) {
                     // the neighbour's interior cell: always in its main part
                     hblk = in + (long long)D * 8 * P;
-                    hoff = cell_off(d, 0, HJ - dj * d.nj, HK - dk * d.nk);
+                    hoff = (unsigned)cell_off(d, 0, HJ - dj * d.nj, HK - dk * d.nk);
                     hsi = SI;
                 }
             }
@@ -199,13 +220,14 @@ struct Marcher {
     }
     // I is the same for every lane of the workgroup, 0 <= I < NI
     __device__ __forceinline__ T col(int v, int I) const {
-        long long o = (long long)v * P + (long long)I * SI + coff;
-        if (PULL) o += (I < ilo ? dlo : 0ll) + (I >= ihi ? dhi : 0ll);
-        return (T)blk[o];
+        const TIN *base = blk + ((long long)v * P + (long long)I * SI);
+        if (PULL) base += (I < ilo ? dlo : 0ll) + (I >= ihi ? dhi : 0ll);
+        return (T)base[coff];
     }
     // interior planes only
     __device__ __forceinline__ T halo(int v, int I) const {
-        return (T)(PULL ? hblk : blk)[(long long)v * P + (long long)I * hsi + hoff];
+        const unsigned o = (unsigned)(I * hsi) + hoff;
+        return (T)((PULL ? hblk : blk) + (long long)v * P)[o];
     }
 };
 
@@ -228,10 +250,13 @@ __device__ __forceinline__ void cell_rhs(const TW (&win)[8][5], LDSF L, const T 
                                          T sinv, T cot, T cr, T ct, T cp, T irho0, T R[8]) {
     auto W = [&](int v, int q) -> T { return (T)win[v][q]; };
     const T rho0c = rho0r[2];
-    auto over_rho0 = [&](T x) -> T { return RECIP ? x * irho0 : x / rho0c; };
+    const T yst = RECIP ? T(0) : div_rcp(st[2]);
+    auto over_rho0 = [&](T x) -> T { return RECIP ? x * irho0 : div_by(x, rho0c, irho0); };
     // d4 of f/sin(theta) along phi (sin(theta) is constant along phi)
     auto d4_over_st = [&](T f0, T f1, T f3, T f4) -> T {
-        return RECIP ? d4(f0, f1, f3, f4, cp) * sinv : d4(f0 / st[2], f1 / st[2], f3 / st[2], f4 / st[2], cp);
+        return RECIP ? d4(f0, f1, f3, f4, cp) * sinv
+                     : d4(div_by(f0, st[2], yst), div_by(f1, st[2], yst), div_by(f3, st[2], yst),
+                          div_by(f4, st[2], yst), cp);
     };
     const T vr = W(1, 2), vt = W(2, 2), vp = W(3, 2);
     const T br = W(4, 2), bt = W(5, 2), bp = W(6, 2);
@@ -416,7 +441,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
         // the FP32 path's reciprocal form (cell_rhs): the stage increment
         // (dt*R)/(5-k) as a product with 1/(5-k)
         constexpr bool RECIP = LEAN;
-        const double rdiv = 1.0 / div;
+        const double rdiv = 1.0 / div, ydiv = div_rcp(div);
 
         T win[8][5];
         T nxt[8], hn[8];
@@ -426,7 +451,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
             for (int q = 0; q < 5; q++) win[v][q] = m.col(v, iA + q);
             hn[v] = m.halo(v, iA + d.ng);
         }
-        const long long ubase = (long long)b * 8 * d.P + m.coff;
+        const long long bbase = (long long)b * 8 * d.P;
         // G ([block][3][interior cells]) at this lane's column; plane i at + i nj nk
         const long long gnn = (long long)d.ni * d.nj * d.nk;
         const double *gcol = GLM ? glm + (b * 3 * gnn + ((long long)(j0 + ty) * d.nk + (k0 + tx))) : nullptr;
@@ -438,7 +463,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
             TB ub[8];
             if (MODE == 0 && LEAN) {
     #pragma unroll
-                for (int v = 0; v < 8; v++) ub[v] = U[ubase + (long long)v * d.P + (long long)I * m.SI];
+                for (int v = 0; v < 8; v++) ub[v] = (U + (bbase + (long long)v * d.P + (long long)I * m.SI))[m.coff];
             }
             // stage this plane: own column centre plus halo strips
     #pragma unroll
@@ -462,7 +487,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                     if (LEAN) return crow[r][II];
                     const double *src = r == 0 ? t.xi : r == 1 ? t.rho0 : r == 2 ? t.gp : r == 3 ? t.gq : r == 4 ? t.rinv
                                       : r == 5 ? t.r2inv : r == 6 ? t.xir2 : r == 7 ? t.heat : t.g_over_rho0;
-                    return r == 9 ? 1.0 / t.rho0[rb + II] : src[rb + II];
+                    return src[rb + II];
                 };
                 double xr[5], rho0r[5], gpr[5], gqr[5];
     #pragma unroll
@@ -475,7 +500,8 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                 auto L = [&](int v, int dj, int dk) -> double { return (double)lds[buf][v][ty + 2 + dj][tx + 2 + dk]; };
                 double R[8];
                 cell_rhs<double, T, RECIP>(win, L, xr, rho0r, gpr, gqr, st, coef(4, I), coef(5, I), coef(6, I),
-                                           coef(7, I), coef(8, I), sinv, cot, cr, ct, cp, RECIP ? coef(9, I) : 1.0, R);
+                                           coef(7, I), coef(8, I), sinv, cot, cr, ct, cp,
+                                           RECIP ? coef(9, I) : div_rcp(rho0r[2]), R);
                 if (MODE == 0) {
                     if constexpr (GLM && sizeof(T) == 8) {
                         // ModDivB_GLM (3_6/ModDivB.f90:27-28): R(B) = R(B) - grad(psi)
@@ -484,14 +510,14 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                         R[5] = R[5] - gi[gnn];
                         R[6] = R[6] - gi[2 * gnn];
                     }
-                    const long long base = (long long)b * 8 * d.P + (long long)I * m.SI + m.coff;
+                    const long long base = bbase + (long long)I * m.SI;
     #pragma unroll
                     for (int v = 0; v < 8; v++) {
                         const long long q = base + (long long)v * d.P;
-                        const double inc = RECIP ? (dt * R[v]) * rdiv : (dt * R[v]) / div;
-                        const double x = (double)(LEAN ? ub[v] : U[q]) + inc;
-                        out[q] = (TOUT)x;
-                        if (SHADOW) shadow[q] = (float)x;
+                        const double inc = RECIP ? (dt * R[v]) * rdiv : div_by(dt * R[v], div, ydiv);
+                        const double x = (double)(LEAN ? ub[v] : (U + q)[m.coff]) + inc;
+                        (out + q)[m.coff] = (TOUT)x;
+                        if (SHADOW) (shadow + q)[m.coff] = (float)x;
                     }
                 } else {
                     const long long nn = (long long)d.ni * d.nj * d.nk;
