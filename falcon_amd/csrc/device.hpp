@@ -85,7 +85,7 @@ inline Dims make_dims(int ni, int nj, int nk, int ng, int nblocks) {
     return d;
 }
 
-// Ghost-fill tables (device), one row per ghost entry: same-panel entries in
+// Ghost-fill tables of the FP32 buffers, one row per ghost entry: same-panel entries in
 // [0, yy_begin), Yin-Yang entries in [yy_begin, n_total), each set in the order
 // of the receiving blocks' target lists.
 struct DevGhosts {
@@ -108,6 +108,15 @@ struct DevGhosts {
     // copies, ghost index g <- D's cell g - (di*ni, dj*nj, dk*nk); -1 where any
     // ghost of that region is filled otherwise.  null: no pull.
     const int32_t *pull;
+};
+
+// Ghost-fill table of the FP64 buffers, in the order of src.
+struct DevGhosts64 {
+    const int32_t *dst;     // block*8*P + cell of the ghost (variable 0); bit 31: a Yin-Yang entry
+    const int32_t *src;     // donor*8*P + cell of the interpolation base (variable 0)
+    const double *w;        // 3 weights per entry
+    const double *rot;      // 2 rotation coefficients per entry (read for Yin-Yang entries only)
+    int n;
 };
 
 struct DevBoundary {
@@ -134,14 +143,15 @@ void launch_stage(const Dims &d, const DevTables &t, const TIN *in, const TB *U,
 // dt R(psi)/div from the stage input (state `in`, psi_in) and Ch, and
 // G = grad(psi_in);
 // diffusion: psi_new = psi + 0.5 dt R_diff(psi) with the speeds of U;
-// ghost fill: the FP64 state's and psi's ghosts in one pass over the FP64
-// ghost tables (psi a scalar: no Yin-Yang rotation).
+// ghost fill: launch_exchange64, with the state's (psi a scalar: no Yin-Yang
+// rotation).
 void launch_glm_speed(const Dims &d, const DevTables &t, const double *U, double *Ch, hipStream_t s);
 void launch_glm_stage(const Dims &d, const DevTables &t, const double *in, const double *Ch, const double *psi_in,
                       const double *psi_n, double *psi_out, double *G, const double *dtp, double div, hipStream_t s);
 void launch_glm_diffusion(const Dims &d, const DevTables &t, const double *U, const double *psi, double *psi_new,
                           const double *dtp, hipStream_t s);
-void launch_exchange_glm(const Dims &d, const DevGhosts &g, double *state, double *psi, hipStream_t s);
+// the FP64 buffers' ghosts and (psi not null) psi's, in one pass over the table
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, hipStream_t s);
 // Uold: U^n for the FP32 path, whose diffusion updates U (= out) in place;
 // null for the FP64 path (U != out)
 template <typename T, typename TIN>
@@ -156,12 +166,10 @@ int march_resident_wgs(int kernel, int precision, int tile);
 // (wgs > 0).  Results do not depend on it; the dt partial minima are
 // one per tile and segment.
 int march_segments(const Dims &d, int tile, int wgs);
-// every ghost entry of g
-template <typename TS>
-void launch_exchange(const Dims &d, const DevGhosts &g, TS *state, hipStream_t s);
+// every ghost entry of the FP32 buffers
+void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s);
 // the entries that kernels reading with pull = g.pull still need
-template <typename TS>
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, TS *state, hipStream_t s);
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, hipStream_t s);
 template <typename TS>
 void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull = nullptr);
 template <typename TS>

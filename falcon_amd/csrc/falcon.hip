@@ -114,7 +114,8 @@ struct falcon_handle {
     hipStream_t stream = nullptr;
     Dims dims{};
     DevTables dt{};
-    DevGhosts gh64{}, gh32{};   // FP64 buffers (exact) and the FP32 deviation path
+    DevGhosts64 gh64{};   // FP64 buffers (exact)
+    DevGhosts gh32{};     // FP32 deviation path
     DevBoundary bnd{};
     // device memory
     DevBuf meta, radial, angular, ghost64[4], ghost32[4], ghost_copy32, ghost_lerp32[2], bnd_list;   // ghost tables
@@ -366,6 +367,71 @@ void upload_radial(falcon_handle *h) {
     h->shadow_valid = false;
 }
 
+// Table of the FP64 ghost fill: every entry, Yin-Yang ones marked, in the
+// order of their base cells' addresses (k_exchange_f64), target-list order
+// where bases coincide.
+void upload_ghosts64(falcon_handle *h) {
+    const Dims &d = h->dims;
+    const std::vector<GhostEntry> &G = h->lay.ghosts;
+    const size_t N = G.size();
+    const int nb = d.nblocks, ng = d.ng;
+    const int nt = std::max(1, std::min(host_threads(), (int)(N / 65536) + 1));
+    auto parallel = [&](auto &&f) {
+        std::vector<std::thread> th;
+        for (int t = 1; t < nt; t++) th.emplace_back([&, t] { f(t); });
+        f(0);
+        for (auto &x : th) x.join();
+    };
+    auto base = [&](const GhostEntry &g) -> int32_t {
+        return (int32_t)((long long)g.donor * 8 * d.P + cell_off(d, g.i0 + ng - 1, g.j0 + ng - 1, g.k0 + ng - 1));
+    };
+    // (base, entry) counted into donors, then sorted within each
+    std::vector<std::vector<size_t>> at(nt, std::vector<size_t>(nb, 0));
+    parallel([&](int t) {
+        for (size_t e = N * t / nt; e < N * (t + 1) / nt; e++) at[t][G[e].donor]++;
+    });
+    std::vector<size_t> first(nb + 1, 0);
+    for (int b = 0; b < nb; b++) {
+        first[b + 1] = first[b];
+        for (int t = 0; t < nt; t++) {
+            const size_t c = at[t][b];
+            at[t][b] = first[b + 1];
+            first[b + 1] += c;
+        }
+    }
+    std::vector<std::pair<int32_t, uint32_t>> key(N);
+    parallel([&](int t) {
+        for (size_t e = N * t / nt; e < N * (t + 1) / nt; e++)
+            key[at[t][G[e].donor]++] = {base(G[e]), (uint32_t)e};
+    });
+    std::vector<int32_t> dst(N), src(N);
+    std::vector<double> w(3 * N), rot(2 * N);
+    parallel([&](int t) {
+        for (int b = t; b < nb; b += nt) {
+            std::sort(key.begin() + first[b], key.begin() + first[b + 1]);
+            for (size_t q = first[b]; q < first[b + 1]; q++) {
+                const GhostEntry &g = G[key[q].second];
+                dst[q] = (int32_t)((uint32_t)((long long)g.recv_block * 8 * d.P +
+                                              cell_off(d, g.gi + ng - 1, g.gj + ng - 1, g.gk + ng - 1)) |
+                                   (g.yy ? 0x80000000u : 0u));
+                src[q] = key[q].first;
+                w[3 * q] = g.w[0]; w[3 * q + 1] = g.w[1]; w[3 * q + 2] = g.w[2];
+                rot[2 * q] = g.rot[0]; rot[2 * q + 1] = g.rot[1];
+            }
+        }
+    });
+    auto up = [&](DevBuf &buf, const void *data, size_t bytes) {
+        buf.alloc(std::max<size_t>(bytes, 16));
+        if (bytes) HIPCHECK(hipMemcpy(buf.p, data, bytes, hipMemcpyHostToDevice));
+    };
+    up(h->ghost64[0], dst.data(), sizeof(int32_t) * N);
+    up(h->ghost64[1], src.data(), sizeof(int32_t) * N);
+    up(h->ghost64[2], w.data(), sizeof(double) * 3 * N);
+    up(h->ghost64[3], rot.data(), sizeof(double) * 2 * N);
+    h->gh64 = DevGhosts64{h->ghost64[0].as<int32_t>(), h->ghost64[1].as<int32_t>(), h->ghost64[2].as<double>(),
+                          h->ghost64[3].as<double>(), (int)N};
+}
+
 void upload_tables(falcon_handle *h) {
     const Tree &t = h->lay.tree;
     const int nb = t.nleaf, NI = h->NI(), NJ = h->NJ(), NK = h->NK(), ng = t.ng;
@@ -410,10 +476,10 @@ void upload_tables(falcon_handle *h) {
     const long long P = h->dims.P;
     auto cell = [&](int i, int j, int k) -> long long { return cell_off(h->dims, i + ng - 1, j + ng - 1, k + ng - 1); };
     if ((long long)nb * 8 * P >= (1ll << 31)) throw Error("state too large for 32-bit ghost offsets");
-    // FP64 buffers: every entry weighted, same-panel entries first, then
-    // Yin-Yang, each in target-list order.  FP32 buffers of the deviation path:
-    // near copies and radial lerps (fp32_copy_lerp), the rest weighted in the
-    // same order.
+    // FP64 buffers: every entry weighted (upload_ghosts64).  FP32 buffers of
+    // the deviation path: near copies and radial lerps (fp32_copy_lerp), the
+    // rest weighted, same-panel entries first, then Yin-Yang, each in
+    // target-list order.
     std::vector<int2> copy32;
     std::vector<std::pair<int2, double>> lerp32;
     fp32_copy_lerp(h, copy32, lerp32);
@@ -449,7 +515,7 @@ void upload_tables(falcon_handle *h) {
         return DevGhosts{bufs[0].as<int32_t>(), bufs[1].as<int32_t>(), bufs[2].as<double>(), bufs[3].as<double>(),
                          0, (int)NG, yy_begin, nullptr, 0, nullptr, nullptr, 0};
     };
-    h->gh64 = weighted([](const GhostEntry &) { return true; }, h->ghost64);
+    upload_ghosts64(h);
     h->gh32 = weighted([&](const GhostEntry &g) { return !fp32_near(g) && !fp32_lerp_r(g); }, h->ghost32);
     up(h->ghost_copy32, copy32.data(), sizeof(int2) * copy32.size());
     up(h->ghost_lerp32[0], lerp_idx.data(), sizeof(int2) * lerp_idx.size());
@@ -579,16 +645,14 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
                                                              nullptr, ts, ws, G);
             });
             timed(h, k < 4 ? K_XSTAGE : K_XSTATE, [&] {
-                if (glm) launch_exchange_glm(d, h->gh64, out[k - 1], pout[k - 1], s);
-                else launch_exchange<double>(d, h->gh64, out[k - 1], s);
+                launch_exchange64(d, h->gh64, out[k - 1], pout[k - 1], s);
             });
         }
         timed(h, K_DIFF, [&] { launch_diffusion<double, double>(d, t, U, U, Un, nullptr, part, dtp, s, nullptr, td, wd); });
         if (glm) timed(h, K_OTHER, [&] { launch_glm_diffusion(d, t, U, P, Pn, dtp, s); });
         timed(h, K_OTHER, [&] { launch_copy_radial<double>(d, h->bnd, U, Un, s); });
         timed(h, K_XSTATE, [&] {
-            if (glm) launch_exchange_glm(d, h->gh64, Un, Pn, s);
-            else launch_exchange<double>(d, h->gh64, Un, s);
+            launch_exchange64(d, h->gh64, Un, Pn, s);
         });
     } else {
         float *S0 = h->S32[0].as<float>(), *S1 = h->S32[1].as<float>();
@@ -600,8 +664,8 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         // only the other ghosts
         const int32_t *pull = h->ghost_pull ? h->gh32.pull : nullptr;
         auto exchange = [&](float *st) {
-            if (pull) launch_exchange_rest<float>(d, h->gh32, st, s);
-            else launch_exchange<float>(d, h->gh32, st, s);
+            if (pull) launch_exchange_rest(d, h->gh32, st, s);
+            else launch_exchange(d, h->gh32, st, s);
         };
         for (int k = 1; k <= 4; k++) {
             timed(h, K_BC, [&] { launch_boundary<float>(d, h->bnd, const_cast<float *>(in[k - 1]), s, pull); });
@@ -630,7 +694,7 @@ void prepare_steps(falcon_handle *h) {
     const long long n = (long long)d.nblocks * 8 * d.P;
     if (h->precision == 1 && !h->shadow_valid) {
         if (!h->u_ghosts_valid) {
-            launch_exchange<double>(d, h->gh64, h->U[h->cur].as<double>(), h->stream);
+            launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, h->stream);
             h->u_ghosts_valid = true;
         }
         launch_to_f32(h->U[h->cur].as<double>(), h->F32[h->cur].as<float>(), n, h->stream);
@@ -638,11 +702,11 @@ void prepare_steps(falcon_handle *h) {
         // ghost fill from the rounded interiors, which is also what the
         // kernels' in-place reads give (rounding the FP64 ghosts instead can
         // differ in the last bit where a weight carries rounding residue)
-        launch_exchange<float>(d, h->gh32, h->F32[h->cur].as<float>(), h->stream);
+        launch_exchange(d, h->gh32, h->F32[h->cur].as<float>(), h->stream);
         h->shadow_valid = true;
     }
     if (h->precision == 0 && !h->u_ghosts_valid) {
-        launch_exchange<double>(d, h->gh64, h->U[h->cur].as<double>(), h->stream);
+        launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, h->stream);
         h->u_ghosts_valid = true;
     }
     if (!h->partials_valid) {
@@ -663,7 +727,7 @@ void after_steps(falcon_handle *h) {
 void refresh_u_ghosts(falcon_handle *h) {
     if (h->u_ghosts_valid) return;
     double *U = h->U[h->cur].as<double>();
-    launch_exchange<double>(h->dims, h->gh64, U, h->stream);
+    launch_exchange64(h->dims, h->gh64, U, nullptr, h->stream);
     launch_boundary<double>(h->dims, h->bnd, U, h->stream);
     h->u_ghosts_valid = true;
 }
@@ -1126,8 +1190,8 @@ int falcon_init_synthetic(falcon_handle_t h, uint64_t seed, double s_amp, double
         launch_synthetic(d, drng.as<double>(), dyin.as<int32_t>(), drows.as<double>(), dmodes.as<SynthMode>(), nm, seed,
                          s_amp, b_ratio, U, dmax.as<double>(), h->stream);
         // the reference driver's two initial fills (3_6/test1.f90:143-144)
-        launch_exchange<double>(d, h->gh64, U, h->stream);
-        launch_exchange<double>(d, h->gh64, U, h->stream);
+        launch_exchange64(d, h->gh64, U, nullptr, h->stream);
+        launch_exchange64(d, h->gh64, U, nullptr, h->stream);
         h->partials_valid = false;
         h->shadow_valid = false;
         h->u_ghosts_valid = true;
@@ -1322,16 +1386,15 @@ int falcon_sendrecv_gc(falcon_handle_t h, int which) {
         h->need_tables();
         ensure_device_tables(h);
         if (which == 0) {
-            if (h->divb)
-                launch_exchange_glm(h->dims, h->gh64, h->U[h->cur].as<double>(), h->psi[h->cur].as<double>(), h->stream);
-            else launch_exchange<double>(h->dims, h->gh64, h->U[h->cur].as<double>(), h->stream);
+            launch_exchange64(h->dims, h->gh64, h->U[h->cur].as<double>(),
+                              h->divb ? h->psi[h->cur].as<double>() : nullptr, h->stream);
             h->shadow_valid = false;
         } else {
             alloc_stage(h);
-            if (h->precision == 0 && h->divb)
-                launch_exchange_glm(h->dims, h->gh64, h->S64[0].as<double>(), h->psiS[0].as<double>(), h->stream);
-            else if (h->precision == 0) launch_exchange<double>(h->dims, h->gh64, h->S64[0].as<double>(), h->stream);
-            else launch_exchange<float>(h->dims, h->gh32, h->S32[0].as<float>(), h->stream);
+            if (h->precision == 0)
+                launch_exchange64(h->dims, h->gh64, h->S64[0].as<double>(),
+                                  h->divb ? h->psiS[0].as<double>() : nullptr, h->stream);
+            else launch_exchange(h->dims, h->gh32, h->S32[0].as<float>(), h->stream);
         }
         check_launch();
         HIPCHECK(hipStreamSynchronize(h->stream));

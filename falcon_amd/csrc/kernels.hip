@@ -946,6 +946,30 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
 
 // ---------------------------------------------------------------- exchange
 
+// the trilinear sum in the term order of ModMath.f90:283-291
+__device__ __forceinline__ double trilinear8(double f000, double f100, double f010, double f001, double f110,
+                                             double f011, double f101, double f111, double wi, double wj, double wk) {
+    double t = f000 * (1.0 - wi) * (1.0 - wj) * (1.0 - wk);
+    t = t + f100 * (wi) * (1.0 - wj) * (1.0 - wk);
+    t = t + f010 * (1.0 - wi) * (wj) * (1.0 - wk);
+    t = t + f001 * (1.0 - wi) * (1.0 - wj) * (wk);
+    t = t + f110 * (wi) * (wj) * (1.0 - wk);
+    t = t + f011 * (1.0 - wi) * (wj) * (wk);
+    t = t + f101 * (wi) * (1.0 - wj) * (wk);
+    t = t + f111 * (wi) * (wj) * (wk);
+    return t;
+}
+
+// ModYinYang_VecConv_1D (3_6/ModYinYang.f90:59-60) on B and v
+__device__ __forceinline__ void yy_rotate(double (&val)[8], double a, double bb) {
+    const double b2 = -(a * val[5]) - bb * val[6];
+    const double b3 = -(a * val[6]) + bb * val[5];
+    val[5] = b2; val[6] = b3;
+    const double v2 = -(a * val[2]) - bb * val[3];
+    const double v3 = -(a * val[3]) + bb * val[2];
+    val[2] = v2; val[3] = v3;
+}
+
 // ModCommunication_SendRecvGC_new (3_6/ModCommunication.f90:678-721) as one
 // table-driven gather: trilinear in the fixed term order of ModMath.f90:283-291
 // with FP64 weights and FP64 accumulation, then the Yin-Yang rotation of v and B
@@ -953,19 +977,12 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
 // donors are read only at interior cells (clamped bases touch a donor ghost only
 // with an exactly-zero weight), so entries are independent.
 //
-// SKIP: a corner whose weight factor is exactly zero contributes f*0 = +-0 to
-// the sum in the reference; its load is skipped and the term taken as +0, which
-// leaves every nonzero result bit-identical.  On the production layouts this
-// removes 60% of the FP64 corner loads and shortens the FP64 fill by 15%.  For
-// the FP32 buffers (whose near-copies go to the copy table) the unpredicated
-// gather measures twice as fast.  A zero-weight corner may then lie on a donor
-// ghost cell that the ghost pull leaves unwritten; the FP32 buffers are zeroed
-// when allocated and written with finite values only, so that term is f*0 = +-0
-// as well.
-// PSI: also psi of GLM divergence cleaning ([block][P], FP64), a scalar
-template <typename TS, bool SKIP, bool PSI = false>
-__global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, TS *__restrict__ st,
-                                                  double *__restrict__ psi = nullptr) {
+// For the FP32 buffers every corner is loaded (a gather that skips the
+// zero-weight ones measures twice the time).  A zero-weight corner may lie on
+// a donor ghost cell that the ghost pull leaves unwritten; the FP32 buffers
+// are zeroed when allocated and written with finite values only, so that term
+// is f*0 = +-0 as well.
+__global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, float *__restrict__ st) {
     const int e = g.first + (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= g.n_total) return;
     const long long P = d.P;
@@ -973,116 +990,98 @@ __global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, TS *__res
     const int SI = (int)d.SI, SJ = d.SJ;
     const int dst = g.dst[e], src = g.src[e];
     const double wi = g.w[3 * (long long)e], wj = g.w[3 * (long long)e + 1], wk = g.w[3 * (long long)e + 2];
-    const bool i0 = !SKIP || wi != 1.0, i1 = !SKIP || wi != 0.0, j0 = !SKIP || wj != 1.0, j1 = !SKIP || wj != 0.0,
-               k0 = !SKIP || wk != 1.0, k1 = !SKIP || wk != 0.0;
     double val[8];
 #pragma unroll
     for (int v = 0; v < 8; v++) {
-        const TS *F = st + src + (long long)v * P;
-        double f000, f100, f010, f001, f110, f011, f101, f111;
-        if constexpr (sizeof(TS) == 8 && SKIP) {
-            // the two phi corners of each (i, j) pair are adjacent: one 16-byte
-            // load per pair (the phi neighbour of a clamped base at the last
-            // interior cell is read in bounds and dropped with its zero weight)
-            auto ld2 = [](const TS *p) -> double2 {
-                double2 r;
-                __builtin_memcpy(&r, p, sizeof(r));
-                return r;
-            };
-            const double2 z = make_double2(0.0, 0.0);
-            const double2 a00 = (i0 && j0) ? ld2(F) : z, a10 = (i1 && j0) ? ld2(F + SI) : z;
-            const double2 a01 = (i0 && j1) ? ld2(F + SJ) : z, a11 = (i1 && j1) ? ld2(F + SI + SJ) : z;
-            f000 = k0 ? a00.x : 0.0; f001 = k1 ? a00.y : 0.0;
-            f100 = k0 ? a10.x : 0.0; f101 = k1 ? a10.y : 0.0;
-            f010 = k0 ? a01.x : 0.0; f011 = k1 ? a01.y : 0.0;
-            f110 = k0 ? a11.x : 0.0; f111 = k1 ? a11.y : 0.0;
-        } else {
-            f000 = (i0 && j0 && k0) ? (double)F[0] : 0.0;
-            f100 = (i1 && j0 && k0) ? (double)F[SI] : 0.0;
-            f010 = (i0 && j1 && k0) ? (double)F[SJ] : 0.0;
-            f001 = (i0 && j0 && k1) ? (double)F[1] : 0.0;
-            f110 = (i1 && j1 && k0) ? (double)F[SI + SJ] : 0.0;
-            f011 = (i0 && j1 && k1) ? (double)F[SJ + 1] : 0.0;
-            f101 = (i1 && j0 && k1) ? (double)F[SI + 1] : 0.0;
-            f111 = (i1 && j1 && k1) ? (double)F[SI + SJ + 1] : 0.0;
-        }
-        double t = f000 * (1.0 - wi) * (1.0 - wj) * (1.0 - wk);
-        t = t + f100 * (wi) * (1.0 - wj) * (1.0 - wk);
-        t = t + f010 * (1.0 - wi) * (wj) * (1.0 - wk);
-        t = t + f001 * (1.0 - wi) * (1.0 - wj) * (wk);
-        t = t + f110 * (wi) * (wj) * (1.0 - wk);
-        t = t + f011 * (1.0 - wi) * (wj) * (wk);
-        t = t + f101 * (wi) * (1.0 - wj) * (wk);
-        t = t + f111 * (wi) * (wj) * (wk);
-        val[v] = t;
+        const float *F = st + src + (long long)v * P;
+        const double f000 = F[0], f100 = F[SI], f010 = F[SJ], f001 = F[1], f110 = F[SI + SJ], f011 = F[SJ + 1],
+                     f101 = F[SI + 1], f111 = F[SI + SJ + 1];
+        val[v] = trilinear8(f000, f100, f010, f001, f110, f011, f101, f111, wi, wj, wk);
     }
-    if (e >= g.yy_begin) {
-        const long long q = 2 * (long long)e;
-        const double a = g.rot[q], bb = g.rot[q + 1];
-        double b2 = -(a * val[5]) - bb * val[6];
-        double b3 = -(a * val[6]) + bb * val[5];
-        val[5] = b2; val[6] = b3;
-        double v2 = -(a * val[2]) - bb * val[3];
-        double v3 = -(a * val[3]) + bb * val[2];
-        val[2] = v2; val[3] = v3;
-    }
+    if (e >= g.yy_begin) yy_rotate(val, g.rot[2 * (long long)e], g.rot[2 * (long long)e + 1]);
 #pragma unroll
-    for (int v = 0; v < 8; v++) st[dst + (long long)v * P] = (TS)val[v];
-    if constexpr (PSI) {
-        // psi has the state's cell layout: the same paired phi-corner loads
-        const double *F = psi + psi_off(d, src);
+    for (int v = 0; v < 8; v++) st[dst + (long long)v * P] = (float)val[v];
+}
+
+// The FP64 buffers' ghosts.  The entries come in the order of their base
+// cells, and runs of kXcdRun workgroups (64 to 256 measure alike, one 6% less) go to one XCD: a donor line is
+// then used by neighbouring lanes and workgroups (the two phi faces read the
+// same line of a row, the Yin-Yang entries the lines of the plain ones) while
+// the L1 or that XCD's L2 holds it.  Bound by HBM: 1536 16^3 blocks read 1731
+// and wrote 479 MB per fill in target-list order (342 us) for 403 MB of
+// donor rows, 383 MB of ghosts and 172 MB of table; sorted, with the Yin-Yang
+// entries behind the plain ones, 881 and 464 MB (277 us), in one sequence and
+// in runs of workgroups 240 to 250 us.  Not kept: staging boxes of donor cells in LDS
+// (368 us: whole boxes are read where the ghosts need their shells), one
+// contiguous range of workgroups per XCD (312 us), non-temporal table loads
+// (no change).
+//
+// SKIP of zero weights: a corner whose weight factor is exactly zero
+// contributes f*0 = +-0 to the reference's sum; it is not loaded and its term
+// is +0, which leaves every nonzero result bit-identical (60% of the corner
+// loads on the production layouts).
+// PSI: also psi of GLM divergence cleaning ([block][P]), a scalar.
+constexpr int kXcdRun = 64;
+template <bool PSI>
+__global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, double *__restrict__ st,
+                                                      double *__restrict__ psi) {
+    int wg = blockIdx.x;
+    const int grp = wg / (8 * kXcdRun), r = wg - grp * 8 * kXcdRun;
+    if ((grp + 1) * 8 * kXcdRun <= (int)gridDim.x) wg = grp * 8 * kXcdRun + (r & 7) * kXcdRun + (r >> 3);
+    const int e = wg * 256 + (int)threadIdx.x;
+    if (e >= g.n) return;
+    const long long P = d.P;
+    // the base cell is interior along phi, so its corners are in the main part
+    const int SI = (int)d.SI, SJ = d.SJ;
+    const int dst0 = g.dst[e], src = g.src[e], dst = dst0 & 0x7fffffff;
+    const double wi = g.w[3 * (long long)e], wj = g.w[3 * (long long)e + 1], wk = g.w[3 * (long long)e + 2];
+    const bool i0 = wi != 1.0, i1 = wi != 0.0, j0 = wj != 1.0, j1 = wj != 0.0, k0 = wk != 1.0, k1 = wk != 0.0;
+    // the two phi corners of each (i, j) pair are adjacent: one 16-byte load
+    // per pair (the phi neighbour of a clamped base at the last interior cell
+    // is read in bounds and dropped with its zero weight)
+    auto value = [&](const double *F) -> double {
         auto ld2 = [](const double *p) -> double2 {
-            double2 r;
-            __builtin_memcpy(&r, p, sizeof(r));
-            return r;
+            double2 v;
+            __builtin_memcpy(&v, p, sizeof(v));
+            return v;
         };
         const double2 z = make_double2(0.0, 0.0);
         const double2 a00 = (i0 && j0) ? ld2(F) : z, a10 = (i1 && j0) ? ld2(F + SI) : z;
         const double2 a01 = (i0 && j1) ? ld2(F + SJ) : z, a11 = (i1 && j1) ? ld2(F + SI + SJ) : z;
-        const double f000 = k0 ? a00.x : 0.0, f001 = k1 ? a00.y : 0.0;
-        const double f100 = k0 ? a10.x : 0.0, f101 = k1 ? a10.y : 0.0;
-        const double f010 = k0 ? a01.x : 0.0, f011 = k1 ? a01.y : 0.0;
-        const double f110 = k0 ? a11.x : 0.0, f111 = k1 ? a11.y : 0.0;
-        double t = f000 * (1.0 - wi) * (1.0 - wj) * (1.0 - wk);
-        t = t + f100 * (wi) * (1.0 - wj) * (1.0 - wk);
-        t = t + f010 * (1.0 - wi) * (wj) * (1.0 - wk);
-        t = t + f001 * (1.0 - wi) * (1.0 - wj) * (wk);
-        t = t + f110 * (wi) * (wj) * (1.0 - wk);
-        t = t + f011 * (1.0 - wi) * (wj) * (wk);
-        t = t + f101 * (wi) * (1.0 - wj) * (wk);
-        t = t + f111 * (wi) * (wj) * (wk);
-        psi[psi_off(d, dst)] = t;
-    }
+        return trilinear8(k0 ? a00.x : 0.0, k0 ? a10.x : 0.0, k0 ? a01.x : 0.0, k1 ? a00.y : 0.0, k0 ? a11.x : 0.0,
+                          k1 ? a01.y : 0.0, k1 ? a10.y : 0.0, k1 ? a11.y : 0.0, wi, wj, wk);
+    };
+    double val[8];
+#pragma unroll
+    for (int v = 0; v < 8; v++) val[v] = value(st + src + (long long)v * P);
+    if (dst0 < 0) yy_rotate(val, g.rot[2 * (long long)e], g.rot[2 * (long long)e + 1]);
+#pragma unroll
+    for (int v = 0; v < 8; v++) st[dst + (long long)v * P] = val[v];
+    // psi has the state's cell layout
+    if constexpr (PSI) psi[psi_off(d, dst)] = value(psi + psi_off(d, src));
 }
 
-// Ghost entries filled by a plain copy, sorted by destination so consecutive
-// lanes copy consecutive phi cells.  For FP64 buffers these are the same-panel
-// entries whose three weights are exactly 0: the weighted sum reduces to the
-// base cell (an interior donor cell, the base being clamped to [1, n]) plus +0
-// from the vanishing terms.  For the FP32 buffers of the deviation path they
-// also include entries whose weights lie within 1e-12 of 0 or 1 (same-level
-// neighbours whose cell centres coincide up to rounding), copied from the
-// nearest donor cell.
-template <typename TS, bool PSI = false>
+// FP32 buffers: ghost entries filled by a plain copy, sorted by destination so
+// consecutive lanes copy consecutive phi cells: the same-panel entries whose
+// weights lie within 1e-12 of 0 or 1 (same-level neighbours whose cell centres
+// coincide up to rounding), copied from the nearest donor cell.
 __global__ void __launch_bounds__(256) k_exchange_copy(Dims d, const int2 *__restrict__ copy, int n,
-                                                       TS *__restrict__ st, double *__restrict__ psi = nullptr) {
+                                                       float *__restrict__ st) {
     const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
     const int2 c = copy[e];
     const long long P = d.P;
-    TS val[8];
+    float val[8];
 #pragma unroll
     for (int v = 0; v < 8; v++) val[v] = st[c.y + (long long)v * P];
 #pragma unroll
-    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = val[v] + TS(0);
-    if constexpr (PSI) psi[psi_off(d, c.x)] = psi[psi_off(d, c.y)] + 0.0;
+    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = val[v] + 0.0f;
 }
 
 // FP32 buffers: same-panel entries whose theta/phi weights lie within 1e-12 of
 // 0 or 1 and whose r weight does not (neighbours across a radial block face,
 // whose radial spacings differ): the two r corners of the weighted sum.
-template <typename TS>
-__global__ void __launch_bounds__(256) k_exchange_lerp(Dims d, DevGhosts g, TS *__restrict__ st) {
+__global__ void __launch_bounds__(256) k_exchange_lerp(Dims d, DevGhosts g, float *__restrict__ st) {
     const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= g.n_lerp) return;
     const int2 c = g.lerp[e];
@@ -1092,11 +1091,11 @@ __global__ void __launch_bounds__(256) k_exchange_lerp(Dims d, DevGhosts g, TS *
     double val[8];
 #pragma unroll
     for (int v = 0; v < 8; v++) {
-        const TS *F = st + c.y + (long long)v * P;
+        const float *F = st + c.y + (long long)v * P;
         val[v] = (double)F[0] * (1.0 - wi) + (double)F[SI] * wi;
     }
 #pragma unroll
-    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = (TS)val[v];
+    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = (float)val[v];
 }
 
 // ---------------------------------------------------------------- boundary
@@ -1549,27 +1548,32 @@ void launch_diffusion_only(const Dims &d, const DevTables &t, const double *U, d
                         (const int32_t *)nullptr, tile, wgs, (const double *)nullptr);
 }
 
-template <typename TS>
-static void exchange_with(const Dims &d, const DevGhosts &g, const int2 *copy, int n_copy, TS *state, hipStream_t s) {
+static void exchange_with(const Dims &d, const DevGhosts &g, const int2 *copy, int n_copy, float *state,
+                          hipStream_t s) {
     if (n_copy > 0)
-        hipLaunchKernelGGL((k_exchange_copy<TS>), dim3((unsigned)((n_copy + 255) / 256)), dim3(256), 0, s, d, copy,
-                           n_copy, state);
+        hipLaunchKernelGGL(k_exchange_copy, dim3((unsigned)((n_copy + 255) / 256)), dim3(256), 0, s, d, copy, n_copy,
+                           state);
     if (g.n_lerp > 0)
-        hipLaunchKernelGGL((k_exchange_lerp<TS>), dim3((unsigned)((g.n_lerp + 255) / 256)), dim3(256), 0, s, d, g, state);
+        hipLaunchKernelGGL(k_exchange_lerp, dim3((unsigned)((g.n_lerp + 255) / 256)), dim3(256), 0, s, d, g, state);
     if (g.n_total > g.first)
-        hipLaunchKernelGGL((k_exchange<TS, sizeof(TS) == 8>), dim3((unsigned)((g.n_total - g.first + 255) / 256)),
-                           dim3(256), 0, s, d, g, state);
+        hipLaunchKernelGGL(k_exchange, dim3((unsigned)((g.n_total - g.first + 255) / 256)), dim3(256), 0, s, d, g,
+                           state);
 }
 
-template <typename TS>
-void launch_exchange(const Dims &d, const DevGhosts &g, TS *state, hipStream_t s) {
+void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s) {
     exchange_with(d, g, g.copy, g.n_copy, state, s);
 }
 
-template <typename TS>
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, TS *state, hipStream_t s) {
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, hipStream_t s) {
     if (!g.pull) throw std::runtime_error("no pull table: use the full exchange");
     exchange_with(d, g, g.copy_rest, g.n_copy_rest, state, s);
+}
+
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, hipStream_t s) {
+    if (g.n <= 0) return;
+    const dim3 grid((unsigned)((g.n + 255) / 256)), wg(256);
+    if (psi) hipLaunchKernelGGL(k_exchange_f64<true>, grid, wg, 0, s, d, g, state, psi);
+    else hipLaunchKernelGGL(k_exchange_f64<false>, grid, wg, 0, s, d, g, state, psi);
 }
 
 template <typename TS>
@@ -1993,16 +1997,6 @@ void launch_glm_diffusion(const Dims &d, const DevTables &t, const double *U, co
     hipLaunchKernelGGL(k_glm_diffusion, dim3(glm_grid(d)), dim3(256), 0, s, d, t, U, psi, psi_new, dtp);
 }
 
-void launch_exchange_glm(const Dims &d, const DevGhosts &g, double *state, double *psi, hipStream_t s) {
-    if (g.n_lerp > 0) throw std::runtime_error("GLM ghost fill: the FP64 ghost tables have no r-only entries");
-    if (g.n_copy > 0)
-        hipLaunchKernelGGL((k_exchange_copy<double, true>), dim3((unsigned)((g.n_copy + 255) / 256)), dim3(256), 0, s, d,
-                           g.copy, g.n_copy, state, psi);
-    if (g.n_total > g.first)
-        hipLaunchKernelGGL((k_exchange<double, true, true>), dim3((unsigned)((g.n_total - g.first + 255) / 256)),
-                           dim3(256), 0, s, d, g, state, psi);
-}
-
 // explicit instantiations: FP64 path, FP32-deviation path
 template void launch_stage<double, double, double, double>(const Dims &, const DevTables &, const double *, const double *, double *, float *, const double *, double, hipStream_t, const int32_t *, int, int, const double *);
 template void launch_stage<float, float, float, float>(const Dims &, const DevTables &, const float *, const float *, float *, float *, const double *, double, hipStream_t, const int32_t *, int, int, const double *);
@@ -2013,9 +2007,6 @@ template void launch_diffusion<double, double>(const Dims &, const DevTables &, 
 template void launch_diffusion<float, float>(const Dims &, const DevTables &, const float *, const double *, double *, float *, double *, const double *, hipStream_t, const int32_t *, int, int, const double *);
 template void launch_diffusion_only<double>(const Dims &, const DevTables &, const double *, double *, hipStream_t, int, int);
 template void launch_diffusion_only<float>(const Dims &, const DevTables &, const double *, double *, hipStream_t, int, int);
-template void launch_exchange<double>(const Dims &, const DevGhosts &, double *, hipStream_t);
-template void launch_exchange<float>(const Dims &, const DevGhosts &, float *, hipStream_t);
-template void launch_exchange_rest<float>(const Dims &, const DevGhosts &, float *, hipStream_t);
 template void launch_boundary<double>(const Dims &, const DevBoundary &, double *, hipStream_t, const int32_t *);
 template void launch_boundary<float>(const Dims &, const DevBoundary &, float *, hipStream_t, const int32_t *);
 template void launch_copy_radial<double>(const Dims &, const DevBoundary &, const double *, double *, hipStream_t);
