@@ -18,6 +18,7 @@
 // state, the ghost interpolation weights and the time step stay FP64.
 #include <algorithm>
 #include <stdexcept>
+#include <type_traits>
 
 #include "device.hpp"
 
@@ -91,50 +92,63 @@ __device__ __forceinline__ double div_by(double x, double b, double y) {
     return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, x), y, q), b, x);
 }
 
-// ModLinReconstruct_minmod (3_6/ModLinReconstruct.f90:37-48) for one triple
+// Smallest t with scale*t >= k in T's rounding: t >= flag_from(scale, k) is
+// that comparison without its product.
 template <typename T>
-__device__ __forceinline__ T minmod(T ul, T u, T ur) {
-    T a = (ur - ul) * T(0.5);
-    T b = T(2) * (ur - u);
-    T c = T(2) * (u - ul);
-    T ab = a * b, bc = b * c;
-    T m1 = ab > T(0) ? ab : T(0);
-    T m2 = bc > T(0) ? bc : T(0);
-    T s = (m1 * m2) * T(1.0e10) - T(1.0e-30f);
-    T half = copysign(T(0.5), s);
-    T fa = fabs(a), fb = fabs(b), fc = fabs(c);
-    T mn = fa < fb ? fa : fb;
+constexpr T flag_from(T scale, T k) {
+    using I = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned>;
+    I t = __builtin_bit_cast(I, (T)(k / scale));
+    while (scale * __builtin_bit_cast(T, t) >= k) t--;
+    while (!(scale * __builtin_bit_cast(T, t) >= k)) t++;
+    return __builtin_bit_cast(T, t);
+}
+
+// Half the slope of ModLinReconstruct_minmod (3_6/ModLinReconstruct.f90:37-48)
+// for one triple (the faces use only the half).  The reference forms a =
+// (ur-ul)/2, b = 2(ur-u), c = 2(u-ul), m1 = max(ab, 0), m2 = max(bc, 0), takes
+// the slope 0 unless m1 m2 1e10 - 1e-30 >= 0 and else the smallest of |a|, |b|,
+// |c| with a's sign.  Powers of two scale exactly, so with A = 2a, B = b/2, C =
+// c/2 the same decisions and values need 16 instead of about 27 operations:
+// ab = AB; bc = 4BC, the 4 in the threshold (FP32, whose m1 m2 may be
+// denormal there, keeps it in bc); AB > 0 wherever BC > 0.  A NaN neighbour
+// below or at the cell gives NaN, as the reference's product with 0 does.
+template <typename T>
+__device__ __forceinline__ T half_slope(T ul, T u, T ur) {
+    constexpr T from = sizeof(T) == 8 ? flag_from<T>(T(4.0e10), T(1.0e-30f)) : flag_from<T>(T(1.0e10), T(1.0e-30f));
+    const T A = ur - ul, B = ur - u, C = u - ul;
+    T m2 = sizeof(T) == 8 ? B * C : (T(4) * B) * C;
+    m2 = sizeof(T) == 8 ? (T)__builtin_fmax((double)m2, 0.0) : (T)__builtin_fmaxf((float)m2, 0.0f);
+    const T f = (A * B) * m2 >= from ? T(1) : T(0);
+    const T fa = fabs(A) * T(0.25), fb = fabs(B), fc = fabs(C);
+    T mn = sizeof(T) == 8 ? (T)__builtin_fmin((double)fa, (double)fb) : (T)__builtin_fminf((float)fa, (float)fb);
     mn = mn < fc ? mn : fc;
-    return (half + T(0.5)) * copysign(mn, a);
+    return f * copysign(mn, A);
 }
 
 // One face of ModDiffusion_Aritificial_1 (3_6/ModDiffusion.f90:50-59) between
-// cell y (value b) and cell x = y+1 (value c); a = y-1, d = x+1.
-// MAX(0.0, NaN) is taken as 0.0 (the comparison below is false for NaN).
-template <typename T>
-__device__ __forceinline__ T face_flux(T a, T b, T c, T d) {
-    T dX = minmod(b, c, d);
-    T dY = minmod(a, b, c);
-    T num = ((c - dX * T(0.5)) - b) - dY * T(0.5);
-    T ph = T(1) + T(2) * (num / (c - b) - T(1));
-    ph = ph > T(0) ? ph : T(0);
-    return ((-T(0.5)) * ph) * num;
-}
-
-// The same face from the two cells' minmod slopes: sY at y (value b), sX at
-// x (value c).  The reference forms every cell's slope once per direction
-// (ModLinReconstruct_minmod over the whole array) and both faces of a cell use
-// it; face_flux recomputes it per face.  RCP (FP32 path): the limiter ratio as
-// a product with the hardware reciprocal of (c - b), whose 1 ulp error is far
-// below the FP32 storage rounding; 0 and +-0 denominators give the same
-// infinities and NaN as the quotient, so the NaN -> 0 rule still applies.
+// cell y (value b, half slope hY) and cell x = y+1 (value c, half slope hX):
+// phi * num, with num = c - sX/2 - b - sY/2 and phi = max(0, 1 + 2 (num/(c-b)
+// - 1)), a NaN taken as 0; the reference's flux is this times -1/2, times the
+// sum of the two speeds, times 1/2.  The factor -1/4 is a power of two: it is
+// applied once to the sum over the faces (kFluxScale) with the same rounding.
+// RCP (FP32 path): the limiter ratio as a product with the hardware reciprocal
+// of (c - b), whose 1 ulp error is far below the FP32 storage rounding; 0 and
+// +-0 denominators give the same infinities and NaN as the quotient, so the
+// NaN -> 0 rule still applies.
+constexpr double kFluxScale = 0.25;
 template <typename T, bool RCP>
-__device__ __forceinline__ T face_flux_s(T b, T c, T sY, T sX) {
-    T num = ((c - sX * T(0.5)) - b) - sY * T(0.5);
-    T q = RCP ? num * (T)__builtin_amdgcn_rcpf((float)(c - b)) : num / (c - b);
-    T ph = T(1) + T(2) * (q - T(1));
-    ph = ph > T(0) ? ph : T(0);
-    return ((-T(0.5)) * ph) * num;
+__device__ __forceinline__ T face_flux(T b, T c, T hY, T hX) {
+    const T num = ((c - hX) - b) - hY;
+    const T q = RCP ? num * (T)__builtin_amdgcn_rcpf((float)(c - b)) : num / (c - b);
+    const T x = q - T(1);
+    const T ph = sizeof(T) == 8 ? (T)__builtin_fmax(__builtin_fma(2.0, (double)x, 1.0), 0.0)
+                                : (T)__builtin_fmaxf(__builtin_fmaf(2.0f, (float)x, 1.0f), 0.0f);
+    return ph * num;
+}
+// the face between b and c of the four cells a, b, c, d
+template <typename T, bool RCP = false>
+__device__ __forceinline__ T face_flux4(T a, T b, T c, T d) {
+    return face_flux<T, RCP>(b, c, half_slope(a, b, c), half_slope(b, c, d));
 }
 
 // Shared r-marching skeleton: loads the column window and the halo'd plane.
@@ -550,8 +564,9 @@ __global__ void __launch_bounds__(TL * TL) k_stage(Dims d, DevTables t, const TI
 
 // The FP64 step's stage (16-edge tiles, one workgroup per tile) held to two
 // wavefronts per SIMD: left to itself the compiler gives it 256 VGPRs plus 2
-// AGPRs, one wavefront per SIMD; held to two it spills two values (12 bytes
-// per lane) and runs in 3.06 instead of 3.94 ms on the 50 M-cell shell.  The
+// AGPRs, one wavefront per SIMD; held to two it spills a few values (36 bytes
+// per lane) and runs in 2.9 instead of 3.9 ms on 12288 16^3 blocks (386 us on
+// 1536, 1.58 GB at 4.1 TB/s: near the memory rate of a copy, 4.7 TB/s).  The
 // other builds either fit two wavefronts already (the FP32 stages) or would
 // spill tens of registers.
 template <typename T, typename TIN, typename TOUT, typename TB, int MODE, bool SHADOW, int TL, bool PERSIST,
@@ -592,38 +607,55 @@ __constant__ double kParTop[8] = {1.0, -1.0, 1.0, 1.0, 1.0, -1.0, -1.0, 1.0};
 // changed the 100-step FP32-vs-FP64 difference only from 5.2e-7 to 5.5e-7
 // (largest variable) and cost 0.8 ms per step.
 
+// A plane takes three phases: half slopes of every cell along theta and phi
+// (each formed once, where the reference's whole-array reconstruction is read
+// by both faces of a cell), then the upper theta and phi face of every cell
+// from its own and its neighbour's half slope, then the cell's update with the
+// lower faces of its neighbours; the radial face and slope are carried from
+// plane to plane.  The halo cells' half slopes (4 tile edges) and the faces on
+// the tile's lower edges are spread one variable a lane over the whole
+// workgroup: done by the first wavefront for all variables, as before, the
+// others waited about a fifth of the plane for it.  FP64 takes the phases in
+// two passes of four variables, so that two workgroups fit a CU's LDS.
+// Bound by vector instructions in FP64 (two thirds busy at two wavefronts per
+// SIMD) and near the memory rate in FP32 (1.5 GB at 4.2 TB/s).  Against one
+// pass that recomputed the slopes per face and kept a five-plane window, with
+// the general divisions and the edges on the first wavefront: FP64 706 -> 476
+// us, FP32 490 -> 360 us on 1536 16^3 blocks; 192 blocks 105 -> 83 and 91 -> 72
+// us.  FP64 held to two wavefronts per SIMD spills 28 bytes per lane; with the
+// eight variables in one pass 124 bytes (607 us).
 template <typename T, typename TIN, int MODE, int TL, bool PERSIST>
-__global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, const TIN *__restrict__ in,
+__global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2))) k_diffusion(Dims d, DevTables t, const TIN *__restrict__ in,
                                                    const double *U, double *out, float *__restrict__ shadow,
                                                    double *__restrict__ partial, const double *__restrict__ dtp,
                                                    const int32_t *__restrict__ pull, const double *__restrict__ Uold,
                                                    int nseg) {
-    // one r-plane with its theta/phi halo; the second barrier of each plane
-    // orders its reuse, so it is not double-buffered
-    constexpr int PL = tile_pl<TL>();
+    constexpr int PL = tile_pl<TL>(), NL = TL * TL;
+    constexpr bool F32 = sizeof(T) == 4;
+    // FP32 path in a step: pulled ghosts, boundary faces from U^n, reciprocals
+    constexpr bool LEAN = F32 && MODE == 0, PULL = LEAN, BFACE = LEAN;
+    // one r-plane with its theta/phi halo; the barriers of a plane order its
+    // reuse, so it is not double-buffered
     __shared__ T lds[8][PL][PL];
-    // theta and phi face fluxes of the plane, each computed once: fj[v][y][x]
-    // is the flux through the lower theta face of tile cell (y, x) (row TJa:
-    // the upper face of the last row), fk[v][y][x] through its lower phi face
-    __shared__ T fj[8][TL + 1][TL];
-    __shared__ T fk[8][TL][TL + 1];
+    // of the pass's variables: half slopes along theta, sj(v, y+1, x) for tile
+    // rows y = -1 .. TJa, and phi, sk(v, y, x+1) for tile columns x = -1 .. TKa;
+    // face fluxes fj(v, y, x) through the lower theta face of tile cell (y, x)
+    // (row TJa: the upper face of the last row), fk(v, y, x) through its lower
+    // phi face
+    constexpr int NV = F32 ? 8 : 4, NSJ = (TL + 2) * TL, NFJ = (TL + 1) * TL;
+    __shared__ T sbuf[2][NV][NSJ];
+    __shared__ T fbuf[2][NV][NFJ];
+    auto sj = [&](int v, int y, int x) -> T & { return sbuf[0][v % NV][y * TL + x]; };
+    auto sk = [&](int v, int y, int x) -> T & { return sbuf[1][v % NV][y * (TL + 2) + x]; };
+    auto fj = [&](int v, int y, int x) -> T & { return fbuf[0][v % NV][y * TL + x]; };
+    auto fk = [&](int v, int y, int x) -> T & { return fbuf[1][v % NV][y * (TL + 1) + x]; };
     __shared__ double red[4];
     // block read in place of this block's ghosts in direction code c (the
-    // pull table's row, -1 where the ghost itself is read); set before the
-    // first barrier of the march
+    // pull table's row, -1 where the ghost itself is read)
     __shared__ int pdir[27];
-    // LEAN (FP32 path, MODE 0): the block's radial rows c_s, xi, sqrt(rho0) are
-    // staged in LDS once per tile, and every global load a plane needs besides
-    // the next plane's window and halo (U^n of the plane, the shifted speed
-    // cells) is issued at the top of the plane, before that prefetch, so no
-    // wait in the plane's arithmetic includes the prefetch
-    constexpr bool LEAN = sizeof(T) == 4 && MODE == 0;
-    __shared__ double drow[3][kMaxNI];
-    // LEAN: the theta and phi minmod slopes of the plane's cells, each formed
-    // once and read by both faces of the cell: sj[v][y+1][x] for tile rows
-    // y = -1 .. TJa, sk[v][y][x+1] for tile columns x = -1 .. TKa
-    __shared__ T sj[LEAN ? 8 : 1][TL + 2][TL];
-    __shared__ T sk[LEAN ? 8 : 1][TL][TL + 2];
+    // the block's radial rows c_s, xi, sqrt(rho0): staged in a step so that no
+    // plane waits on a load issued after its prefetch
+    __shared__ double drow[3][MODE == 0 ? kMaxNI : 1];
     const int ntk = (d.nk + TL - 1) / TL, tpb = ((d.nj + TL - 1) / TL) * ntk;
     const int ntot = d.nblocks * tpb * nseg;
     // PERSIST: a grid smaller than the tile count (a persistent launch) takes
@@ -635,279 +667,266 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
         const int tcol = tile / nseg, seg = tile - tcol * nseg;
         const int iA = seg * d.ni / nseg, iB = (seg + 1) * d.ni / nseg;
         const int b = tcol / tpb;
-        if (sizeof(T) == 4 && MODE == 0 && threadIdx.x < 27) pdir[threadIdx.x] = pull ? pull[b * 27 + threadIdx.x] : -1;
+        if (PULL && threadIdx.x < 27) pdir[threadIdx.x] = pull ? pull[b * 27 + threadIdx.x] : -1;
         const int trem = tcol - b * tpb;
         const int tj = trem / ntk, tk = trem - tj * ntk;
         const int j0 = tj * TL, k0 = tk * TL;
         const int TJa = min(TL, d.nj - j0), TKa = min(TL, d.nk - k0);
-        const int tx = threadIdx.x & (TL - 1), ty = threadIdx.x / TL;
+        const int lane = threadIdx.x, tx = lane & (TL - 1), ty = lane / TL;
 
-        constexpr bool PULL = sizeof(T) == 4 && MODE == 0;
         Marcher<T, TIN, PULL, TL> m;
         m.init(d, in, b, j0, k0, TJa, TKa, pull);
         const long long rb = (long long)b * d.NI, tb = (long long)b * d.NJ;
-        if (LEAN) {
-            for (int I = threadIdx.x; I < d.NI; I += TL * TL) {
+        if constexpr (MODE == 0) {
+            for (int I = lane; I < d.NI; I += NL) {
                 drow[0][I] = t.cs[rb + I];
                 drow[1][I] = t.xi[rb + I];
                 drow[2][I] = t.sqrt_rho0[rb + I];
             }
         }
-        // radial rows at plane I: LDS (LEAN) or the tables
-        auto cs_at = [&](int I) -> double { return LEAN ? drow[0][I] : t.cs[rb + I]; };
-        auto xi_at = [&](int I) -> double { return LEAN ? drow[1][I] : t.xi[rb + I]; };
-        auto sr_at = [&](int I) -> double { return LEAN ? drow[2][I] : t.sqrt_rho0[rb + I]; };
+        auto cs_at = [&](int I) -> double { return MODE == 0 ? drow[0][MODE == 0 ? I : 0] : t.cs[rb + I]; };
+        auto xi_at = [&](int I) -> double { return MODE == 0 ? drow[1][MODE == 0 ? I : 0] : t.xi[rb + I]; };
         const BlockMeta mt = t.meta[b];
         const T dxi = (T)mt.dxi, dxj = (T)mt.dxj, dxk = (T)mt.dxk;
-        const T rdxi = LEAN ? (T)__builtin_amdgcn_rcpf((float)dxi) : T(0);
+        // the face sums are divided by the cell lengths: products with hardware
+        // reciprocals (LEAN), div_by (FP64, the correctly rounded quotient) or
+        // plain divisions
+        auto recip = [](T x) -> T {
+            if constexpr (!F32) return div_rcp(x);
+            else return (T)__builtin_amdgcn_rcpf((float)x);
+        };
+        auto over = [](T f, T x, T y) -> T {
+            if constexpr (!F32) return div_by(f, x, y);
+            else return LEAN ? f * y : f / x;
+        };
+        const T ydxi = recip(dxi);
         double hmin = INFINITY;
         const double sint64 = m.act ? t.sint[tb + m.J] : 1.0;
         const T sintc = m.act ? (T)t.sint[tb + m.J] : T(1);
         const double dt = MODE == 0 ? *dtp : 0.0;
+        const double dts = (0.5 * kFluxScale) * dt;
+        __syncthreads();   // pdir, drow
 
-        T win[8][5];
-        T nxt[8], hn[8];
-        // the upper r-face flux of plane i is the lower r-face flux of plane i+1:
-        // same four values, same speed sum (speed at the upper cell first), so it
-        // is carried instead of recomputed.  The same holds for the theta and phi
-        // faces between neighbouring lanes, which go through fj / fk.
-        T fr[8];
-        T sr[8];   // LEAN: radial slope of the cell above this plane's (carried)
-        bool have_fr = false;
-        // FP32 path: U before the diffusion on the previous plane (the top
-        // boundary face reads it after that plane has been updated in place)
-        constexpr bool BFACE = MODE == 0 && sizeof(T) == 4;
-        double uprev[8];
-        const bool bot = BFACE && (mt.flags & 1), topb = BFACE && (mt.flags & 2);
-    #pragma unroll
-        for (int v = 0; v < 8; v++) {
-    #pragma unroll
-            for (int q = 0; q < 5; q++) win[v][q] = (LEAN || m.act) ? m.col(v, iA + q) : T(0);
-            hn[v] = (LEAN || m.hv) ? m.halo(v, iA + d.ng) : T(0);
-            fr[v] = T(0);
-        }
-        // a ghost in a direction listed in the pull table is the same-level
-        // neighbour's interior cell, translated by n
-        auto at = [&](int v, int II, int JJ, int KK) -> T {
-            int B = b;
+        // Column (JJ, KK) of variable v from padded plane II, which lies in radial
+        // direction di of the block (-1, 0, 1: below, inside, above its interior):
+        // address of that plane, and the plane pitch.  A ghost in a direction listed
+        // in the pull table is the same-level neighbour's interior cell, translated
+        // by n.
+        struct Col {
+            const TIN *p;
+            int pitch;
+        };
+        auto column = [&](int v, int II, int JJ, int KK, int di) -> Col {
+            int B = b, sh = 0;
             if (PULL) {
-                const int di = II < d.ng ? -1 : (II >= d.ng + d.ni ? 1 : 0);
                 const int dj = JJ < d.ng ? -1 : (JJ >= d.ng + d.nj ? 1 : 0);
                 const int dk = KK < d.ng ? -1 : (KK >= d.ng + d.nk ? 1 : 0);
                 const int D = pdir[(di + 1) * 9 + (dj + 1) * 3 + (dk + 1)];
                 if ((di | dj | dk) && D >= 0) {
                     B = D;
-                    II -= di * d.ni; JJ -= dj * d.nj; KK -= dk * d.nk;
+                    sh = di * d.ni; JJ -= dj * d.nj; KK -= dk * d.nk;
                 }
             }
-            return (T)in[((long long)B * 8 + v) * d.P + cell_off(d, II, JJ, KK)];
+            Col c;
+            c.pitch = (KK >= d.ng && KK < d.ng + d.nk) ? (int)d.SI : d.NJ * 2 * d.ng;
+            c.p = in + ((long long)B * 8 + v) * d.P + cell_off(d, 0, JJ, KK) + (long long)(II - sh) * c.pitch;
+            return c;
         };
-        // faces on the tile's lower edges: lanes 0 .. TL-1 take the theta face
-        // below row 0 in column x = lane, lanes TL .. 2TL-1 the phi face left of
-        // column 0 in row y = lane - TL.  Such a face's four-cell stencil lies in
-        // the LDS plane at (bstart, step bstep); its speed cells are (bJ0, bK0) on
-        // the upper side and (bJ1, bK1) on the lower side.
-        const int lane = threadIdx.x;
-        const bool bact = lane < TL ? lane < TKa : (lane < 2 * TL && lane - TL < TJa);
-        const bool bj = lane < TL;
-        const int bx = bj ? lane : 0, by = bj ? 0 : lane - TL;
-        const int bstart = bj ? bx + 2 : (by + 2) * PL, bstep = bj ? PL : 1;
+        // |value| of the column's plane; the column steps to the next plane
+        auto step = [](Col &c) -> T {
+            const T x = fabs((T)*c.p);
+            c.p += c.pitch;
+            return x;
+        };
+        // Speeds |v_d| + c_s are read where the reference reads them (transverse
+        // index - ng): (I-2, J, K-2) and (I-2, J+1, K-2) for theta, (I-2, J-2, K)
+        // and (I-2, J-2, K+1) for phi, (., J-2, K-2) for r.  Inactive lanes read at
+        // the tile's first column.
+        const int J = m.act ? m.J : j0 + d.ng, K = m.act ? m.K : k0 + d.ng;
+        // faces on the tile's lower edges, one (position, variables) a lane:
+        // positions 0 .. TL-1 are the theta faces below row 0, TL .. 2TL-1 the phi
+        // faces left of column 0; the lane's variables are ev, ev + EV, ...
+        constexpr int EV = NL / (2 * TL);
+        const int ep = lane & (2 * TL - 1), ev = lane / (2 * TL);
+        const bool bj = ep < TL;
+        const int bx = bj ? ep : 0, by = bj ? 0 : ep - TL;
+        const bool bact = bj ? bx < TKa : by < TJa;
         const int bvar = bj ? 2 : 3;
-        const int bJ0 = bj ? j0 + d.ng : j0 + by + d.ng - 2, bK0 = bj ? k0 + bx + d.ng - 2 : k0 + d.ng;
+        const int bJ0 = !bact ? j0 + d.ng : bj ? j0 + d.ng : j0 + by + d.ng - 2,
+                  bK0 = !bact ? k0 + d.ng : bj ? k0 + bx + d.ng - 2 : k0 + d.ng;
         const int bJ1 = bj ? bJ0 - 1 : bJ0, bK1 = bj ? bK0 : bK0 - 1;
+        Col q20, q2p, q30, q3p, q1, qe0, qe1;
+        auto theta_phi_columns = [&](int II, int di) {
+            q20 = column(2, II, J, K - 2, di);
+            q2p = column(2, II, J + 1, K - 2, di);
+            q30 = column(3, II, J - 2, K, di);
+            q3p = column(3, II, J - 2, K + 1, di);
+            qe0 = column(bvar, II, bJ0, bK0, di);
+            qe1 = column(bvar, II, bJ1, bK1, di);
+        };
+        // planes I - 2 = i of the theta and phi speeds leave the ghost range at i = ng
+        theta_phi_columns(iA, iA < d.ng ? -1 : 0);
+        // |v_r| of the radial faces' cells at planes I - 1 (first plane), I and I + 1
+        q1 = column(1, iA + d.ng - 1, J - 2, K - 2, iA == 0 ? -1 : 0);
+        const T v1m = step(q1);
+        if (iA == 0) q1 = column(1, d.ng, J - 2, K - 2, 0);
+        T v1c = step(q1), v1n;
+
+        // window: this plane and the two above it
+        T w0[8], w1[8], w2[8];
+        T nxt[8], hn[8];
+        // the upper r-face of plane i is the lower r-face of plane i+1: same four
+        // values, same speed sum (speed at the upper cell first); carried with the
+        // half slope of the cell above
+        T fr[8], sr[8];
+        // FP32 path: U before the diffusion on the previous plane (the top
+        // boundary face reads it after that plane has been updated in place)
+        double uprev[8];
+        const bool bot = BFACE && (mt.flags & 1), topb = BFACE && (mt.flags & 2);
+        const long long bbase = (long long)b * 8 * d.P;
+        {
+            const T cm = v1m + (T)cs_at(iA + d.ng - 1);
+            const T cc = v1c + (T)cs_at(iA + d.ng);
+    #pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const T a = m.col(v, iA), c = m.col(v, iA + 1);
+                w0[v] = m.col(v, iA + 2);
+                w1[v] = m.col(v, iA + 3);
+                w2[v] = m.col(v, iA + 4);
+                hn[v] = m.halo(v, iA + d.ng);
+                sr[v] = half_slope(c, w0[v], w1[v]);
+                fr[v] = face_flux<T, LEAN>(c, w0[v], half_slope(a, c, w0[v]), sr[v]) * (cc + cm);
+                if (BFACE && bot && iA == 0) {
+                    // lower face of the first cell: ghosts 0 and -1 mirror cells 1 and 2 of U^n
+                    const long long q = bbase + (long long)d.ng * m.SI + (long long)v * d.P + m.coff;
+                    const double p = kParBottom[v];
+                    const double g0 = p * Uold[q], gm1 = p * Uold[q + m.SI];
+                    fr[v] = (T)(face_flux4<double>(gm1, g0, U[q], U[q + m.SI]) * (double)(cc + cm));
+                }
+            }
+        }
 
         for (int i = iA; i < iB; i++) {
             const int I = i + d.ng;
-            // LEAN: U^n of the plane and |v_d| at the shifted speed cells, issued
-            // before the prefetch (inactive lanes read at the tile's first column)
+            // U^n of the plane (LEAN; FP64's is the input itself) and |v_d| at the
+            // shifted speed cells, issued before the prefetch
             double ucur[8];
-            T a20 = T(0), a2p = T(0), a30 = T(0), a3p = T(0), a1m = T(0), a10 = T(0), a1p = T(0), as0 = T(0),
-              as1 = T(0);
             if (LEAN) {
-                const int J = m.act ? m.J : j0 + d.ng, K = m.act ? m.K : k0 + d.ng;
-                const long long base = (long long)b * 8 * d.P + (long long)I * m.SI + m.coff;
     #pragma unroll
-                for (int v = 0; v < 8; v++) ucur[v] = U[base + (long long)v * d.P];
-                a20 = fabs(at(2, I - 2, J, K - 2));
-                a2p = fabs(at(2, I - 2, J + 1, K - 2));
-                a30 = fabs(at(3, I - 2, J - 2, K));
-                a3p = fabs(at(3, I - 2, J - 2, K + 1));
-                a1m = fabs(at(1, I - 1, J - 2, K - 2));
-                a10 = fabs(at(1, I, J - 2, K - 2));
-                a1p = fabs(at(1, I + 1, J - 2, K - 2));
-                if (bact) {
-                    as0 = fabs(at(bvar, I - 2, bJ0, bK0));
-                    as1 = fabs(at(bvar, I - 2, bJ1, bK1));
-                }
+                for (int v = 0; v < 8; v++) ucur[v] = (U + (bbase + (long long)v * d.P + (long long)I * m.SI))[m.coff];
             }
+            if (i == d.ng) theta_phi_columns(i, 0);
+            if (i == d.ni - 1) q1 = column(1, I + 1, J - 2, K - 2, 1);
+            const T a20 = step(q20), a2p = step(q2p), a30 = step(q30), a3p = step(q3p);
+            const T ae0 = step(qe0), ae1 = step(qe1);
+            v1n = step(q1);
     #pragma unroll
             for (int v = 0; v < 8; v++) {
-                if (m.act) lds[v][ty + 2][tx + 2] = win[v][2];
+                if (m.act) lds[v][ty + 2][tx + 2] = w0[v];
                 if (m.hv) lds[v][m.hly][m.hlx] = hn[v];
             }
-            const bool more = i + 1 < iB;
             const int In = min(I + 3, d.NI - 1), Ih = min(I + 1, d.NI - 1);
     #pragma unroll
             for (int v = 0; v < 8; v++) {
-                nxt[v] = (LEAN || (m.act && more)) ? m.col(v, In) : T(0);
-                hn[v] = (LEAN || (m.hv && more)) ? m.halo(v, Ih) : T(0);
+                nxt[v] = m.col(v, In);
+                hn[v] = m.halo(v, Ih);
             }
             __syncthreads();
-            const T csI2 = (T)cs_at(I - 2);
             auto Lv = [&](int v, int dj, int dk) -> T { return lds[v][ty + 2 + dj][tx + 2 + dk]; };
-            if (m.act) {
-                const int J = m.J, K = m.K;
-                // speeds |v_d| + c_s at the cells the reference reads (see above)
-                const T c20 = (LEAN ? a20 : fabs(at(2, I - 2, J, K - 2))) + csI2;
-                const T c2p = (LEAN ? a2p : fabs(at(2, I - 2, J + 1, K - 2))) + csI2;
-                const T c30 = (LEAN ? a30 : fabs(at(3, I - 2, J - 2, K))) + csI2;
-                const T c3p = (LEAN ? a3p : fabs(at(3, I - 2, J - 2, K + 1))) + csI2;
-                if (LEAN) {
-                    // this cell's slopes; its faces are formed after the barrier
+            const T csI2 = (T)cs_at(i), csI = (T)cs_at(I), csIp = (T)cs_at(I + 1);
+            const T S2 = (a2p + csI2) + (a20 + csI2), S3 = (a3p + csI2) + (a30 + csI2);
+            const T Se = (ae0 + csI2) + (ae1 + csI2);
+            const T S1 = (v1n + csIp) + (v1c + csI);
+            const T xic = (T)xi_at(I);
+            const T L2 = dxj * xic;
+            const T L3 = (dxk * xic) * sintc;
+            const T y2 = recip(L2), y3 = recip(L3);
+            const long long base = bbase + (long long)I * m.SI;
+            const long long nn = (long long)d.ni * d.nj * d.nk;
+            const long long rbase = (long long)b * 8 * nn + ((long long)i * d.nj + (j0 + ty)) * d.nk + (k0 + tx);
+            double vv = 0.0, bb2 = 0.0;   // |v|^2 and |B|^2 of the new state, summed in component order
     #pragma unroll
-                    for (int v = 0; v < 8; v++) {
-                        sj[v][ty + 1][tx] = minmod(Lv(v, -1, 0), Lv(v, 0, 0), Lv(v, 1, 0));
-                        sk[v][ty][tx + 1] = minmod(Lv(v, 0, -1), Lv(v, 0, 0), Lv(v, 0, 1));
-                    }
-                } else {
+            for (int p0 = 0; p0 < 8; p0 += NV) {
+                if (m.act) {
     #pragma unroll
-                    for (int v = 0; v < 8; v++) {
-                        // upper theta face (the lower one of the cell at row + 1)
-                        fj[v][ty + 1][tx] =
-                            (face_flux(Lv(v, -1, 0), Lv(v, 0, 0), Lv(v, 1, 0), Lv(v, 2, 0)) * (c2p + c20)) * T(0.5);
-                        // upper phi face
-                        fk[v][ty][tx + 1] =
-                            (face_flux(Lv(v, 0, -1), Lv(v, 0, 0), Lv(v, 0, 1), Lv(v, 0, 2)) * (c3p + c30)) * T(0.5);
+                    for (int v = p0; v < p0 + NV; v++) {
+                        sj(v, ty + 1, tx) = half_slope(Lv(v, -1, 0), w0[v], Lv(v, 1, 0));
+                        sk(v, ty, tx + 1) = half_slope(Lv(v, 0, -1), w0[v], Lv(v, 0, 1));
                     }
                 }
-            }
-            if (LEAN) {
-                // slopes of the halo cells next to the tile: rows -1 and TJa (theta),
-                // columns -1 and TKa (phi), lanes 0 .. 4*TL-1
-                const int q = lane / TL, x = lane - q * TL;
-                if (q < 4 && x < (q < 2 ? TKa : TJa)) {
-                    // LDS plane index of the slope cell and the step to its neighbours
-                    const int y = q == 0 ? -1 : (q == 1 ? TJa : x), xx = q < 2 ? x : (q == 2 ? -1 : TKa);
-                    const int st = q < 2 ? PL : 1;
+                // halo cells next to the tile: rows -1 and TJa (theta), columns -1 and TKa (phi)
     #pragma unroll
-                    for (int v = 0; v < 8; v++) {
+                for (int h = lane; h < 4 * TL * NV; h += NL) {
+                    const int v = p0 + h / (4 * TL), q = (h / TL) & 3, x = h & (TL - 1);
+                    if (x < (q < 2 ? TKa : TJa)) {
+                        const int y = q == 0 ? -1 : (q == 1 ? TJa : x), xx = q < 2 ? x : (q == 2 ? -1 : TKa);
+                        const int st = q < 2 ? PL : 1;
                         const T *pc = &lds[v][y + 2][xx + 2];
-                        const T sl = minmod(pc[-st], pc[0], pc[st]);
-                        if (q < 2) sj[v][y + 1][x] = sl;
-                        else sk[v][x][xx + 1] = sl;
+                        const T sl = half_slope(pc[-st], pc[0], pc[st]);
+                        if (q < 2) sj(v, y + 1, x) = sl;
+                        else sk(v, x, xx + 1) = sl;
                     }
                 }
                 __syncthreads();
                 if (m.act) {
-                    const T c20 = a20 + csI2, c2p = a2p + csI2, c30 = a30 + csI2, c3p = a3p + csI2;
     #pragma unroll
-                    for (int v = 0; v < 8; v++) {
-                        fj[v][ty + 1][tx] =
-                            (face_flux_s<T, true>(Lv(v, 0, 0), Lv(v, 1, 0), sj[v][ty + 1][tx], sj[v][ty + 2][tx]) *
-                             (c2p + c20)) * T(0.5);
-                        fk[v][ty][tx + 1] =
-                            (face_flux_s<T, true>(Lv(v, 0, 0), Lv(v, 0, 1), sk[v][ty][tx + 1], sk[v][ty][tx + 2]) *
-                             (c3p + c30)) * T(0.5);
+                    for (int v = p0; v < p0 + NV; v++) {
+                        fj(v, ty + 1, tx) = face_flux<T, LEAN>(w0[v], Lv(v, 1, 0), sj(v, ty + 1, tx), sj(v, ty + 2, tx)) * S2;
+                        fk(v, ty, tx + 1) = face_flux<T, LEAN>(w0[v], Lv(v, 0, 1), sk(v, ty, tx + 1), sk(v, ty, tx + 2)) * S3;
                     }
                 }
-            }
-            if (bact) {
-                // the lower face of the edge cell
-                const T s0 = (LEAN ? as0 : fabs(at(bvar, I - 2, bJ0, bK0))) + csI2;
-                const T s1 = (LEAN ? as1 : fabs(at(bvar, I - 2, bJ1, bK1))) + csI2;
+                if (bact) {
     #pragma unroll
-                for (int v = 0; v < 8; v++) {
-                    const T *pv = &lds[v][0][0] + bstart;
-                    T f;
-                    if (LEAN)
-                        f = face_flux_s<T, true>(pv[bstep], pv[2 * bstep], bj ? sj[v][0][bx] : sk[v][by][0],
-                                                 bj ? sj[v][1][bx] : sk[v][by][1]);
-                    else
-                        f = face_flux(pv[0], pv[bstep], pv[2 * bstep], pv[3 * bstep]);
-                    f = (f * (s0 + s1)) * T(0.5);
-                    if (bj) fj[v][0][bx] = f;
-                    else fk[v][by][0] = f;
+                    for (int v = p0 + ev; v < p0 + NV; v += EV) {
+                        const T *pv = &lds[v][by + 2][bx + 2];
+                        const T lo = bj ? pv[-PL] : pv[-1];
+                        const T f = face_flux<T, LEAN>(lo, pv[0], bj ? sj(v, 0, bx) : sk(v, by, 0),
+                                                       bj ? sj(v, 1, bx) : sk(v, by, 1)) * Se;
+                        if (bj) fj(v, 0, bx) = f;
+                        else fk(v, by, 0) = f;
+                    }
                 }
-            }
-            __syncthreads();
-            if (m.act) {
-                const int J = m.J, K = m.K;
-                const T csI = (T)cs_at(I), csIm = (T)cs_at(I - 1), csIp = (T)cs_at(I + 1);
-                const T c1m = (LEAN ? a1m : fabs(at(1, I - 1, J - 2, K - 2))) + csIm;
-                const T c10 = (LEAN ? a10 : fabs(at(1, I, J - 2, K - 2))) + csI;
-                const T c1p = (LEAN ? a1p : fabs(at(1, I + 1, J - 2, K - 2))) + csIp;
-                const T xic = (T)xi_at(I);
-                const T L2 = dxj * xic;
-                const T L3 = (dxk * xic) * sintc;
-                // LEAN: the face sums scaled by hardware reciprocals of the lengths
-                const T rL2 = LEAN ? (T)__builtin_amdgcn_rcpf((float)L2) : T(0);
-                const T rL3 = LEAN ? (T)__builtin_amdgcn_rcpf((float)L3) : T(0);
-                const long long base = (long long)b * 8 * d.P + (long long)I * m.SI + m.coff;
-                const long long nn = (long long)d.ni * d.nj * d.nk;
-                const long long rbase = (long long)b * 8 * nn + ((long long)i * d.nj + (j0 + ty)) * d.nk + (k0 + tx);
-                double vv = 0.0, bb2 = 0.0;   // |v|^2 and |B|^2 of the new state, summed in component order
+                __syncthreads();
+                if (m.act) {
     #pragma unroll
-                for (int v = 0; v < 8; v++) {
-                    T r = T(0);
-                    T f0, f1;
-                    if (LEAN) {
-                        // radial slopes of this cell and the one above; the latter is
-                        // carried to the next plane
-                        const T sc = have_fr ? sr[v] : minmod(win[v][1], win[v][2], win[v][3]);
-                        const T su = minmod(win[v][2], win[v][3], win[v][4]);
-                        f0 = have_fr ? fr[v]
-                                     : (face_flux_s<T, true>(win[v][1], win[v][2],
-                                                             minmod(win[v][0], win[v][1], win[v][2]), sc) *
-                                        (c10 + c1m)) * T(0.5);
-                        f1 = (face_flux_s<T, true>(win[v][2], win[v][3], sc, su) * (c1p + c10)) * T(0.5);
+                    for (int v = p0; v < p0 + NV; v++) {
+                        const T su = half_slope(w0[v], w1[v], w2[v]);
+                        const T f0 = fr[v];
+                        T f1 = face_flux<T, LEAN>(w0[v], w1[v], sr[v], su) * S1;
                         sr[v] = su;
-                    } else {
-                        f0 = have_fr ? fr[v]
-                                     : (face_flux(win[v][0], win[v][1], win[v][2], win[v][3]) * (c10 + c1m)) * T(0.5);
-                        f1 = (face_flux(win[v][1], win[v][2], win[v][3], win[v][4]) * (c1p + c10)) * T(0.5);
-                    }
-                    if (BFACE && bot && i == 0) {
-                        // lower face of the first cell: ghosts 0 and -1 mirror cells 1 and 2 of U^n
-                        const long long q = base + (long long)v * d.P;
-                        const double p = kParBottom[v];
-                        const double g0 = p * Uold[q], gm1 = p * Uold[q + m.SI];
-                        f0 = (T)((face_flux<double>(gm1, g0, ucur[v], U[q + m.SI]) * (double)(c10 + c1m)) * 0.5);
-                    }
-                    if (BFACE && topb && i == d.ni - 1) {
-                        // upper face of the last cell: ghosts ni+1 and ni+2 mirror cells ni and ni-1 of U^n
-                        const long long q = base + (long long)v * d.P;
-                        const double p = kParTop[v];
-                        const double g1 = p * Uold[q], g2 = p * Uold[q - m.SI];
-                        f1 = (T)((face_flux<double>(uprev[v], ucur[v], g1, g2) * (double)(c1p + c10)) * 0.5);
-                    }
-                    fr[v] = f1;
-                    if (LEAN) {
-                        r = r + (f0 - f1) * rdxi;
-                        r = r + (fj[v][ty][tx] - fj[v][ty + 1][tx]) * rL2;
-                        r = r + (fk[v][ty][tx] - fk[v][ty][tx + 1]) * rL3;
-                    } else {
-                        r = r + (f0 - f1) / dxi;
-                        r = r + (fj[v][ty][tx] - fj[v][ty + 1][tx]) / L2;
-                        r = r + (fk[v][ty][tx] - fk[v][ty][tx + 1]) / L3;
-                    }
-                    if (MODE == 0) {
-                        const long long q = base + (long long)v * d.P;
-                        const double x = (LEAN ? ucur[v] : U[q]) + (0.5 * dt) * (double)r;
-                        out[q] = x;
-                        if (shadow) shadow[q] = (float)x;
-                        if (v == 1) vv = x * x;
-                        if (v == 2 || v == 3) vv = vv + x * x;
-                        if (v == 4) bb2 = x * x;
-                        if (v == 5 || v == 6) bb2 = bb2 + x * x;
-                    } else {
-                        out[rbase + (long long)v * nn] = (double)r;
+                        if (BFACE && topb && i == d.ni - 1) {
+                            // upper face of the last cell: ghosts ni+1 and ni+2 mirror cells ni and ni-1 of U^n
+                            const long long q = base + (long long)v * d.P + m.coff;
+                            const double p = kParTop[v];
+                            const double g1 = p * Uold[q], g2 = p * Uold[q - m.SI];
+                            f1 = (T)(face_flux4<double>(uprev[v], ucur[v], g1, g2) * (double)S1);
+                        }
+                        fr[v] = f1;
+                        T r = T(0);
+                        r = r + over(f1 - f0, dxi, ydxi);
+                        r = r + over(fj(v, ty + 1, tx) - fj(v, ty, tx), L2, y2);
+                        r = r + over(fk(v, ty, tx + 1) - fk(v, ty, tx), L3, y3);
+                        if (MODE == 0) {
+                            const long long q = base + (long long)v * d.P;
+                            const double x = (LEAN ? ucur[v] : (double)w0[v]) + dts * (double)r;
+                            (out + q)[m.coff] = x;
+                            if (LEAN) (shadow + q)[m.coff] = (float)x;
+                            if (v == 1) vv = x * x;
+                            if (v == 2 || v == 3) vv = vv + x * x;
+                            if (v == 4) bb2 = x * x;
+                            if (v == 5 || v == 6) bb2 = bb2 + x * x;
+                        } else {
+                            out[rbase + (long long)v * nn] = kFluxScale * (double)r;
+                        }
                     }
                 }
+            }
+            if (m.act) {
                 if (MODE == 0) {
                     // ModWaveSpeed_Dynamo (3_6/ModWaveSpeed.f90:12-24) on the new state and
                     // h_LLL (3_6/ModBlock.f90:420-422), as k_dt_tile computes them
                     double w = cs_at(I) + sqrt(vv);
-                    w = w + sqrt(bb2) / sr_at(I);
+                    w = w + sqrt(bb2) / drow[2][I];
                     const double xi = xi_at(I);
                     double h = mt.dxi, h2 = xi * mt.dxj, h3 = (xi * sint64) * mt.dxk;
                     h = h < h2 ? h : h2;
@@ -916,11 +935,10 @@ __global__ void __launch_bounds__(TL * TL) k_diffusion(Dims d, DevTables t, cons
                     hmin = x < hmin ? x : hmin;
                 }
             }
-            have_fr = true;
+            v1c = v1n;
     #pragma unroll
             for (int v = 0; v < 8; v++) {
-                win[v][0] = win[v][1]; win[v][1] = win[v][2]; win[v][2] = win[v][3]; win[v][3] = win[v][4];
-                win[v][4] = nxt[v];
+                w0[v] = w1[v]; w1[v] = w2[v]; w2[v] = nxt[v];
                 if (BFACE) uprev[v] = ucur[v];
             }
         }
@@ -1536,8 +1554,11 @@ template <typename T, typename TIN>
 void launch_diffusion(const Dims &d, const DevTables &t, const TIN *in, const double *U, double *out, float *shadow,
                       double *partial, const double *dtp, hipStream_t s, const int32_t *pull, int tile, int wgs,
                       const double *Uold) {
-    if (sizeof(T) == 4 && (U != out || !Uold || d.ni < 2))
-        throw std::runtime_error("FP32 diffusion: updates the state in place, needs U^n and ni >= 2");
+    check_stage_ni(d);
+    if (sizeof(T) == 4 && (U != out || !Uold || !shadow || d.ni < 2))
+        throw std::runtime_error("FP32 diffusion: updates the state in place, needs U^n, the FP32 copy and ni >= 2");
+    if (sizeof(T) == 8 && ((const void *)in != (const void *)U || out == U || shadow))
+        throw std::runtime_error("FP64 diffusion: updates its input into another buffer");
     diffusion_any<0, T>(d, t, in, U, out, shadow, partial, dtp, s, pull, tile, wgs, Uold);
 }
 
@@ -1955,24 +1976,28 @@ __global__ void __launch_bounds__(256) k_glm_diffusion(Dims d, DevTables t, cons
     const double c10 = fabs(V1[s1]) + cs[I];
     const double c1p = fabs(V1[s1 + pI]) + cs[I + 1];
     const double p0 = Pb[q];
-    const double f0 = (face_flux(Pb[q - 2 * SI], Pb[q - SI], p0, Pb[q + SI]) * (c10 + c1m)) * 0.5;
-    const double f1 = (face_flux(Pb[q - SI], p0, Pb[q + SI], Pb[q + 2 * SI]) * (c1p + c10)) * 0.5;
+    // half slopes of the cell and its neighbours along one axis, then its two faces
+    auto faces = [&](double m2, double m1, double p1, double p2, double slo, double shi, double &lo, double &hi) {
+        const double s0 = half_slope(m1, p0, p1);
+        lo = face_flux<double, false>(m1, p0, half_slope(m2, m1, p0), s0) * slo;
+        hi = face_flux<double, false>(p0, p1, s0, half_slope(p0, p1, p2)) * shi;
+    };
+    double f0, f1, fj0, fj1, fk0, fk1;
+    faces(Pb[q - 2 * SI], Pb[q - SI], Pb[q + SI], Pb[q + 2 * SI], c10 + c1m, c1p + c10, f0, f1);
     const double csI2 = cs[I - 2];
     const double c2m = fabs(V2[s2 - pJ]) + csI2, c20 = fabs(V2[s2]) + csI2, c2p = fabs(V2[s2 + pJ]) + csI2;
-    const double fj0 = (face_flux(Pb[q - 2 * SJ], Pb[q - SJ], p0, Pb[q + SJ]) * (c20 + c2m)) * 0.5;
-    const double fj1 = (face_flux(Pb[q - SJ], p0, Pb[q + SJ], Pb[q + 2 * SJ]) * (c2p + c20)) * 0.5;
+    faces(Pb[q - 2 * SJ], Pb[q - SJ], Pb[q + SJ], Pb[q + 2 * SJ], c20 + c2m, c2p + c20, fj0, fj1);
     const double c3m = fabs(V3[cell_off(d, I - 2, J - 2, K - 1)]) + csI2, c30 = fabs(V3[cell_off(d, I - 2, J - 2, K)]) + csI2,
                  c3p = fabs(V3[cell_off(d, I - 2, J - 2, K + 1)]) + csI2;
-    const double fk0 = (face_flux(Pb[km2], Pb[km1], p0, Pb[kp1]) * (c30 + c3m)) * 0.5;
-    const double fk1 = (face_flux(Pb[km1], p0, Pb[kp1], Pb[kp2]) * (c3p + c30)) * 0.5;
+    faces(Pb[km2], Pb[km1], Pb[kp1], Pb[kp2], c30 + c3m, c3p + c30, fk0, fk1);
     const double xic = t.xi[rb + I];
     const double L2 = mt.dxj * xic;
     const double L3 = (mt.dxk * xic) * t.sint[tb + J];
     double r = 0.0;
-    r = r + (f0 - f1) / mt.dxi;
-    r = r + (fj0 - fj1) / L2;
-    r = r + (fk0 - fk1) / L3;
-    psi_new[(long long)g.b * d.P + q] = p0 + (0.5 * *dtp) * r;
+    r = r + (f1 - f0) / mt.dxi;
+    r = r + (fj1 - fj0) / L2;
+    r = r + (fk1 - fk0) / L3;
+    psi_new[(long long)g.b * d.P + q] = p0 + ((0.5 * kFluxScale) * *dtp) * r;
 }
 
 static unsigned glm_grid(const Dims &d) {
