@@ -85,24 +85,24 @@ inline Dims make_dims(int ni, int nj, int nk, int ng, int nblocks) {
     return d;
 }
 
-// Ghost-fill tables of the FP32 buffers, one row per ghost entry: same-panel entries in
-// [0, yy_begin), Yin-Yang entries in [yy_begin, n_total), each set in the order
-// of the receiving blocks' target lists.
+// Entries of one kind of the FP32 buffers' ghost fill.  The first n_face fill
+// ghosts outside the block along one axis, all that the stage kernel reads; the
+// others, ghosts beyond an edge or a corner, are read by the diffusion's
+// shifted speed cells only.  Both parts are in the order of src.
+struct DevFill {
+    const int2 *idx;        // (dst, src): block*8*P + cell of the ghost and of its (base) source cell, variable 0
+    int n, n_face;
+};
+// Ghost-fill tables of the FP32 buffers (device)
 struct DevGhosts {
-    const int32_t *dst;     // block*8*P + cell of the ghost (variable 0)
-    const int32_t *src;     // donor*8*P + cell of the interpolation base (variable 0)
-    const double *w;        // 3 weights per entry
-    const double *rot;      // 2 rotation coefficients per entry (read for Yin-Yang entries only)
-    int first, n_total, yy_begin;  // weighted entries [first, n_total): same-panel, then Yin-Yang from yy_begin
-    const int2 *copy;       // (dst, src) of the entries filled by a plain copy, sorted by dst
-    int n_copy;
-    const int2 *lerp;       // (dst, src) of the entries interpolated along r only, sorted by dst
+    DevFill weighted;       // trilinear; bit 31 of dst: a Yin-Yang entry
+    const double *w;        // 3 weights per weighted entry
+    const double *rot;      // 2 rotation coefficients per weighted entry (read for Yin-Yang entries only)
+    DevFill lerp;           // interpolated along r only
     const double *lerp_w;   // their r weight
-    int n_lerp;
-    // copies whose ghosts the consuming kernels read in place (see pull below),
-    // sorted by dst
-    const int2 *copy_rest;
-    int n_copy_rest;
+    DevFill copy;           // plain copies (every one: n_face is not used)
+    // copies whose ghosts the consuming kernels do not read in place (see pull below)
+    DevFill copy_rest;
     // pull[R*27 + (di+1)*9 + (dj+1)*3 + (dk+1)]: the same-level block D whose
     // interior holds all ghosts of block R in direction (di,dj,dk) as plain
     // copies, ghost index g <- D's cell g - (di*ni, dj*nj, dk*nk); -1 where any
@@ -110,13 +110,16 @@ struct DevGhosts {
     const int32_t *pull;
 };
 
-// Ghost-fill table of the FP64 buffers, in the order of src.
+// Ghost-fill table of the FP64 buffers: first the ghosts outside the block
+// along one axis (n_face), then those beyond an edge or a corner, both in the
+// order of src (see DevFill).
 struct DevGhosts64 {
+    const int32_t *all;     // every entry's index, in the order of src
     const int32_t *dst;     // block*8*P + cell of the ghost (variable 0); bit 31: a Yin-Yang entry
     const int32_t *src;     // donor*8*P + cell of the interpolation base (variable 0)
     const double *w;        // 3 weights per entry
     const double *rot;      // 2 rotation coefficients per entry (read for Yin-Yang entries only)
-    int n;
+    int n, n_face;
 };
 
 struct DevBoundary {
@@ -150,8 +153,9 @@ void launch_glm_stage(const Dims &d, const DevTables &t, const double *in, const
                       const double *psi_n, double *psi_out, double *G, const double *dtp, double div, hipStream_t s);
 void launch_glm_diffusion(const Dims &d, const DevTables &t, const double *U, const double *psi, double *psi_new,
                           const double *dtp, hipStream_t s);
-// the FP64 buffers' ghosts and (psi not null) psi's, in one pass over the table
-void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, hipStream_t s);
+// the FP64 buffers' ghosts and (psi not null) psi's, in one pass over the
+// table; faces: only the ghosts outside the block along one axis
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s);
 // Uold: U^n for the FP32 path, whose diffusion updates U (= out) in place;
 // null for the FP64 path (U != out)
 template <typename T, typename TIN>
@@ -168,8 +172,9 @@ int march_resident_wgs(int kernel, int precision, int tile);
 int march_segments(const Dims &d, int tile, int wgs);
 // every ghost entry of the FP32 buffers
 void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s);
-// the entries that kernels reading with pull = g.pull still need
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, hipStream_t s);
+// the entries that kernels reading with pull = g.pull still need; faces: only
+// the ghosts outside the block along one axis
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s);
 template <typename TS>
 void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull = nullptr);
 template <typename TS>

@@ -118,7 +118,7 @@ struct falcon_handle {
     DevGhosts gh32{};     // FP32 deviation path
     DevBoundary bnd{};
     // device memory
-    DevBuf meta, radial, angular, ghost64[4], ghost32[4], ghost_copy32, ghost_lerp32[2], bnd_list;   // ghost tables
+    DevBuf meta, radial, angular, ghost64[5], ghost32[3], ghost_copy32, ghost_lerp32[2], bnd_list;   // ghost tables
     DevBuf ghost_rest32, ghost_pull32;   // copies not read in place, pull table (FP32 path)
     bool ghost_pull = true;              // FP32 step: kernels read same-level ghost copies in place
     bool device_tables = false;          // falcon_set_gc_all builds the ghost tables on the device
@@ -161,8 +161,8 @@ struct falcon_handle {
 
     ~falcon_handle() {
         if (graph) (void)hipGraphExecDestroy(graph);
-        DevBuf *all[] = {&meta, &radial, &angular, &ghost64[0], &ghost64[1], &ghost64[2], &ghost64[3], &ghost32[0],
-                         &ghost32[1], &ghost32[2], &ghost32[3], &ghost_copy32, &ghost_lerp32[0], &ghost_lerp32[1],
+        DevBuf *all[] = {&meta, &radial, &angular, &ghost64[0], &ghost64[1], &ghost64[2], &ghost64[3], &ghost64[4], &ghost32[0],
+                         &ghost32[1], &ghost32[2], &ghost_copy32, &ghost_lerp32[0], &ghost_lerp32[1],
                          &bnd_list, &ghost_rest32, &ghost_pull32,
 
                          &U[0], &U[1], &F32[0], &F32[1], &S64[0], &S64[1], &S32[0], &S32[1], &dtp, &partial, &rbuf, &diffbuf, &scanbuf,
@@ -367,9 +367,15 @@ void upload_radial(falcon_handle *h) {
     h->shadow_valid = false;
 }
 
-// Table of the FP64 ghost fill: every entry, Yin-Yang ones marked, in the
-// order of their base cells' addresses (k_exchange_f64), target-list order
-// where bases coincide.
+// Whether a padded cell lies outside the block's interior along one axis only.
+bool face_ghost(const Dims &d, int I, int J, int K) {
+    const int n = (I < d.ng || I >= d.ng + d.ni) + (J < d.ng || J >= d.ng + d.nj) + (K < d.ng || K >= d.ng + d.nk);
+    return n == 1;
+}
+
+// Table of the FP64 ghost fill (DevGhosts64): every entry, Yin-Yang ones
+// marked, face ghosts before the others, in the order of their base cells'
+// addresses (k_exchange_f64), target-list order where bases coincide.
 void upload_ghosts64(falcon_handle *h) {
     const Dims &d = h->dims;
     const std::vector<GhostEntry> &G = h->lay.ghosts;
@@ -385,13 +391,16 @@ void upload_ghosts64(falcon_handle *h) {
     auto base = [&](const GhostEntry &g) -> int32_t {
         return (int32_t)((long long)g.donor * 8 * d.P + cell_off(d, g.i0 + ng - 1, g.j0 + ng - 1, g.k0 + ng - 1));
     };
+    auto bucket = [&](const GhostEntry &g) -> int {
+        return g.donor + (face_ghost(d, g.gi + ng - 1, g.gj + ng - 1, g.gk + ng - 1) ? 0 : nb);
+    };
     // (base, entry) counted into donors, then sorted within each
-    std::vector<std::vector<size_t>> at(nt, std::vector<size_t>(nb, 0));
+    std::vector<std::vector<size_t>> at(nt, std::vector<size_t>(2 * nb, 0));
     parallel([&](int t) {
-        for (size_t e = N * t / nt; e < N * (t + 1) / nt; e++) at[t][G[e].donor]++;
+        for (size_t e = N * t / nt; e < N * (t + 1) / nt; e++) at[t][bucket(G[e])]++;
     });
-    std::vector<size_t> first(nb + 1, 0);
-    for (int b = 0; b < nb; b++) {
+    std::vector<size_t> first(2 * nb + 1, 0);
+    for (int b = 0; b < 2 * nb; b++) {
         first[b + 1] = first[b];
         for (int t = 0; t < nt; t++) {
             const size_t c = at[t][b];
@@ -402,12 +411,12 @@ void upload_ghosts64(falcon_handle *h) {
     std::vector<std::pair<int32_t, uint32_t>> key(N);
     parallel([&](int t) {
         for (size_t e = N * t / nt; e < N * (t + 1) / nt; e++)
-            key[at[t][G[e].donor]++] = {base(G[e]), (uint32_t)e};
+            key[at[t][bucket(G[e])]++] = {base(G[e]), (uint32_t)e};
     });
-    std::vector<int32_t> dst(N), src(N);
+    std::vector<int32_t> dst(N), src(N), all(N);
     std::vector<double> w(3 * N), rot(2 * N);
     parallel([&](int t) {
-        for (int b = t; b < nb; b += nt) {
+        for (int b = t; b < 2 * nb; b += nt) {
             std::sort(key.begin() + first[b], key.begin() + first[b + 1]);
             for (size_t q = first[b]; q < first[b + 1]; q++) {
                 const GhostEntry &g = G[key[q].second];
@@ -420,6 +429,14 @@ void upload_ghosts64(falcon_handle *h) {
             }
         }
     });
+    // the two parts of each donor merged
+    parallel([&](int t) {
+        for (int b = t; b < nb; b += nt) {
+            size_t f = first[b], o = first[nb + b], q = f + (o - first[nb]);
+            while (f < first[b + 1] || o < first[nb + b + 1])
+                all[q++] = (int32_t)(o == first[nb + b + 1] || (f < first[b + 1] && src[f] <= src[o]) ? f++ : o++);
+        }
+    });
     auto up = [&](DevBuf &buf, const void *data, size_t bytes) {
         buf.alloc(std::max<size_t>(bytes, 16));
         if (bytes) HIPCHECK(hipMemcpy(buf.p, data, bytes, hipMemcpyHostToDevice));
@@ -428,8 +445,9 @@ void upload_ghosts64(falcon_handle *h) {
     up(h->ghost64[1], src.data(), sizeof(int32_t) * N);
     up(h->ghost64[2], w.data(), sizeof(double) * 3 * N);
     up(h->ghost64[3], rot.data(), sizeof(double) * 2 * N);
-    h->gh64 = DevGhosts64{h->ghost64[0].as<int32_t>(), h->ghost64[1].as<int32_t>(), h->ghost64[2].as<double>(),
-                          h->ghost64[3].as<double>(), (int)N};
+    up(h->ghost64[4], all.data(), sizeof(int32_t) * N);
+    h->gh64 = DevGhosts64{h->ghost64[4].as<int32_t>(), h->ghost64[0].as<int32_t>(), h->ghost64[1].as<int32_t>(), h->ghost64[2].as<double>(),
+                          h->ghost64[3].as<double>(), (int)N, (int)first[nb]};
 }
 
 void upload_tables(falcon_handle *h) {
@@ -471,70 +489,93 @@ void upload_tables(falcon_handle *h) {
     dt.g_over_rho0 = R + 6 * rs; dt.xir2 = R + 7 * rs; dt.heat = R + 8 * rs; dt.cs = R + 9 * rs; dt.sqrt_rho0 = R + 10 * rs;
     dt.sint = A; dt.sinv = A + as; dt.cot = A + 2 * as;
 
-    // ghost entries: same-panel first, then Yin-Yang, each in target-list order
     const auto &G = h->lay.ghosts;
     const long long P = h->dims.P;
     auto cell = [&](int i, int j, int k) -> long long { return cell_off(h->dims, i + ng - 1, j + ng - 1, k + ng - 1); };
     if ((long long)nb * 8 * P >= (1ll << 31)) throw Error("state too large for 32-bit ghost offsets");
     // FP64 buffers: every entry weighted (upload_ghosts64).  FP32 buffers of
     // the deviation path: near copies and radial lerps (fp32_copy_lerp), the
-    // rest weighted, same-panel entries first, then Yin-Yang, each in
-    // target-list order.
+    // rest weighted.
     std::vector<int2> copy32;
     std::vector<std::pair<int2, double>> lerp32;
     fp32_copy_lerp(h, copy32, lerp32);
-    std::vector<int2> lerp_idx(lerp32.size());
-    std::vector<double> lerp_w(lerp32.size());
-    for (size_t q = 0; q < lerp32.size(); q++) { lerp_idx[q] = lerp32[q].first; lerp_w[q] = lerp32[q].second; }
     auto up = [&](DevBuf &buf, const void *data, size_t bytes) {
         buf.alloc(std::max<size_t>(bytes, 16));
         if (bytes) HIPCHECK(hipMemcpy(buf.p, data, bytes, hipMemcpyHostToDevice));
     };
-    // weighted table of the entries passing `keep`, plain then Yin-Yang
-    auto weighted = [&](auto keep, DevBuf *bufs) -> DevGhosts {
-        std::vector<size_t> order;
-        for (int pass = 0; pass < 2; pass++)
-            for (size_t e = 0; e < G.size(); e++)
-                if (G[e].yy == pass && keep(G[e])) order.push_back(e);
-        const size_t NG = order.size();
-        int yy_begin = 0;
-        while (yy_begin < (int)NG && !G[order[yy_begin]].yy) yy_begin++;
-        std::vector<int32_t> dst(NG), src(NG);
-        std::vector<double> w(3 * NG), rot(2 * NG);
-        for (size_t q = 0; q < NG; q++) {
-            const GhostEntry &e = G[order[q]];
-            dst[q] = (int32_t)((long long)e.recv_block * 8 * P + cell(e.gi, e.gj, e.gk));
-            src[q] = (int32_t)((long long)e.donor * 8 * P + cell(e.i0, e.j0, e.k0));
-            w[3 * q] = e.w[0]; w[3 * q + 1] = e.w[1]; w[3 * q + 2] = e.w[2];
-            rot[2 * q] = e.rot[0]; rot[2 * q + 1] = e.rot[1];
-        }
-        up(bufs[0], dst.data(), sizeof(int32_t) * NG);
-        up(bufs[1], src.data(), sizeof(int32_t) * NG);
-        up(bufs[2], w.data(), sizeof(double) * 3 * NG);
-        up(bufs[3], rot.data(), sizeof(double) * 2 * NG);
-        return DevGhosts{bufs[0].as<int32_t>(), bufs[1].as<int32_t>(), bufs[2].as<double>(), bufs[3].as<double>(),
-                         0, (int)NG, yy_begin, nullptr, 0, nullptr, nullptr, 0};
+    // ghosts outside the block along one axis come first, each part in the
+    // order of the sources (DevFill)
+    auto is_face = [&](int32_t dst) {
+        int I, J, K;
+        cell_ijk(h->dims, dst % (8 * P), I, J, K);
+        return face_ghost(h->dims, I, J, K);
+    };
+    auto by_source = [&](auto &v, auto &&idx) -> int {
+        const auto mid = std::partition(v.begin(), v.end(), [&](const auto &x) { return is_face(idx(x).x & 0x7fffffff); });
+        auto less = [&](const auto &x, const auto &y) {
+            return idx(x).y != idx(y).y ? idx(x).y < idx(y).y : idx(x).x < idx(y).x;
+        };
+        std::sort(v.begin(), mid, less);
+        std::sort(mid, v.end(), less);
+        return (int)(mid - v.begin());
     };
     upload_ghosts64(h);
-    h->gh32 = weighted([&](const GhostEntry &g) { return !fp32_near(g) && !fp32_lerp_r(g); }, h->ghost32);
-    up(h->ghost_copy32, copy32.data(), sizeof(int2) * copy32.size());
-    up(h->ghost_lerp32[0], lerp_idx.data(), sizeof(int2) * lerp_idx.size());
-    up(h->ghost_lerp32[1], lerp_w.data(), sizeof(double) * lerp_w.size());
-    h->gh32.copy = h->ghost_copy32.as<int2>();
-    h->gh32.n_copy = (int)copy32.size();
-    h->gh32.lerp = h->ghost_lerp32[0].as<int2>();
-    h->gh32.lerp_w = h->ghost_lerp32[1].as<double>();
-    h->gh32.n_lerp = (int)lerp_idx.size();
-
+    DevGhosts &g32 = h->gh32;
+    {
+        // a base on an axis's last cell (weight 0 there) becomes the cell before it
+        // with weight 1, so that no corner is a ghost of the donor (k_exchange_f32)
+        const int n3[3] = {t.ni, t.nj, t.nk};
+        auto inside = [&](GhostEntry g) -> GhostEntry {
+            int32_t *base[3] = {&g.i0, &g.j0, &g.k0};
+            for (int a = 0; a < 3; a++)
+                if (*base[a] == n3[a] && n3[a] > 1) { --*base[a]; g.w[a] += 1.0; }
+            return g;
+        };
+        std::vector<std::pair<int2, uint32_t>> wt;
+        for (size_t e = 0; e < G.size(); e++) {
+            if (fp32_near(G[e]) || fp32_lerp_r(G[e])) continue;
+            const GhostEntry g = inside(G[e]);
+            const int32_t dst = (int32_t)((long long)g.recv_block * 8 * P + cell(g.gi, g.gj, g.gk));
+            wt.push_back({make_int2((int32_t)((uint32_t)dst | (g.yy ? 0x80000000u : 0u)),
+                                    (int32_t)((long long)g.donor * 8 * P + cell(g.i0, g.j0, g.k0))), (uint32_t)e});
+        }
+        const int nf = by_source(wt, [](const auto &x) -> const int2 & { return x.first; });
+        std::vector<int2> idx(wt.size());
+        std::vector<double> w(3 * wt.size()), rot(2 * wt.size());
+        for (size_t q = 0; q < wt.size(); q++) {
+            const GhostEntry g = inside(G[wt[q].second]);
+            idx[q] = wt[q].first;
+            w[3 * q] = g.w[0]; w[3 * q + 1] = g.w[1]; w[3 * q + 2] = g.w[2];
+            rot[2 * q] = g.rot[0]; rot[2 * q + 1] = g.rot[1];
+        }
+        up(h->ghost32[0], idx.data(), sizeof(int2) * idx.size());
+        up(h->ghost32[1], w.data(), sizeof(double) * w.size());
+        up(h->ghost32[2], rot.data(), sizeof(double) * rot.size());
+        g32.weighted = {h->ghost32[0].as<int2>(), (int)idx.size(), nf};
+        g32.w = h->ghost32[1].as<double>();
+        g32.rot = h->ghost32[2].as<double>();
+    }
+    {
+        const int nf = by_source(lerp32, [](const auto &x) -> const int2 & { return x.first; });
+        std::vector<int2> idx(lerp32.size());
+        std::vector<double> w(lerp32.size());
+        for (size_t q = 0; q < lerp32.size(); q++) { idx[q] = lerp32[q].first; w[q] = lerp32[q].second; }
+        up(h->ghost_lerp32[0], idx.data(), sizeof(int2) * idx.size());
+        up(h->ghost_lerp32[1], w.data(), sizeof(double) * w.size());
+        g32.lerp = {h->ghost_lerp32[0].as<int2>(), (int)idx.size(), nf};
+        g32.lerp_w = h->ghost_lerp32[1].as<double>();
+    }
     {
         std::vector<int32_t> pull;
         std::vector<int2> rest;
         build_pull_table(h, copy32, pull, rest);
+        const int nf = by_source(rest, [](const int2 &x) -> const int2 & { return x; });
+        up(h->ghost_copy32, copy32.data(), sizeof(int2) * copy32.size());
         up(h->ghost_rest32, rest.data(), sizeof(int2) * rest.size());
         up(h->ghost_pull32, pull.data(), sizeof(int32_t) * pull.size());
-        h->gh32.copy_rest = h->ghost_rest32.as<int2>();
-        h->gh32.n_copy_rest = (int)rest.size();
-        h->gh32.pull = h->ghost_pull32.as<int32_t>();
+        g32.copy = {h->ghost_copy32.as<int2>(), (int)copy32.size(), (int)copy32.size()};
+        g32.copy_rest = {h->ghost_rest32.as<int2>(), (int)rest.size(), nf};
+        g32.pull = h->ghost_pull32.as<int32_t>();
     }
 
     std::vector<int32_t> bl;
@@ -645,14 +686,16 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
                                                              nullptr, ts, ws, G);
             });
             timed(h, k < 4 ? K_XSTAGE : K_XSTATE, [&] {
-                launch_exchange64(d, h->gh64, out[k - 1], pout[k - 1], s);
+                // the stage buffers' ghosts beyond edges and corners are left out: the
+                // diffusion alone reads such ghosts (its shifted speed cells), the state's
+                launch_exchange64(d, h->gh64, out[k - 1], pout[k - 1], k < 4, s);
             });
         }
         timed(h, K_DIFF, [&] { launch_diffusion<double, double>(d, t, U, U, Un, nullptr, part, dtp, s, nullptr, td, wd); });
         if (glm) timed(h, K_OTHER, [&] { launch_glm_diffusion(d, t, U, P, Pn, dtp, s); });
         timed(h, K_OTHER, [&] { launch_copy_radial<double>(d, h->bnd, U, Un, s); });
         timed(h, K_XSTATE, [&] {
-            launch_exchange64(d, h->gh64, Un, Pn, s);
+            launch_exchange64(d, h->gh64, Un, Pn, false, s);
         });
     } else {
         float *S0 = h->S32[0].as<float>(), *S1 = h->S32[1].as<float>();
@@ -661,10 +704,12 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         float *out[3] = {S0, S1, S0};
         // with the pull table, the stage and diffusion kernels read same-level
         // ghost copies from the neighbours' interiors and the exchange fills
-        // only the other ghosts
+        // only the other ghosts.  Those beyond a block's edges and corners are left
+        // out of the stage buffers: the diffusion alone reads them (its shifted
+        // speed cells, and through the first stage's radial mirror of them)
         const int32_t *pull = h->ghost_pull ? h->gh32.pull : nullptr;
-        auto exchange = [&](float *st) {
-            if (pull) launch_exchange_rest(d, h->gh32, st, s);
+        auto exchange = [&](float *st, bool faces) {
+            if (pull) launch_exchange_rest(d, h->gh32, st, faces, s);
             else launch_exchange(d, h->gh32, st, s);
         };
         for (int k = 1; k <= 4; k++) {
@@ -675,16 +720,16 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
                 timed(h, K_STAGE, [&] {
                     launch_stage<float, float, float, float>(d, t, in[k - 1], F, out[k - 1], nullptr, dtp, div, s, pull, ts, ws);
                 });
-                timed(h, K_XSTAGE, [&] { exchange(out[k - 1]); });
+                timed(h, K_XSTAGE, [&] { exchange(out[k - 1], true); });
             } else {
                 // U^n stays in U: the diffusion's boundary faces read it
                 timed(h, K_STAGE,
                       [&] { launch_stage<float, float, double, double>(d, t, in[3], U, Un, F, dtp, div, s, pull, ts, ws); });
-                timed(h, K_XSTATE, [&] { exchange(F); });
+                timed(h, K_XSTATE, [&] { exchange(F, false); });
             }
         }
         timed(h, K_DIFF, [&] { launch_diffusion<float, float>(d, t, F, Un, Un, Fn, part, dtp, s, pull, td, wd, U); });
-        timed(h, K_XSTATE, [&] { exchange(Fn); });
+        timed(h, K_XSTATE, [&] { exchange(Fn, false); });
     }
 }
 
@@ -694,7 +739,7 @@ void prepare_steps(falcon_handle *h) {
     const long long n = (long long)d.nblocks * 8 * d.P;
     if (h->precision == 1 && !h->shadow_valid) {
         if (!h->u_ghosts_valid) {
-            launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, h->stream);
+            launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, false, h->stream);
             h->u_ghosts_valid = true;
         }
         launch_to_f32(h->U[h->cur].as<double>(), h->F32[h->cur].as<float>(), n, h->stream);
@@ -706,7 +751,7 @@ void prepare_steps(falcon_handle *h) {
         h->shadow_valid = true;
     }
     if (h->precision == 0 && !h->u_ghosts_valid) {
-        launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, h->stream);
+        launch_exchange64(d, h->gh64, h->U[h->cur].as<double>(), nullptr, false, h->stream);
         h->u_ghosts_valid = true;
     }
     if (!h->partials_valid) {
@@ -727,7 +772,7 @@ void after_steps(falcon_handle *h) {
 void refresh_u_ghosts(falcon_handle *h) {
     if (h->u_ghosts_valid) return;
     double *U = h->U[h->cur].as<double>();
-    launch_exchange64(h->dims, h->gh64, U, nullptr, h->stream);
+    launch_exchange64(h->dims, h->gh64, U, nullptr, false, h->stream);
     launch_boundary<double>(h->dims, h->bnd, U, h->stream);
     h->u_ghosts_valid = true;
 }
@@ -1190,8 +1235,8 @@ int falcon_init_synthetic(falcon_handle_t h, uint64_t seed, double s_amp, double
         launch_synthetic(d, drng.as<double>(), dyin.as<int32_t>(), drows.as<double>(), dmodes.as<SynthMode>(), nm, seed,
                          s_amp, b_ratio, U, dmax.as<double>(), h->stream);
         // the reference driver's two initial fills (3_6/test1.f90:143-144)
-        launch_exchange64(d, h->gh64, U, nullptr, h->stream);
-        launch_exchange64(d, h->gh64, U, nullptr, h->stream);
+        launch_exchange64(d, h->gh64, U, nullptr, false, h->stream);
+        launch_exchange64(d, h->gh64, U, nullptr, false, h->stream);
         h->partials_valid = false;
         h->shadow_valid = false;
         h->u_ghosts_valid = true;
@@ -1368,10 +1413,9 @@ int falcon_set_ghost_pull(falcon_handle_t h, int on) {
         }
         if (on && !h->ghost_pull) {
             // With the pull on, the ghosts that the kernels read in place are
-            // never written again, yet the FP32 Yin-Yang gather reads some of
-            // them as zero-weight corners (f * 0).  Whatever a run without the
-            // pull left there (a diverged run's NaN included) is cleared: the
-            // FP32 buffers restart from zeros and the shadow of U is rebuilt.
+            // never written again.  Whatever a run without the pull left there (a
+            // diverged run's NaN included) is cleared: the FP32 buffers restart
+            // from zeros and the shadow of U is rebuilt.
             if (h->stream) HIPCHECK(hipStreamSynchronize(h->stream));
             for (DevBuf *b : {&h->S32[0], &h->S32[1], &h->F32[0], &h->F32[1]})
                 if (b->p) HIPCHECK(hipMemset(b->p, 0, b->bytes));
@@ -1387,13 +1431,13 @@ int falcon_sendrecv_gc(falcon_handle_t h, int which) {
         ensure_device_tables(h);
         if (which == 0) {
             launch_exchange64(h->dims, h->gh64, h->U[h->cur].as<double>(),
-                              h->divb ? h->psi[h->cur].as<double>() : nullptr, h->stream);
+                              h->divb ? h->psi[h->cur].as<double>() : nullptr, false, h->stream);
             h->shadow_valid = false;
         } else {
             alloc_stage(h);
             if (h->precision == 0)
                 launch_exchange64(h->dims, h->gh64, h->S64[0].as<double>(),
-                                  h->divb ? h->psiS[0].as<double>() : nullptr, h->stream);
+                                  h->divb ? h->psiS[0].as<double>() : nullptr, false, h->stream);
             else launch_exchange(h->dims, h->gh32, h->S32[0].as<float>(), h->stream);
         }
         check_launch();
@@ -1501,10 +1545,21 @@ int falcon_check_state(falcon_handle_t h, int which, int64_t *n_nan, int32_t *wh
             if (h->divb) launch_nan_scan_psi(d, h->psi[h->cur].as<double>(), w, h->stream);
         } else if (h->precision == 0) {
             if (!h->S64[0].p) throw Error("falcon_check_state: no stage buffer yet");
+            // the ghosts beyond edges and corners that the steps leave out
+            if (h->dt.meta) {
+                launch_exchange64(d, h->gh64, h->S64[0].as<double>(), h->divb ? h->psiS[0].as<double>() : nullptr, false,
+                                  h->stream);
+                launch_boundary<double>(d, h->bnd, h->S64[0].as<double>(), h->stream);
+            }
             launch_nan_scan<double>(d, h->S64[0].as<double>(), w, h->stream);
             if (h->divb) launch_nan_scan_psi(d, h->psiS[0].as<double>(), w, h->stream);
         } else {
             if (!h->S32[0].p) throw Error("falcon_check_state: no stage buffer yet");
+            // the ghosts beyond edges and corners that the steps leave out
+            if (h->ghost_pull && h->dt.meta) {
+                launch_exchange_rest(d, h->gh32, h->S32[0].as<float>(), false, h->stream);
+                launch_boundary<float>(d, h->bnd, h->S32[0].as<float>(), h->stream, h->gh32.pull);
+            }
             launch_nan_scan<float>(d, h->S32[0].as<float>(), w, h->stream);
         }
         check_launch();
@@ -1756,7 +1811,7 @@ int falcon_profile_step(falcon_handle_t h, int nsteps, double cfl, double *out_m
 int falcon_device_bytes(falcon_handle_t h, int64_t *bytes) {
     return guard([&] {
         const DevBuf *all[] = {&h->meta, &h->radial, &h->angular, &h->ghost64[0], &h->ghost64[1], &h->ghost64[2],
-                               &h->ghost64[3], &h->ghost32[0], &h->ghost32[1], &h->ghost32[2], &h->ghost32[3],
+                               &h->ghost64[3], &h->ghost64[4], &h->ghost32[0], &h->ghost32[1], &h->ghost32[2],
                                &h->ghost_copy32, &h->ghost_lerp32[0], &h->ghost_lerp32[1],
                                &h->ghost_rest32, &h->ghost_pull32,
                                &h->bnd_list, &h->U[0], &h->U[1], &h->F32[0], &h->F32[1], &h->S64[0], &h->S64[1],

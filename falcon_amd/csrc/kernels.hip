@@ -995,30 +995,83 @@ __device__ __forceinline__ void yy_rotate(double (&val)[8], double a, double bb)
 // donors are read only at interior cells (clamped bases touch a donor ghost only
 // with an exactly-zero weight), so entries are independent.
 //
-// For the FP32 buffers every corner is loaded (a gather that skips the
-// zero-weight ones measures twice the time).  A zero-weight corner may lie on
-// a donor ghost cell that the ghost pull leaves unwritten; the FP32 buffers
-// are zeroed when allocated and written with finite values only, so that term
-// is f*0 = +-0 as well.
-__global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, float *__restrict__ st) {
-    const int e = g.first + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (e >= g.n_total) return;
+//
+// Workgroup of a fill in the order of its sources: runs of kXcdRun workgroups
+// go to one XCD, whose L2 then holds the lines they share.
+constexpr int kXcdRun = 64;
+__device__ __forceinline__ int xcd_run(int wg, int n) {
+    const int grp = wg / (8 * kXcdRun), r = wg - grp * 8 * kXcdRun;
+    return (grp + 1) * 8 * kXcdRun <= n ? grp * 8 * kXcdRun + (r & 7) * kXcdRun + (r >> 3) : wg;
+}
+
+// The FP32 buffers' ghosts: workgroups [0, nw) take the weighted entries, the
+// next nl the radial lerps, the rest the copies, so the three kinds run
+// together instead of in three launches with three tails.
+//   weighted: every corner is loaded (a gather that skips the zero-weight ones
+//     measures twice the time); a base on an axis's last cell, whose upper
+//     corner would be a ghost that this launch fills, is in the table as the
+//     cell before it with weight 1;
+//   lerp: same-panel entries whose theta/phi weights lie within 1e-12 of 0 or
+//     1 and whose r weight does not (neighbours across a radial block face,
+//     whose radial spacings differ): the two r corners of the weighted sum;
+//   copy: same-panel entries whose weights lie within 1e-12 of 0 or 1
+//     (same-level neighbours whose cell centres coincide up to rounding), from
+//     the nearest donor cell.
+// Bound by HBM and, on small layouts, by launch and tail.  Three launches in
+// target-list and destination order took 95 us on 1536 16^3 blocks (500 MB),
+// 71 us on 528 refined ones, 20 us on 648 8^3 ones; one launch in source order
+// 81, 59 and 13 us, its face ghosts alone 52, 42 and 9 us.
+__global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFill copy, int nwe, int nle, int nce,
+                                                      float *__restrict__ st) {
+    const int nw = (nwe + 255) / 256, nl = (nle + 255) / 256, nc = (nce + 255) / 256;
     const long long P = d.P;
-    // the base cell is interior along phi, so its corners are in the main part
+    // a base cell is interior along phi, so its corners are in the main part
     const int SI = (int)d.SI, SJ = d.SJ;
-    const int dst = g.dst[e], src = g.src[e];
-    const double wi = g.w[3 * (long long)e], wj = g.w[3 * (long long)e + 1], wk = g.w[3 * (long long)e + 2];
-    double val[8];
+    int wg = blockIdx.x;
+    if (wg < nw) {
+        const int e = xcd_run(wg, nw) * 256 + (int)threadIdx.x;
+        if (e >= nwe) return;
+        const int2 c = g.weighted.idx[e];
+        const double wi = g.w[3 * (long long)e], wj = g.w[3 * (long long)e + 1], wk = g.w[3 * (long long)e + 2];
+        double val[8];
 #pragma unroll
-    for (int v = 0; v < 8; v++) {
-        const float *F = st + src + (long long)v * P;
-        const double f000 = F[0], f100 = F[SI], f010 = F[SJ], f001 = F[1], f110 = F[SI + SJ], f011 = F[SJ + 1],
-                     f101 = F[SI + 1], f111 = F[SI + SJ + 1];
-        val[v] = trilinear8(f000, f100, f010, f001, f110, f011, f101, f111, wi, wj, wk);
+        for (int v = 0; v < 8; v++) {
+            const float *F = st + c.y + (long long)v * P;
+            const double f000 = F[0], f100 = F[SI], f010 = F[SJ], f001 = F[1], f110 = F[SI + SJ], f011 = F[SJ + 1],
+                         f101 = F[SI + 1], f111 = F[SI + SJ + 1];
+            val[v] = trilinear8(f000, f100, f010, f001, f110, f011, f101, f111, wi, wj, wk);
+        }
+        if (c.x < 0) yy_rotate(val, g.rot[2 * (long long)e], g.rot[2 * (long long)e + 1]);
+#pragma unroll
+        for (int v = 0; v < 8; v++) st[(c.x & 0x7fffffff) + (long long)v * P] = (float)val[v];
+        return;
     }
-    if (e >= g.yy_begin) yy_rotate(val, g.rot[2 * (long long)e], g.rot[2 * (long long)e + 1]);
+    wg -= nw;
+    if (wg < nl) {
+        const int e = xcd_run(wg, nl) * 256 + (int)threadIdx.x;
+        if (e >= nle) return;
+        const int2 c = g.lerp.idx[e];
+        const double wi = g.lerp_w[e];
+        float f0[8], f1[8];
 #pragma unroll
-    for (int v = 0; v < 8; v++) st[dst + (long long)v * P] = (float)val[v];
+        for (int v = 0; v < 8; v++) {
+            const float *F = st + c.y + (long long)v * P;
+            f0[v] = F[0];
+            f1[v] = F[SI];
+        }
+#pragma unroll
+        for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = (float)((double)f0[v] * (1.0 - wi) + (double)f1[v] * wi);
+        return;
+    }
+    wg -= nl;
+    const int e = xcd_run(wg, nc) * 256 + (int)threadIdx.x;
+    if (e >= nce) return;
+    const int2 c = copy.idx[e];
+    float val[8];
+#pragma unroll
+    for (int v = 0; v < 8; v++) val[v] = st[c.y + (long long)v * P];
+#pragma unroll
+    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = val[v] + 0.0f;
 }
 
 // The FP64 buffers' ghosts.  The entries come in the order of their base
@@ -1029,7 +1082,9 @@ __global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, float *__
 // and wrote 479 MB per fill in target-list order (342 us) for 403 MB of
 // donor rows, 383 MB of ghosts and 172 MB of table; sorted, with the Yin-Yang
 // entries behind the plain ones, 881 and 464 MB (277 us), in one sequence and
-// in runs of workgroups 240 to 250 us.  Not kept: staging boxes of donor cells in LDS
+// in runs of workgroups 240 to 250 us, the face ghosts alone 205 us.  A full
+// fill takes both parts of the table through `all`, in one sequence (one part
+// after the other reads their shared lines twice: 302 us).  Not kept: staging boxes of donor cells in LDS
 // (368 us: whole boxes are read where the ghosts need their shells), one
 // contiguous range of workgroups per XCD (312 us), non-temporal table loads
 // (no change).
@@ -1039,15 +1094,12 @@ __global__ void __launch_bounds__(256) k_exchange(Dims d, DevGhosts g, float *__
 // is +0, which leaves every nonzero result bit-identical (60% of the corner
 // loads on the production layouts).
 // PSI: also psi of GLM divergence cleaning ([block][P]), a scalar.
-constexpr int kXcdRun = 64;
 template <bool PSI>
-__global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, double *__restrict__ st,
-                                                      double *__restrict__ psi) {
-    int wg = blockIdx.x;
-    const int grp = wg / (8 * kXcdRun), r = wg - grp * 8 * kXcdRun;
-    if ((grp + 1) * 8 * kXcdRun <= (int)gridDim.x) wg = grp * 8 * kXcdRun + (r & 7) * kXcdRun + (r >> 3);
-    const int e = wg * 256 + (int)threadIdx.x;
-    if (e >= g.n) return;
+__global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, const int32_t *__restrict__ all,
+                                                      int n, double *__restrict__ st, double *__restrict__ psi) {
+    int e = xcd_run(blockIdx.x, gridDim.x) * 256 + (int)threadIdx.x;
+    if (e >= n) return;
+    if (all) e = all[e];
     const long long P = d.P;
     // the base cell is interior along phi, so its corners are in the main part
     const int SI = (int)d.SI, SJ = d.SJ;
@@ -1077,43 +1129,6 @@ __global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, dou
     for (int v = 0; v < 8; v++) st[dst + (long long)v * P] = val[v];
     // psi has the state's cell layout
     if constexpr (PSI) psi[psi_off(d, dst)] = value(psi + psi_off(d, src));
-}
-
-// FP32 buffers: ghost entries filled by a plain copy, sorted by destination so
-// consecutive lanes copy consecutive phi cells: the same-panel entries whose
-// weights lie within 1e-12 of 0 or 1 (same-level neighbours whose cell centres
-// coincide up to rounding), copied from the nearest donor cell.
-__global__ void __launch_bounds__(256) k_exchange_copy(Dims d, const int2 *__restrict__ copy, int n,
-                                                       float *__restrict__ st) {
-    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (e >= n) return;
-    const int2 c = copy[e];
-    const long long P = d.P;
-    float val[8];
-#pragma unroll
-    for (int v = 0; v < 8; v++) val[v] = st[c.y + (long long)v * P];
-#pragma unroll
-    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = val[v] + 0.0f;
-}
-
-// FP32 buffers: same-panel entries whose theta/phi weights lie within 1e-12 of
-// 0 or 1 and whose r weight does not (neighbours across a radial block face,
-// whose radial spacings differ): the two r corners of the weighted sum.
-__global__ void __launch_bounds__(256) k_exchange_lerp(Dims d, DevGhosts g, float *__restrict__ st) {
-    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (e >= g.n_lerp) return;
-    const int2 c = g.lerp[e];
-    const double wi = g.lerp_w[e];
-    const long long P = d.P;
-    const int SI = (int)d.SI;   // the donor cell is interior along phi (main part)
-    double val[8];
-#pragma unroll
-    for (int v = 0; v < 8; v++) {
-        const float *F = st + c.y + (long long)v * P;
-        val[v] = (double)F[0] * (1.0 - wi) + (double)F[SI] * wi;
-    }
-#pragma unroll
-    for (int v = 0; v < 8; v++) st[c.x + (long long)v * P] = (float)val[v];
 }
 
 // ---------------------------------------------------------------- boundary
@@ -1569,32 +1584,30 @@ void launch_diffusion_only(const Dims &d, const DevTables &t, const double *U, d
                         (const int32_t *)nullptr, tile, wgs, (const double *)nullptr);
 }
 
-static void exchange_with(const Dims &d, const DevGhosts &g, const int2 *copy, int n_copy, float *state,
-                          hipStream_t s) {
-    if (n_copy > 0)
-        hipLaunchKernelGGL(k_exchange_copy, dim3((unsigned)((n_copy + 255) / 256)), dim3(256), 0, s, d, copy, n_copy,
-                           state);
-    if (g.n_lerp > 0)
-        hipLaunchKernelGGL(k_exchange_lerp, dim3((unsigned)((g.n_lerp + 255) / 256)), dim3(256), 0, s, d, g, state);
-    if (g.n_total > g.first)
-        hipLaunchKernelGGL(k_exchange, dim3((unsigned)((g.n_total - g.first + 255) / 256)), dim3(256), 0, s, d, g,
-                           state);
+static void exchange32(const Dims &d, const DevGhosts &g, const DevFill &copy, bool faces, float *state,
+                       hipStream_t s) {
+    auto n = [&](const DevFill &f) { return faces ? f.n_face : f.n; };
+    const int nw = n(g.weighted), nl = n(g.lerp), nc = n(copy);
+    const unsigned wgs = (unsigned)((nw + 255) / 256 + (nl + 255) / 256 + (nc + 255) / 256);
+    if (wgs) hipLaunchKernelGGL(k_exchange_f32, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state);
 }
 
 void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s) {
-    exchange_with(d, g, g.copy, g.n_copy, state, s);
+    exchange32(d, g, g.copy, false, state, s);
 }
 
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, hipStream_t s) {
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s) {
     if (!g.pull) throw std::runtime_error("no pull table: use the full exchange");
-    exchange_with(d, g, g.copy_rest, g.n_copy_rest, state, s);
+    exchange32(d, g, g.copy_rest, faces, state, s);
 }
 
-void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, hipStream_t s) {
-    if (g.n <= 0) return;
-    const dim3 grid((unsigned)((g.n + 255) / 256)), wg(256);
-    if (psi) hipLaunchKernelGGL(k_exchange_f64<true>, grid, wg, 0, s, d, g, state, psi);
-    else hipLaunchKernelGGL(k_exchange_f64<false>, grid, wg, 0, s, d, g, state, psi);
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s) {
+    const int n = faces ? g.n_face : g.n;
+    if (n <= 0) return;
+    const dim3 grid((unsigned)((n + 255) / 256)), wg(256);
+    const int32_t *all = faces ? nullptr : g.all;
+    if (psi) hipLaunchKernelGGL(k_exchange_f64<true>, grid, wg, 0, s, d, g, all, n, state, psi);
+    else hipLaunchKernelGGL(k_exchange_f64<false>, grid, wg, 0, s, d, g, all, n, state, psi);
 }
 
 template <typename TS>
