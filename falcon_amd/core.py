@@ -253,7 +253,7 @@ class Shell:
         _check(self.L.falcon_set_state(self.h, ib, _p(u)))
 
     def get_state(self, ib):
-        out = np.zeros((8,) + self.pad[::-1])
+        out = np.empty((8,) + self.pad[::-1])
         _check(self.L.falcon_get_state(self.h, ib, _p(out)))
         return out
 
@@ -519,7 +519,7 @@ class HeatSolver:
         return it, rel, sec.value
 
     def get_T(self, sys=0):
-        out = np.zeros(self.shape[1:])
+        out = np.empty(self.shape[1:])
         _check(self.L.falcon_heat_get_T(self.s.h, sys, _p(out)))
         return out
 

@@ -184,6 +184,8 @@ void launch_copy_radial(const Dims &d, const DevBoundary &b, const TS *src, TS *
 void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile,
                        int nseg);
 void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile, int nseg);
+// nvar variables of one block ([nvar][P], cell_off layout) in Fortran order into pinned host memory
+void launch_block_to_host(const Dims &d, const double *src, int nvar, double *dst, hipStream_t s);
 void launch_to_f32(const double *src, float *dst, long long n, hipStream_t s);
 void launch_set_scalar(double *p, double v, hipStream_t s);
 // NaN scan of a padded state (see k_nan_scan): w[0] counts, w[1] first position;

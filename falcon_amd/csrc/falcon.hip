@@ -131,6 +131,7 @@ struct falcon_handle {
     DevBuf psi[2], psiS[2], glmG, glmC;
     DevBuf diffbuf;          // falcon_state_diff's reduction words
     DevBuf scanbuf;          // falcon_check_state's count and first position
+    double *pinned = nullptr;      // host staging of the block read-backs (read_block), made on first use
     int cur = 0;             // index of the current state buffer in U[]
     // validity of derived device data
     bool partials_valid = false;   // partial[] holds min(h/v_wave) of U[cur]
@@ -168,6 +169,7 @@ struct falcon_handle {
                          &U[0], &U[1], &F32[0], &F32[1], &S64[0], &S64[1], &S32[0], &S32[1], &dtp, &partial, &rbuf, &diffbuf, &scanbuf,
                          &psi[0], &psi[1], &psiS[0], &psiS[1], &glmG, &glmC};
         for (DevBuf *b : all) b->free();
+        if (pinned) (void)hipHostFree(pinned);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -196,7 +198,7 @@ struct falcon_handle {
 
 namespace {
 
-// host Fortran (i fastest) <-> device block variables (cell_off) for one block
+// host Fortran (i fastest) -> device block variables (cell_off) for one block
 void fortran_to_device(const double *src, double *dst, const Dims &d) {
     const size_t P = (size_t)d.P;
     for (int v = 0; v < 8; v++)
@@ -205,15 +207,6 @@ void fortran_to_device(const double *src, double *dst, const Dims &d) {
                 for (int I = 0; I < d.NI; I++)
                     dst[v * P + cell_off(d, I, J, K)] = src[v * P + (size_t)I + (size_t)d.NI * (J + (size_t)d.NJ * K)];
 }
-void device_to_fortran(const double *src, double *dst, const Dims &d) {
-    const size_t P = (size_t)d.P;
-    for (int v = 0; v < 8; v++)
-        for (int K = 0; K < d.NK; K++)
-            for (int J = 0; J < d.NJ; J++)
-                for (int I = 0; I < d.NI; I++)
-                    dst[v * P + (size_t)I + (size_t)d.NI * (J + (size_t)d.NJ * K)] = src[v * P + cell_off(d, I, J, K)];
-}
-
 // FP32 buffers of the deviation path: same-panel ghost entries whose weights
 // lie within 1e-12 of 0 or 1 (same-level neighbours whose cell centres
 // coincide up to rounding) are plain copies from the nearest donor cell;
@@ -779,6 +772,22 @@ void refresh_u_ghosts(falcon_handle *h) {
 
 void check_launch() { HIPCHECK(hipGetLastError()); }
 
+// nvar variables of one block to the caller in Fortran order: transposed by the
+// GPU into a pinned buffer that the handle keeps (at most 4 MB, or one variable
+// where that is more), then copied.  Synchronises the stream.
+void read_block(falcon_handle *h, const double *src, int nvar, double *dst) {
+    const size_t P = (size_t)h->dims.P;
+    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(8, (size_t)4194304 / (P * sizeof(double))));
+    if (!h->pinned) HIPCHECK(hipHostMalloc((void **)&h->pinned, sizeof(double) * P * chunk, hipHostMallocDefault));
+    for (int v = 0; v < nvar; v += chunk) {
+        const int n = std::min(chunk, nvar - v);
+        launch_block_to_host(h->dims, src + v * P, n, h->pinned, h->stream);
+        check_launch();
+        HIPCHECK(hipStreamSynchronize(h->stream));
+        std::memcpy(dst + v * P, h->pinned, sizeof(double) * P * n);
+    }
+}
+
 }  // namespace
 
 // host Fortran order (i fastest) <-> device [i][j][k] (k fastest) for m^3 blocks
@@ -1121,12 +1130,8 @@ int falcon_get_state(falcon_handle_t h, int ib, double *prim) {
         h->need_tables();
         h->check_block(ib);
         const size_t P = (size_t)h->dims.P;
-        std::vector<double> tmp(8 * P);
         if (h->dt.meta) refresh_u_ghosts(h);
-        HIPCHECK(hipStreamSynchronize(h->stream));
-        HIPCHECK(hipMemcpy(tmp.data(), h->U[h->cur].as<double>() + (size_t)ib * 8 * P, sizeof(double) * 8 * P,
-                           hipMemcpyDeviceToHost));
-        device_to_fortran(tmp.data(), prim, h->dims);
+        read_block(h, h->U[h->cur].as<double>() + (size_t)ib * 8 * P, 8, prim);
     });
 }
 
@@ -1176,15 +1181,7 @@ int falcon_get_psi(falcon_handle_t h, int ib, double *psi) {
         h->need_tables();
         h->check_block(ib);
         if (h->divb != 1) throw Error("psi is stepped only with GLM divergence cleaning (falcon_set_divb(h, 1))");
-        const Dims &d = h->dims;
-        std::vector<double> tmp((size_t)d.P);
-        HIPCHECK(hipStreamSynchronize(h->stream));
-        HIPCHECK(hipMemcpy(tmp.data(), h->psi[h->cur].as<double>() + (size_t)ib * d.P, sizeof(double) * d.P,
-                           hipMemcpyDeviceToHost));
-        for (int K = 0; K < d.NK; K++)
-            for (int J = 0; J < d.NJ; J++)
-                for (int I = 0; I < d.NI; I++)
-                    psi[(size_t)I + (size_t)d.NI * (J + (size_t)d.NJ * K)] = tmp[cell_off(d, I, J, K)];
+        read_block(h, h->psi[h->cur].as<double>() + (size_t)ib * (size_t)h->dims.P, 1, psi);
     });
 }
 
@@ -1880,14 +1877,9 @@ int falcon_pfss_set_magnetogram(falcon_handle_t h, const double *br) {
         const long long mm = (long long)m * m;
         h->pfss_br.assign(br, br + t.bottom.size() * mm);
         // b = Br S on the first radial cell of each bottom block (3_5/ModPFSS.f90:43-44)
-        std::vector<double> b(H.cells(), 0.0);
-        for (size_t q = 0; q < t.bottom.size(); q++)
-            for (int k = 0; k < m; k++)
-                for (int j = 0; j < m; j++) {
-                    const long long f = (long long)q * mm + (long long)k * m + j;
-                    b[(long long)t.bottom[q] * mm * m + (long long)j * m + k] = br[f] * t.area[f];
-                }
-        H.set_rhs(b);
+        std::vector<double> flux(h->pfss_br.size());
+        for (size_t f = 0; f < flux.size(); f++) flux[f] = br[f] * t.area[f];
+        H.set_rhs_bottom(t.bottom, flux);
     });
 }
 
@@ -1921,10 +1913,7 @@ int falcon_pfss_solve(falcon_handle_t h, double tol, int max_iter, int32_t *iter
 
 int falcon_pfss_get_phi(falcon_handle_t h, double *phi) {
     return guard([&] {
-        HeatSolver &H = need_pfss(h);
-        std::vector<double> dev;
-        H.get_solution(0, dev);
-        heat_to_host(dev.data(), phi, H.m(), (long long)dev.size() / ((long long)H.m() * H.m() * H.m()));
+        need_pfss(h).get_solution_host(0, phi);
     });
 }
 
@@ -1934,14 +1923,13 @@ int falcon_pfss_field(falcon_handle_t h, double *B) {
         const PfssTables &t = h->pfss;
         const int m = t.m, nb = h->lay.tree.nleaf;
         const long long mm = (long long)m * m;
-        std::vector<double> bot((size_t)nb * mm, 0.0), dev;
+        std::vector<double> bot((size_t)nb * mm, 0.0);
         for (size_t q = 0; q < t.bottom.size(); q++)
             for (int k = 0; k < m; k++)
                 for (int j = 0; j < m; j++)
                     bot[(long long)t.bottom[q] * mm + (long long)j * m + k] =
                         h->pfss_br[(long long)q * mm + (long long)k * m + j] * t.dr[t.bottom[q]];
-        H.pfss_field(bot, t.geo, dev);
-        heat_to_host(dev.data(), B, m, 3LL * nb);
+        H.pfss_field(bot, t.geo, B);
     });
 }
 
@@ -1974,10 +1962,7 @@ int falcon_heat_set_dt(falcon_handle_t h, const double *dt) {
 int falcon_heat_set_T(falcon_handle_t h, const double *T) {
     return guard([&] {
         HeatSolver &H = need_heat(h);
-        const long long n = H.cells() * H.nsys();
-        std::vector<double> dev(n);
-        heat_to_device(T, dev.data(), H.m(), n / ((long long)H.m() * H.m() * H.m()));
-        H.set_rhs_from_T(dev);
+        H.set_rhs_from_host_T(T);
     });
 }
 
@@ -2019,9 +2004,7 @@ int falcon_heat_get_T(falcon_handle_t h, int sys, double *T) {
     return guard([&] {
         HeatSolver &H = need_heat(h);
         if (sys < 0 || sys >= H.nsys()) throw Error("system index out of range");
-        std::vector<double> dev;
-        H.get_solution(sys, dev);
-        heat_to_host(dev.data(), T, H.m(), (long long)dev.size() / ((long long)H.m() * H.m() * H.m()));
+        H.get_solution_host(sys, T);
     });
 }
 

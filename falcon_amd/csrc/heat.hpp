@@ -62,10 +62,14 @@ class HeatSolver {
     void set_dt(const std::vector<double> &dt);
     void set_rhs_from_T(const std::vector<double> &T);   // system-major, per block [i][j][k]
     void set_rhs(const std::vector<double> &b);          // the right-hand side itself, same layout
-    // B = -grad(x) of system 0 at every finest-level cell, [block][3][i][j][k]
+    // the same from the caller's T: system-major, per block in Fortran order (i fastest)
+    void set_rhs_from_host_T(const double *T);
+    // b = flux (per bottom block, j fastest) on the first radial cells of the given blocks, 0 elsewhere
+    void set_rhs_bottom(const std::vector<int32_t> &bottom, const std::vector<double> &flux);
+    // B = -grad(x) of system 0 at every finest-level cell, [block][3][k][j][i]
     // (PFSS field; bot: per block and bottom-face cell (j, k) the ghost offset
     // Br dr of the domain's bottom, geo: see build_pfss_tables)
-    void pfss_field(const std::vector<double> &bot, const std::vector<double> &geo, std::vector<double> &B);
+    void pfss_field(const std::vector<double> &bot, const std::vector<double> &geo, double *B);
     void apply(const std::vector<double> &x, std::vector<double> &y);
     // z = M r, one V-cycle, system-major interior vectors (parity tests)
     void vcycle_host(const std::vector<double> &r, std::vector<double> &z);
@@ -73,7 +77,7 @@ class HeatSolver {
     // mode kSolvePlain / kSolveLearned (needs a corrector) / kSolveRecord (plain
     // FCG that appends training records to rec)
     HeatResult solve(double tol, int max_iter, int mode, HeatRecord *rec);
-    void get_solution(int s, std::vector<double> &T) const;
+    void get_solution_host(int s, double *T) const;      // per block in Fortran order (i fastest)
     void get_rhs(int s, std::vector<double> &b) const;
     void set_corrector(HeatCorrector *c);
     // finest-level smoothing sweeps of the V-cycle used with the learned
