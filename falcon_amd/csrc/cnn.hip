@@ -14,8 +14,8 @@
 // Layouts: images x/out [img][4096] float; activations and their gradients
 // [img][4096][16] bfloat16 (channel fastest); voxel v = (i*16 + j)*16 + k.
 // LDS planes: x [18][18] with a zero halo; forward activations [16][16][16]
-// (k-shifts by DPP, out-of-block lines skipped); gradient kernels [18][18][16]
-// with a zero halo.
+// (k-shifts by DPP, out-of-block lines skipped); the gradient kernels' carves are
+// described there.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,8 +46,8 @@ namespace {
 constexpr int PL = 18 * 18;                 // plane with halo
 constexpr int OFF_W1 = 0, OFF_B1 = 432, OFF_W2 = 448, OFF_B2 = 7360, OFF_W3 = 7376, OFF_B3 = 7808;
 // packed operand images of the 16x16x32 form, 64 lanes x 8 bf16 per MFMA step:
-// P1 layer-1 forward (1 step), Q3 layer-3 data gradient (1), Q2 layer-2 data gradient (14)
-constexpr int PK_P1 = 0, PK_Q3 = 64, PK_Q2 = 128, PK_TOTAL = PK_Q2 + 14 * 64;
+// Q3 layer-3 data gradient (1 step), Q2 layer-2 data gradient (14)
+constexpr int PK_Q3 = 0, PK_Q2 = 64, PK_TOTAL = PK_Q2 + 14 * 64;
 
 // forward operand images (bf16 elements, lane-major):
 //   L1  [3 di][64] x 4: 16x16x16 A, rows co, K = the 9 (dj,dk) taps of plane offset di
@@ -63,8 +63,6 @@ constexpr int PF_L1 = 0, PF_L2A = PF_L1 + 3 * 64 * 4, PF_L2B = PF_L2A + 9 * 64 *
 constexpr int HGRP = 18 * 4, HROW = 4 * HGRP, HPL = 18 * HROW;
 constexpr int kFwdWaves = 8;                // wavefronts per image (16 / kFwdWaves k-lines each)
 constexpr int F_H1 = 0, F_H2 = 3 * HPL, F_X = 6 * HPL, F_TOTAL = F_X + 3 * PL;
-// single-layer LDS carve: ring of 3 input planes + zero plane
-constexpr int S_IN = 0, S_Z = 3 * PL * 16, S_TOTAL = 4 * PL * 16;
 
 __device__ __forceinline__ uint16_t f2bf(float f) {
     uint32_t u = __float_as_uint(f);
@@ -87,26 +85,24 @@ __device__ __forceinline__ uint32_t shr1(uint32_t v) { return (uint32_t)__builti
 __device__ __forceinline__ uint32_t shl1(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xf, 0xf, false); }
 __device__ __forceinline__ float shr1f(float v) { return __uint_as_float(shr1(__float_as_uint(v))); }
 __device__ __forceinline__ float shl1f(float v) { return __uint_as_float(shl1(__float_as_uint(v))); }
-__device__ __forceinline__ void tap_off(int t, int &di, int &dj, int &dk) {
-    di = t / 9 - 1;
-    dj = (t / 3) % 3 - 1;
-    dk = t % 3 - 1;
-}
 __device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
     return make_uint2((uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16), (uint32_t)f2bf(c) | ((uint32_t)f2bf(d) << 16));
 }
 __device__ __forceinline__ float relu(float a) { return a > 0.0f ? a : 0.0f; }
 
 // ------------------------------------------------------------------ packing
+// the gradient images, then the forward images, in one launch
+__device__ __forceinline__ void pack_forward(const float *__restrict__ p, uint16_t *__restrict__ pk, int q);
+
 __global__ void __launch_bounds__(256) k_cnn_pack(const float *__restrict__ p, uint16_t *__restrict__ pk) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= PK_TOTAL * 8) return;
+    if (q >= PK_TOTAL * 8) {
+        pack_forward(p, pk + PK_TOTAL * 8, q - PK_TOTAL * 8);
+        return;
+    }
     const int e = q & 7, entry = q >> 3, lane = entry & 63, row = lane & 15, g = lane >> 4;
     float w = 0.0f;
-    if (entry < PK_Q3) {                                   // P1: k = tap, row = co
-        const int t = 8 * g + e;
-        if (t < 27) w = p[OFF_W1 + t * 16 + row];
-    } else if (entry < PK_Q2) {                            // Q3: k = tap (flipped), row = ci of layer 3
+    if (entry < PK_Q2) {                            // Q3: k = tap (flipped), row = ci of layer 3
         const int t = 8 * g + e;
         if (t < 27) w = p[OFF_W3 + (26 - t) * 16 + row];
     } else {                                               // Q2: k = (t flipped, co), row = ci of layer 2
@@ -116,8 +112,7 @@ __global__ void __launch_bounds__(256) k_cnn_pack(const float *__restrict__ p, u
     pk[q] = f2bf(w);
 }
 
-__global__ void __launch_bounds__(256) k_cnn_packf(const float *__restrict__ p, uint16_t *__restrict__ pk) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pack_forward(const float *__restrict__ p, uint16_t *__restrict__ pk, int q) {
     if (q >= PF_TOTAL) return;
     float w = 0.0f;
     if (q < PF_L2A) {                                      // L1: W1[t = 9 di + s][co]
@@ -180,7 +175,8 @@ __device__ __forceinline__ f4 mfma32(uint4 a, uint4 b, f4 c) {
 template <bool STORE, bool HEAT, int NW>
 __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x, float *__restrict__ out,
                                                  const uint16_t *__restrict__ pf, const float *__restrict__ prm,
-                                                 uint16_t *__restrict__ h1g, uint16_t *__restrict__ h2g, HeatIO hio) {
+                                                 uint16_t *__restrict__ h1g, uint16_t *__restrict__ h2g, HeatIO hio,
+                                                 const long long *__restrict__ idx) {
     __shared__ __align__(16) uint16_t sm[F_TOTAL];
     const long long img = blockIdx.x;
     double sc = 1.0;
@@ -232,7 +228,7 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
     // and the 4 channels 4g .. 4g+3 at k
     const int oA = (2 * (g & 1)) * HGRP + (g < 2 ? n : n + 2) * 4;
     const int oB = g * HGRP + (n + 1) * 4;
-    const float *X = x + img * 4096;
+    const float *X = x + (STORE && idx ? idx[img] : img) * 4096;   // idx: the batch's images of a training set
     __syncthreads();
 
     // Planes -1 and 16 (the block's zero padding in i) are ring slots holding
@@ -378,81 +374,114 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
 
 // ------------------------------------------------------------------ data gradients
 // gout[v][c] = (mask[v][c] > 0) ? sum_{t,ci} Wq[t][ci][c] gin[v + off_t][ci] : 0, stored as bfloat16.
-// CIN = 1: gin is the float output gradient (layer 3, weights Q3); CIN = 16: gin is
-// the bfloat16 layer-2 output gradient (weights Q2).
-template <int CIN>
-__global__ void __launch_bounds__(256) k_cnn_dgrad(const void *__restrict__ gin_, const uint16_t *__restrict__ mask,
-                                                   uint16_t *__restrict__ gout, const us8 *__restrict__ pk) {
-    __shared__ __align__(16) uint16_t sm[S_TOTAL];
+// A workgroup takes 4 i-planes of an image (blockIdx.y), one per wavefront, and
+// stages them with a halo once: 4 workgroups per image fill the chip at the
+// training batches (128 images, 256 CUs), and no barrier follows the staging.
+constexpr int DPL = 4;                      // output planes per workgroup
+
+// Layer 3 -> 2 (gin: the float output gradient, weights Q3): one MFMA per
+// k-line, K = the 27 taps.  Bound by the LDS gather of the taps; their offsets
+// are formed once per lane, a line's row is an immediate.  128
+// images: 48 -> 11.5 us against one workgroup per image with the offsets formed per read.
+__global__ void __launch_bounds__(256) k_cnn_dgrad1(const float *__restrict__ gin, const uint16_t *__restrict__ mask,
+                                                    uint16_t *__restrict__ gout, const us8 *__restrict__ pk) {
+    __shared__ __align__(16) uint16_t sm[(DPL + 2) * PL];
     const long long img = blockIdx.x;
+    const int p0 = blockIdx.y * DPL;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, kk = lane & 15;
-    constexpr int S = CIN == 1 ? 1 : 14;
-    constexpr int STRIDE = CIN == 1 ? 1 : 16;   // elements per voxel in an LDS plane
-    for (int q = tid; q < S_TOTAL / 2; q += 256) reinterpret_cast<uint32_t *>(sm)[q] = 0u;
-    us8 w[S];
+    float v[DPL + 2];
 #pragma unroll
-    for (int s = 0; s < S; s++) w[s] = pk[(CIN == 1 ? PK_Q3 : PK_Q2) + s * 64 + lane];
+    for (int q = 0; q < DPL + 2; q++) {
+        const int i = p0 - 1 + q;
+        v[q] = i >= 0 && i < 16 ? gin[img * 4096 + i * 256 + tid] : 0.0f;
+    }
+    const us8 w = pk[PK_Q3 + lane];
+    for (int q = tid; q < (DPL + 2) * PL / 2; q += 256) reinterpret_cast<uint32_t *>(sm)[q] = 0u;
     __syncthreads();
+#pragma unroll
+    for (int q = 0; q < DPL + 2; q++) sm[q * PL + ((tid >> 4) + 1) * 18 + (tid & 15) + 1] = f2bf(v[q]);
+    __syncthreads();
+    const uint16_t *src[8];
+    bool on[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int t = 8 * g + e;
+        on[e] = t < 27;
+        src[e] = sm + (on[e] ? (wave + t / 9) * PL + (t / 3) % 3 * 18 + t % 3 + kk : 0);
+    }
+    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        us8 b;
+#pragma unroll
+        for (int e = 0; e < 8; e++) b[e] = on[e] ? src[e][j * 18] : (uint16_t)0;
+        const f4 acc = mfma(w, b, f4{0.0f, 0.0f, 0.0f, 0.0f});
+        const uint2 mk = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
+        const float m0 = bf2f((uint16_t)(mk.x & 0xffffu)), m1 = bf2f((uint16_t)(mk.x >> 16)),
+                    m2 = bf2f((uint16_t)(mk.y & 0xffffu)), m3 = bf2f((uint16_t)(mk.y >> 16));
+        *reinterpret_cast<uint2 *>(gout + o0 + j * 256) = pack4(m0 > 0.0f ? acc[0] : 0.0f, m1 > 0.0f ? acc[1] : 0.0f,
+                                                                m2 > 0.0f ? acc[2] : 0.0f, m3 > 0.0f ? acc[3] : 0.0f);
+    }
+}
 
-    auto load = [&](int q) {
-        const int j = tid >> 4, k = tid & 15;
-        const long long v = img * 4096 + (q * 16 + j) * 16 + k;
-        uint16_t *dst = sm + S_IN + (q % 3) * PL * STRIDE + ((j + 1) * 18 + k + 1) * STRIDE;
-        if (CIN == 1) {
-            dst[0] = f2bf(reinterpret_cast<const float *>(gin_)[v]);
-        } else {
-            const uint4 *src = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(gin_) + v * 16);
-            reinterpret_cast<uint4 *>(dst)[0] = src[0];
-            reinterpret_cast<uint4 *>(dst)[1] = src[1];
+// Layer 2 -> 1 (gin: the bfloat16 layer-2 output gradient, weights Q2): 14
+// MFMAs per k-line in one chain, K = (tap pair, channel).  LDS [plane][channel
+// half][18][18][8]: the lanes of a 16-byte read are consecutive (no bank
+// conflicts); bound by those reads, 14 per line and wavefront.  128
+// images: 53 -> 14.7 us against one workgroup per image on [voxel][16] planes.
+__global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict__ gin, const uint16_t *__restrict__ mask,
+                                                     uint16_t *__restrict__ gout, const us8 *__restrict__ pk) {
+    constexpr int HP = PL * 8;              // elements per half plane
+    __shared__ __align__(16) uint16_t sm[(DPL + 2) * 2 * HP];
+    const long long img = blockIdx.x;
+    const int p0 = blockIdx.y * DPL;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, kk = lane & 15;
+    uint4 v[DPL + 2][2];
+#pragma unroll
+    for (int q = 0; q < DPL + 2; q++) {
+        const int i = p0 - 1 + q;
+        const uint4 *src = reinterpret_cast<const uint4 *>(gin + (img * 4096 + (long long)i * 256) * 16);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            v[q][h] = i >= 0 && i < 16 ? src[h * 256 + tid] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    us8 w[14];
+#pragma unroll
+    for (int s = 0; s < 14; s++) w[s] = pk[PK_Q2 + s * 64 + lane];
+    for (int q = tid; q < (DPL + 2) * 2 * PL; q += 256) reinterpret_cast<uint4 *>(sm)[q] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < DPL + 2; q++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            // element h * 256 + tid of the plane: voxel e >> 1, channel half e & 1
+            const int e = h * 256 + tid, vx = e >> 1;
+            *reinterpret_cast<uint4 *>(sm + (q * 2 + (e & 1)) * HP + (((vx >> 4) + 1) * 18 + (vx & 15) + 1) * 8) = v[q][h];
         }
-    };
-    auto plane = [&](int q) -> const uint16_t * {
-        return (q < 0 || q > 15) ? sm + S_Z : sm + S_IN + (q % 3) * PL * STRIDE;
-    };
-
-    load(0);
-    for (int p = 0; p <= 15; p++) {
-        if (p + 1 <= 15) load(p + 1);
-        __syncthreads();
+    __syncthreads();
+    // slot s of this lane is tap 2 s + (g >> 1) (27: none)
+    int off[14];
 #pragma unroll
-        for (int jl = 0; jl < 4; jl++) {
-            const int j = wave + 4 * jl;
-            f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (CIN == 1) {
-                us8 b;
+    for (int s = 0; s < 14; s++) {
+        const int t = 2 * s + (g >> 1), u = t < 27 ? t : 0;
+        off[s] = ((wave + u / 9) * 2 + (g & 1)) * HP + ((u / 3) % 3 * 18 + u % 3 + kk) * 8;
+    }
+    const bool last = g < 2;
+    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
+#pragma unroll 4
+    for (int j = 0; j < 16; j++) {
+        const uint2 mk = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int t = 8 * g + e;
-                    uint16_t val = 0;
-                    if (t < 27) {
-                        int di, dj, dk;
-                        tap_off(t, di, dj, dk);
-                        val = plane(p + di)[(j + dj + 1) * 18 + kk + dk + 1];
-                    }
-                    b[e] = val;
-                }
-                acc = mfma(w[0], b, acc);
-            } else {
-#pragma unroll
-                for (int s = 0; s < S; s++) {
-                    const int t = 2 * s + (g >> 1);
-                    const uint16_t *src = sm + S_Z;
-                    if (t < 27) {
-                        int di, dj, dk;
-                        tap_off(t, di, dj, dk);
-                        src = plane(p + di) + ((j + dj + 1) * 18 + kk + dk + 1) * 16 + 8 * (g & 1);
-                    }
-                    acc = mfma(w[s], *reinterpret_cast<const us8 *>(src), acc);
-                }
-            }
-            const long long o = (img * 4096 + (p * 16 + j) * 16 + kk) * 16 + 4 * g;
-            const uint2 mk = *reinterpret_cast<const uint2 *>(mask + o);
-            const float m0 = bf2f((uint16_t)(mk.x & 0xffffu)), m1 = bf2f((uint16_t)(mk.x >> 16)),
-                        m2 = bf2f((uint16_t)(mk.y & 0xffffu)), m3 = bf2f((uint16_t)(mk.y >> 16));
-            *reinterpret_cast<uint2 *>(gout + o) = pack4(m0 > 0.0f ? acc[0] : 0.0f, m1 > 0.0f ? acc[1] : 0.0f,
-                                                         m2 > 0.0f ? acc[2] : 0.0f, m3 > 0.0f ? acc[3] : 0.0f);
+        for (int s = 0; s < 14; s++) {
+            uint4 b = *reinterpret_cast<const uint4 *>(sm + off[s] + j * 144);
+            if (s == 13) b = last ? b : make_uint4(0u, 0u, 0u, 0u);
+            acc = mfma(w[s], __builtin_bit_cast(us8, b), acc);
         }
-        __syncthreads();
+        const float m0 = bf2f((uint16_t)(mk.x & 0xffffu)), m1 = bf2f((uint16_t)(mk.x >> 16)),
+                    m2 = bf2f((uint16_t)(mk.y & 0xffffu)), m3 = bf2f((uint16_t)(mk.y >> 16));
+        *reinterpret_cast<uint2 *>(gout + o0 + j * 256) = pack4(m0 > 0.0f ? acc[0] : 0.0f, m1 > 0.0f ? acc[1] : 0.0f,
+                                                                m2 > 0.0f ? acc[2] : 0.0f, m3 > 0.0f ? acc[3] : 0.0f);
     }
 }
 
@@ -462,155 +491,275 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad(const void *__restrict__ gin_
 //   L = 2: dW2[t][ci][co] = sum_v h1[v+t][ci] g2[v][co]
 //   L = 1: dW1[t][co] = sum_v x[v+t] g1[v][co]        (in = x float)
 // and the bias gradient of the layer, sum_v g[v][co].
-// D[co][n] = sum over 32-voxel chunks of A[co][voxel] B[voxel][n]; n = ci
-// (L = 2, 3; taps spread over the 4 waves) or n = tap (L = 1; wave w < 2 holds
-// taps 16w .. 16w+15).
+// D[co][n] = sum over 32-voxel chunks (2 k-lines, in the order of the planes)
+// of A[co][voxel] B[voxel][n]; n = ci of one tap (L = 2, 3) or n = tap (L = 1).
+// An MFMA lane needs 8 consecutive voxels of one channel, the activations are
+// channel-fastest: the planes are turned on their way into LDS ([channel][j][k],
+// 4 voxels x 4 channels per lane), so an operand is one 16-byte read; gathering
+// it 2 bytes at a time bound the three passes before: 221 us for 128 images, this
+// one 47 us (37 images 211 -> 27 us).
+// Layers 2 and 3: a workgroup takes the 9 taps of one plane offset di, wavefront
+// w < 3 the 3 taps of dj = w - 1, whose operands are one row read and its
+// shifts by one voxel in registers (v_alignbit); planes are double-buffered,
+// one barrier each.  Layer 1: x with a halo in 3 copies shifted in k (every
+// tap's 8 voxels aligned), wavefront w < 2 holds taps 16w .. 16w+15.  All in
+// one launch: blockIdx.y = 0 .. 2 layer 2, 3 .. 5 layer 3, 6 layer 1, so a
+// small batch still spreads over 7 workgroups per image.
+constexpr int WA_CH = 16 * 16 + 8, WA_PL = 16 * WA_CH;           // g planes: rows of 16, channels 528 bytes apart
+constexpr int WB_ROW = 24, WB_CH = 18 * WB_ROW + 8, WB_PL = 16 * WB_CH;   // input planes: 8 zeros, 16 voxels; channels 880 bytes apart
+constexpr int WX_CP = 18 * 18 * 16;                              // one shifted copy of x
+constexpr int W_TOTAL = 3 * WX_CP + 2 * WA_PL > 2 * (WA_PL + WB_PL) ? 3 * WX_CP + 2 * WA_PL : 2 * (WA_PL + WB_PL);
+
+struct Quad {                               // 4 voxels x 4 channels
+    uint2 v[4];
+    __device__ __forceinline__ void load(const uint16_t *src, int plane, int tid) {
+        const uint16_t *p = src + ((plane * 64 + (tid >> 2)) * 4) * 16 + 4 * (tid & 3);
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const uint2 *>(p + u * 16);
+    }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = make_uint2(0u, 0u);
+    }
+    // channel c of the 4 as its 4 voxels, channels `stride` elements apart
+    __device__ __forceinline__ void store(uint16_t *dst, int stride) const {
+        const uint32_t lo = 0xffffu, hi = 0xffff0000u;
+        *reinterpret_cast<uint2 *>(dst) = make_uint2((v[0].x & lo) | (v[1].x << 16), (v[2].x & lo) | (v[3].x << 16));
+        *reinterpret_cast<uint2 *>(dst + stride) = make_uint2((v[0].x >> 16) | (v[1].x & hi), (v[2].x >> 16) | (v[3].x & hi));
+        *reinterpret_cast<uint2 *>(dst + 2 * stride) = make_uint2((v[0].y & lo) | (v[1].y << 16), (v[2].y & lo) | (v[3].y << 16));
+        *reinterpret_cast<uint2 *>(dst + 3 * stride) = make_uint2((v[0].y >> 16) | (v[1].y & hi), (v[2].y >> 16) | (v[3].y & hi));
+    }
+};
+
+// sum of a row of 16 bf16 voxels onto s, in order
+__device__ __forceinline__ float row_sum(const uint16_t *row, float s) {
+    const uint4 a = reinterpret_cast<const uint4 *>(row)[0], b = reinterpret_cast<const uint4 *>(row)[1];
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        s += __uint_as_float(w[k] << 16);
+        s += __uint_as_float(w[k] & 0xffff0000u);
+    }
+    return s;
+}
+
 template <int L>
-__global__ void __launch_bounds__(256) k_cnn_wgrad(const void *__restrict__ in_, const void *__restrict__ g_,
-                                                   float *__restrict__ part) {
-    constexpr int ISTR = L == 1 ? 1 : 16;       // input elements per voxel
-    constexpr int GCH = L == 3 ? 1 : 16;        // gradient channels
-    __shared__ __align__(16) uint16_t sIn[4 * PL * ISTR];   // ring of 3 + zero plane
-    __shared__ __align__(16) uint16_t sG[256 * GCH];        // gradient plane, [j][k][c]
-    __shared__ float sBias[16][16];
-    const long long img = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
-    for (int q = tid; q < 4 * PL * ISTR / 2; q += 256) reinterpret_cast<uint32_t *>(sIn)[q] = 0u;
-    const uint16_t *zp = sIn + 3 * PL * ISTR;
-
-    auto load_in = [&](int q) {
-        const int j = tid >> 4, k = tid & 15;
-        const long long v = img * 4096 + (q * 16 + j) * 16 + k;
-        uint16_t *dst = sIn + (q % 3) * PL * ISTR + ((j + 1) * 18 + k + 1) * ISTR;
-        if (L == 1) {
-            dst[0] = f2bf(reinterpret_cast<const float *>(in_)[v]);
-        } else {
-            const uint4 *src = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(in_) + v * 16);
-            reinterpret_cast<uint4 *>(dst)[0] = src[0];
-            reinterpret_cast<uint4 *>(dst)[1] = src[1];
-        }
+__device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, const void *__restrict__ g_, int di,
+                                           float *__restrict__ P, uint16_t *sm, float (*sBias)[16], float *sF) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
+              n = lane & 15;
+    const int vg = tid >> 2, j4 = vg >> 2, k4 = 4 * (vg & 3), c4 = 4 * (tid & 3);
+    for (int q = tid; q < 2 * (WA_PL + WB_PL) / 8; q += 256) reinterpret_cast<uint4 *>(sm)[q] = make_uint4(0u, 0u, 0u, 0u);
+    Quad qa, qb;
+    float gf = 0.0f;
+    auto fetch = [&](int p) {
+        if (L == 2) qa.load(reinterpret_cast<const uint16_t *>(g_), p, tid);
+        else gf = reinterpret_cast<const float *>(g_)[p * 256 + tid];
+        const int q = p + di;
+        if (q >= 0 && q < 16) qb.load(in, q, tid);
+        else qb.clear();
     };
-    auto plane = [&](int q) -> const uint16_t * { return (q < 0 || q > 15) ? zp : sIn + (q % 3) * PL * ISTR; };
-
-    f4 acc[7];
+    auto stage = [&](int p) {
+        uint16_t *A = sm + (p & 1) * (WA_PL + WB_PL), *B = A + WA_PL;
+        if (L == 2) {
+            qa.store(A + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+        } else {
+            A[tid] = f2bf(gf);
+            sF[(p & 1) * 256 + tid] = gf;
+        }
+        qb.store(B + c4 * WB_CH + (j4 + 1) * WB_ROW + 8 + k4, WB_CH);
+    };
+    f4 acc[3];
 #pragma unroll
-    for (int a = 0; a < 7; a++) acc[a] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int a = 0; a < 3; a++) acc[a] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float bias_acc = 0.0f;    // thread tid: channel tid & 15, voxels of its plane rows (tid >> 4)
+    fetch(0);
     __syncthreads();
-    load_in(0);
-    for (int p = 0; p <= 15; p++) {
-        if (p + 1 <= 15) load_in(p + 1);
-        {   // gradient plane p
-            const int j = tid >> 4, k = tid & 15;
-            const long long v = img * 4096 + (p * 16 + j) * 16 + k;
-            if (L == 3) {
-                sG[tid] = f2bf(reinterpret_cast<const float *>(g_)[v]);
-            } else {
-                const uint4 *src = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(g_) + v * 16);
-                reinterpret_cast<uint4 *>(sG + tid * 16)[0] = src[0];
-                reinterpret_cast<uint4 *>(sG + tid * 16)[1] = src[1];
-            }
-        }
+    stage(0);
+    for (int p = 0; p < 16; p++) {
         __syncthreads();
-        {   // bias: thread (c = tid & 15, row = tid >> 4) sums its row of 16 voxels
+        if (p + 1 < 16) fetch(p + 1);
+        const uint16_t *A = sm + (p & 1) * (WA_PL + WB_PL), *B = A + WA_PL;
+        if (di == 0) {
             const int c = tid & 15, jr = tid >> 4;
-            if (L == 3) {
-                if (c == 0)
-                    for (int k = 0; k < 16; k++) bias_acc += reinterpret_cast<const float *>(g_)[img * 4096 + (p * 16 + jr) * 16 + k];
-            } else {
-                for (int k = 0; k < 16; k++) bias_acc += bf2f(sG[(jr * 16 + k) * 16 + c]);
-            }
-        }
-#pragma unroll 1
-        for (int ch = 0; ch < 8; ch++) {          // 32-voxel chunk: lines 2ch, 2ch+1
-            const int jj = 2 * ch + (g >> 1), k0 = 8 * (g & 1);
-            us8 a;                                 // A[co = n][voxels 8g..8g+7]
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int vv = jj * 16 + k0 + e;
-                a[e] = (L == 3) ? (n == 0 ? sG[vv] : (uint16_t)0) : sG[vv * 16 + n];
-            }
-            if (L == 1) {
-                if (wave < 2) {
-                    const int t = 16 * wave + n;
-                    us8 b;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        uint16_t val = 0;
-                        if (t < 27) {
-                            int di, dj, dk;
-                            tap_off(t, di, dj, dk);
-                            val = plane(p + di)[(jj + dj + 1) * 18 + k0 + e + dk + 1];
-                        }
-                        b[e] = val;
-                    }
-                    acc[0] = mfma(a, b, acc[0]);
-                }
-            } else {
-#pragma unroll
-                for (int a7 = 0; a7 < 7; a7++) {
-                    const int t = wave + 4 * a7;
-                    if (t < 27) {
-                        int di, dj, dk;
-                        tap_off(t, di, dj, dk);
-                        const uint16_t *P = plane(p + di);
-                        us8 b;
-#pragma unroll
-                        for (int e = 0; e < 8; e++) b[e] = P[((jj + dj + 1) * 18 + k0 + e + dk + 1) * 16 + n];
-                        acc[a7] = mfma(a, b, acc[a7]);
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    float *P = part + img * (long long)kCnnParams;
-    // D[co = 4g + r][n]
-    if (L == 1) {
-        if (wave < 2) {
-            const int t = 16 * wave + n;
-            if (t < 27)
-                for (int r = 0; r < 4; r++) P[OFF_W1 + t * 16 + 4 * g + r] = acc[0][r];
-        }
-    } else {
-        for (int a7 = 0; a7 < 7; a7++) {
-            const int t = wave + 4 * a7;
-            if (t >= 27) continue;
             if (L == 2) {
-                for (int r = 0; r < 4; r++) P[OFF_W2 + (t * 16 + n) * 16 + 4 * g + r] = acc[a7][r];
+                bias_acc = row_sum(A + c * WA_CH + jr * 16, bias_acc);
+            } else if (c == 0) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) bias_acc += sF[(p & 1) * 256 + jr * 16 + k];
+            }
+        }
+        if (wave < 3) {
+#pragma unroll
+            for (int ch = 0; ch < 8; ch++) {
+                const int jj = 2 * ch + (g >> 1), k0 = 8 * (g & 1);
+                uint4 a;
+                if (L == 2) {
+                    a = *reinterpret_cast<const uint4 *>(A + n * WA_CH + jj * 16 + k0);
+                } else {
+                    a = *reinterpret_cast<const uint4 *>(A + jj * 16 + k0);
+                    if (n != 0) a = make_uint4(0u, 0u, 0u, 0u);
+                }
+                const uint16_t *row = B + n * WB_CH + (jj + wave) * WB_ROW + 8 + k0;
+                const uint4 b = *reinterpret_cast<const uint4 *>(row);
+                const uint32_t pv = *reinterpret_cast<const uint32_t *>(row - 2), nx = *reinterpret_cast<const uint32_t *>(row + 8);
+                const uint32_t s1 = __builtin_amdgcn_alignbit(b.y, b.x, 16), s2 = __builtin_amdgcn_alignbit(b.z, b.y, 16),
+                               s3 = __builtin_amdgcn_alignbit(b.w, b.z, 16);
+                acc[0] = mfma32(a, make_uint4(__builtin_amdgcn_alignbit(b.x, pv, 16), s1, s2, s3), acc[0]);
+                acc[1] = mfma32(a, b, acc[1]);
+                acc[2] = mfma32(a, make_uint4(s1, s2, s3, __builtin_amdgcn_alignbit(nx, b.w, 16)), acc[2]);
+            }
+        }
+        if (p + 1 < 16) stage(p + 1);
+    }
+    // D[co = 4g + r][n]
+    if (wave < 3) {
+#pragma unroll
+        for (int dk = 0; dk < 3; dk++) {
+            const int t = (di + 1) * 9 + wave * 3 + dk;
+            if (L == 2) {
+                for (int r = 0; r < 4; r++) P[OFF_W2 + (t * 16 + n) * 16 + 4 * g + r] = acc[dk][r];
             } else if (g == 0) {
-                P[OFF_W3 + t * 16 + n] = acc[a7][0];
+                P[OFF_W3 + t * 16 + n] = acc[dk][0];
             }
         }
     }
+    if (di == 0) {
+        sBias[tid >> 4][tid & 15] = bias_acc;
+        __syncthreads();
+        if (tid < 16) {
+            float s = 0.0f;
+            for (int r = 0; r < 16; r++) s += sBias[r][tid];
+            if (L == 2) P[OFF_B2 + tid] = s;
+            else if (tid == 0) P[OFF_B3] = s;
+        }
+    }
+}
+
+__device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const uint16_t *__restrict__ g1,
+                                            float *__restrict__ P, uint16_t *sm, float (*sBias)[16]) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
+              n = lane & 15;
+    const int vg = tid >> 2, j4 = vg >> 2, k4 = 4 * (vg & 3), c4 = 4 * (tid & 3);
+    uint16_t *xs = sm + 2 * WA_PL;
+    float xv[16];
+#pragma unroll
+    for (int p = 0; p < 16; p++) xv[p] = x[p * 256 + tid];
+    for (int q = tid; q < 3 * WX_CP / 8; q += 256) reinterpret_cast<uint4 *>(xs)[q] = make_uint4(0u, 0u, 0u, 0u);
+    Quad qa;
+    qa.load(g1, 0, tid);
+    __syncthreads();
+    // copy dk + 1, row (plane + 1, j + 1): element k holds x at k + dk
+#pragma unroll
+    for (int p = 0; p < 16; p++) {
+        const uint16_t v = f2bf(xv[p]);
+        uint16_t *row = xs + ((p + 1) * 18 + (tid >> 4) + 1) * 16;
+        const int k = tid & 15;
+        if (k < 15) row[k + 1] = v;
+        row[WX_CP + k] = v;
+        if (k > 0) row[2 * WX_CP + k - 1] = v;
+    }
+    qa.store(sm + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+    const int t = 16 * wave + n;
+    const bool on = t < 27;
+    const int u = on ? t : 0;
+    const uint16_t *src = xs + (u % 3) * WX_CP + ((u / 9) * 18 + (u / 3) % 3) * 16;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float bias_acc = 0.0f;
+    for (int p = 0; p < 16; p++) {
+        __syncthreads();
+        if (p + 1 < 16) qa.load(g1, p + 1, tid);
+        const uint16_t *A = sm + (p & 1) * WA_PL;
+        bias_acc = row_sum(A + (tid & 15) * WA_CH + (tid >> 4) * 16, bias_acc);
+        if (wave < 2) {
+#pragma unroll
+            for (int ch = 0; ch < 8; ch++) {
+                const int jj = 2 * ch + (g >> 1), k0 = 8 * (g & 1);
+                const uint4 a = *reinterpret_cast<const uint4 *>(A + n * WA_CH + jj * 16 + k0);
+                uint4 b = *reinterpret_cast<const uint4 *>(src + (p * 18 + jj) * 16 + k0);
+                if (!on) b = make_uint4(0u, 0u, 0u, 0u);
+                acc = mfma32(a, b, acc);
+            }
+        }
+        if (p + 1 < 16) qa.store(sm + ((p + 1) & 1) * WA_PL + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+    }
+    if (wave < 2 && on)
+        for (int r = 0; r < 4; r++) P[OFF_W1 + t * 16 + 4 * g + r] = acc[r];
     sBias[tid >> 4][tid & 15] = bias_acc;
     __syncthreads();
     if (tid < 16) {
         float s = 0.0f;
         for (int r = 0; r < 16; r++) s += sBias[r][tid];
-        if (L == 1) P[OFF_B1 + tid] = s;
-        else if (L == 2) P[OFF_B2 + tid] = s;
-        else if (tid == 0) P[OFF_B3] = s;
+        P[OFF_B1 + tid] = s;
     }
 }
 
-// grad[q] = sum over images of part[img][q], fixed order, FP64
-__global__ void __launch_bounds__(256) k_cnn_reduce(const float *__restrict__ part, int nimg, double *__restrict__ grad) {
+__global__ void __launch_bounds__(256) k_cnn_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ h1,
+                                                   const uint16_t *__restrict__ h2, const uint16_t *__restrict__ g1,
+                                                   const uint16_t *__restrict__ g2, const float *__restrict__ g3,
+                                                   float *__restrict__ part, const long long *__restrict__ idx) {
+    __shared__ __align__(16) uint16_t sm[W_TOTAL];
+    __shared__ float sBias[16][16], sF[512];
+    const long long img = blockIdx.x, v = img * 4096;
+    const int job = blockIdx.y;
+    float *P = part + img * (long long)kCnnParams;
+    if (job < 3) wgrad_taps<2>(h1 + v * 16, g2 + v * 16, job - 1, P, sm, sBias, sF);
+    else if (job < 6) wgrad_taps<3>(h2 + v * 16, g3 + v, job - 4, P, sm, sBias, sF);
+    else wgrad_first(x + (idx ? idx[img] : img) * 4096, g1 + v * 16, P, sm, sBias);
+}
+
+// grad[q] = sum over images of part[img][q], fixed order, FP64, 16 images in
+// flight (the additions keep their order, the loads do not wait for them)
+__device__ __forceinline__ double part_sum(const float *__restrict__ part, int nimg, int q) {
+    double s = 0.0;
+    for (int i0 = 0; i0 < nimg; i0 += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = i0 + i < nimg ? part[(long long)(i0 + i) * kCnnParams + q] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (i0 + i < nimg) s += (double)v[i];
+    }
+    return s;
+}
+__global__ void __launch_bounds__(64) k_cnn_reduce(const float *__restrict__ part, int nimg, double *__restrict__ grad) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < kCnnParams) grad[q] = part_sum(part, nimg, q);
+}
+
+// end of a training step: the gradient sums go straight into Adam's update;
+// one more workgroup adds the batch's loss partials (x scale x weight) to
+// loss[0], which `first` starts
+__global__ void __launch_bounds__(64) k_cnn_update(const float *__restrict__ part, int nimg, float *__restrict__ p,
+                                                   float *__restrict__ m, float *__restrict__ v, float lr, float c1,
+                                                   float c2, const double *__restrict__ lpart, int nl, double scale,
+                                                   double weight, bool first, double *__restrict__ loss) {
+    if (blockIdx.x == gridDim.x - 1) {
+        double s = 0.0;
+        for (int i = threadIdx.x; i < nl; i += 64) s += lpart[i];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+        if (threadIdx.x == 0) loss[0] = (first ? 0.0 : loss[0]) + (s * scale) * weight;
+        return;
+    }
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= kCnnParams) return;
-    double s = 0.0;
-    for (int i = 0; i < nimg; i++) s += (double)part[(long long)i * kCnnParams + q];
-    grad[q] = s;
+    const float g = (float)part_sum(part, nimg, q);
+    const float mm = 0.9f * m[q] + 0.1f * g, vv = 0.999f * v[q] + 0.001f * g * g;
+    m[q] = mm;
+    v[q] = vv;
+    p[q] = p[q] - lr * (mm * c1) / (sqrtf(vv * c2) + 1e-8f);
 }
 
 // g3 = 2 (out - y) / N ; loss partials sum (out - y)^2
+// (every loss: y of image b is that of the training set's image idx[b])
 __global__ void __launch_bounds__(256) k_cnn_loss(const float *__restrict__ out, const float *__restrict__ y, long long n,
-                                                  float *__restrict__ g3, double *__restrict__ part) {
+                                                  float *__restrict__ g3, double *__restrict__ part,
+                                                  const long long *__restrict__ idx) {
     __shared__ double red[4];
     double acc = 0.0;
     const float sc = (float)(2.0 / (double)n);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        const float d = out[i] - y[i];
+        const float d = out[i] - y[idx[i >> 12] * 4096 + (i & 4095)];
         g3[i] = sc * d;
         acc += (double)d * (double)d;
     }
@@ -629,13 +778,15 @@ __global__ void __launch_bounds__(256) k_cnn_loss(const float *__restrict__ out,
 // images blockIdx.x, blockIdx.x + gridDim.x, ...
 __global__ void __launch_bounds__(256) k_cnn_loss_h1(const float *__restrict__ out, const float *__restrict__ y,
                                                      int nimg, float alpha, float wi, float wj, float wk, float sc,
-                                                     float *__restrict__ g3, double *__restrict__ part) {
+                                                     float *__restrict__ g3, double *__restrict__ part,
+                                                     const long long *__restrict__ idx) {
     __shared__ float dl[4096];
     __shared__ double red[4];
     double acc = 0.0;
     for (int img = blockIdx.x; img < nimg; img += gridDim.x) {
         const long long o = (long long)img * 4096;
-        for (int c = threadIdx.x; c < 4096; c += 256) dl[c] = out[o + c] - y[o + c];
+        const float *Y = y + idx[img] * 4096;
+        for (int c = threadIdx.x; c < 4096; c += 256) dl[c] = out[o + c] - Y[c];
         __syncthreads();
         for (int c = threadIdx.x; c < 4096; c += 256) {
             const int i = c >> 8, j = (c >> 4) & 15, k = c & 15;
@@ -670,7 +821,8 @@ __global__ void __launch_bounds__(256) k_cnn_loss_h1(const float *__restrict__ o
 // Images with <c,Ac> or <e,Ae> zero contribute nothing.
 __global__ void __launch_bounds__(256) k_cnn_loss_cos(const float *__restrict__ out, const float *__restrict__ y,
                                                       int nimg, float alpha, float wi, float wj, float wk, float sc,
-                                                      float *__restrict__ g3, double *__restrict__ part) {
+                                                      float *__restrict__ g3, double *__restrict__ part,
+                                                     const long long *__restrict__ idx) {
     __shared__ float cl[4096], el[4096];
     __shared__ double red[3][4];
     double lacc = 0.0;
@@ -679,7 +831,7 @@ __global__ void __launch_bounds__(256) k_cnn_loss_cos(const float *__restrict__ 
         const long long o = (long long)img * 4096;
         for (int c = threadIdx.x; c < 4096; c += 256) {
             cl[c] = out[o + c];
-            el[c] = y[o + c];
+            el[c] = y[idx[img] * 4096 + c];
         }
         __syncthreads();
         // A v at cell c, v in LDS
@@ -724,32 +876,6 @@ __global__ void __launch_bounds__(256) k_cnn_loss_cos(const float *__restrict__ 
     if (threadIdx.x == 0) part[blockIdx.x] = lacc;
 }
 
-__global__ void k_cnn_sum(const double *__restrict__ part, int n, double scale, double *__restrict__ out) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double s = 0.0;
-    for (int i = 0; i < n; i++) s += part[i];
-    *out = s * scale;
-}
-
-__global__ void __launch_bounds__(256) k_cnn_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-                                                  const double *__restrict__ grad, float lr, float c1, float c2) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= kCnnParams) return;
-    const float g = (float)grad[q];
-    const float mm = 0.9f * m[q] + 0.1f * g, vv = 0.999f * v[q] + 0.001f * g * g;
-    m[q] = mm;
-    v[q] = vv;
-    p[q] = p[q] - lr * (mm * c1) / (sqrtf(vv * c2) + 1e-8f);
-}
-
-// batch gather: dst[b][4096] = src[idx[b]][4096]
-__global__ void __launch_bounds__(256) k_cnn_gather(const float *__restrict__ src, const long long *__restrict__ idx,
-                                                    float *__restrict__ dst) {
-    const long long b = blockIdx.x;
-    const long long s = idx[b];
-    for (int v = threadIdx.x; v < 4096; v += 256) dst[b * 4096 + v] = src[s * 4096 + v];
-}
-
 }  // namespace
 
 // ------------------------------------------------------------------ host class
@@ -766,8 +892,7 @@ CnnModel::CnnModel() {
 
 CnnModel::~CnnModel() {
     for (void *p : {(void *)params_, (void *)adam_m_, (void *)adam_v_, (void *)grad_, packed_, (void *)loss_part_,
-                    (void *)h1_, (void *)h2_, (void *)g2_, (void *)g1_, (void *)out_, (void *)g3_, (void *)part_,
-                    (void *)xb_, (void *)yb_})
+                    (void *)h1_, (void *)h2_, (void *)g2_, (void *)g1_, (void *)out_, (void *)g3_, (void *)part_})
         if (p) (void)hipFree(p);
 }
 
@@ -800,17 +925,14 @@ void CnnModel::get_params(float *p) const {
 
 void CnnModel::pack(hipStream_t stream) {
     if (packed_valid_) return;
-    hipLaunchKernelGGL(k_cnn_pack, dim3((PK_TOTAL * 8 + 255) / 256), dim3(256), 0, stream, (const float *)params_,
-                       (uint16_t *)packed_);
-    hipLaunchKernelGGL(k_cnn_packf, dim3((PF_TOTAL + 255) / 256), dim3(256), 0, stream, (const float *)params_,
-                       (uint16_t *)packed_ + PK_TOTAL * 8);
+    hipLaunchKernelGGL(k_cnn_pack, dim3((PK_TOTAL * 8 + PF_TOTAL + 255) / 256), dim3(256), 0, stream,
+                       (const float *)params_, (uint16_t *)packed_);
     packed_valid_ = true;
 }
 
 void CnnModel::ensure_batch(int nimg) {
     if (nimg <= max_batch_) return;
-    for (void *p : {(void *)h1_, (void *)h2_, (void *)g2_, (void *)g1_, (void *)out_, (void *)g3_, (void *)part_,
-                    (void *)xb_, (void *)yb_})
+    for (void *p : {(void *)h1_, (void *)h2_, (void *)g2_, (void *)g1_, (void *)out_, (void *)g3_, (void *)part_})
         if (p) CCHECK(hipFree(p));
     const size_t n = (size_t)nimg;
     CCHECK(hipMalloc(&h1_, n * 4096 * 16 * sizeof(uint16_t)));
@@ -819,8 +941,6 @@ void CnnModel::ensure_batch(int nimg) {
     CCHECK(hipMalloc(&g1_, n * 4096 * 16 * sizeof(uint16_t)));
     CCHECK(hipMalloc(&out_, n * 4096 * sizeof(float)));
     CCHECK(hipMalloc(&g3_, n * 4096 * sizeof(float)));
-    CCHECK(hipMalloc(&xb_, n * 4096 * sizeof(float)));
-    CCHECK(hipMalloc(&yb_, n * 4096 * sizeof(float)));
     CCHECK(hipMalloc(&part_, n * kCnnParams * sizeof(float)));
     max_batch_ = nimg;
 }
@@ -830,7 +950,7 @@ void CnnModel::infer(const float *x, float *out, long long nimg, hipStream_t str
     pack(stream);
     hipLaunchKernelGGL((k_cnn_fwd<false, false, kFwdWaves>), dim3((unsigned)nimg), dim3(64 * kFwdWaves), 0, stream, x, out,
                        (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_,
-                       (uint16_t *)nullptr, (uint16_t *)nullptr, HeatIO{});
+                       (uint16_t *)nullptr, (uint16_t *)nullptr, HeatIO{}, (const long long *)nullptr);
 }
 
 void CnnModel::infer_heat(const float *x, const double *scale, int scale_stride, int nb, long long istride, double *c,
@@ -840,69 +960,59 @@ void CnnModel::infer_heat(const float *x, const double *scale, int scale_stride,
     HeatIO hio{scale, scale_stride, nb, istride, c, active};
     hipLaunchKernelGGL((k_cnn_fwd<false, true, kFwdWaves>), dim3((unsigned)nimg), dim3(64 * kFwdWaves), 0, stream, x, (float *)nullptr,
                        (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_,
-                       (uint16_t *)nullptr, (uint16_t *)nullptr, hio);
+                       (uint16_t *)nullptr, (uint16_t *)nullptr, hio, (const long long *)nullptr);
 }
 
-void CnnModel::backward(const float *x, int nimg, hipStream_t stream) {
-    hipLaunchKernelGGL((k_cnn_dgrad<1>), dim3(nimg), dim3(256), 0, stream, (const void *)g3_, (const uint16_t *)h2_, g2_,
+void CnnModel::backward(const float *x, const float *g3, const long long *idx, int nimg, hipStream_t stream) {
+    hipLaunchKernelGGL(k_cnn_dgrad1, dim3(nimg, 16 / DPL), dim3(256), 0, stream, g3, (const uint16_t *)h2_, g2_,
                        (const us8 *)packed_);
-    hipLaunchKernelGGL((k_cnn_dgrad<16>), dim3(nimg), dim3(256), 0, stream, (const void *)g2_, (const uint16_t *)h1_, g1_,
-                       (const us8 *)packed_);
-    hipLaunchKernelGGL((k_cnn_wgrad<3>), dim3(nimg), dim3(256), 0, stream, (const void *)h2_, (const void *)g3_, part_);
-    hipLaunchKernelGGL((k_cnn_wgrad<2>), dim3(nimg), dim3(256), 0, stream, (const void *)h1_, (const void *)g2_, part_);
-    hipLaunchKernelGGL((k_cnn_wgrad<1>), dim3(nimg), dim3(256), 0, stream, (const void *)x, (const void *)g1_, part_);
-    hipLaunchKernelGGL(k_cnn_reduce, dim3((kCnnParams + 255) / 256), dim3(256), 0, stream, (const float *)part_, nimg,
-                       grad_);
+    hipLaunchKernelGGL(k_cnn_dgrad16, dim3(nimg, 16 / DPL), dim3(256), 0, stream, (const uint16_t *)g2_,
+                       (const uint16_t *)h1_, g1_, (const us8 *)packed_);
+    hipLaunchKernelGGL(k_cnn_wgrad, dim3(nimg, 7), dim3(256), 0, stream, x, (const uint16_t *)h1_, (const uint16_t *)h2_,
+                       (const uint16_t *)g1_, (const uint16_t *)g2_, g3, part_, idx);
 }
 
 void CnnModel::gradient(const float *x, const float *gout, int nimg, double *grad_host, hipStream_t stream) {
     ensure_batch(nimg);
     pack(stream);
     hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg), dim3(64 * kFwdWaves), 0, stream, x, out_,
-                       (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{});
-    CCHECK(hipMemcpyAsync(g3_, gout, sizeof(float) * 4096 * (size_t)nimg, hipMemcpyDeviceToDevice, stream));
-    backward(x, nimg, stream);
+                       (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{}, (const long long *)nullptr);
+    backward(x, gout, nullptr, nimg, stream);
+    hipLaunchKernelGGL(k_cnn_reduce, dim3((kCnnParams + 63) / 64), dim3(64), 0, stream, (const float *)part_, nimg, grad_);
     CCHECK(hipStreamSynchronize(stream));
     CCHECK(hipMemcpy(grad_host, grad_, sizeof(double) * kCnnParams, hipMemcpyDeviceToHost));
 }
 
-double CnnModel::train_step(const float *x, const float *y, int nimg, double lr, hipStream_t stream) {
-    ensure_batch(nimg);
+void CnnModel::train_step(const float *x, const float *y, const long long *idx, int nimg, double lr, bool first,
+                          hipStream_t stream) {
     pack(stream);
     hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg), dim3(64 * kFwdWaves), 0, stream, x, out_,
-                       (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{});
+                       (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{}, idx);
     const long long n = 4096LL * nimg;
+    int nwg = nimg < 1024 ? nimg : 1024;
+    double scale = 1.0 / (double)n;
     if (h1_alpha_ >= 0.0 && loss_cos_) {
         // mean over the images of the scale-free loss
-        const int nwg = nimg < 1024 ? nimg : 1024;
+        scale = 1.0 / (double)nimg;
         hipLaunchKernelGGL(k_cnn_loss_cos, dim3(nwg), dim3(256), 0, stream, (const float *)out_, y, nimg,
-                           (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2],
-                           (float)(1.0 / (double)nimg), g3_, loss_part_);
-        hipLaunchKernelGGL(k_cnn_sum, dim3(1), dim3(64), 0, stream, (const double *)loss_part_, nwg,
-                           1.0 / (double)nimg, loss_part_ + 1024);
+                           (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2], (float)scale, g3_,
+                           loss_part_, idx);
     } else if (h1_alpha_ >= 0.0) {
-        const int nwg = nimg < 1024 ? nimg : 1024;
         hipLaunchKernelGGL(k_cnn_loss_h1, dim3(nwg), dim3(256), 0, stream, (const float *)out_, y, nimg,
-                           (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2],
-                           (float)(1.0 / (double)n), g3_, loss_part_);
-        hipLaunchKernelGGL(k_cnn_sum, dim3(1), dim3(64), 0, stream, (const double *)loss_part_, nwg, 1.0 / (double)n,
-                           loss_part_ + 1024);
+                           (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2], (float)scale, g3_,
+                           loss_part_, idx);
     } else {
-        hipLaunchKernelGGL(k_cnn_loss, dim3(1024), dim3(256), 0, stream, (const float *)out_, y, n, g3_, loss_part_);
-        hipLaunchKernelGGL(k_cnn_sum, dim3(1), dim3(64), 0, stream, (const double *)loss_part_, 1024, 1.0 / (double)n,
-                           loss_part_ + 1024);
+        nwg = 1024;
+        hipLaunchKernelGGL(k_cnn_loss, dim3(nwg), dim3(256), 0, stream, (const float *)out_, y, n, g3_, loss_part_, idx);
     }
-    backward(x, nimg, stream);
+    backward(x, g3_, idx, nimg, stream);
     adam_t_++;
     const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)adam_t_)));
     const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)adam_t_)));
-    hipLaunchKernelGGL(k_cnn_adam, dim3((kCnnParams + 255) / 256), dim3(256), 0, stream, params_, adam_m_, adam_v_,
-                       (const double *)grad_, (float)lr, c1, c2);
+    hipLaunchKernelGGL(k_cnn_update, dim3((kCnnParams + 63) / 64 + 1), dim3(64), 0, stream, (const float *)part_, nimg,
+                       params_, adam_m_, adam_v_, (float)lr, c1, c2, (const double *)loss_part_, nwg, scale, (double)nimg,
+                       first, loss_part_ + 1024);
     packed_valid_ = false;
-    double loss = 0.0;
-    CCHECK(hipMemcpyAsync(&loss, loss_part_ + 1024, sizeof(double), hipMemcpyDeviceToHost, stream));
-    CCHECK(hipStreamSynchronize(stream));
-    return loss;
 }
 
 double CnnModel::train(const float *x, const float *y, long long nimg, int epochs, int batch, double lr, uint64_t seed,
@@ -916,23 +1026,29 @@ double CnnModel::train(const float *x, const float *y, long long nimg, int epoch
     CCHECK(hipMalloc(&didx, sizeof(long long) * nimg));
     double last = 0.0;
     try {
+        // the steps run on without the host: the loss adds up on the device
+        // and is read once, the batches are read in place by index
+        long long seen = 0;
         for (int ep = 0; ep < epochs; ep++) {
             // learning rate decays linearly from lr to lr/10 over the epochs
             const double lr_ep = epochs > 1 ? lr * (1.0 - 0.9 * (double)ep / (double)(epochs - 1)) : lr;
             for (long long i = 0; i < nimg; i++) idx[i] = i;
             std::shuffle(idx.begin(), idx.end(), rng);
+            CCHECK(hipStreamSynchronize(stream));     // the previous epoch's steps read didx
             CCHECK(hipMemcpy(didx, idx.data(), sizeof(long long) * nimg, hipMemcpyHostToDevice));
-            double tot = 0.0;
-            long long seen = 0;
+            seen = 0;
             for (long long b0 = 0; b0 + batch <= nimg; b0 += batch) {
-                hipLaunchKernelGGL(k_cnn_gather, dim3(batch), dim3(256), 0, stream, x, (const long long *)(didx + b0), xb_);
-                hipLaunchKernelGGL(k_cnn_gather, dim3(batch), dim3(256), 0, stream, y, (const long long *)(didx + b0), yb_);
-                tot += train_step(xb_, yb_, batch, lr_ep, stream) * batch;
+                train_step(x, y, didx + b0, batch, lr_ep, b0 == 0, stream);
                 seen += batch;
             }
-            last = seen ? tot / (double)seen : 0.0;
+            CCHECK(hipGetLastError());
         }
+        double tot = 0.0;
+        CCHECK(hipStreamSynchronize(stream));
+        CCHECK(hipMemcpy(&tot, loss_part_ + 1024, sizeof(double), hipMemcpyDeviceToHost));
+        last = seen ? tot / (double)seen : 0.0;
     } catch (...) {
+        (void)hipStreamSynchronize(stream);
         (void)hipFree(didx);
         throw;
     }

@@ -33,8 +33,6 @@ class CnnModel : public HeatCorrector {
     void prepare(hipStream_t stream) override { pack(stream); }
     // sum over the batch of the gradient of sum(gout * out) (device x/gout, host grad)
     void gradient(const float *x, const float *gout, int nimg, double *grad_host, hipStream_t stream);
-    // one Adam step on the mean squared error over a batch (device x, y); returns the loss
-    double train_step(const float *x, const float *y, int nimg, double lr, hipStream_t stream);
     // epochs over nimg device images in shuffled minibatches, learning rate decaying
     // linearly to lr/10; returns the last epoch's mean loss
     double train(const float *x, const float *y, long long nimg, int epochs, int batch, double lr, uint64_t seed,
@@ -54,14 +52,19 @@ class CnnModel : public HeatCorrector {
   private:
     void ensure_batch(int nimg);
     void pack(hipStream_t stream);
-    void backward(const float *x, int nimg, hipStream_t stream);   // from g3 in ws_g3_ into grad_
+    // from the output gradient g3 into the images' parts of the parameter gradient (idx: images of x, null: 0 .. nimg - 1)
+    void backward(const float *x, const float *g3, const long long *idx, int nimg, hipStream_t stream);
+    // one Adam step on the loss over the images idx of the device arrays x, y;
+    // nimg times the loss is added to loss_part_[1024] (first: starts it)
+    void train_step(const float *x, const float *y, const long long *idx, int nimg, double lr, bool first,
+                    hipStream_t stream);
     float *params_ = nullptr, *adam_m_ = nullptr, *adam_v_ = nullptr;
     double *grad_ = nullptr;
     void *packed_ = nullptr;      // MFMA operand images of the weights (fwd and data-gradient forms)
     bool packed_valid_ = false;
     int max_batch_ = 0;
     uint16_t *h1_ = nullptr, *h2_ = nullptr, *g2_ = nullptr, *g1_ = nullptr;
-    float *out_ = nullptr, *g3_ = nullptr, *part_ = nullptr, *xb_ = nullptr, *yb_ = nullptr;
+    float *out_ = nullptr, *g3_ = nullptr, *part_ = nullptr;
     double *loss_part_ = nullptr;
     long long adam_t_ = 0;
     double h1_alpha_ = -1.0, h1_w_[3] = {1.0, 1.0, 1.0};

@@ -253,3 +253,24 @@ def test_learned_fcg_on_the_locally_refined_shell_32_systems():
         x1 = hs.get_T(k)
         assert np.linalg.norm(x1 - x0[k]) / np.linalg.norm(x0[k]) < 1e-7
     s.close()
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 33])
+def test_batch_gradient_is_the_sum_of_its_images(n):
+    """Every image's gradient is formed by workgroups of its own and the batch
+    adds them in FP64 in order: the batch's equals that sum bit for bit, with
+    zero-border, constant and very small images among them."""
+    s = _shell()
+    c = Cnn(s)
+    c.params = _params(8)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, 16, 16, 16)).astype(np.float32)
+    gout = rng.standard_normal((n, 16, 16, 16)).astype(np.float32)
+    x[0, :, :, 1:15] = 0.0
+    gout[-1, 1:15] *= np.float32(1e-30)
+    print("[cnn gradient sum]", n, flush=True)
+    g = c.gradient(x, gout)
+    tot = np.zeros(NP)
+    for k in range(n):
+        tot = tot + c.gradient(x[k:k + 1], gout[k:k + 1])
+    assert np.array_equal(g, tot)
