@@ -577,10 +577,72 @@ __global__ void __launch_bounds__(256) k_hdot(long long n, const double *__restr
     block_partials<2>(v, partial, s);
 }
 
-// sum of nwg partials per (system, pair), fixed order
+// Per-system scalars on the device, kSc slots each:
+// [0] alpha = <p,r>/<p,q>, [1] beta = <z,q>/gamma, [2] gamma = <p,q>,
+// [3] feature scale of the learned correction, [4] its step along c, [5] <b,b>,
+// [6] <z,q> of the V-cycle output.
+constexpr int kSc = 8;
+enum {
+    kScNone = -1,
+    kScAlpha = 0,     // alpha and gamma (dots: [0]=<p,q>, [1]=<p,r>)
+    kScBeta = 1,      // beta (dots: [0]=<z,q>)
+    kScStep = 2,      // correction step <c,r'>/<c,Ac> (dots: [0]=<c,r'>, [1]=<c,Ac>), 0 unless <c,Ac> > 0
+    kScFeature = 3,   // feature scale sqrt(sum / ncell) (dots: [0]=sum (r'/diag)^2)
+    kScNorm = 4,      // <b,b> (dots: [0])
+    kScBetaStep = 5,  // beta of the learned direction, <z + a c, q>/gamma = (<z,q> + a <c,q>)/gamma, from [6], [4] and dots[2] = <c,q>
+    kScZq = 6,        // [6] = <z,q> of the V-cycle output (dots: [0])
+    kScBetaBlocks = 7, // beta of the learned direction with per-block steps (dots: [0] = sum_b a_b <c_b,q_b>)
+    kScConverge = 8   // the convergence test (dots: [0]=<r,r>)
+};
+// Convergence on the device: an active system counts the iteration, stores
+// ||r||/||b|| and is deactivated at tol (or on a non-finite residual), which
+// takes it off the count of active systems.
+struct Converge {
+    double tol;
+    int *iters, *nactive;
+    double *relres;
+};
+__device__ __forceinline__ void scalar_step(int what, int s, const double *__restrict__ dots, double *__restrict__ S,
+                                            int *__restrict__ active, double ncell, const Converge &cv) {
+    const bool on = active[s] != 0;
+    if (what == kScAlpha) {
+        S[2] = dots[0];
+        S[0] = on ? dots[1] / dots[0] : 0.0;
+    } else if (what == kScBeta) {
+        S[1] = on ? dots[0] / S[2] : 0.0;
+    } else if (what == kScStep) {
+        const double num = dots[0], den = dots[1];
+        const double a = num / den;
+        S[4] = (on && den > 0.0 && a == a && a < 1e300 && a > -1e300) ? a : 0.0;
+    } else if (what == kScFeature) {
+        S[3] = on ? sqrt(dots[0] / ncell) : 0.0;
+    } else if (what == kScNorm) {
+        S[5] = dots[0];
+    } else if (what == kScBetaStep) {
+        S[1] = on ? (S[6] + S[4] * dots[2]) / S[2] : 0.0;
+    } else if (what == kScZq) {
+        S[6] = dots[0];
+    } else if (what == kScBetaBlocks) {
+        S[1] = on ? (S[6] + dots[0]) / S[2] : 0.0;
+    } else if (what == kScConverge && on) {
+        const double rel = sqrt(dots[0] / S[5]);
+        cv.iters[s] = cv.iters[s] + 1;
+        cv.relres[s] = rel;
+        if (rel <= cv.tol || !(rel == rel) || rel > 1e300) {
+            active[s] = 0;
+            atomicSub(cv.nactive, 1);
+        }
+    }
+}
+
+// sum of nwg partials per (system, pair), fixed order, and the scalars formed
+// from the sums by the workgroup's first thread (a launch of its own for each
+// cost 4.4 us per use, 3 uses per iteration)
 __global__ void __launch_bounds__(256) k_hdot_final(const double *__restrict__ partial, int nwg, int npairs,
-                                                   double *__restrict__ out) {
-    __shared__ double red[4];
+                                                   double *__restrict__ out, int what, int what2,
+                                                   double *__restrict__ sc, int *__restrict__ active, double ncell,
+                                                   Converge cv) {
+    __shared__ double red[3][4];
     const int s = blockIdx.x;
     for (int p = 0; p < npairs; p++) {
         const double *P = partial + ((long long)s * 3 + p) * nwg;
@@ -590,78 +652,17 @@ __global__ void __launch_bounds__(256) k_hdot_final(const double *__restrict__ p
         if (w < nwg) v0 += P[w];
         double v = v0 + v1;
         for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-        __syncthreads();
-        if (threadIdx.x == 0) out[s * 3 + p] = ((red[0] + red[1]) + red[2]) + red[3];
-        __syncthreads();
+        if ((threadIdx.x & 63) == 0) red[p][threadIdx.x >> 6] = v;
     }
-}
-
-// Per-system scalars on the device (one thread per system), kSc slots each:
-// [0] alpha = <p,r>/<p,q>, [1] beta = <z,q>/gamma, [2] gamma = <p,q>,
-// [3] feature scale of the learned correction, [4] its step along c, [5] <b,b>,
-// [6] <z,q> of the V-cycle output.
-constexpr int kSc = 8;
-// what 0: alpha and gamma (dots: [0]=<p,q>, [1]=<p,r>)
-// what 1: beta (dots: [0]=<z,q>)
-// what 2: correction step <c,r'>/<c,Ac> (dots: [0]=<c,r'>, [1]=<c,Ac>), 0 unless <c,Ac> > 0
-// what 3: feature scale sqrt(sum / ncell) (dots: [0]=sum (r'/diag)^2)
-// what 4: <b,b> (dots: [0])
-// what 5: beta of the learned direction from [6], [4] and dots[2] = <c,q>
-// what 6: [6] = <z,q> (dots: [0])
-// what 7: beta of the learned direction with per-block steps (dots: [0] = sum_b a_b <c_b,q_b>)
-__global__ void k_hscalars(int what, int nsys, const double *__restrict__ dots, double *__restrict__ sc,
-                           const int *__restrict__ active, double ncell) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys) return;
-    double *S = sc + kSc * s;
-    if (what == 0) {
-        S[2] = dots[3 * s];
-        S[0] = active[s] ? dots[3 * s + 1] / dots[3 * s] : 0.0;
-    } else if (what == 1) {
-        S[1] = active[s] ? dots[3 * s] / S[2] : 0.0;
-    } else if (what == 2) {
-        const double num = dots[3 * s], den = dots[3 * s + 1];
-        const double a = num / den;
-        S[4] = (active[s] && den > 0.0 && a == a && a < 1e300 && a > -1e300) ? a : 0.0;
-    } else if (what == 3) {
-        S[3] = active[s] ? sqrt(dots[3 * s] / ncell) : 0.0;
-    } else if (what == 4) {
-        S[5] = dots[3 * s];
-    } else if (what == 7) {
-        // beta of the learned direction with per-block steps: (<z,q> + sum_b a_b <c_b,q_b>)/gamma
-        S[1] = active[s] ? (S[6] + dots[3 * s]) / S[2] : 0.0;
-    } else if (what == 5) {
-        // beta of the learned direction: <z + a c, q>/gamma = (<z,q> + a <c,q>)/gamma
-        S[1] = active[s] ? (S[6] + S[4] * dots[3 * s + 2]) / S[2] : 0.0;
-    } else {
-        S[6] = dots[3 * s];                 // <z, q> of the V-cycle output
-    }
-}
-
-// Convergence on the device (one workgroup): for every system still active,
-// count the iteration, store ||r||/||b|| and deactivate it at tol (or on a
-// non-finite residual); out[0] = number of systems left active.
-__global__ void __launch_bounds__(256) k_hconverge(int nsys, const double *__restrict__ dots,
-                                                   const double *__restrict__ sc, double tol, int *__restrict__ active,
-                                                   int *__restrict__ iters, double *__restrict__ relres,
-                                                   int *__restrict__ out) {
-    __shared__ int cnt[256];
-    int c = 0;
-    for (int s = threadIdx.x; s < nsys; s += blockDim.x) {
-        if (!active[s]) continue;
-        const double rel = sqrt(dots[3 * s] / sc[kSc * s + 5]);
-        iters[s] = iters[s] + 1;
-        relres[s] = rel;
-        if (rel <= tol || !(rel == rel) || rel > 1e300) active[s] = 0;
-        else c++;
-    }
-    cnt[threadIdx.x] = c;
     __syncthreads();
     if (threadIdx.x == 0) {
-        int t = 0;
-        for (int k = 0; k < (int)blockDim.x; k++) t += cnt[k];
-        out[0] = t;
+        double dots[3] = {0.0, 0.0, 0.0};
+        for (int p = 0; p < npairs; p++) {
+            dots[p] = ((red[p][0] + red[p][1]) + red[p][2]) + red[p][3];
+            out[s * 3 + p] = dots[p];
+        }
+        if (what != kScNone) scalar_step(what, s, dots, sc + kSc * s, active, ncell, cv);
+        if (what2 != kScNone) scalar_step(what2, s, dots, sc + kSc * s, active, ncell, cv);
     }
 }
 
@@ -919,7 +920,7 @@ struct HeatSolver::Impl {
     double *ablk = nullptr;
     // captured FCG iteration per mode (plain, learned) and device-side convergence state
     hipGraphExec_t graph[2] = {nullptr, nullptr};
-    double graph_tol[2] = {0.0, 0.0};   // tolerance baked into each captured k_hconverge
+    double graph_tol[2] = {0.0, 0.0};   // tolerance baked into each captured convergence test
     bool use_graph = true;
     int learned_iters = 0;              // directions built with the learned correction (0: all)
     int *iters_dev = nullptr, *nactive_dev = nullptr;
@@ -939,13 +940,11 @@ struct HeatSolver::Impl {
     void ensure_learned();
     void features(double *z);
     void learned_correction(bool first);
-    void final_dots(int npairs, unsigned nwg) {
+    // sums of npairs dots over nwg workgroups' partials, then the scalars what, what2
+    void final_dots(int npairs, unsigned nwg, int what, int what2 = kScNone, double tol = 0.0) {
         hipLaunchKernelGGL(k_hdot_final, dim3((unsigned)nsys), dim3(256), 0, stream, (const double *)partial, (int)nwg,
-                           npairs, dots);
-    }
-    void scalars(int what, double ncell = 0.0) {
-        hipLaunchKernelGGL(k_hscalars, dim3((nsys + 63) / 64), dim3(64), 0, stream, what, nsys, (const double *)dots, sc,
-                           (const int *)active, ncell);
+                           npairs, dots, what, what2, sc, active, (double)ist(0),
+                           Converge{tol, iters_dev, nactive_dev, relres_dev});
     }
     int pre = 2, post = 2;
     // coarsest level: Jacobi-preconditioned CG to r.z <= coarse_tol^2 (r.z)_0
@@ -1339,8 +1338,7 @@ void HeatSolver::Impl::ensure_learned() {
 // square) in sc[3]
 void HeatSolver::Impl::features(double *z) {
     launch_march(0, z, OpFeat{rp, xin, r, nullptr}, partial);
-    final_dots(1, march_wgs(0));
-    scalars(3, (double)ist(0));
+    final_dots(1, march_wgs(0), kScFeature);
 }
 
 // c = scale * net(features / scale) and its step a = <c,r'>/<c,Ac> (sc[4]);
@@ -1352,15 +1350,10 @@ void HeatSolver::Impl::learned_correction(bool first) {
         const unsigned nwg = march_wgs(0);
         hipLaunchKernelGGL(k_hblockstep, dim3((nwg + 255) / 256, (unsigned)nsys), dim3(256), 0, stream, (int)nwg, nb,
                            partial, ablk, (const int *)active);
-        if (!first) {
-            final_dots(1, nwg);
-            scalars(7);
-        }
+        if (!first) final_dots(1, nwg, kScBetaBlocks);
         return;
     }
-    final_dots(3, march_wgs(0));
-    scalars(2);
-    if (!first) scalars(5);
+    final_dots(3, march_wgs(0), kScStep, first ? kScNone : kScBetaStep);
 }
 
 HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec) {
@@ -1386,8 +1379,7 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
                        ni * ns);
     hipLaunchKernelGGL(k_hdot, I.grid_elem(), dim3(256), 0, I.stream, ni, (const double *)I.b, (const double *)I.b,
                        (const double *)nullptr, (const double *)nullptr, 1, (const int *)nullptr, I.partial, ni);
-    I.final_dots(1, I.elem_wgs());
-    I.scalars(4);
+    I.final_dots(1, I.elem_wgs(), kScNorm);
     std::vector<double> bn(3 * ns);
     HCHECK(hipMemcpyAsync(bn.data(), I.dots, sizeof(double) * 3 * ns, hipMemcpyDeviceToHost, I.stream));
     HCHECK(hipStreamSynchronize(I.stream));
@@ -1399,6 +1391,7 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         nact += act[s];
     }
     HCHECK(hipMemcpy(I.active, act.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
+    HCHECK(hipMemcpy(I.nactive_dev, &nact, sizeof(int), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_hizero, dim3((ns + 255) / 256), dim3(256), 0, I.stream, I.iters_dev, ns);
 
     auto record = [&](const double *z) {
@@ -1435,10 +1428,7 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         double *z = nullptr;
         if (lrn) {
             const unsigned nwg = I.vcycle(I.r, z, I.learned_pre0, I.learned_post0, first ? nullptr : I.q);
-            if (!first) {
-                I.final_dots(1, nwg);
-                I.scalars(6);                // <z, q>
-            }
+            if (!first) I.final_dots(1, nwg, kScZq);
             I.features(z);
             I.learned_correction(first);     // step a and (unless first) beta
             hipLaunchKernelGGL(k_hupdate_p2, g0, dim3(256), 0, I.stream, ni, I.p, (const double *)z, (const double *)I.cc,
@@ -1448,10 +1438,7 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         }
         const int pre0 = recording ? I.learned_pre0 : I.pre, post0 = recording ? I.learned_post0 : I.post;
         const unsigned nwg = I.vcycle(I.r, z, pre0, post0, first ? nullptr : I.q);
-        if (!first) {
-            I.final_dots(1, nwg);
-            I.scalars(1);
-        }
+        if (!first) I.final_dots(1, nwg, kScBeta);
         if (recording) {
             I.features(z);
             record(z);
@@ -1459,16 +1446,13 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         hipLaunchKernelGGL(k_hupdate_p, g0, dim3(256), 0, I.stream, ni, I.p, (const double *)z, (const double *)I.sc,
                            (const int *)I.active, ni, first ? 0 : 1);
     };
-    // one FCG iteration; the convergence test runs on the device (k_hconverge)
+    // one FCG iteration; the convergence test runs on the device (k_hdot_final)
     auto body = [&](bool lrn) {
         I.apply0(I.p, I.q, I.r);                         // q = A p with <p,q>, <p,r>
-        I.final_dots(2, I.march_wgs(0));
-        I.scalars(0);
+        I.final_dots(2, I.march_wgs(0), kScAlpha);
         hipLaunchKernelGGL(k_hupdate_xr, I.grid_elem(), dim3(256), 0, I.stream, ni, I.x, I.r, (const double *)I.p,
                            (const double *)I.q, (const double *)I.sc, (const int *)I.active, I.partial, ni);
-        I.final_dots(1, I.elem_wgs());
-        hipLaunchKernelGGL(k_hconverge, dim3(1), dim3(256), 0, I.stream, ns, (const double *)I.dots, (const double *)I.sc,
-                           tol, I.active, I.iters_dev, I.relres_dev, I.nactive_dev);
+        I.final_dots(1, I.elem_wgs(), kScConverge, kScNone, tol);
         precond_direction(false, lrn);
     };
     // directions 0 .. nlearn-1 come from the learned correction, later ones
