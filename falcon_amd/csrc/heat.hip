@@ -61,6 +61,7 @@ struct HLev {
     const double *V, *Ai, *Aj, *Ak, *off;   // [block][i][j] coefficient tables
     const int2 *gsw;        // per face ghost: (donor base cell or -1, weights index or -1 = copy)
     const double *gw;       // 3 weights per weighted ghost
+    const double *diag;     // [system][block][i][j]: V/dt + off (k_hdiag)
 };
 
 struct Cell {
@@ -78,15 +79,24 @@ __device__ __forceinline__ Cell cell_of(const HLev &L, long long c) {
     return r;
 }
 
-// the field a stencil reads
-struct Field {
+// the field a stencil reads: a stored vector, or (FIRST) the damped Jacobi
+// value from x = 0, (omega r)/diag, formed where it is read
+template <bool FIRST>
+struct FieldT {
     const double *x;
-    __device__ __forceinline__ double operator()(long long c) const { return x[c]; }
+    const double *diag;     // of the system (FIRST)
+    int lm;
+    double omega;
+    __device__ __forceinline__ double value(long long c, double v) const { return FIRST ? (omega * v) / diag[c >> lm] : v; }
+    __device__ __forceinline__ double operator()(long long c) const { return value(c, x[c]); }
 };
+typedef FieldT<false> Field;
 
-__device__ __forceinline__ double diag_at(const HLev &L, const Cell &q, double inv_dt) {
-    const long long t2 = ((long long)q.b << (2 * L.lm)) + (q.i << L.lm) + q.j;
-    return L.V[t2] * inv_dt + L.off[t2];
+// diag[s][t2] = V/dt + off of every system (whenever dt changes)
+__global__ void __launch_bounds__(256) k_hdiag(HLev L, double *__restrict__ diag, const double *__restrict__ inv_dt,
+                                               long long n2) {
+    const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < n2) diag[blockIdx.y * n2 + c] = L.V[c] * inv_dt[blockIdx.y] + L.off[c];
 }
 
 // Block partial sums of NP per-thread values into partial[s][p][blockIdx.x].
@@ -115,20 +125,34 @@ __device__ __forceinline__ int xcd_group(int w, int nwg) {
     return x * q + (x < r ? x : r) + (w >> 3);
 }
 
+// its inverse: the workgroup that takes group g
+__device__ __forceinline__ int xcd_slot(int g, int nwg) {
+    const int q = nwg >> 3, r = nwg & 7;
+    const int x = g < r * (q + 1) ? g / (q + 1) : r + (g - r * (q + 1)) / (q > 0 ? q : 1);
+    return ((g - (x * q + (x < r ? x : r))) << 3) + x;
+}
+
 // ---- block-tile stencil kernels
-// A workgroup of 256 threads owns 256/m^2 whole blocks (one for m = 16);
-// thread (block, j, k) owns the column i = 0..m-1 (lanes of one i-plane are
-// consecutive, so every load instruction is coalesced).  Phase 1 issues every
-// load at once: the 6 ghost-table entries per thread, the x column, the op's
-// input columns and the workgroup's coefficient tables.  Phase 2 gathers the
-// face ghosts (1536 per workgroup for any m: the first donor of every entry,
-// then the rest of the weighted ones) and stores the x tile (plane-major:
-// tile[i][thread]), the ghosts and the coefficients in LDS.  Phase 3 applies
-// the operator from registers (i +- 1) and LDS (j, k +- 1, ghosts, coefficients).
+// A workgroup of 256 threads owns the C = m/S planes i0 .. i0 + C - 1 of
+// 256/m^2 whole blocks (one for m = 16); thread (block, j, k) owns the column
+// of those planes (lanes of one i-plane are consecutive, so every load
+// instruction is coalesced).  Phase 1 issues every load at once: the ghost-table
+// entries, the x column with the planes before and after it, the op's input
+// columns and the coefficient tables of the planes.  Phase 2 gathers the face
+// ghosts (the first donor of every entry, then the rest of the weighted ones);
+// those of the theta and phi faces go to LDS with the coefficients, those of
+// the radial faces stay with their column's thread.  Phase 3 applies the
+// operator from registers (i +- 1) and lane exchanges (j, k +- 1).
+// S = 2 for m >= 4 (1 below: a thread keeps the i pair of a restriction): a whole 16^3 block per
+// workgroup took 130 to 162 VGPRs and 39 KB of LDS, three workgroups per CU
+// whose phases ran in step.  On 6.3 M cells: sweep 50 -> 37 us, operator with
+// dots 53 -> 43, restriction 43 -> 32 (4.1 TB/s of algorithmic traffic); the
+// first two sweeps 77 -> 55 us in one pass.
 
 // trilinear inter/extrapolation inside the donor block from base cell c, in
 // the term order of ModMath.f90:283-291 (weights may lie in [-0.5, 1.5]); f0 = X(c)
-__device__ __forceinline__ double trilinear(const HLev &L, const Field &X, long long c, int wid, double f0) {
+template <class F>
+__device__ __forceinline__ double trilinear(const HLev &L, const F &X, long long c, int wid, double f0) {
     const double wi = L.gw[3 * wid], wj = L.gw[3 * wid + 1], wk = L.gw[3 * wid + 2];
     const long long S1 = L.m, SI = (long long)L.m * L.m;
     const double f1 = X(c + SI), f2 = X(c + S1), f3 = X(c + 1), f4 = X(c + SI + S1), f5 = X(c + S1 + 1),
@@ -199,17 +223,26 @@ struct OpApplyDot {              // c.r', c.Ac, c.q (Ac itself is not stored)
     }
 };
 
+// planes per thread
+template <int LM>
+struct Planes {
+    static constexpr int LS = LM < 2 ? 0 : 1;   // log2(S)
+    static constexpr int LC = LM - LS, C = 1 << LC, S = 1 << LS;
+};
 // LDS layout (doubles): edge rows of the x tile (m = 16 only: the first and
-// last j-row of every wavefront, [wave][2][i][k]), face ghosts [6 * 256],
-// coefficient tables Ai [bpw][m+1][m], Aj [bpw][m][m+1], Ak, V, off [bpw][m][m]
+// last j-row of every wavefront, [wave][2][i][k]), theta and phi face ghosts
+// [block][4][i][m], coefficient tables Ai [bpw][C+1][m], Aj [bpw][C][m+1], Ak
+// and diag [bpw][C][m]
 template <int LM>
 struct TileLds {
-    static constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM);
-    static constexpr int NE = LM == 4 ? 4 * 2 * 16 * 16 : 0;
-    static constexpr int G0 = NE, CI = G0 + 6 * 256, NI = bpw * (m + 1) * m, CJ = CI + NI, NJ = bpw * m * (m + 1),
-                         CK = CJ + NJ, CV = CK + bpw * mm, CO = CV + bpw * mm, SIZE = CO + bpw * mm;
+    static constexpr int m = 1 << LM, C = Planes<LM>::C, bpw = 256 >> (2 * LM);
+    static constexpr int NE = LM == 4 ? 4 * 2 * C * 16 : 0;
+    static constexpr int NG = bpw * 4 * C * m;
+    static constexpr int G0 = NE, CI = G0 + NG, NI = bpw * (C + 1) * m, CJ = CI + NI, NJ = bpw * C * (m + 1),
+                         CK = CJ + NJ, NK = bpw * C * m, CD = CK + NK, SIZE = CD + NK;
     static constexpr int NC = SIZE - CI;              // coefficient doubles
     static constexpr int NCT = (NC + 255) / 256;      // per thread
+    static constexpr int NGT = (NG + 255) / 256;      // ghosts per thread
 };
 
 // x of lane l - 1 / l + 1 within rows of 16 lanes (DPP row shifts)
@@ -221,60 +254,87 @@ __device__ __forceinline__ double dpp_d(double v) {
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// phases 1-2: col = the thread's x column, a0 / a1 its columns of in0 / in1,
-// sm = tile + ghosts + coefficients.  Ends with a barrier.
-template <int LM, bool IN0, bool IN1>
-__device__ __forceinline__ void load_tile(const HLev &L, const Field &F, int b0, bool own, long long cb,
-                                          const double *__restrict__ in0, const double *__restrict__ in1, long long so,
-                                          double (&col)[1 << LM], double (&a0)[1 << LM], double (&a1)[1 << LM],
-                                          double *__restrict__ sm) {
+// phases 1-2: col[1 .. C] = the thread's x column, col[0] and col[C + 1] its
+// radial neighbours, a0 / a1 its columns of in0 / in1, sm = edge rows + ghosts +
+// coefficients.  FIRST: x is formed from in0 = r, which a0 returns.  Ends with a
+// barrier.
+template <int LM, bool FIRST, bool IN0, bool IN1>
+__device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F, const double *__restrict__ diag, int b0,
+                                          int h, bool own, long long cb, const double *__restrict__ in0,
+                                          const double *__restrict__ in1, long long so,
+                                          double (&col)[Planes<LM>::C + 2], double (&a0)[Planes<LM>::C],
+                                          double (&a1)[Planes<LM>::C], double *__restrict__ sm) {
     using T = TileLds<LM>;
-    constexpr int m = T::m, mm = T::mm, bpw = T::bpw;
+    constexpr int m = T::m, mm = m * m, bpw = T::bpw, C = T::C, LC = Planes<LM>::LC, S = Planes<LM>::S;
     const int tid = threadIdx.x;
     const int nbw = L.nb - b0 < bpw ? L.nb - b0 : bpw;
-    const int ng = nbw * 6 * mm;
-    const int2 *E = L.gsw + (long long)b0 * 6 * mm;
-    int2 e[6];
+    const int lb = tid >> (2 * LM), jk = tid & (mm - 1), i0 = h * C;
+    const int2 none = make_int2(-1, -1);
+    // theta and phi face ghosts of the planes, in the LDS order
+    int2 e[T::NGT];
 #pragma unroll
-    for (int u = 0; u < 6; u++) {
-        const int g = tid + 256 * u;
-        e[u] = g < ng ? E[g] : make_int2(-1, -1);
+    for (int u = 0; u < T::NGT; u++) {
+        const int q = tid + 256 * u, t = q & (m - 1), il = (q >> LM) & (C - 1), f = (q >> (LM + LC)) & 3,
+                  b = q >> (LM + LC + 2);
+        e[u] = q < T::NG && b < nbw ? L.gsw[((long long)(b0 + b) * 6 + 2 + f) * mm + (i0 + il) * m + t] : none;
     }
+    // radial faces: the block's own ghosts, or its planes of the neighbouring part
+    const int2 *Er = L.gsw + (long long)(b0 + lb) * 6 * mm + jk;
+    const int2 elo = own && h == 0 ? Er[0] : none, ehi = own && h == S - 1 ? Er[mm] : none;
+    const long long c0 = cb + (long long)i0 * mm;
+    double xr[C + 2], dg[C + 2];
 #pragma unroll
-    for (int i = 0; i < m; i++) {
-        const long long c = cb + (long long)i * mm;
-        col[i] = own ? F(c) : 0.0;
-        if (IN0) a0[i] = own ? in0[so + c] : 0.0;
-        if (IN1) a1[i] = own ? in1[so + c] : 0.0;
+    for (int i = 0; i < C + 2; i++) {
+        const bool in = own && (i > 0 || h > 0) && (i < C + 1 || h < S - 1);
+        const long long c = c0 + (long long)(i - 1) * mm;
+        xr[i] = in ? F.x[c] : 0.0;
+        if (FIRST) dg[i] = in ? diag[c >> LM] : 1.0;
+        if (i > 0 && i < C + 1) {
+            if (IN0 && !FIRST) a0[i - 1] = own ? in0[so + c] : 0.0;
+            if (IN1) a1[i - 1] = own ? in1[so + c] : 0.0;
+        }
     }
-    // coefficient tables of the workgroup's blocks: 5 contiguous ranges
+    // coefficient tables of the planes
     double cf[T::NCT];
 #pragma unroll
     for (int u = 0; u < T::NCT; u++) {
         const int q = tid + 256 * u;
         double v = 0.0;
         if (q < T::NI) {
-            if (q < nbw * (m + 1) * m) v = L.Ai[(long long)b0 * (m + 1) * m + q];
+            constexpr int w = (C + 1) * m;
+            const int b = q / w, r = q - b * w;
+            if (b < nbw) v = L.Ai[(long long)(b0 + b) * (m + 1) * m + i0 * m + r];
         } else if (q < T::NI + T::NJ) {
-            const int r = q - T::NI;
-            if (r < nbw * m * (m + 1)) v = L.Aj[(long long)b0 * m * (m + 1) + r];
+            constexpr int w = C * (m + 1);
+            const int r0 = q - T::NI, b = r0 / w, r = r0 - b * w;
+            if (b < nbw) v = L.Aj[(long long)(b0 + b) * m * (m + 1) + i0 * (m + 1) + r];
         } else if (q < T::NC) {
-            const int r = q - T::NI - T::NJ, which = r / (bpw * mm), w = r - which * (bpw * mm);
-            const double *src = which == 0 ? L.Ak : (which == 1 ? L.V : L.off);
-            if (w < nbw * mm) v = src[((long long)b0 << (2 * LM)) + w];
+            const int r0 = q - T::NI - T::NJ, which = r0 >= T::NK, r1 = which ? r0 - T::NK : r0;
+            const int b = r1 >> (LM + LC), r = r1 & (C * m - 1);
+            if (b < nbw) v = (which ? diag : L.Ak)[((long long)(b0 + b) << (2 * LM)) + i0 * m + r];
         }
         cf[u] = v;
     }
     // ghosts: the first donor value of every entry, then the weighted ones
-    double f0[6];
+    double f0[T::NGT];
 #pragma unroll
-    for (int u = 0; u < 6; u++) f0[u] = e[u].x >= 0 ? F(e[u].x) : 0.0;
+    for (int u = 0; u < T::NGT; u++) f0[u] = e[u].x >= 0 ? F(e[u].x) : 0.0;
+    double flo = elo.x >= 0 ? F(elo.x) : 0.0, fhi = ehi.x >= 0 ? F(ehi.x) : 0.0;
 #pragma unroll
-    for (int u = 0; u < 6; u++) {
+    for (int u = 0; u < T::NGT; u++) {
         double g = f0[u];
         if (e[u].y >= 0) g = trilinear(L, F, e[u].x, e[u].y, f0[u]);
-        sm[T::G0 + tid + 256 * u] = g;
+        if (tid + 256 * u < T::NG) sm[T::G0 + tid + 256 * u] = g;
     }
+    if (elo.y >= 0) flo = trilinear(L, F, elo.x, elo.y, flo);
+    if (ehi.y >= 0) fhi = trilinear(L, F, ehi.x, ehi.y, fhi);
+#pragma unroll
+    for (int i = 0; i < C + 2; i++) {
+        col[i] = FIRST ? (F.omega * xr[i]) / dg[i] : xr[i];
+        if (FIRST && i > 0 && i < C + 1) a0[i - 1] = xr[i];
+    }
+    if (h == 0) col[0] = flo;
+    if (h == S - 1) col[C + 1] = fhi;
 #pragma unroll
     for (int u = 0; u < T::NCT; u++)
         if (tid + 256 * u < T::NC) sm[T::CI + tid + 256 * u] = cf[u];
@@ -284,45 +344,44 @@ __device__ __forceinline__ void load_tile(const HLev &L, const Field &F, int b0,
         if (l < 16 || l >= 48) {
             const int side = l < 16 ? 0 : 1;
 #pragma unroll
-            for (int i = 0; i < m; i++) sm[((w * 2 + side) * 16 + i) * 16 + (l & 15)] = col[i];
+            for (int i = 0; i < C; i++) sm[((w * 2 + side) * C + i) * 16 + (l & 15)] = col[i + 1];
         }
     }
     __syncthreads();
 }
 
-// A x at cell i of the thread's column: i +- 1 from col, k +- 1 from the
+// A x at plane i of the thread's column: i +- 1 from col, k +- 1 from the
 // neighbouring lanes (DPP), j +- 1 from the lanes m apart (within the
 // wavefront; for m = 16 the wavefront's first / last row reads the LDS edge
 // rows of the neighbouring wavefront), face ghosts and coefficients from LDS.
 // Every lane of the workgroup calls it (cross-lane operations).
 template <int LM>
-__device__ __forceinline__ double tile_apply(const double *__restrict__ sm, const double (&col)[1 << LM], int i, int lb,
-                                             int j, int k, double inv_dt, double &diag) {
+__device__ __forceinline__ double tile_apply(const double *__restrict__ sm, const double (&col)[Planes<LM>::C + 2], int i,
+                                             int lb, int j, int k, double &diag) {
     using T = TileLds<LM>;
-    constexpr int m = T::m, mm = T::mm;
+    constexpr int m = T::m, C = T::C;
     const int t = threadIdx.x, lane = t & 63;
-    const int g = T::G0 + lb * 6 * mm;
-    const double x0 = col[i];
+    const double *G = sm + T::G0 + lb * 4 * C * m + i * m;       // face f at f * C * m
+    const double x0 = col[i + 1];
     const double dkm = dpp_d<0x111>(x0), dkp = dpp_d<0x101>(x0);
     double djm = __shfl(x0, (lane - m) & 63), djp = __shfl(x0, (lane + m) & 63);
     if (LM == 4) {
         const int w = t >> 6;
-        if (lane < 16 && w > 0) djm = sm[(((w - 1) * 2 + 1) * 16 + i) * 16 + k];
-        if (lane >= 48 && w < 3) djp = sm[(((w + 1) * 2 + 0) * 16 + i) * 16 + k];
+        if (lane < 16 && w > 0) djm = sm[(((w - 1) * 2 + 1) * C + i) * 16 + k];
+        if (lane >= 48 && w < 3) djp = sm[(((w + 1) * 2 + 0) * C + i) * 16 + k];
     }
-    const double xim = i > 0 ? col[i > 0 ? i - 1 : 0] : sm[g + j * m + k];
-    const double xip = i < m - 1 ? col[i < m - 1 ? i + 1 : 0] : sm[g + mm + j * m + k];
-    const double xjm = j > 0 ? djm : sm[g + 2 * mm + i * m + k];
-    const double xjp = j < m - 1 ? djp : sm[g + 3 * mm + i * m + k];
-    const double xkm = k > 0 ? dkm : sm[g + 4 * mm + i * m + j];
-    const double xkp = k < m - 1 ? dkp : sm[g + 5 * mm + i * m + j];
-    const double *ai = sm + T::CI + lb * (m + 1) * m;
-    const double *aj = sm + T::CJ + lb * m * (m + 1);
-    const int t2 = lb * mm + i * m + j;
+    const double xim = col[i], xip = col[i + 2];
+    const double xjm = j > 0 ? djm : G[k];
+    const double xjp = j < m - 1 ? djp : G[C * m + k];
+    const double xkm = k > 0 ? dkm : G[2 * C * m + j];
+    const double xkp = k < m - 1 ? dkp : G[3 * C * m + j];
+    const double *ai = sm + T::CI + lb * (C + 1) * m;
+    const double *aj = sm + T::CJ + lb * C * (m + 1);
+    const int t2 = lb * C * m + i * m + j;
     const double cim = ai[i * m + j], cip = ai[(i + 1) * m + j];
     const double cjm = aj[i * (m + 1) + j], cjp = aj[i * (m + 1) + j + 1];
     const double ck = sm[T::CK + t2];
-    diag = sm[T::CV + t2] * inv_dt + sm[T::CO + t2];
+    diag = sm[T::CD + t2];
     double nb = cim * xim + cip * xip;
     nb = nb + cjm * xjm + cjp * xjp;
     nb = nb + ck * xkm + ck * xkp;
@@ -330,31 +389,35 @@ __device__ __forceinline__ double tile_apply(const double *__restrict__ sm, cons
 }
 
 // One operator pass over every cell of a level: op.cell at each cell, dot
-// products per workgroup into partial (when given).
-template <int LM, class OP>
-__global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict__ x, const double *__restrict__ inv_dt,
-                                                const int *__restrict__ active, long long istride, OP op,
-                                                double *__restrict__ partial) {
-    constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM);
+// products per workgroup into partial (when given).  FIRST (Jacobi sweeps): x
+// is the first sweep's result from zero, formed from op.in0 = r, so the first
+// two sweeps are one pass.
+template <int LM, bool FIRST, class OP>
+__global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict__ x, const int *__restrict__ active,
+                                                long long istride, OP op, double omega, double *__restrict__ partial) {
+    constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM), C = Planes<LM>::C, S = Planes<LM>::S;
     __shared__ double sm[TileLds<LM>::SIZE];
     const int s = blockIdx.y;
     if (!active[s]) return;
     const int tid = threadIdx.x;
     const int lb = tid >> (2 * LM), j = (tid >> LM) & (m - 1), k = tid & (m - 1);
-    const int b0 = xcd_group(blockIdx.x, gridDim.x) * bpw, b = b0 + lb;
+    const int w = xcd_group(blockIdx.x, gridDim.x), h = w & (S - 1);
+    const int b0 = (w >> Planes<LM>::LS) * bpw, b = b0 + lb;
     const bool own = b < L.nb;
-    const Field F{x + s * istride};
+    const double *D = L.diag + s * ((long long)L.nb << (2 * LM));
     const long long so = s * istride;
+    const FieldT<FIRST> F{(FIRST ? op.in0 : x) + so, D, LM, omega};
     const long long cb = ((long long)b << (3 * LM)) + (j << LM) + k;
-    double col[m], a0[m], a1[m];
-    load_tile<LM, OP::IN0, OP::IN1>(L, F, b0, own, cb, op.in0, op.in1, so, col, a0, a1, sm);
+    double col[C + 2], a0[C], a1[C];
+    load_tile<LM, FIRST, OP::IN0, OP::IN1>(L, F, D, b0, h, own, cb, op.in0, op.in1, so, col, a0, a1, sm);
     double v[OP::NP] = {};
-    const double idt = inv_dt[s];
 #pragma unroll
-    for (int i = 0; i < m; i++) {
+    for (int i = 0; i < C; i++) {
         double diag;
-        const double ax = tile_apply<LM>(sm, col, i, lb, j, k, idt, diag);
-        if (own) op.cell(so + cb + (long long)i * mm, col[i], ax, diag, OP::IN0 ? a0[i] : 0.0, OP::IN1 ? a1[i] : 0.0, v);
+        const double ax = tile_apply<LM>(sm, col, i, lb, j, k, diag);
+        if (own)
+            op.cell(so + cb + (long long)(h * C + i) * mm, col[i + 1], ax, diag, OP::IN0 ? a0[i] : 0.0,
+                    OP::IN1 ? a1[i] : 0.0, v);
     }
     if (partial) block_partials<OP::NP>(v, partial, s);
 }
@@ -366,30 +429,31 @@ __global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict
 // by lane shuffles, the i pair from the thread's own column.
 template <int LM>
 __global__ void __launch_bounds__(256) k_hresrestrict(HLev L, const double *__restrict__ x, const double *__restrict__ r,
-                                                      double *__restrict__ rc, const double *__restrict__ inv_dt,
-                                                      const int *__restrict__ active, long long istride,
-                                                      long long cstride) {
-    constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM), LC = LM - 1;
+                                                      double *__restrict__ rc, const int *__restrict__ active,
+                                                      long long istride, long long cstride) {
+    constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM), LC = LM - 1, C = Planes<LM>::C, S = Planes<LM>::S;
+    static_assert(C >= 2, "an i pair of children belongs to one thread");
     __shared__ double sm[TileLds<LM>::SIZE];
     const int s = blockIdx.y;
     if (!active[s]) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int lb = tid >> (2 * LM), j = (tid >> LM) & (m - 1), k = tid & (m - 1);
-    const int b0 = xcd_group(blockIdx.x, gridDim.x) * bpw, b = b0 + lb;
+    const int w = xcd_group(blockIdx.x, gridDim.x), h = w & (S - 1);
+    const int b0 = (w >> Planes<LM>::LS) * bpw, b = b0 + lb;
     const bool own = b < L.nb;
-    const Field F{x + s * istride};
+    const double *D = L.diag + s * ((long long)L.nb << (2 * LM));
     const long long so = s * istride;
+    const Field F{x + so, D, LM, 0.0};
     const long long cb = ((long long)b << (3 * LM)) + (j << LM) + k;
-    double col[m], a0[m], a1[m];
-    load_tile<LM, true, false>(L, F, b0, own, cb, r, nullptr, so, col, a0, a1, sm);
-    const double idt = inv_dt[s];
+    double col[C + 2], a0[C], a1[C];
+    load_tile<LM, false, true, false>(L, F, D, b0, h, own, cb, r, nullptr, so, col, a0, a1, sm);
     const bool out = own && !(j & 1) && !(k & 1);
     double *R = rc + s * cstride + ((long long)b << (3 * LC)) + ((j >> 1) << LC) + (k >> 1);
 #pragma unroll
-    for (int ic = 0; ic < m / 2; ic++) {
+    for (int ic = 0; ic < C / 2; ic++) {
         double diag;
-        const double ax0 = tile_apply<LM>(sm, col, 2 * ic, lb, j, k, idt, diag);
-        const double ax1 = tile_apply<LM>(sm, col, 2 * ic + 1, lb, j, k, idt, diag);
+        const double ax0 = tile_apply<LM>(sm, col, 2 * ic, lb, j, k, diag);
+        const double ax1 = tile_apply<LM>(sm, col, 2 * ic + 1, lb, j, k, diag);
         const double o0 = own ? a0[2 * ic] - ax0 : 0.0, o1 = own ? a0[2 * ic + 1] - ax1 : 0.0;
         const double k0 = __shfl(o0, (lane + 1) & 63, 64), k1 = __shfl(o1, (lane + 1) & 63, 64);
         const double j0 = __shfl(o0, (lane + m) & 63, 64), j1 = __shfl(o1, (lane + m) & 63, 64);
@@ -397,20 +461,20 @@ __global__ void __launch_bounds__(256) k_hresrestrict(HLev L, const double *__re
         double t = 0.0;
         t += o0; t += k0; t += j0; t += q0;
         t += o1; t += k1; t += j1; t += q1;
-        if (out) R[(long long)ic << (2 * LC)] = t;
+        if (out) R[(long long)(h * (C / 2) + ic) << (2 * LC)] = t;
     }
 }
 
 // Jacobi from x = 0: y = (omega r)/diag (the damped Jacobi value at x = 0)
 __global__ void __launch_bounds__(256) k_hjacobi0(HLev L, const double *__restrict__ r, double *__restrict__ y,
-                                                  const double *__restrict__ inv_dt, const int *__restrict__ active,
+                                                  const int *__restrict__ active,
                                                   long long istride, double omega) {
     const int s = blockIdx.y;
     if (!active[s]) return;
     const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= (long long)L.nb * L.M3) return;
     const long long io = s * istride + c;
-    y[io] = (omega * r[io]) / diag_at(L, cell_of(L, c), inv_dt[s]);
+    y[io] = (omega * r[io]) / L.diag[s * (((long long)L.nb * L.M3) >> L.lm) + (c >> L.lm)];
 }
 
 // Linear prolongation, stored: fine cell (i, j, k) of level LM adds
@@ -436,7 +500,7 @@ __global__ void __launch_bounds__(256) k_hprolong_lin(HLev Lc, double *__restric
     const int ic = i >> 1, jc = j >> 1, kc = k >> 1;
     const int si = (i & 1) ? 1 : -1, sj = (j & 1) ? 1 : -1, sk = (k & 1) ? 1 : -1;
     const double *Z = zc + s * cstride;
-    const Field F{Z};
+    const Field F{Z, nullptr, 0, 0.0};
     const long long cb = ((long long)b << (3 * LC)) + (ic << (2 * LC)) + (jc << LC) + kc;
     const double z0 = Z[cb];
     const int2 *E = Lc.gsw + (long long)b * 6 * mmc;
@@ -783,7 +847,7 @@ __global__ void __launch_bounds__(256) k_pfss_field(HLev L, const double *__rest
     { const int i = q.k; q.k = q.i; q.i = i; }
     const int m = L.m;
     const long long mm = (long long)m * m, cb = (long long)q.b * L.M3, c = cb + ((long long)q.i * m + q.j) * m + q.k;
-    const Field F{x};
+    const Field F{x, nullptr, 0, 0.0};
     // the face ghost of face f (i-, i+, j-, j+, k-, k+) at in-face position (t1, t2)
     auto ghost = [&](int f, int t1, int t2) -> double {
         const int2 e = L.gsw[((long long)q.b * 6 + f) * mm + (long long)t1 * m + t2];
@@ -848,8 +912,8 @@ __global__ void __launch_bounds__(256) k_hupdate_p2(long long n, double *__restr
     p[io] = (z[io] + a * cc[io]) - be * p[io];
 }
 
-// Per-block correction steps (16^3 blocks, one block per workgroup of the
-// correction's dot pass): a_b = <c_b,r'_b>/<c_b,(Ac)_b> (0 unless the
+// Per-block correction steps (16^3 blocks, S consecutive workgroups of the
+// correction's dot pass each): a_b = <c_b,r'_b>/<c_b,(Ac)_b> (0 unless the
 // denominator is positive), and in partial slot 0 the block's a_b <c_b,q_b>
 __global__ void __launch_bounds__(256) k_hblockstep(int nwg, int nb, double *__restrict__ partial,
                                                     double *__restrict__ ablk, const int *__restrict__ active) {
@@ -857,9 +921,20 @@ __global__ void __launch_bounds__(256) k_hblockstep(int nwg, int nb, double *__r
     if (!active[s]) return;
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= nwg) return;
-    const int b = xcd_group(w, nwg);
+    // the S workgroups of a block: its parts' sums in order, by the first of them
+    constexpr int S = Planes<4>::S;
+    const int g = xcd_group(w, nwg), b = g / S;
+    if (g % S) return;
     double *P = partial + (long long)s * 3 * nwg;
-    const double num = P[w], den = P[nwg + w], cq = P[2 * nwg + w];
+    int o[S];
+    for (int h = 0; h < S; h++) o[h] = xcd_slot(g + h, nwg);
+    double num = P[o[0]], den = P[nwg + o[0]], cq = P[2 * nwg + o[0]];
+    for (int h = 1; h < S; h++) {
+        num += P[o[h]];
+        den += P[nwg + o[h]];
+        cq += P[2 * nwg + o[h]];
+        P[o[h]] = 0.0;
+    }
     const double a = num / den;
     const double ab = (den > 0.0 && a == a && a < 1e300 && a > -1e300) ? a : 0.0;
     ablk[(long long)s * nb + b] = ab;
@@ -933,7 +1008,7 @@ struct HeatSolver::Impl {
     // and elementwise (kElem cells each); their dot partials are per workgroup
     unsigned march_wgs(int l) const {
         const int bpw = 256 >> (2 * L[l].lm);
-        return (unsigned)((nb + bpw - 1) / bpw);
+        return (unsigned)((nb + bpw - 1) / bpw) << (L[l].lm < 2 ? 0 : 1);      // x Planes<LM>::S
     }
     unsigned elem_wgs() const { return (unsigned)((ist(0) + kElem - 1) / kElem); }
     dim3 grid_elem() const { return dim3(elem_wgs(), (unsigned)nsys); }
@@ -985,19 +1060,19 @@ struct HeatSolver::Impl {
         std::vector<int> one(nsys, 1);
         HCHECK(hipMemcpy(active, one.data(), sizeof(int) * nsys, hipMemcpyHostToDevice));
     }
-    template <class OP>
+    template <bool FIRST = false, class OP>
     void launch_march(int l, const double *x_, const OP &op, double *part) {
         const dim3 g(march_wgs(l), (unsigned)nsys);
         const HLev &D = L[l];
-        const double *idt = inv_dt;
         const int *ac = active;
         const long long is = ist(l);
+        const double om = omega;
         switch (D.lm) {
-            case 0: hipLaunchKernelGGL((k_hmarch<0, OP>), g, dim3(256), 0, stream, D, x_, idt, ac, is, op, part); break;
-            case 1: hipLaunchKernelGGL((k_hmarch<1, OP>), g, dim3(256), 0, stream, D, x_, idt, ac, is, op, part); break;
-            case 2: hipLaunchKernelGGL((k_hmarch<2, OP>), g, dim3(256), 0, stream, D, x_, idt, ac, is, op, part); break;
-            case 3: hipLaunchKernelGGL((k_hmarch<3, OP>), g, dim3(256), 0, stream, D, x_, idt, ac, is, op, part); break;
-            case 4: hipLaunchKernelGGL((k_hmarch<4, OP>), g, dim3(256), 0, stream, D, x_, idt, ac, is, op, part); break;
+            case 0: hipLaunchKernelGGL((k_hmarch<0, FIRST, OP>), g, dim3(256), 0, stream, D, x_, ac, is, op, om, part); break;
+            case 1: hipLaunchKernelGGL((k_hmarch<1, FIRST, OP>), g, dim3(256), 0, stream, D, x_, ac, is, op, om, part); break;
+            case 2: hipLaunchKernelGGL((k_hmarch<2, FIRST, OP>), g, dim3(256), 0, stream, D, x_, ac, is, op, om, part); break;
+            case 3: hipLaunchKernelGGL((k_hmarch<3, FIRST, OP>), g, dim3(256), 0, stream, D, x_, ac, is, op, om, part); break;
+            case 4: hipLaunchKernelGGL((k_hmarch<4, FIRST, OP>), g, dim3(256), 0, stream, D, x_, ac, is, op, om, part); break;
             default: throw std::runtime_error("heat blocks are at most 16^3");
         }
     }
@@ -1005,13 +1080,13 @@ struct HeatSolver::Impl {
     void restrict_residual(int l) {
         const dim3 g(march_wgs(l), (unsigned)nsys);
         const HLev &D = L[l];
-        const double *z = Z[l], *rr = R[l], *idt = inv_dt;
+        const double *z = Z[l], *rr = R[l];
         const int *ac = active;
         switch (D.lm) {
-            case 1: hipLaunchKernelGGL(k_hresrestrict<1>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], idt, ac, ist(l), ist(l + 1)); break;
-            case 2: hipLaunchKernelGGL(k_hresrestrict<2>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], idt, ac, ist(l), ist(l + 1)); break;
-            case 3: hipLaunchKernelGGL(k_hresrestrict<3>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], idt, ac, ist(l), ist(l + 1)); break;
-            case 4: hipLaunchKernelGGL(k_hresrestrict<4>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], idt, ac, ist(l), ist(l + 1)); break;
+            case 1: hipLaunchKernelGGL(k_hresrestrict<1>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], ac, ist(l), ist(l + 1)); break;
+            case 2: hipLaunchKernelGGL(k_hresrestrict<2>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], ac, ist(l), ist(l + 1)); break;
+            case 3: hipLaunchKernelGGL(k_hresrestrict<3>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], ac, ist(l), ist(l + 1)); break;
+            case 4: hipLaunchKernelGGL(k_hresrestrict<4>, g, dim3(256), 0, stream, D, z, rr, R[l + 1], ac, ist(l), ist(l + 1)); break;
             default: throw std::runtime_error("no restriction below 2^3 cells per block");
         }
     }
@@ -1027,10 +1102,25 @@ struct HeatSolver::Impl {
         else launch_march(l, Z[l], OpJacobi<false>{Z2[l], R[l], nullptr, omega}, nullptr);
         std::swap(Z[l], Z2[l]);
     }
+    // the first two sweeps from zero in one pass: Z[l] = sweep of omega R[l] / diag
+    void sweep01(int l) {
+        launch_march<true>(l, nullptr, OpJacobi<false>{Z2[l], R[l], nullptr, omega}, nullptr);
+        std::swap(Z[l], Z2[l]);
+    }
     // first sweep from zero: Z[l] = omega R[l] / diag
     void sweep0(int l) {
         hipLaunchKernelGGL(k_hjacobi0, grid_cells(l), dim3(256), 0, stream, L[l], (const double *)R[l], Z[l],
-                           (const double *)inv_dt, (const int *)active, ist(l), omega);
+                           (const int *)active, ist(l), omega);
+    }
+    // the levels' diagonals at the current 1/dt
+    void diagonals() {
+        for (int l = 0; l < nlev; l++) {
+            const long long n2 = (long long)nb * L[l].m * L[l].m;
+            hipLaunchKernelGGL(k_hdiag, dim3((unsigned)((n2 + 255) / 256), (unsigned)nsys), dim3(256), 0, stream, L[l],
+                               const_cast<double *>(L[l].diag), (const double *)inv_dt, n2);
+        }
+        HCHECK(hipGetLastError());
+        HCHECK(hipStreamSynchronize(stream));
     }
 
     // zf (level l) += linear prolongation of level l+1
@@ -1071,8 +1161,9 @@ struct HeatSolver::Impl {
             if (sweeps == 0) {
                 zero(Z[l], ist(l) * nsys);
             } else {
-                sweep0(l);
-                for (int s = 1; s < sweeps; s++) sweep(l, nullptr);
+                if (sweeps == 1) sweep0(l);
+                else sweep01(l);
+                for (int s = 2; s < sweeps; s++) sweep(l, nullptr);
             }
             restrict_residual(l);
         }
@@ -1166,6 +1257,8 @@ void HeatSolver::setup(const Layout &lay, const HeatParams &hp, int nsys, int nt
     I.tmp = I.dalloc(I.ist(0) * nsys);
     I.p = I.dalloc(I.ist(0) * nsys);
     I.inv_dt = I.dalloc(nsys);
+    for (int l = 0; l < I.nlev; l++) I.L[l].diag = I.dalloc((size_t)nsys * I.nb * I.L[l].m * I.L[l].m);
+    I.diagonals();
     I.partial = I.dalloc((size_t)nsys * 3 * std::max(I.march_wgs(0), I.elem_wgs()));
     I.dots = I.dalloc((size_t)nsys * 3);
     I.sc = I.dalloc((size_t)nsys * kSc);
@@ -1223,6 +1316,7 @@ void HeatSolver::set_dt(const std::vector<double> &dt) {
     std::vector<double> inv(I.nsys);
     for (int s = 0; s < I.nsys; s++) inv[s] = 1.0 / dt[s];
     HCHECK(hipMemcpy(I.inv_dt, inv.data(), sizeof(double) * I.nsys, hipMemcpyHostToDevice));
+    I.diagonals();
 }
 
 void HeatSolver::set_rhs_from_T(const std::vector<double> &T) {

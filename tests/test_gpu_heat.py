@@ -175,3 +175,22 @@ def test_graph_follows_a_tolerance_change():
     print("tol change", it10.tolist(), it6_g.tolist(), it6_e.tolist(), flush=True)
     assert np.array_equal(it6_g, it6_e) and np.array_equal(rel6_g, rel6_e)
     assert (rel6_g <= 1e-6).all() and (it6_g < it10).all()
+
+
+# blocks of every edge the kernels are built for, numbers of blocks that leave a
+# workgroup's last blocks empty, and 24, 1800 and 2880 rows on the coarsest level
+# (one and two rows per thread, and the form for any number)
+@pytest.mark.parametrize("edge,split,sweeps_dt", [(2, (1, 2, 6), 40.0), (4, (1, 2, 6), 40.0), (16, (1, 2, 6), 100.0),
+                                                  (2, (3, 10, 30), 100.0), (2, (4, 12, 30), 1000.0)])
+def test_operator_and_vcycle_bitexact_for_block_edges(edge, split, sweeps_dt):
+    lay = {"ni": edge, "nj": edge, "nk": edge, "ng": 2, "r_rsun": configs.R_RANGE, "ops": [("split", split)]}
+    H = pyoracle.HeatOracle(pyoracle.Oracle(lay), KAPPA0, RREF)
+    hs = HeatSolver(Shell(lay), KAPPA0, RREF, 2)
+    dt = np.array([1.0, sweeps_dt]) * H.dt_explicit
+    hs.set_dt(dt)
+    r = np.random.default_rng(edge).standard_normal(hs.shape)
+    print("[heat edges]", edge, split, flush=True)
+    y, z = hs.apply(r), hs.vcycle(r)
+    for k in range(2):
+        assert np.array_equal(y[k], H.apply(dt[k], r[k])), (edge, k)
+        assert np.array_equal(z[k], H.vcycle(dt[k], r[k])), (edge, k)
