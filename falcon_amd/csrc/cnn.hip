@@ -507,6 +507,7 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
 // small batch still spreads over 7 workgroups per image.
 constexpr int WA_CH = 16 * 16 + 8, WA_PL = 16 * WA_CH;           // g planes: rows of 16, channels 528 bytes apart
 constexpr int WB_ROW = 24, WB_CH = 18 * WB_ROW + 8, WB_PL = 16 * WB_CH;   // input planes: 8 zeros, 16 voxels; channels 880 bytes apart
+constexpr int WDEPTH = 2;                                        // planes in flight
 constexpr int WX_CP = 18 * 18 * 16;                              // one shifted copy of x
 constexpr int W_TOTAL = 3 * WX_CP + 2 * WA_PL > 2 * (WA_PL + WB_PL) ? 3 * WX_CP + 2 * WA_PL : 2 * (WA_PL + WB_PL);
 
@@ -550,35 +551,39 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
               n = lane & 15;
     const int vg = tid >> 2, j4 = vg >> 2, k4 = 4 * (vg & 3), c4 = 4 * (tid & 3);
     for (int q = tid; q < 2 * (WA_PL + WB_PL) / 8; q += 256) reinterpret_cast<uint4 *>(sm)[q] = make_uint4(0u, 0u, 0u, 0u);
-    Quad qa, qb;
-    float gf = 0.0f;
-    auto fetch = [&](int p) {
-        if (L == 2) qa.load(reinterpret_cast<const uint16_t *>(g_), p, tid);
-        else gf = reinterpret_cast<const float *>(g_)[p * 256 + tid];
+    // planes p + 1 .. p + WDEPTH are on their way while plane p is computed
+    Quad qa[WDEPTH], qb[WDEPTH];
+    float gf[WDEPTH];
+    auto fetch = [&](int p, int u) {
+        if (L == 2) qa[u].load(reinterpret_cast<const uint16_t *>(g_), p, tid);
+        else gf[u] = reinterpret_cast<const float *>(g_)[p * 256 + tid];
         const int q = p + di;
-        if (q >= 0 && q < 16) qb.load(in, q, tid);
-        else qb.clear();
+        qb[u].load(in, q < 0 ? 0 : (q > 15 ? 15 : q), tid);
     };
-    auto stage = [&](int p) {
+    auto stage = [&](int p, int u) {
         uint16_t *A = sm + (p & 1) * (WA_PL + WB_PL), *B = A + WA_PL;
         if (L == 2) {
-            qa.store(A + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+            qa[u].store(A + c4 * WA_CH + j4 * 16 + k4, WA_CH);
         } else {
-            A[tid] = f2bf(gf);
-            sF[(p & 1) * 256 + tid] = gf;
+            A[tid] = f2bf(gf[u]);
+            sF[(p & 1) * 256 + tid] = gf[u];
         }
-        qb.store(B + c4 * WB_CH + (j4 + 1) * WB_ROW + 8 + k4, WB_CH);
+        if (p + di < 0 || p + di > 15) qb[u].clear();      // beyond the block: zeros
+        qb[u].store(B + c4 * WB_CH + (j4 + 1) * WB_ROW + 8 + k4, WB_CH);
     };
     f4 acc[3];
 #pragma unroll
     for (int a = 0; a < 3; a++) acc[a] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float bias_acc = 0.0f;    // thread tid: channel tid & 15, voxels of its plane rows (tid >> 4)
-    fetch(0);
+    const uint32_t row0 = n == 0 ? 0xffffffffu : 0u;      // layer 3: the only row of A
+#pragma unroll
+    for (int u = 0; u < WDEPTH; u++) fetch(u, u);
     __syncthreads();
-    stage(0);
+    stage(0, 0);
+#pragma unroll WDEPTH
     for (int p = 0; p < 16; p++) {
         __syncthreads();
-        if (p + 1 < 16) fetch(p + 1);
+        if (p + WDEPTH < 16) fetch(p + WDEPTH, p % WDEPTH);
         const uint16_t *A = sm + (p & 1) * (WA_PL + WB_PL), *B = A + WA_PL;
         if (di == 0) {
             const int c = tid & 15, jr = tid >> 4;
@@ -590,27 +595,35 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
             }
         }
         if (wave < 3) {
+            // all operands of 4 chunks are read before the first is used
+            const uint16_t *Ap = A + (L == 2 ? n * WA_CH : 0) + (g >> 1) * 16 + 8 * (g & 1);
+            const uint16_t *Bp = B + n * WB_CH + (wave + (g >> 1)) * WB_ROW + 8 + 8 * (g & 1);
 #pragma unroll
-            for (int ch = 0; ch < 8; ch++) {
-                const int jj = 2 * ch + (g >> 1), k0 = 8 * (g & 1);
-                uint4 a;
-                if (L == 2) {
-                    a = *reinterpret_cast<const uint4 *>(A + n * WA_CH + jj * 16 + k0);
-                } else {
-                    a = *reinterpret_cast<const uint4 *>(A + jj * 16 + k0);
-                    if (n != 0) a = make_uint4(0u, 0u, 0u, 0u);
+            for (int c0 = 0; c0 < 8; c0 += 4) {
+                uint4 a[4], b[4];
+                uint32_t pv[4], nx[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    a[u] = *reinterpret_cast<const uint4 *>(Ap + (c0 + u) * 32);
+                    const uint16_t *row = Bp + (c0 + u) * 2 * WB_ROW;
+                    b[u] = *reinterpret_cast<const uint4 *>(row);
+                    pv[u] = *reinterpret_cast<const uint32_t *>(row - 2);
+                    nx[u] = *reinterpret_cast<const uint32_t *>(row + 8);
                 }
-                const uint16_t *row = B + n * WB_CH + (jj + wave) * WB_ROW + 8 + k0;
-                const uint4 b = *reinterpret_cast<const uint4 *>(row);
-                const uint32_t pv = *reinterpret_cast<const uint32_t *>(row - 2), nx = *reinterpret_cast<const uint32_t *>(row + 8);
-                const uint32_t s1 = __builtin_amdgcn_alignbit(b.y, b.x, 16), s2 = __builtin_amdgcn_alignbit(b.z, b.y, 16),
-                               s3 = __builtin_amdgcn_alignbit(b.w, b.z, 16);
-                acc[0] = mfma32(a, make_uint4(__builtin_amdgcn_alignbit(b.x, pv, 16), s1, s2, s3), acc[0]);
-                acc[1] = mfma32(a, b, acc[1]);
-                acc[2] = mfma32(a, make_uint4(s1, s2, s3, __builtin_amdgcn_alignbit(nx, b.w, 16)), acc[2]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (L == 3) a[u] = make_uint4(a[u].x & row0, a[u].y & row0, a[u].z & row0, a[u].w & row0);
+                    const uint32_t s1 = __builtin_amdgcn_alignbit(b[u].y, b[u].x, 16),
+                                   s2 = __builtin_amdgcn_alignbit(b[u].z, b[u].y, 16),
+                                   s3 = __builtin_amdgcn_alignbit(b[u].w, b[u].z, 16);
+                    acc[0] = mfma32(a[u], make_uint4(__builtin_amdgcn_alignbit(b[u].x, pv[u], 16), s1, s2, s3), acc[0]);
+                    acc[1] = mfma32(a[u], b[u], acc[1]);
+                    acc[2] = mfma32(a[u], make_uint4(s1, s2, s3, __builtin_amdgcn_alignbit(nx[u], b[u].w, 16)), acc[2]);
+                }
             }
         }
-        if (p + 1 < 16) stage(p + 1);
+        if (p + 1 < 16) stage(p + 1, (p + 1) % WDEPTH);
     }
     // D[co = 4g + r][n]
     if (wave < 3) {
@@ -646,8 +659,9 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
 #pragma unroll
     for (int p = 0; p < 16; p++) xv[p] = x[p * 256 + tid];
     for (int q = tid; q < 3 * WX_CP / 8; q += 256) reinterpret_cast<uint4 *>(xs)[q] = make_uint4(0u, 0u, 0u, 0u);
-    Quad qa;
-    qa.load(g1, 0, tid);
+    Quad qa[WDEPTH];
+#pragma unroll
+    for (int u = 0; u < WDEPTH; u++) qa[u].load(g1, u, tid);
     __syncthreads();
     // copy dk + 1, row (plane + 1, j + 1): element k holds x at k + dk
 #pragma unroll
@@ -659,29 +673,36 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
         row[WX_CP + k] = v;
         if (k > 0) row[2 * WX_CP + k - 1] = v;
     }
-    qa.store(sm + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+    qa[0].store(sm + c4 * WA_CH + j4 * 16 + k4, WA_CH);
     const int t = 16 * wave + n;
     const bool on = t < 27;
+    const uint32_t taps = on ? 0xffffffffu : 0u;
     const int u = on ? t : 0;
     const uint16_t *src = xs + (u % 3) * WX_CP + ((u / 9) * 18 + (u / 3) % 3) * 16;
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     float bias_acc = 0.0f;
+#pragma unroll WDEPTH
     for (int p = 0; p < 16; p++) {
         __syncthreads();
-        if (p + 1 < 16) qa.load(g1, p + 1, tid);
+        if (p + WDEPTH < 16) qa[p % WDEPTH].load(g1, p + WDEPTH, tid);
         const uint16_t *A = sm + (p & 1) * WA_PL;
         bias_acc = row_sum(A + (tid & 15) * WA_CH + (tid >> 4) * 16, bias_acc);
         if (wave < 2) {
 #pragma unroll
-            for (int ch = 0; ch < 8; ch++) {
-                const int jj = 2 * ch + (g >> 1), k0 = 8 * (g & 1);
-                const uint4 a = *reinterpret_cast<const uint4 *>(A + n * WA_CH + jj * 16 + k0);
-                uint4 b = *reinterpret_cast<const uint4 *>(src + (p * 18 + jj) * 16 + k0);
-                if (!on) b = make_uint4(0u, 0u, 0u, 0u);
-                acc = mfma32(a, b, acc);
+            for (int c0 = 0; c0 < 8; c0 += 4) {
+                uint4 a[4], b[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    a[u] = *reinterpret_cast<const uint4 *>(A + n * WA_CH + (2 * (c0 + u) + (g >> 1)) * 16 + 8 * (g & 1));
+                    b[u] = *reinterpret_cast<const uint4 *>(src + (p * 18 + 2 * (c0 + u) + (g >> 1)) * 16 + 8 * (g & 1));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    acc = mfma32(a[u], make_uint4(b[u].x & taps, b[u].y & taps, b[u].z & taps, b[u].w & taps), acc);
             }
         }
-        if (p + 1 < 16) qa.store(sm + ((p + 1) & 1) * WA_PL + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+        if (p + 1 < 16) qa[(p + 1) % WDEPTH].store(sm + ((p + 1) & 1) * WA_PL + c4 * WA_CH + j4 * 16 + k4, WA_CH);
     }
     if (wave < 2 && on)
         for (int r = 0; r < 4; r++) P[OFF_W1 + t * 16 + 4 * g + r] = acc[r];
@@ -694,7 +715,7 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
     }
 }
 
-__global__ void __launch_bounds__(256) k_cnn_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ h1,
+__global__ void __launch_bounds__(256, 3) k_cnn_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ h1,
                                                    const uint16_t *__restrict__ h2, const uint16_t *__restrict__ g1,
                                                    const uint16_t *__restrict__ g2, const float *__restrict__ g3,
                                                    float *__restrict__ part, const long long *__restrict__ idx) {
@@ -708,18 +729,27 @@ __global__ void __launch_bounds__(256) k_cnn_wgrad(const float *__restrict__ x, 
     else wgrad_first(x + (idx ? idx[img] : img) * 4096, g1 + v * 16, P, sm, sBias);
 }
 
-// grad[q] = sum over images of part[img][q], fixed order, FP64, 16 images in
+// grad[q] = sum over images of part[img][q], fixed order, FP64, 32 images in
 // flight (the additions keep their order, the loads do not wait for them)
 __device__ __forceinline__ double part_sum(const float *__restrict__ part, int nimg, int q) {
     double s = 0.0;
-    for (int i0 = 0; i0 < nimg; i0 += 16) {
-        float v[16];
+    const float *P = part + q;
+    int i0 = 0;
+    for (; i0 + 32 <= nimg; i0 += 32, P += 32LL * kCnnParams) {
+        float v[32];
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = i0 + i < nimg ? part[(long long)(i0 + i) * kCnnParams + q] : 0.0f;
+        for (int i = 0; i < 32; i++) v[i] = P[(long long)i * kCnnParams];
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (i0 + i < nimg) s += (double)v[i];
+        for (int i = 0; i < 32; i++) s += (double)v[i];
     }
+    for (; i0 + 4 <= nimg; i0 += 4, P += 4LL * kCnnParams) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = P[(long long)i * kCnnParams];
+#pragma unroll
+        for (int i = 0; i < 4; i++) s += (double)v[i];
+    }
+    for (; i0 < nimg; i0++, P += kCnnParams) s += (double)P[0];
     return s;
 }
 __global__ void __launch_bounds__(64) k_cnn_reduce(const float *__restrict__ part, int nimg, double *__restrict__ grad) {
