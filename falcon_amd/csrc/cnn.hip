@@ -151,6 +151,9 @@ __device__ __forceinline__ void pack_forward(const float *__restrict__ p, uint16
 //     taps (accumulated over di), combined by DPP shifts (dk) and lane shuffles
 //     (dj) into the output line.
 // STORE also writes h1/h2 (channel-fastest) for the backward pass.
+// A march is a serial chain of planes: 37 to 42 us per image alone on a CU.  An
+// image is cut in i segments (each recomputes the planes its first needs, the
+// same bits) while they still get a CU each, see fwd_segments.
 struct HeatIO {                 // solver form of the forward (HEAT = true)
     const double *scale;       // per system, stride scale_stride
     int scale_stride, nb;
@@ -179,6 +182,9 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
                                                  const long long *__restrict__ idx) {
     __shared__ __align__(16) uint16_t sm[F_TOTAL];
     const long long img = blockIdx.x;
+    // output planes pa .. pb - 1 of the image (blockIdx.y of gridDim.y segments):
+    // the march starts with the h1 plane two before and ends with the one two after
+    const int pa = 16 * blockIdx.y / gridDim.y, pb = 16 * (blockIdx.y + 1) / gridDim.y, first = pa > 2 ? pa - 2 : 0;
     double sc = 1.0;
     float inv_sc = 1.0f;
     if (HEAT) {
@@ -244,9 +250,12 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
         sm[F_X + (q % 3) * PL + (xj + 1) * 18 + xk + 1] = cvt1(HEAT ? v * inv_sc : v);
     };
 
-    if (xl) store_x(0, fetch_x(0));
-    float xnext = xl ? fetch_x(1) : 0.0f;
-    for (int step = 0; step <= 17; step++) {
+    if (xl) {
+        if (first > 0) store_x(first - 1, fetch_x(first - 1));
+        store_x(first, fetch_x(first));
+    }
+    float xnext = xl ? fetch_x(first + 1) : 0.0f;
+    for (int step = first; step <= pb + 1; step++) {
         if (xl && step + 1 <= 16) {
             store_x(step + 1, xnext);
             if (step + 2 <= 16) xnext = fetch_x(step + 2);
@@ -284,7 +293,7 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
                 const uint2 o = cvt4(relu(acc[jj][0] + bb1[0]), relu(acc[jj][1] + bb1[1]), relu(acc[jj][2] + bb1[2]),
                                      relu(acc[jj][3] + bb1[3]));
                 *reinterpret_cast<uint2 *>(sm + F_H1 + (p % 3) * HPL + (j + 1) * HROW + oB) = o;
-                if (STORE) *reinterpret_cast<uint2 *>(h1g + ((img * 4096 + (p * 16 + j) * 16 + n) * 16 + 4 * g)) = o;
+                if (STORE && p >= pa && p < pb) *reinterpret_cast<uint2 *>(h1g + ((img * 4096 + (p * 16 + j) * 16 + n) * 16 + 4 * g)) = o;
             }
         }
         __syncthreads();
@@ -293,7 +302,7 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
             for (int jj = 0; jj < LPW; jj++)
                 *reinterpret_cast<uint2 *>(sm + F_H2 + (16 % 3) * HPL + (j0 + jj + 1) * HROW + oB) = make_uint2(0u, 0u);
         }
-        if (step >= 1 && step <= 16) {          // h2 plane step-1
+        if (step > first + (pa > 0) && step <= 16) {          // h2 plane step-1
             const int p = step - 1;
             // the 16x16x32 and 16x16x16 products accumulate in separate chains
             // (an accumulator is never shared by MFMAs of different shapes)
@@ -332,11 +341,11 @@ __global__ void __launch_bounds__(64 * NW) k_cnn_fwd(const float *__restrict__ x
                 const f4 a = acc[jj] + acc16[jj];
                 const uint2 o = cvt4(relu(a[0] + bb2[0]), relu(a[1] + bb2[1]), relu(a[2] + bb2[2]), relu(a[3] + bb2[3]));
                 *reinterpret_cast<uint2 *>(sm + F_H2 + (p % 3) * HPL + (j + 1) * HROW + oB) = o;
-                if (STORE) *reinterpret_cast<uint2 *>(h2g + ((img * 4096 + (p * 16 + j) * 16 + n) * 16 + 4 * g)) = o;
+                if (STORE && p >= pa && p < pb) *reinterpret_cast<uint2 *>(h2g + ((img * 4096 + (p * 16 + j) * 16 + n) * 16 + 4 * g)) = o;
             }
         }
         __syncthreads();
-        if (step >= 2) {                        // output plane step-2
+        if (step >= pa + 2) {                   // output plane step-2
             const int p = step - 2;
             f4 D[LPW + 2];
 #pragma unroll
@@ -382,13 +391,18 @@ constexpr int DPL = 4;                      // output planes per workgroup
 // Layer 3 -> 2 (gin: the float output gradient, weights Q3): one MFMA per
 // k-line, K = the 27 taps.  Bound by the LDS gather of the taps; their offsets
 // are formed once per lane, a line's row is an immediate.  128
-// images: 48 -> 11.5 us against one workgroup per image with the offsets formed per read.
+// images: 48 -> 9.7 us against one workgroup per image with the offsets formed
+// per read and the masks read where they are used (loads now come first).
 __global__ void __launch_bounds__(256) k_cnn_dgrad1(const float *__restrict__ gin, const uint16_t *__restrict__ mask,
                                                     uint16_t *__restrict__ gout, const us8 *__restrict__ pk) {
     __shared__ __align__(16) uint16_t sm[(DPL + 2) * PL];
     const long long img = blockIdx.x;
     const int p0 = blockIdx.y * DPL;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, kk = lane & 15;
+    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
+    uint2 mk[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) mk[j] = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
     float v[DPL + 2];
 #pragma unroll
     for (int q = 0; q < DPL + 2; q++) {
@@ -409,16 +423,14 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad1(const float *__restrict__ gi
         on[e] = t < 27;
         src[e] = sm + (on[e] ? (wave + t / 9) * PL + (t / 3) % 3 * 18 + t % 3 + kk : 0);
     }
-    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
 #pragma unroll
     for (int j = 0; j < 16; j++) {
         us8 b;
 #pragma unroll
         for (int e = 0; e < 8; e++) b[e] = on[e] ? src[e][j * 18] : (uint16_t)0;
         const f4 acc = mfma(w, b, f4{0.0f, 0.0f, 0.0f, 0.0f});
-        const uint2 mk = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
-        const float m0 = bf2f((uint16_t)(mk.x & 0xffffu)), m1 = bf2f((uint16_t)(mk.x >> 16)),
-                    m2 = bf2f((uint16_t)(mk.y & 0xffffu)), m3 = bf2f((uint16_t)(mk.y >> 16));
+        const float m0 = bf2f((uint16_t)(mk[j].x & 0xffffu)), m1 = bf2f((uint16_t)(mk[j].x >> 16)),
+                    m2 = bf2f((uint16_t)(mk[j].y & 0xffffu)), m3 = bf2f((uint16_t)(mk[j].y >> 16));
         *reinterpret_cast<uint2 *>(gout + o0 + j * 256) = pack4(m0 > 0.0f ? acc[0] : 0.0f, m1 > 0.0f ? acc[1] : 0.0f,
                                                                 m2 > 0.0f ? acc[2] : 0.0f, m3 > 0.0f ? acc[3] : 0.0f);
     }
@@ -428,7 +440,7 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad1(const float *__restrict__ gi
 // MFMAs per k-line in one chain, K = (tap pair, channel).  LDS [plane][channel
 // half][18][18][8]: the lanes of a 16-byte read are consecutive (no bank
 // conflicts); bound by those reads, 14 per line and wavefront.  128
-// images: 53 -> 14.7 us against one workgroup per image on [voxel][16] planes.
+// images: 53 -> 15 us against one workgroup per image on [voxel][16] planes.
 __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict__ gin, const uint16_t *__restrict__ mask,
                                                      uint16_t *__restrict__ gout, const us8 *__restrict__ pk) {
     constexpr int HP = PL * 8;              // elements per half plane
@@ -436,6 +448,10 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
     const long long img = blockIdx.x;
     const int p0 = blockIdx.y * DPL;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, kk = lane & 15;
+    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
+    uint2 mk[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) mk[j] = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
     uint4 v[DPL + 2][2];
 #pragma unroll
     for (int q = 0; q < DPL + 2; q++) {
@@ -467,10 +483,8 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
         off[s] = ((wave + u / 9) * 2 + (g & 1)) * HP + ((u / 3) % 3 * 18 + u % 3 + kk) * 8;
     }
     const bool last = g < 2;
-    const long long o0 = (img * 4096 + ((p0 + wave) * 16) * 16 + kk) * 16 + 4 * g;
-#pragma unroll 4
+#pragma unroll
     for (int j = 0; j < 16; j++) {
-        const uint2 mk = *reinterpret_cast<const uint2 *>(mask + o0 + j * 256);
         f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 14; s++) {
@@ -478,8 +492,8 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
             if (s == 13) b = last ? b : make_uint4(0u, 0u, 0u, 0u);
             acc = mfma(w[s], __builtin_bit_cast(us8, b), acc);
         }
-        const float m0 = bf2f((uint16_t)(mk.x & 0xffffu)), m1 = bf2f((uint16_t)(mk.x >> 16)),
-                    m2 = bf2f((uint16_t)(mk.y & 0xffffu)), m3 = bf2f((uint16_t)(mk.y >> 16));
+        const float m0 = bf2f((uint16_t)(mk[j].x & 0xffffu)), m1 = bf2f((uint16_t)(mk[j].x >> 16)),
+                    m2 = bf2f((uint16_t)(mk[j].y & 0xffffu)), m3 = bf2f((uint16_t)(mk[j].y >> 16));
         *reinterpret_cast<uint2 *>(gout + o0 + j * 256) = pack4(m0 > 0.0f ? acc[0] : 0.0f, m1 > 0.0f ? acc[1] : 0.0f,
                                                                 m2 > 0.0f ? acc[2] : 0.0f, m3 > 0.0f ? acc[3] : 0.0f);
     }
@@ -497,7 +511,7 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
 // channel-fastest: the planes are turned on their way into LDS ([channel][j][k],
 // 4 voxels x 4 channels per lane), so an operand is one 16-byte read; gathering
 // it 2 bytes at a time bound the three passes before: 221 us for 128 images, this
-// one 47 us (37 images 211 -> 27 us).
+// one 36 us (37 images 211 -> 19 us).
 // Layers 2 and 3: a workgroup takes the 9 taps of one plane offset di, wavefront
 // w < 3 the 3 taps of dj = w - 1, whose operands are one row read and its
 // shifts by one voxel in registers (v_alignbit); planes are double-buffered,
@@ -505,11 +519,15 @@ __global__ void __launch_bounds__(256) k_cnn_dgrad16(const uint16_t *__restrict_
 // tap's 8 voxels aligned), wavefront w < 2 holds taps 16w .. 16w+15.  All in
 // one launch: blockIdx.y = 0 .. 2 layer 2, 3 .. 5 layer 3, 6 layer 1, so a
 // small batch still spreads over 7 workgroups per image.
+// 40 KB of LDS and at most 128 VGPRs: 4 workgroups per CU hold the 896 of 128
+// images in one round.
 constexpr int WA_CH = 16 * 16 + 8, WA_PL = 16 * WA_CH;           // g planes: rows of 16, channels 528 bytes apart
-constexpr int WB_ROW = 24, WB_CH = 18 * WB_ROW + 8, WB_PL = 16 * WB_CH;   // input planes: 8 zeros, 16 voxels; channels 880 bytes apart
+constexpr int WB_ROW = 20, WB_CH = 18 * WB_ROW + 4, WB_PL = 16 * WB_CH;   // input planes: 4 zeros, 16 voxels; channels 728 bytes apart
 constexpr int WDEPTH = 2;                                        // planes in flight
 constexpr int WX_CP = 18 * 18 * 16;                              // one shifted copy of x
-constexpr int W_TOTAL = 3 * WX_CP + 2 * WA_PL > 2 * (WA_PL + WB_PL) ? 3 * WX_CP + 2 * WA_PL : 2 * (WA_PL + WB_PL);
+constexpr int W_TOTAL = 2 * (WA_PL + WB_PL);
+static_assert(W_TOTAL >= 3 * WX_CP + WA_PL, "layer 1's three copies of x and one g plane");
+static_assert(WA_PL >= 256 + 2 * 256 + 16 * 16 * 2, "layer 3's g plane in two types");
 
 struct Quad {                               // 4 voxels x 4 channels
     uint2 v[4];
@@ -546,7 +564,7 @@ __device__ __forceinline__ float row_sum(const uint16_t *row, float s) {
 
 template <int L>
 __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, const void *__restrict__ g_, int di,
-                                           float *__restrict__ P, uint16_t *sm, float (*sBias)[16], float *sF) {
+                                           float *__restrict__ P, uint16_t *sm) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
               n = lane & 15;
     const int vg = tid >> 2, j4 = vg >> 2, k4 = 4 * (vg & 3), c4 = 4 * (tid & 3);
@@ -566,10 +584,10 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
             qa[u].store(A + c4 * WA_CH + j4 * 16 + k4, WA_CH);
         } else {
             A[tid] = f2bf(gf[u]);
-            sF[(p & 1) * 256 + tid] = gf[u];
+            reinterpret_cast<float *>(A + 256)[tid] = gf[u];
         }
         if (p + di < 0 || p + di > 15) qb[u].clear();      // beyond the block: zeros
-        qb[u].store(B + c4 * WB_CH + (j4 + 1) * WB_ROW + 8 + k4, WB_CH);
+        qb[u].store(B + c4 * WB_CH + (j4 + 1) * WB_ROW + 4 + k4, WB_CH);
     };
     f4 acc[3];
 #pragma unroll
@@ -591,13 +609,13 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
                 bias_acc = row_sum(A + c * WA_CH + jr * 16, bias_acc);
             } else if (c == 0) {
 #pragma unroll
-                for (int k = 0; k < 16; k++) bias_acc += sF[(p & 1) * 256 + jr * 16 + k];
+                for (int k = 0; k < 16; k++) bias_acc += reinterpret_cast<const float *>(A + 256)[jr * 16 + k];
             }
         }
         if (wave < 3) {
             // all operands of 4 chunks are read before the first is used
             const uint16_t *Ap = A + (L == 2 ? n * WA_CH : 0) + (g >> 1) * 16 + 8 * (g & 1);
-            const uint16_t *Bp = B + n * WB_CH + (wave + (g >> 1)) * WB_ROW + 8 + 8 * (g & 1);
+            const uint16_t *Bp = B + n * WB_CH + (wave + (g >> 1)) * WB_ROW + 4 + 8 * (g & 1);
 #pragma unroll
             for (int c0 = 0; c0 < 8; c0 += 4) {
                 uint4 a[4], b[4];
@@ -606,7 +624,8 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
                 for (int u = 0; u < 4; u++) {
                     a[u] = *reinterpret_cast<const uint4 *>(Ap + (c0 + u) * 32);
                     const uint16_t *row = Bp + (c0 + u) * 2 * WB_ROW;
-                    b[u] = *reinterpret_cast<const uint4 *>(row);
+                    const uint2 lo = *reinterpret_cast<const uint2 *>(row), hi = *reinterpret_cast<const uint2 *>(row + 4);
+                    b[u] = make_uint4(lo.x, lo.y, hi.x, hi.y);
                     pv[u] = *reinterpret_cast<const uint32_t *>(row - 2);
                     nx[u] = *reinterpret_cast<const uint32_t *>(row + 8);
                 }
@@ -638,6 +657,8 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
         }
     }
     if (di == 0) {
+        __syncthreads();
+        float (*sBias)[16] = reinterpret_cast<float (*)[16]>(sm);
         sBias[tid >> 4][tid & 15] = bias_acc;
         __syncthreads();
         if (tid < 16) {
@@ -650,11 +671,11 @@ __device__ __forceinline__ void wgrad_taps(const uint16_t *__restrict__ in, cons
 }
 
 __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const uint16_t *__restrict__ g1,
-                                            float *__restrict__ P, uint16_t *sm, float (*sBias)[16]) {
+                                            float *__restrict__ P, uint16_t *sm) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
               n = lane & 15;
     const int vg = tid >> 2, j4 = vg >> 2, k4 = 4 * (vg & 3), c4 = 4 * (tid & 3);
-    uint16_t *xs = sm + 2 * WA_PL;
+    uint16_t *xs = sm + WA_PL;
     float xv[16];
 #pragma unroll
     for (int p = 0; p < 16; p++) xv[p] = x[p * 256 + tid];
@@ -685,7 +706,7 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
     for (int p = 0; p < 16; p++) {
         __syncthreads();
         if (p + WDEPTH < 16) qa[p % WDEPTH].load(g1, p + WDEPTH, tid);
-        const uint16_t *A = sm + (p & 1) * WA_PL;
+        const uint16_t *A = sm;
         bias_acc = row_sum(A + (tid & 15) * WA_CH + (tid >> 4) * 16, bias_acc);
         if (wave < 2) {
 #pragma unroll
@@ -702,10 +723,12 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
                     acc = mfma32(a[u], make_uint4(b[u].x & taps, b[u].y & taps, b[u].z & taps, b[u].w & taps), acc);
             }
         }
-        if (p + 1 < 16) qa[(p + 1) % WDEPTH].store(sm + ((p + 1) & 1) * WA_PL + c4 * WA_CH + j4 * 16 + k4, WA_CH);
+        __syncthreads();
+        if (p + 1 < 16) qa[(p + 1) % WDEPTH].store(sm + c4 * WA_CH + j4 * 16 + k4, WA_CH);
     }
     if (wave < 2 && on)
         for (int r = 0; r < 4; r++) P[OFF_W1 + t * 16 + 4 * g + r] = acc[r];
+    float (*sBias)[16] = reinterpret_cast<float (*)[16]>(sm);      // (the last plane's barrier is behind)
     sBias[tid >> 4][tid & 15] = bias_acc;
     __syncthreads();
     if (tid < 16) {
@@ -715,18 +738,17 @@ __device__ __forceinline__ void wgrad_first(const float *__restrict__ x, const u
     }
 }
 
-__global__ void __launch_bounds__(256, 3) k_cnn_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ h1,
+__global__ void __launch_bounds__(256, 4) k_cnn_wgrad(const float *__restrict__ x, const uint16_t *__restrict__ h1,
                                                    const uint16_t *__restrict__ h2, const uint16_t *__restrict__ g1,
                                                    const uint16_t *__restrict__ g2, const float *__restrict__ g3,
                                                    float *__restrict__ part, const long long *__restrict__ idx) {
     __shared__ __align__(16) uint16_t sm[W_TOTAL];
-    __shared__ float sBias[16][16], sF[512];
     const long long img = blockIdx.x, v = img * 4096;
     const int job = blockIdx.y;
     float *P = part + img * (long long)kCnnParams;
-    if (job < 3) wgrad_taps<2>(h1 + v * 16, g2 + v * 16, job - 1, P, sm, sBias, sF);
-    else if (job < 6) wgrad_taps<3>(h2 + v * 16, g3 + v, job - 4, P, sm, sBias, sF);
-    else wgrad_first(x + (idx ? idx[img] : img) * 4096, g1 + v * 16, P, sm, sBias);
+    if (job < 3) wgrad_taps<2>(h1 + v * 16, g2 + v * 16, job - 1, P, sm);
+    else if (job < 6) wgrad_taps<3>(h2 + v * 16, g3 + v, job - 4, P, sm);
+    else wgrad_first(x + (idx ? idx[img] : img) * 4096, g1 + v * 16, P, sm);
 }
 
 // grad[q] = sum over images of part[img][q], fixed order, FP64, 32 images in
@@ -806,19 +828,19 @@ __global__ void __launch_bounds__(256) k_cnn_loss(const float *__restrict__ out,
 // w) that weighs the error's variation instead of its offset.
 // g3 = (dL/d out) * sc; loss partials per workgroup.  One workgroup walks
 // images blockIdx.x, blockIdx.x + gridDim.x, ...
-__global__ void __launch_bounds__(256) k_cnn_loss_h1(const float *__restrict__ out, const float *__restrict__ y,
+__global__ void __launch_bounds__(1024) k_cnn_loss_h1(const float *__restrict__ out, const float *__restrict__ y,
                                                      int nimg, float alpha, float wi, float wj, float wk, float sc,
                                                      float *__restrict__ g3, double *__restrict__ part,
                                                      const long long *__restrict__ idx) {
     __shared__ float dl[4096];
-    __shared__ double red[4];
+    __shared__ double red[16];
     double acc = 0.0;
     for (int img = blockIdx.x; img < nimg; img += gridDim.x) {
         const long long o = (long long)img * 4096;
         const float *Y = y + idx[img] * 4096;
-        for (int c = threadIdx.x; c < 4096; c += 256) dl[c] = out[o + c] - Y[c];
+        for (int c = threadIdx.x; c < 4096; c += 1024) dl[c] = out[o + c] - Y[c];
         __syncthreads();
-        for (int c = threadIdx.x; c < 4096; c += 256) {
+        for (int c = threadIdx.x; c < 4096; c += 1024) {
             const int i = c >> 8, j = (c >> 4) & 15, k = c & 15;
             const float d = dl[c];
             float g = alpha * d;
@@ -839,7 +861,11 @@ __global__ void __launch_bounds__(256) k_cnn_loss_h1(const float *__restrict__ o
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (threadIdx.x == 0) {
+        double l = red[0];
+        for (int w = 1; w < 16; w++) l += red[w];
+        part[blockIdx.x] = l;
+    }
 }
 
 // Scale-free form of the same norm, per image: with A = alpha I + sum_a w_a
@@ -975,10 +1001,16 @@ void CnnModel::ensure_batch(int nimg) {
     max_batch_ = nimg;
 }
 
+// segments of the forward march: 4 of 8 steps up to 64 images, 2 of 10 and 12 up
+// to 128 (256 workgroups of 64 KB LDS, one per CU), 1 of 18 beyond, where the
+// recomputed planes would cost more than idle CUs.  37 images 38 -> 22 us, with
+// the activations stored 42 -> 25; 128 images 39 -> 29.
+static unsigned fwd_segments(long long nimg) { return nimg <= 64 ? 4 : (nimg <= 128 ? 2 : 1); }
+
 void CnnModel::infer(const float *x, float *out, long long nimg, hipStream_t stream) {
     if (nimg <= 0) return;
     pack(stream);
-    hipLaunchKernelGGL((k_cnn_fwd<false, false, kFwdWaves>), dim3((unsigned)nimg), dim3(64 * kFwdWaves), 0, stream, x, out,
+    hipLaunchKernelGGL((k_cnn_fwd<false, false, kFwdWaves>), dim3((unsigned)nimg, fwd_segments(nimg)), dim3(64 * kFwdWaves), 0, stream, x, out,
                        (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_,
                        (uint16_t *)nullptr, (uint16_t *)nullptr, HeatIO{}, (const long long *)nullptr);
 }
@@ -1005,7 +1037,7 @@ void CnnModel::backward(const float *x, const float *g3, const long long *idx, i
 void CnnModel::gradient(const float *x, const float *gout, int nimg, double *grad_host, hipStream_t stream) {
     ensure_batch(nimg);
     pack(stream);
-    hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg), dim3(64 * kFwdWaves), 0, stream, x, out_,
+    hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg, fwd_segments(nimg)), dim3(64 * kFwdWaves), 0, stream, x, out_,
                        (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{}, (const long long *)nullptr);
     backward(x, gout, nullptr, nimg, stream);
     hipLaunchKernelGGL(k_cnn_reduce, dim3((kCnnParams + 63) / 64), dim3(64), 0, stream, (const float *)part_, nimg, grad_);
@@ -1016,7 +1048,7 @@ void CnnModel::gradient(const float *x, const float *gout, int nimg, double *gra
 void CnnModel::train_step(const float *x, const float *y, const long long *idx, int nimg, double lr, bool first,
                           hipStream_t stream) {
     pack(stream);
-    hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg), dim3(64 * kFwdWaves), 0, stream, x, out_,
+    hipLaunchKernelGGL((k_cnn_fwd<true, false, kFwdWaves>), dim3(nimg, fwd_segments(nimg)), dim3(64 * kFwdWaves), 0, stream, x, out_,
                        (const uint16_t *)packed_ + PK_TOTAL * 8, (const float *)params_, h1_, h2_, HeatIO{}, idx);
     const long long n = 4096LL * nimg;
     int nwg = nimg < 1024 ? nimg : 1024;
@@ -1028,7 +1060,7 @@ void CnnModel::train_step(const float *x, const float *y, const long long *idx, 
                            (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2], (float)scale, g3_,
                            loss_part_, idx);
     } else if (h1_alpha_ >= 0.0) {
-        hipLaunchKernelGGL(k_cnn_loss_h1, dim3(nwg), dim3(256), 0, stream, (const float *)out_, y, nimg,
+        hipLaunchKernelGGL(k_cnn_loss_h1, dim3(nwg), dim3(1024), 0, stream, (const float *)out_, y, nimg,
                            (float)h1_alpha_, (float)h1_w_[0], (float)h1_w_[1], (float)h1_w_[2], (float)scale, g3_,
                            loss_part_, idx);
     } else {
