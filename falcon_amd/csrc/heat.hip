@@ -61,7 +61,7 @@ struct HLev {
     const double *V, *Ai, *Aj, *Ak, *off;   // [block][i][j] coefficient tables
     const int2 *gsw;        // per face ghost: (donor base cell or -1, weights index or -1 = copy)
     const double *gw;       // 3 weights per weighted ghost
-    const double *diag;     // [system][block][i][j]: V/dt + off (k_hdiag)
+    const double2 *diag;    // [system][block][i][j]: d = V/dt + off and 1/d for div_by (k_hdiag)
 };
 
 struct Cell {
@@ -84,19 +84,25 @@ __device__ __forceinline__ Cell cell_of(const HLev &L, long long c) {
 template <bool FIRST>
 struct FieldT {
     const double *x;
-    const double *diag;     // of the system (FIRST)
+    const double2 *diag;    // of the system (FIRST)
     int lm;
     double omega;
-    __device__ __forceinline__ double value(long long c, double v) const { return FIRST ? (omega * v) / diag[c >> lm] : v; }
-    __device__ __forceinline__ double operator()(long long c) const { return value(c, x[c]); }
+    __device__ __forceinline__ double operator()(long long c) const {
+        const double v = x[c];
+        if (!FIRST) return v;
+        const double2 d = diag[c >> lm];
+        return div_by(omega * v, d.x, d.y);
+    }
 };
 typedef FieldT<false> Field;
 
-// diag[s][t2] = V/dt + off of every system (whenever dt changes)
-__global__ void __launch_bounds__(256) k_hdiag(HLev L, double *__restrict__ diag, const double *__restrict__ inv_dt,
+// diag[s][t2] = V/dt + off of every system and its reciprocal (whenever dt changes)
+__global__ void __launch_bounds__(256) k_hdiag(HLev L, double2 *__restrict__ diag, const double *__restrict__ inv_dt,
                                                long long n2) {
     const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n2) diag[blockIdx.y * n2 + c] = L.V[c] * inv_dt[blockIdx.y] + L.off[c];
+    if (c >= n2) return;
+    const double d = L.V[c] * inv_dt[blockIdx.y] + L.off[c];
+    diag[blockIdx.y * n2 + c] = make_double2(d, div_rcp(d));
 }
 
 // Block partial sums of NP per-thread values into partial[s][p][blockIdx.x].
@@ -168,7 +174,7 @@ __device__ __forceinline__ double trilinear(const HLev &L, const F &X, long long
     return t;
 }
 
-// Per-cell epilogues: (io, x, A x, diag, in0, in1) -> stores and NP dot terms.
+// Per-cell epilogues: (io, x, A x, (diag, 1/diag), in0, in1) -> stores and NP dot terms.
 // IN0 / IN1: whether the op reads its input vectors in0 / in1 at the cell.
 template <bool DOT>
 struct OpApply {                 // y = A x; DOT: x.y, x.r
@@ -176,7 +182,7 @@ struct OpApply {                 // y = A x; DOT: x.y, x.r
     const double *in0, *in1;     // r (DOT); unused
     static constexpr int NP = 2;
     static constexpr bool IN0 = DOT, IN1 = false;
-    __device__ __forceinline__ void cell(long long io, double x, double ax, double, double r, double,
+    __device__ __forceinline__ void cell(long long io, double x, double ax, double2, double r, double,
                                          double (&v)[NP]) const {
         y[io] = ax;
         if (DOT) { v[0] += x * ax; v[1] += x * r; }
@@ -189,9 +195,9 @@ struct OpJacobi {                // y = x + omega (r - A x)/diag; DOT: y.dq
     double omega;
     static constexpr int NP = 1;
     static constexpr bool IN0 = true, IN1 = DOT;
-    __device__ __forceinline__ void cell(long long io, double x, double ax, double diag, double r, double dq,
+    __device__ __forceinline__ void cell(long long io, double x, double ax, double2 diag, double r, double dq,
                                          double (&v)[NP]) const {
-        const double yn = x + omega * (r - ax) / diag;
+        const double yn = x + div_by(omega * (r - ax), diag.x, diag.y);
         y[io] = yn;
         if (DOT) v[0] += yn * dq;
     }
@@ -202,11 +208,11 @@ struct OpFeat {                  // r' = r - A z, u = r'/diag (float), u.u
     const double *in0, *in1;     // r; unused
     static constexpr int NP = 1;
     static constexpr bool IN0 = true, IN1 = false;
-    __device__ __forceinline__ void cell(long long io, double, double ax, double diag, double r, double,
+    __device__ __forceinline__ void cell(long long io, double, double ax, double2 diag, double r, double,
                                          double (&v)[NP]) const {
         const double res = r - ax;
         rp[io] = res;
-        const double w = res / diag;
+        const double w = div_by(res, diag.x, diag.y);
         u[io] = (float)w;
         v[0] += w * w;
     }
@@ -215,7 +221,7 @@ struct OpApplyDot {              // c.r', c.Ac, c.q (Ac itself is not stored)
     const double *in0, *in1;     // r'; q
     static constexpr int NP = 3;
     static constexpr bool IN0 = true, IN1 = true;
-    __device__ __forceinline__ void cell(long long, double x, double ax, double, double rp, double q,
+    __device__ __forceinline__ void cell(long long, double x, double ax, double2, double rp, double q,
                                          double (&v)[NP]) const {
         v[0] += x * rp;
         v[1] += x * ax;
@@ -232,15 +238,16 @@ struct Planes {
 // LDS layout (doubles): edge rows of the x tile (m = 16 only: the first and
 // last j-row of every wavefront, [wave][2][i][k]), theta and phi face ghosts
 // [block][4][i][m], coefficient tables Ai [bpw][C+1][m], Aj [bpw][C][m+1], Ak
-// and diag [bpw][C][m]
+// [bpw][C][m], diag and 1/diag in pairs [bpw][C][m]
 template <int LM>
 struct TileLds {
     static constexpr int m = 1 << LM, C = Planes<LM>::C, bpw = 256 >> (2 * LM);
     static constexpr int NE = LM == 4 ? 4 * 2 * C * 16 : 0;
     static constexpr int NG = bpw * 4 * C * m;
     static constexpr int G0 = NE, CI = G0 + NG, NI = bpw * (C + 1) * m, CJ = CI + NI, NJ = bpw * C * (m + 1),
-                         CK = CJ + NJ, NK = bpw * C * m, CD = CK + NK, SIZE = CD + NK;
-    static constexpr int NC = SIZE - CI;              // coefficient doubles
+                         CK = CJ + NJ, NK = bpw * C * m, CD = (CK + NK + 1) & ~1, SIZE = CD + 2 * NK;
+    static constexpr int NC = CK + NK - CI;           // coefficient doubles (diag apart)
+    static constexpr int NDT = (NK + 255) / 256;      // diagonals per thread
     static constexpr int NCT = (NC + 255) / 256;      // per thread
     static constexpr int NGT = (NG + 255) / 256;      // ghosts per thread
 };
@@ -259,7 +266,7 @@ __device__ __forceinline__ double dpp_d(double v) {
 // coefficients.  FIRST: x is formed from in0 = r, which a0 returns.  Ends with a
 // barrier.
 template <int LM, bool FIRST, bool IN0, bool IN1>
-__device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F, const double *__restrict__ diag, int b0,
+__device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F, const double2 *__restrict__ diag, int b0,
                                           int h, bool own, long long cb, const double *__restrict__ in0,
                                           const double *__restrict__ in1, long long so,
                                           double (&col)[Planes<LM>::C + 2], double (&a0)[Planes<LM>::C],
@@ -282,13 +289,14 @@ __device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F,
     const int2 *Er = L.gsw + (long long)(b0 + lb) * 6 * mm + jk;
     const int2 elo = own && h == 0 ? Er[0] : none, ehi = own && h == S - 1 ? Er[mm] : none;
     const long long c0 = cb + (long long)i0 * mm;
-    double xr[C + 2], dg[C + 2];
+    double xr[C + 2];
+    double2 dg[C + 2];
 #pragma unroll
     for (int i = 0; i < C + 2; i++) {
         const bool in = own && (i > 0 || h > 0) && (i < C + 1 || h < S - 1);
         const long long c = c0 + (long long)(i - 1) * mm;
         xr[i] = in ? F.x[c] : 0.0;
-        if (FIRST) dg[i] = in ? diag[c >> LM] : 1.0;
+        if (FIRST) dg[i] = in ? diag[c >> LM] : make_double2(1.0, 1.0);
         if (i > 0 && i < C + 1) {
             if (IN0 && !FIRST) a0[i - 1] = own ? in0[so + c] : 0.0;
             if (IN1) a1[i - 1] = own ? in1[so + c] : 0.0;
@@ -309,11 +317,16 @@ __device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F,
             const int r0 = q - T::NI, b = r0 / w, r = r0 - b * w;
             if (b < nbw) v = L.Aj[(long long)(b0 + b) * m * (m + 1) + i0 * (m + 1) + r];
         } else if (q < T::NC) {
-            const int r0 = q - T::NI - T::NJ, which = r0 >= T::NK, r1 = which ? r0 - T::NK : r0;
-            const int b = r1 >> (LM + LC), r = r1 & (C * m - 1);
-            if (b < nbw) v = (which ? diag : L.Ak)[((long long)(b0 + b) << (2 * LM)) + i0 * m + r];
+            const int r0 = q - T::NI - T::NJ, b = r0 >> (LM + LC), r = r0 & (C * m - 1);
+            if (b < nbw) v = L.Ak[((long long)(b0 + b) << (2 * LM)) + i0 * m + r];
         }
         cf[u] = v;
+    }
+    double2 cd[T::NDT];
+#pragma unroll
+    for (int u = 0; u < T::NDT; u++) {
+        const int q = tid + 256 * u, b = q >> (LM + LC), r = q & (C * m - 1);
+        cd[u] = q < T::NK && b < nbw ? diag[((long long)(b0 + b) << (2 * LM)) + i0 * m + r] : make_double2(1.0, 1.0);
     }
     // ghosts: the first donor value of every entry, then the weighted ones
     double f0[T::NGT];
@@ -330,7 +343,7 @@ __device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F,
     if (ehi.y >= 0) fhi = trilinear(L, F, ehi.x, ehi.y, fhi);
 #pragma unroll
     for (int i = 0; i < C + 2; i++) {
-        col[i] = FIRST ? (F.omega * xr[i]) / dg[i] : xr[i];
+        col[i] = FIRST ? div_by(F.omega * xr[i], dg[i].x, dg[i].y) : xr[i];
         if (FIRST && i > 0 && i < C + 1) a0[i - 1] = xr[i];
     }
     if (h == 0) col[0] = flo;
@@ -338,6 +351,9 @@ __device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F,
 #pragma unroll
     for (int u = 0; u < T::NCT; u++)
         if (tid + 256 * u < T::NC) sm[T::CI + tid + 256 * u] = cf[u];
+#pragma unroll
+    for (int u = 0; u < T::NDT; u++)
+        if (tid + 256 * u < T::NK) *reinterpret_cast<double2 *>(sm + T::CD + 2 * (tid + 256 * u)) = cd[u];
     if (LM == 4) {
         // wavefront edge rows: lanes 0-15 (j = 4w) and 48-63 (j = 4w + 3)
         const int w = tid >> 6, l = tid & 63;
@@ -357,7 +373,7 @@ __device__ __forceinline__ void load_tile(const HLev &L, const FieldT<FIRST> &F,
 // Every lane of the workgroup calls it (cross-lane operations).
 template <int LM>
 __device__ __forceinline__ double tile_apply(const double *__restrict__ sm, const double (&col)[Planes<LM>::C + 2], int i,
-                                             int lb, int j, int k, double &diag) {
+                                             int lb, int j, int k, double2 &diag) {
     using T = TileLds<LM>;
     constexpr int m = T::m, C = T::C;
     const int t = threadIdx.x, lane = t & 63;
@@ -381,11 +397,11 @@ __device__ __forceinline__ double tile_apply(const double *__restrict__ sm, cons
     const double cim = ai[i * m + j], cip = ai[(i + 1) * m + j];
     const double cjm = aj[i * (m + 1) + j], cjp = aj[i * (m + 1) + j + 1];
     const double ck = sm[T::CK + t2];
-    diag = sm[T::CD + t2];
+    diag = *reinterpret_cast<const double2 *>(sm + T::CD + 2 * t2);
     double nb = cim * xim + cip * xip;
     nb = nb + cjm * xjm + cjp * xjp;
     nb = nb + ck * xkm + ck * xkp;
-    return diag * x0 - nb;
+    return diag.x * x0 - nb;
 }
 
 // One operator pass over every cell of a level: op.cell at each cell, dot
@@ -396,7 +412,7 @@ template <int LM, bool FIRST, class OP>
 __global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict__ x, const int *__restrict__ active,
                                                 long long istride, OP op, double omega, double *__restrict__ partial) {
     constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM), C = Planes<LM>::C, S = Planes<LM>::S;
-    __shared__ double sm[TileLds<LM>::SIZE];
+    __shared__ __align__(16) double sm[TileLds<LM>::SIZE];
     const int s = blockIdx.y;
     if (!active[s]) return;
     const int tid = threadIdx.x;
@@ -404,7 +420,7 @@ __global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict
     const int w = xcd_group(blockIdx.x, gridDim.x), h = w & (S - 1);
     const int b0 = (w >> Planes<LM>::LS) * bpw, b = b0 + lb;
     const bool own = b < L.nb;
-    const double *D = L.diag + s * ((long long)L.nb << (2 * LM));
+    const double2 *D = L.diag + s * ((long long)L.nb << (2 * LM));
     const long long so = s * istride;
     const FieldT<FIRST> F{(FIRST ? op.in0 : x) + so, D, LM, omega};
     const long long cb = ((long long)b << (3 * LM)) + (j << LM) + k;
@@ -413,7 +429,7 @@ __global__ void __launch_bounds__(256) k_hmarch(HLev L, const double *__restrict
     double v[OP::NP] = {};
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        double diag;
+        double2 diag;
         const double ax = tile_apply<LM>(sm, col, i, lb, j, k, diag);
         if (own)
             op.cell(so + cb + (long long)(h * C + i) * mm, col[i + 1], ax, diag, OP::IN0 ? a0[i] : 0.0,
@@ -433,7 +449,7 @@ __global__ void __launch_bounds__(256) k_hresrestrict(HLev L, const double *__re
                                                       long long istride, long long cstride) {
     constexpr int m = 1 << LM, mm = m * m, bpw = 256 >> (2 * LM), LC = LM - 1, C = Planes<LM>::C, S = Planes<LM>::S;
     static_assert(C >= 2, "an i pair of children belongs to one thread");
-    __shared__ double sm[TileLds<LM>::SIZE];
+    __shared__ __align__(16) double sm[TileLds<LM>::SIZE];
     const int s = blockIdx.y;
     if (!active[s]) return;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -441,7 +457,7 @@ __global__ void __launch_bounds__(256) k_hresrestrict(HLev L, const double *__re
     const int w = xcd_group(blockIdx.x, gridDim.x), h = w & (S - 1);
     const int b0 = (w >> Planes<LM>::LS) * bpw, b = b0 + lb;
     const bool own = b < L.nb;
-    const double *D = L.diag + s * ((long long)L.nb << (2 * LM));
+    const double2 *D = L.diag + s * ((long long)L.nb << (2 * LM));
     const long long so = s * istride;
     const Field F{x + so, D, LM, 0.0};
     const long long cb = ((long long)b << (3 * LM)) + (j << LM) + k;
@@ -451,7 +467,7 @@ __global__ void __launch_bounds__(256) k_hresrestrict(HLev L, const double *__re
     double *R = rc + s * cstride + ((long long)b << (3 * LC)) + ((j >> 1) << LC) + (k >> 1);
 #pragma unroll
     for (int ic = 0; ic < C / 2; ic++) {
-        double diag;
+        double2 diag;
         const double ax0 = tile_apply<LM>(sm, col, 2 * ic, lb, j, k, diag);
         const double ax1 = tile_apply<LM>(sm, col, 2 * ic + 1, lb, j, k, diag);
         const double o0 = own ? a0[2 * ic] - ax0 : 0.0, o1 = own ? a0[2 * ic + 1] - ax1 : 0.0;
@@ -474,7 +490,8 @@ __global__ void __launch_bounds__(256) k_hjacobi0(HLev L, const double *__restri
     const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= (long long)L.nb * L.M3) return;
     const long long io = s * istride + c;
-    y[io] = (omega * r[io]) / L.diag[s * (((long long)L.nb * L.M3) >> L.lm) + (c >> L.lm)];
+    const double2 d = L.diag[s * (((long long)L.nb * L.M3) >> L.lm) + (c >> L.lm)];
+    y[io] = div_by(omega * r[io], d.x, d.y);
 }
 
 // Linear prolongation, stored: fine cell (i, j, k) of level LM adds
@@ -571,13 +588,14 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
     const int s = blockIdx.x;
     if (!active[s]) return;
     const int nb = L.nb, t = threadIdx.x;
-    const double *dgs = L.diag + (long long)s * nb;
+    const double2 *dgs = L.diag + (long long)s * nb;
     double *X = x + s * stride;
     const double *B = rhs + s * stride;
     int set = 0;
     if (K > 0) {
         constexpr int KK = K > 0 ? K : 1;
-        double xv[KK], r[KK], pv[KK], ap[KK], dg[KK], cf[KK][5];
+        double xv[KK], r[KK], pv[KK], ap[KK], cf[KK][5];
+        double2 dg[KK];
         int2 e[KK][3];                     // donors of the 6 faces (no donor: itself, its coefficient is 0)
         bool on[KK];
         double acc = 0.0;
@@ -587,7 +605,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
             on[u] = b < nb;
             const int bb = on[u] ? b : 0;
             r[u] = on[u] ? B[bb] : 0.0;
-            dg[u] = on[u] ? dgs[bb] : 1.0;
+            dg[u] = on[u] ? dgs[bb] : make_double2(1.0, 1.0);
             cf[u][0] = L.Ai[2 * bb]; cf[u][1] = L.Ai[2 * bb + 1];
             cf[u][2] = L.Aj[2 * bb]; cf[u][3] = L.Aj[2 * bb + 1];
             cf[u][4] = L.Ak[bb];
@@ -597,7 +615,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
         }
 #pragma unroll
         for (int u = 0; u < KK; u++) {
-            const double z = r[u] / dg[u];
+            const double z = div_by(r[u], dg[u].x, dg[u].y);
             pv[u] = z;
             xv[u] = 0.0;
             if (on[u]) {
@@ -621,7 +639,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
                 double nbv = cf[u][0] * g[0] + cf[u][1] * g[1];
                 nbv = nbv + cf[u][2] * g[2] + cf[u][3] * g[3];
                 nbv = nbv + cf[u][4] * g[4] + cf[u][4] * g[5];
-                ap[u] = dg[u] * pv[u] - nbv;
+                ap[u] = dg[u].x * pv[u] - nbv;
                 acc += pv[u] * ap[u];
             }
             const double pAp = wg1024_sum(acc, red, set);
@@ -633,7 +651,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
                 if (!on[u]) continue;
                 xv[u] = xv[u] + alpha * pv[u];
                 r[u] = r[u] - alpha * ap[u];
-                ap[u] = r[u] / dg[u];
+                ap[u] = div_by(r[u], dg[u].x, dg[u].y);
                 acc += r[u] * ap[u];
             }
             const double rzn = wg1024_sum(acc, red, set);
@@ -657,7 +675,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
     for (int b = t; b < nb; b += 1024) {
         const double r = B[b];
         R[b] = r;
-        const double z = r / dgs[b];
+        const double z = div_by(r, dgs[b].x, dgs[b].y);
         Pv[b] = z;
         X[b] = 0.0;
         acc += r * z;
@@ -679,7 +697,7 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
             double nbv = cim * g[0] + cip * g[1];
             nbv = nbv + cjm * g[2] + cjp * g[3];
             nbv = nbv + ck * g[4] + ck * g[5];
-            const double ap = dgs[b] * Pv[b] - nbv;
+            const double ap = dgs[b].x * Pv[b] - nbv;
             AP[b] = ap;
             acc += Pv[b] * ap;
         }
@@ -691,12 +709,12 @@ __global__ void __launch_bounds__(1024) k_hcoarse_cg(HLev L, const double *__res
             X[b] = X[b] + alpha * Pv[b];
             const double r = R[b] - alpha * AP[b];
             R[b] = r;
-            acc += r * (r / dgs[b]);
+            acc += r * div_by(r, dgs[b].x, dgs[b].y);
         }
         const double rzn = wg1024_sum(acc, red, set);
         const double beta = rzn / rz;
         rz = rzn;
-        for (int b = t; b < nb; b += 1024) Pv[b] = R[b] / dgs[b] + beta * Pv[b];
+        for (int b = t; b < nb; b += 1024) Pv[b] = div_by(R[b], dgs[b].x, dgs[b].y) + beta * Pv[b];
         __syncthreads();   // every p before the next product reads its neighbours
     }
 }
@@ -1207,7 +1225,7 @@ struct HeatSolver::Impl {
         for (int l = 0; l < nlev; l++) {
             const long long n2 = (long long)nb * L[l].m * L[l].m;
             hipLaunchKernelGGL(k_hdiag, dim3((unsigned)((n2 + 255) / 256), (unsigned)nsys), dim3(256), 0, stream, L[l],
-                               const_cast<double *>(L[l].diag), (const double *)inv_dt, n2);
+                               const_cast<double2 *>(L[l].diag), (const double *)inv_dt, n2);
         }
         HCHECK(hipGetLastError());
         HCHECK(hipStreamSynchronize(stream));
@@ -1352,7 +1370,7 @@ void HeatSolver::setup(const Layout &lay, const HeatParams &hp, int nsys, int nt
     I.tmp = I.dalloc(I.ist(0) * nsys);
     I.p = I.dalloc(I.ist(0) * nsys);
     I.inv_dt = I.dalloc(nsys);
-    for (int l = 0; l < I.nlev; l++) I.L[l].diag = I.dalloc((size_t)nsys * I.nb * I.L[l].m * I.L[l].m);
+    for (int l = 0; l < I.nlev; l++) I.L[l].diag = (const double2 *)I.dalloc((size_t)nsys * I.nb * I.L[l].m * I.L[l].m * 2);
     I.diagonals();
     I.partial = I.dalloc((size_t)nsys * 3 * std::max(I.march_wgs(0), I.elem_wgs()));
     I.dots = I.dalloc((size_t)nsys * 3);

@@ -75,23 +75,6 @@ __device__ __forceinline__ double d4(double fm2, double fm1, double fp1, double 
     return c * (__builtin_fma(-8.0, fm1, __builtin_fma(8.0, fp1, -fp2)) + fm2);
 }
 
-// x / b for many x and one b: y = 1/b by two Newton steps on the hardware
-// reciprocal, then Markstein's correction of x*y by its exact remainder: the
-// correctly rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990) in 3
-// operations per x, where the general division takes 11 (the same steps with
-// a rescaling of operands near the ends of the exponent range, which neither
-// the background's and metric's divisors nor values above 1e-290 reach).  The
-// fix-up gives zeros, infinities and NaN as the division does.
-__device__ __forceinline__ double div_rcp(double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-    return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
-}
-__device__ __forceinline__ double div_by(double x, double b, double y) {
-    const double q = x * y;
-    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, x), y, q), b, x);
-}
-
 // Smallest t with scale*t >= k in T's rounding: t >= flag_from(scale, k) is
 // that comparison without its product.
 template <typename T>
