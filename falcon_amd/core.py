@@ -460,12 +460,12 @@ class Pfss:
         return it.value, rel.value, sec.value
 
     def phi(self):
-        out = np.zeros(self.shape)
+        out = np.empty(self.shape)
         _check(self.L.falcon_pfss_get_phi(self.s.h, _p(out)))
         return out
 
     def field(self):
-        out = np.zeros((self.shape[0], 3) + self.shape[1:])
+        out = np.empty((self.shape[0], 3) + self.shape[1:])
         _check(self.L.falcon_pfss_field(self.s.h, _p(out)))
         return out
 

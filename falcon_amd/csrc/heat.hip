@@ -37,6 +37,7 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -750,14 +751,12 @@ __global__ void __launch_bounds__(256) k_hdot(long long n, const double *__restr
 }
 
 // Per-system scalars on the device, kSc slots each:
-// [0] alpha = <p,r>/<p,q>, [1] beta = <z,q>/gamma, [2] gamma = <p,q>,
+// [0] alpha = <p,r>/<p,q>, [1] beta of the learned direction, [2] gamma = <p,q>,
 // [3] feature scale of the learned correction, [4] its step along c, [5] <b,b>,
 // [6] <z,q> of the V-cycle output.
 constexpr int kSc = 8;
 enum {
     kScNone = -1,
-    kScAlpha = 0,     // alpha and gamma (dots: [0]=<p,q>, [1]=<p,r>)
-    kScBeta = 1,      // beta (dots: [0]=<z,q>)
     kScStep = 2,      // correction step <c,r'>/<c,Ac> (dots: [0]=<c,r'>, [1]=<c,Ac>), 0 unless <c,Ac> > 0
     kScFeature = 3,   // feature scale sqrt(sum / ncell) (dots: [0]=sum (r'/diag)^2)
     kScNorm = 4,      // <b,b> (dots: [0])
@@ -777,12 +776,7 @@ struct Converge {
 __device__ __forceinline__ void scalar_step(int what, int s, const double *__restrict__ dots, double *__restrict__ S,
                                             int *__restrict__ active, double ncell, const Converge &cv) {
     const bool on = active[s] != 0;
-    if (what == kScAlpha) {
-        S[2] = dots[0];
-        S[0] = on ? dots[1] / dots[0] : 0.0;
-    } else if (what == kScBeta) {
-        S[1] = on ? dots[0] / S[2] : 0.0;
-    } else if (what == kScStep) {
+    if (what == kScStep) {
         const double num = dots[0], den = dots[1];
         const double a = num / den;
         S[4] = (on && den > 0.0 && a == a && a < 1e300 && a > -1e300) ? a : 0.0;
@@ -807,32 +801,33 @@ __device__ __forceinline__ void scalar_step(int what, int s, const double *__res
     }
 }
 
-// sum of nwg partials per (system, pair), fixed order, and the scalars formed
-// from the sums by the workgroup's first thread (a launch of its own for each
-// cost 4.4 us per use, 3 uses per iteration)
+// one dot product of a system from its workgroups' partials, fixed order, in
+// the first thread of a 256-thread workgroup (red: the caller's, one per pair)
+__device__ __forceinline__ double sum_partials(const double *__restrict__ P, int nwg, double (&red)[4]) {
+    double v0 = 0.0, v1 = 0.0;
+    int w = threadIdx.x;
+    for (; w + 256 < nwg; w += 512) { v0 += P[w]; v1 += P[w + 256]; }
+    if (w < nwg) v0 += P[w];
+    double v = v0 + v1;
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+// sum of nwg partials per (system, pair) and the scalars formed from the sums
+// by the workgroup's first thread (a launch of its own for each cost 4.4 us per
+// use, 3 uses per iteration)
 __global__ void __launch_bounds__(256) k_hdot_final(const double *__restrict__ partial, int nwg, int npairs,
                                                    double *__restrict__ out, int what, int what2,
                                                    double *__restrict__ sc, int *__restrict__ active, double ncell,
                                                    Converge cv) {
     __shared__ double red[3][4];
     const int s = blockIdx.x;
-    for (int p = 0; p < npairs; p++) {
-        const double *P = partial + ((long long)s * 3 + p) * nwg;
-        double v0 = 0.0, v1 = 0.0;
-        int w = threadIdx.x;
-        for (; w + 256 < nwg; w += 512) { v0 += P[w]; v1 += P[w + 256]; }
-        if (w < nwg) v0 += P[w];
-        double v = v0 + v1;
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if ((threadIdx.x & 63) == 0) red[p][threadIdx.x >> 6] = v;
-    }
-    __syncthreads();
+    double dots[3] = {0.0, 0.0, 0.0};
+    for (int p = 0; p < npairs; p++) dots[p] = sum_partials(partial + ((long long)s * 3 + p) * nwg, nwg, red[p]);
     if (threadIdx.x == 0) {
-        double dots[3] = {0.0, 0.0, 0.0};
-        for (int p = 0; p < npairs; p++) {
-            dots[p] = ((red[p][0] + red[p][1]) + red[p][2]) + red[p][3];
-            out[s * 3 + p] = dots[p];
-        }
+        for (int p = 0; p < npairs; p++) out[s * 3 + p] = dots[p];
         if (what != kScNone) scalar_step(what, s, dots, sc + kSc * s, active, ncell, cv);
         if (what2 != kScNone) scalar_step(what2, s, dots, sc + kSc * s, active, ncell, cv);
     }
@@ -843,14 +838,26 @@ __global__ void k_hizero(int *__restrict__ a, int n) {
     if (i < n) a[i] = 0;
 }
 
-// x += alpha p ; r -= alpha q, and partial sums of r.r
+// Where an update needs a scalar of dots that its predecessor left in partial
+// sums, every workgroup adds the nwg partials itself (they come from the L2; the
+// same order as k_hdot_final's): the sum's own launch took 4.6 to 5.4 us, twice an
+// iteration; solve of 6.3 M cells 8.36 -> 8.20 ms, PFSS 4.48 -> 4.44.
+// x += alpha p ; r -= alpha q with alpha = <p,r>/<p,q> (dots 1 and 0 of pin,
+// gamma = <p,q> kept for beta), and partial sums of r.r into partial
 __global__ void __launch_bounds__(256) k_hupdate_xr(long long n, double *__restrict__ x, double *__restrict__ r,
                                                     const double *__restrict__ p, const double *__restrict__ q,
-                                                    const double *__restrict__ sc, const int *__restrict__ active,
-                                                    double *__restrict__ partial, long long istride) {
+                                                    const double *__restrict__ pin, int nwg, double *__restrict__ sc,
+                                                    const int *__restrict__ active, double *__restrict__ partial,
+                                                    long long istride) {
+    __shared__ double red[2][4];
     const int s = blockIdx.y;
     if (!active[s]) return;
-    const double a = sc[kSc * s];
+    const double pq = sum_partials(pin + (long long)s * 3 * nwg, nwg, red[0]);
+    const double a = sum_partials(pin + ((long long)s * 3 + 1) * nwg, nwg, red[1]) / pq;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[kSc * s] = a;
+        sc[kSc * s + 2] = pq;
+    }
     double v[1] = {0.0};
     const long long c0 = (long long)blockIdx.x * kElem + threadIdx.x;
 #pragma unroll 4
@@ -867,17 +874,25 @@ __global__ void __launch_bounds__(256) k_hupdate_xr(long long n, double *__restr
     block_partials<1>(v, partial, s);
 }
 
-// p = z - beta p; beta = 0 starts a fresh direction
+// p = z - beta p, beta = <z,q>/gamma (dot 0 of partial); beta = 0 (no partials)
+// starts a fresh direction
 __global__ void __launch_bounds__(256) k_hupdate_p(long long n, double *__restrict__ p, const double *__restrict__ z,
+                                                   const double *__restrict__ partial, int nwg,
                                                    const double *__restrict__ sc, const int *__restrict__ active,
-                                                   long long istride, int use_beta) {
+                                                   long long istride) {
+    __shared__ double red[4];
     const int s = blockIdx.y;
     if (!active[s]) return;
-    const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const double be = use_beta ? sc[kSc * s + 1] : 0.0;
-    const long long io = s * istride + c;
-    p[io] = z[io] - be * p[io];
+    const double be = nwg ? sum_partials(partial + (long long)s * 3 * nwg, nwg, red) / sc[kSc * s + 2] : 0.0;
+    const long long c0 = (long long)blockIdx.x * kElem + threadIdx.x;
+#pragma unroll 4
+    for (int u = 0; u < kElem / 256; u++) {
+        const long long c = c0 + 256 * u;
+        if (c < n) {
+            const long long io = s * istride + c;
+            p[io] = z[io] - be * p[io];
+        }
+    }
 }
 
 // Vectors at the host boundary: the caller's arrays hold each block in Fortran
@@ -1092,7 +1107,7 @@ struct HeatSolver::Impl {
     std::vector<double *> Z, Z2, R;
     // level-0 FCG arrays
     double *x = nullptr, *r = nullptr, *p = nullptr, *q = nullptr, *b = nullptr, *tmp = nullptr;
-    double *inv_dt = nullptr, *partial = nullptr, *dots = nullptr, *sc = nullptr;
+    double *inv_dt = nullptr, *partial = nullptr, *partial2 = nullptr, *dots = nullptr, *sc = nullptr;
     double *field = nullptr;         // PFSS field and its tables (allocated on first use)
     int *active = nullptr;
     // learned correction work arrays (allocated on first use)
@@ -1124,8 +1139,9 @@ struct HeatSolver::Impl {
     void features(double *z);
     void learned_correction(bool first);
     // sums of npairs dots over nwg workgroups' partials, then the scalars what, what2
-    void final_dots(int npairs, unsigned nwg, int what, int what2 = kScNone, double tol = 0.0) {
-        hipLaunchKernelGGL(k_hdot_final, dim3((unsigned)nsys), dim3(256), 0, stream, (const double *)partial, (int)nwg,
+    void final_dots(int npairs, unsigned nwg, int what, int what2 = kScNone, double tol = 0.0,
+                    const double *part = nullptr) {
+        hipLaunchKernelGGL(k_hdot_final, dim3((unsigned)nsys), dim3(256), 0, stream, part ? part : partial, (int)nwg,
                            npairs, dots, what, what2, sc, active, (double)ist(0),
                            Converge{tol, iters_dev, nactive_dev, relres_dev});
     }
@@ -1373,6 +1389,7 @@ void HeatSolver::setup(const Layout &lay, const HeatParams &hp, int nsys, int nt
     for (int l = 0; l < I.nlev; l++) I.L[l].diag = (const double2 *)I.dalloc((size_t)nsys * I.nb * I.L[l].m * I.L[l].m * 2);
     I.diagonals();
     I.partial = I.dalloc((size_t)nsys * 3 * std::max(I.march_wgs(0), I.elem_wgs()));
+    I.partial2 = I.dalloc((size_t)nsys * 3 * I.elem_wgs());   // <r,r> of the update, which reads partial
     I.dots = I.dalloc((size_t)nsys * 3);
     I.sc = I.dalloc((size_t)nsys * kSc);
     void *a = nullptr;
@@ -1457,13 +1474,47 @@ void HeatSolver::set_rhs_from_host_T(const double *T) {
     HCHECK(hipStreamSynchronize(I.stream));
 }
 
+// Output pages of the caller's array touched by several threads while the GPU
+// prepares the copy: a fresh array's page faults (each page is cleared) otherwise
+// run one by one inside the copy.  Read-back of 50 MB 5.0 -> 3.9 ms.  Below 32 MB
+// the allocator hands out pages it has used before, and the threads cost more
+// than they give (17 MB: 1.0 -> 1.1 ms).
+namespace {
+struct Prefault {
+    std::vector<std::thread> t;
+    Prefault(void *dst, size_t bytes) {
+        const size_t n = std::min(8u, std::max(1u, std::thread::hardware_concurrency() / 2));
+        if (bytes < (32u << 20) || n < 2) return;
+        char *p = (char *)dst;
+        t.reserve(n);
+        try {
+            for (size_t k = 0; k < n; k++) {
+                char *lo = p + bytes * k / n, *hi = p + bytes * (k + 1) / n;
+                t.emplace_back([lo, hi] {
+                    for (volatile char *q = lo; q < hi; q += 4096) *q = *q;
+                });
+            }
+        } catch (const std::system_error &) {
+            // no more threads: the copy faults the rest in
+        }
+    }
+    void join() {
+        for (auto &x : t) x.join();
+        t.clear();
+    }
+    ~Prefault() { join(); }
+};
+}  // namespace
+
 void HeatSolver::get_solution_host(int s, double *T) const {
     const Impl &I = *d;
     const long long n = I.ist(0);
+    Prefault pages(T, sizeof(double) * n);
     hipLaunchKernelGGL(k_hreorder<false>, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, I.stream, I.L[0],
                        (const double *)(I.x + s * n), I.tmp, (const double *)nullptr, n);
     HCHECK(hipGetLastError());
     HCHECK(hipStreamSynchronize(I.stream));
+    pages.join();
     HCHECK(hipMemcpy(T, I.tmp, sizeof(double) * n, hipMemcpyDeviceToHost));
 }
 
@@ -1489,6 +1540,7 @@ void HeatSolver::pfss_field(const std::vector<double> &bot, const std::vector<do
     if ((long long)bot.size() != (long long)I.nb * I.L[0].m * I.L[0].m ||
         (long long)geo.size() != (long long)I.nb * (2 * I.L[0].m + 3))
         throw std::runtime_error("pfss_field: table sizes do not match the layout");
+    Prefault pages(B, sizeof(double) * 3 * n);
     if (!I.field) I.field = I.dalloc(3 * n + bot.size() + geo.size());
     double *dbot = I.field + 3 * n, *dgeo = dbot + bot.size();
     HCHECK(hipMemcpy(dbot, bot.data(), sizeof(double) * bot.size(), hipMemcpyHostToDevice));
@@ -1497,6 +1549,7 @@ void HeatSolver::pfss_field(const std::vector<double> &bot, const std::vector<do
                        (const double *)I.x, (const double *)dbot, (const double *)dgeo, I.field);
     HCHECK(hipGetLastError());
     HCHECK(hipStreamSynchronize(I.stream));
+    pages.join();
     HCHECK(hipMemcpy(B, I.field, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
 }
 
@@ -1645,21 +1698,20 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         }
         const int pre0 = recording ? I.learned_pre0 : I.pre, post0 = recording ? I.learned_post0 : I.post;
         const unsigned nwg = I.vcycle(I.r, z, pre0, post0, first ? nullptr : I.q);
-        if (!first) I.final_dots(1, nwg, kScBeta);
+        hipLaunchKernelGGL(k_hupdate_p, I.grid_elem(), dim3(256), 0, I.stream, ni, I.p, (const double *)z,
+                           (const double *)I.partial, first ? 0 : (int)nwg, (const double *)I.sc, (const int *)I.active, ni);
         if (recording) {
             I.features(z);
             record(z);
         }
-        hipLaunchKernelGGL(k_hupdate_p, g0, dim3(256), 0, I.stream, ni, I.p, (const double *)z, (const double *)I.sc,
-                           (const int *)I.active, ni, first ? 0 : 1);
     };
     // one FCG iteration; the convergence test runs on the device (k_hdot_final)
     auto body = [&](bool lrn) {
         I.apply0(I.p, I.q, I.r);                         // q = A p with <p,q>, <p,r>
-        I.final_dots(2, I.march_wgs(0), kScAlpha);
         hipLaunchKernelGGL(k_hupdate_xr, I.grid_elem(), dim3(256), 0, I.stream, ni, I.x, I.r, (const double *)I.p,
-                           (const double *)I.q, (const double *)I.sc, (const int *)I.active, I.partial, ni);
-        I.final_dots(1, I.elem_wgs(), kScConverge, kScNone, tol);
+                           (const double *)I.q, (const double *)I.partial, (int)I.march_wgs(0), I.sc, (const int *)I.active,
+                           I.partial2, ni);
+        I.final_dots(1, I.elem_wgs(), kScConverge, kScNone, tol, I.partial2);
         precond_direction(false, lrn);
     };
     // directions 0 .. nlearn-1 come from the learned correction, later ones
