@@ -144,6 +144,20 @@ struct DevBoundary {
     int n;
 };
 
+// radial ghosts formed in a fill's launch (none where bnd.n is 0): the mirror
+// of the buffer's interior columns, or with src all radial ghosts of src
+struct FillTail {
+    DevBoundary bnd{nullptr, 0};
+    const void *src = nullptr;
+};
+// dt from the partial minima, formed in a boundary launch (none where partial is null)
+struct DtFinal {
+    const double *partial = nullptr;
+    int n = 0;
+    double cfl = 0.0;
+    double *dtp = nullptr;
+};
+
 // launchers (kernels.hip)
 // pull (null: none): the pull table of DevGhosts; ghosts of `in` in the
 // directions it lists are read from the neighbour's interior instead.
@@ -172,7 +186,8 @@ void launch_glm_diffusion(const Dims &d, const DevTables &t, const double *U, co
                           const double *dtp, hipStream_t s);
 // the FP64 buffers' ghosts and (psi not null) psi's, in one pass over the
 // table; faces: only the ghosts outside the block along one axis
-void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s);
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s,
+                       const FillTail &tail = FillTail{});
 // Uold: U^n for the FP32 path, whose diffusion updates U (= out) in place;
 // null for the FP64 path (U != out)
 template <typename T, typename TIN>
@@ -188,18 +203,19 @@ int march_resident_wgs(int kernel, int precision, int tile);
 // one per tile and segment.
 int march_segments(const Dims &d, int tile, int wgs);
 // every ghost entry of the FP32 buffers
-void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s);
+void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s, const FillTail &tail = FillTail{});
 // the entries that kernels reading with pull = g.pull still need; faces: only
 // the ghosts outside the block along one axis
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s);
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s,
+                          const FillTail &tail = FillTail{});
 template <typename TS>
-void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull = nullptr);
-template <typename TS>
-void launch_copy_radial(const Dims &d, const DevBoundary &b, const TS *src, TS *dst, hipStream_t s);
+void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull = nullptr,
+                     const DtFinal &dt = DtFinal{});
 // nseg: the radial segments of the diffusion's tiles (march_segments): one
 // partial minimum per tile and segment
 void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, double *partial, hipStream_t s, int tile,
                        int nseg);
+DtFinal dt_final_args(const Dims &d, const double *partial, double *dtp, double cfl, int tile, int nseg);
 void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile, int nseg);
 // nvar variables of one block ([nvar][P], cell_off layout) in Fortran order into pinned host memory
 void launch_block_to_host(const Dims &d, const double *src, int nvar, double *dst, hipStream_t s);

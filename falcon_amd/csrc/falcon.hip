@@ -650,10 +650,12 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
     double *dtp = h->dtp.as<double>(), *part = h->partial.as<double>();
     const int ts = h->tile_stage[h->precision], td = h->tile_diff[h->precision];
     const int ws = h->wgs_stage[h->precision], wd = h->wgs_diff[h->precision];
-    timed(h, K_DT, [&] {
-        if (h->fixed_dt > 0) launch_set_scalar(dtp, h->fixed_dt, s);
-        else launch_dt_final(d, part, dtp, cfl, s, td, march_segments(d, td, wd));
-    });
+    // dt is formed in the launch of the state's radial boundary, the stage
+    // buffers' radial ghosts in their fills
+    DtFinal dtf;
+    if (h->fixed_dt > 0) timed(h, K_DT, [&] { launch_set_scalar(dtp, h->fixed_dt, s); });
+    else dtf = dt_final_args(d, part, dtp, cfl, td, march_segments(d, td, wd));
+    const FillTail mirror{h->bnd, nullptr};
     if (h->precision == 0) {
         double *S0 = h->S64[0].as<double>(), *S1 = h->S64[1].as<double>();
         const double *in[4] = {U, S0, S1, S0};
@@ -670,7 +672,7 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         if (glm) timed(h, K_OTHER, [&] { launch_glm_speed(d, t, U, Ch, s); });
         for (int k = 1; k <= 4; k++) {
             const double div = (double)(5.0f - (float)k);
-            timed(h, K_BC, [&] { launch_boundary<double>(d, h->bnd, const_cast<double *>(in[k - 1]), s); });
+            if (k == 1) timed(h, K_BC, [&] { launch_boundary<double>(d, h->bnd, U, s, nullptr, dtf); });
             if (glm)
                 timed(h, K_OTHER,
                       [&] { launch_glm_stage(d, t, in[k - 1], Ch, pin[k - 1], P, pout[k - 1], G, dtp, div, s); });
@@ -681,15 +683,12 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
             timed(h, k < 4 ? K_XSTAGE : K_XSTATE, [&] {
                 // the stage buffers' ghosts beyond edges and corners are left out: the
                 // diffusion alone reads such ghosts (its shifted speed cells), the state's
-                launch_exchange64(d, h->gh64, out[k - 1], pout[k - 1], k < 4, s);
+                launch_exchange64(d, h->gh64, out[k - 1], pout[k - 1], k < 4, s, k < 4 ? mirror : FillTail{});
             });
         }
         timed(h, K_DIFF, [&] { launch_diffusion<double, double>(d, t, U, U, Un, nullptr, part, dtp, s, nullptr, td, wd); });
         if (glm) timed(h, K_OTHER, [&] { launch_glm_diffusion(d, t, U, P, Pn, dtp, s); });
-        timed(h, K_OTHER, [&] { launch_copy_radial<double>(d, h->bnd, U, Un, s); });
-        timed(h, K_XSTATE, [&] {
-            launch_exchange64(d, h->gh64, Un, Pn, false, s);
-        });
+        timed(h, K_XSTATE, [&] { launch_exchange64(d, h->gh64, Un, Pn, false, s, FillTail{h->bnd, U}); });
     } else {
         float *S0 = h->S32[0].as<float>(), *S1 = h->S32[1].as<float>();
         float *F = h->F32[cur].as<float>(), *Fn = h->F32[1 - cur].as<float>();
@@ -702,11 +701,12 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         // speed cells, and through the first stage's radial mirror of them)
         const int32_t *pull = h->ghost_pull ? h->gh32.pull : nullptr;
         auto exchange = [&](float *st, bool faces) {
-            if (pull) launch_exchange_rest(d, h->gh32, st, faces, s);
-            else launch_exchange(d, h->gh32, st, s);
+            const FillTail tail = faces ? mirror : FillTail{};
+            if (pull) launch_exchange_rest(d, h->gh32, st, faces, s, tail);
+            else launch_exchange(d, h->gh32, st, s, tail);
         };
         for (int k = 1; k <= 4; k++) {
-            timed(h, K_BC, [&] { launch_boundary<float>(d, h->bnd, const_cast<float *>(in[k - 1]), s, pull); });
+            if (k == 1) timed(h, K_BC, [&] { launch_boundary<float>(d, h->bnd, F, s, pull, dtf); });
             const double div = (double)(5.0f - (float)k);
             if (k < 4) {
                 // intermediate stage values are FP32 temporaries: base = FP32 copy of U^n
@@ -1542,7 +1542,7 @@ int falcon_check_state(falcon_handle_t h, int which, int64_t *n_nan, int32_t *wh
             if (h->divb) launch_nan_scan_psi(d, h->psi[h->cur].as<double>(), w, h->stream);
         } else if (h->precision == 0) {
             if (!h->S64[0].p) throw Error("falcon_check_state: no stage buffer yet");
-            // the ghosts beyond edges and corners that the steps leave out
+            // the ghosts beyond edges and corners and of the radial ghost planes' columns that the steps leave out
             if (h->dt.meta) {
                 launch_exchange64(d, h->gh64, h->S64[0].as<double>(), h->divb ? h->psiS[0].as<double>() : nullptr, false,
                                   h->stream);
@@ -1552,10 +1552,11 @@ int falcon_check_state(falcon_handle_t h, int which, int64_t *n_nan, int32_t *wh
             if (h->divb) launch_nan_scan_psi(d, h->psiS[0].as<double>(), w, h->stream);
         } else {
             if (!h->S32[0].p) throw Error("falcon_check_state: no stage buffer yet");
-            // the ghosts beyond edges and corners that the steps leave out
-            if (h->ghost_pull && h->dt.meta) {
-                launch_exchange_rest(d, h->gh32, h->S32[0].as<float>(), false, h->stream);
-                launch_boundary<float>(d, h->bnd, h->S32[0].as<float>(), h->stream, h->gh32.pull);
+            // the ghosts beyond edges and corners and of the radial ghost planes' columns that the steps leave out
+            if (h->dt.meta) {
+                const int32_t *pull = h->ghost_pull ? h->gh32.pull : nullptr;
+                if (pull) launch_exchange_rest(d, h->gh32, h->S32[0].as<float>(), false, h->stream);
+                launch_boundary<float>(d, h->bnd, h->S32[0].as<float>(), h->stream, pull);
             }
             launch_nan_scan<float>(d, h->S32[0].as<float>(), w, h->stream);
         }

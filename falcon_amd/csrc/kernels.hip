@@ -979,6 +979,37 @@ __device__ __forceinline__ void yy_rotate(double (&val)[8], double a, double bb)
 // with an exactly-zero weight), so entries are independent.
 //
 //
+// The radial ghosts that go with a fill, formed by workgroups behind those of the
+// entries (they read and write other cells: interior and radial-ghost planes,
+// where no entry has its target or a loaded corner).  On their own each was a
+// launch of 4 to 8 us between kernels.
+// mirror: the radial ghosts of a stage buffer, its interior columns alone (the
+//   stage kernels read no other ghost of those planes); parities as k_boundary;
+// copy: the radial ghosts of `src` (all columns) into the buffer.
+template <typename TS>
+__device__ __forceinline__ void fill_tail(const Dims &d, const FillTail &tail, TS *st, unsigned id) {
+    const bool mirror = tail.src == nullptr;
+    const unsigned nk = (unsigned)(mirror ? d.nk : d.NK), nj = (unsigned)(mirror ? d.nj : d.NJ), ng = (unsigned)d.ng;
+    if (id >= (unsigned)tail.bnd.n * ng * nj * nk) return;
+    unsigned r = id / nk;
+    const int k = (int)(id - r * nk) + (mirror ? d.ng : 0);
+    const unsigned q = r / nj;
+    const int j = (int)(r - q * nj) + (mirror ? d.ng : 0);
+    const unsigned e = q / ng;
+    const int g = (int)(q - e * ng);
+    const int b = tail.bnd.list[e] >> 1, side = tail.bnd.list[e] & 1;
+    const int dI = side ? d.ni + d.ng + g : g, sI = side ? d.ni + d.ng - 1 - g : 2 * d.ng - 1 - g;
+    const long long base = (long long)b * 8 * d.P, dst = base + cell_off(d, dI, j, k);
+    const long long so = mirror ? base + cell_off(d, sI, j, k) : dst;
+    const TS *S = mirror ? st : (const TS *)tail.src;
+    const unsigned neg = !mirror ? 0u : (side ? 0x62u : 0x12u);   // as k_boundary
+    TS x[8];
+#pragma unroll
+    for (int v = 0; v < 8; v++) x[v] = S[so + (long long)v * d.P];
+#pragma unroll
+    for (int v = 0; v < 8; v++) st[dst + (long long)v * d.P] = ((neg >> v) & 1u) ? -x[v] : x[v];
+}
+
 // Workgroup of a fill in the order of its sources: runs of kXcdRun workgroups
 // go to one XCD, whose L2 then holds the lines they share.
 constexpr int kXcdRun = 64;
@@ -1005,7 +1036,7 @@ __device__ __forceinline__ int xcd_run(int wg, int n) {
 // 71 us on 528 refined ones, 20 us on 648 8^3 ones; one launch in source order
 // 81, 59 and 13 us, its face ghosts alone 52, 42 and 9 us.
 __global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFill copy, int nwe, int nle, int nce,
-                                                      float *__restrict__ st) {
+                                                      float *__restrict__ st, FillTail tail) {
     const int nw = (nwe + 255) / 256, nl = (nle + 255) / 256, nc = (nce + 255) / 256;
     const long long P = d.P;
     // a base cell is interior along phi, so its corners are in the main part
@@ -1047,6 +1078,10 @@ __global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFi
         return;
     }
     wg -= nl;
+    if (wg >= nc) {
+        fill_tail(d, tail, st, (unsigned)(wg - nc) * 256u + threadIdx.x);
+        return;
+    }
     const int e = xcd_run(wg, nc) * 256 + (int)threadIdx.x;
     if (e >= nce) return;
     const int2 c = copy.idx[e];
@@ -1079,8 +1114,14 @@ __global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFi
 // PSI: also psi of GLM divergence cleaning ([block][P]), a scalar.
 template <bool PSI>
 __global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, const int32_t *__restrict__ all,
-                                                      int n, double *__restrict__ st, double *__restrict__ psi) {
-    int e = xcd_run(blockIdx.x, gridDim.x) * 256 + (int)threadIdx.x;
+                                                      int n, double *__restrict__ st, double *__restrict__ psi,
+                                                      FillTail tail) {
+    const int nx = (n + 255) / 256;
+    if ((int)blockIdx.x >= nx) {
+        fill_tail(d, tail, st, (blockIdx.x - (unsigned)nx) * 256u + threadIdx.x);
+        return;
+    }
+    int e = xcd_run(blockIdx.x, nx) * 256 + (int)threadIdx.x;
     if (e >= n) return;
     if (all) e = all[e];
     const long long P = d.P;
@@ -1114,6 +1155,27 @@ __global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, con
     if constexpr (PSI) psi[psi_off(d, dst)] = value(psi + psi_off(d, src));
 }
 
+// dt = min(1.e20, CFL * min) of the partial minima, by one workgroup
+__device__ __forceinline__ void dt_final(const double *__restrict__ partial, int n, double cfl, double *__restrict__ dtp) {
+    double mn = INFINITY;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) mn = partial[i] < mn ? partial[i] : mn;
+    for (int off = 32; off > 0; off >>= 1) {
+        double o = __shfl_down(mn, off, 64);
+        mn = o < mn ? o : mn;
+    }
+    __shared__ double red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mn;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double r = red[0];
+        for (int w = 1; w < (int)(blockDim.x >> 6); w++) r = red[w] < r ? red[w] : r;
+        // dt = min(1.e20, CFL*min) (3_6/ModTimeStep.f90:254-262)
+        double dt = cfl * r;
+        const double big = (double)1.0e20f;
+        dtp[0] = dt < big ? dt : big;
+    }
+}
+
 // ---------------------------------------------------------------- boundary
 
 // ModBoundary_Dynamo_primitives (3_6/ModBoundary.f90:10-55): radial mirror of
@@ -1123,15 +1185,19 @@ __global__ void __launch_bounds__(256) k_exchange_f64(Dims d, DevGhosts64 g, con
 // direction are read from the same-level neighbour's interior.
 template <typename TS>
 __global__ void __launch_bounds__(256) k_boundary(Dims d, DevBoundary bl, TS *__restrict__ st,
-                                                  const int32_t *__restrict__ pull) {
-    const long long plane = (long long)d.NJ * d.NK;
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long per = (long long)d.ng * plane;
-    if (tid >= per * bl.n) return;
+                                                  const int32_t *__restrict__ pull, DtFinal dt) {
+    // a step's first launch: its last workgroup forms dt
+    if (dt.partial && blockIdx.x == gridDim.x - 1) {
+        dt_final(dt.partial, dt.n, dt.cfl, dt.dtp);
+        return;
+    }
+    const unsigned plane = (unsigned)(d.NJ * d.NK), per = (unsigned)d.ng * plane;
+    const unsigned tid = blockIdx.x * 256u + threadIdx.x;
+    if (tid >= per * (unsigned)bl.n) return;
     const int e = (int)(tid / per);
-    const long long rem = tid - (long long)e * per;
+    const unsigned rem = tid - (unsigned)e * per;
     const int g = (int)(rem / plane);
-    const long long jk = rem - (long long)g * plane;
+    const unsigned jk = rem - (unsigned)g * plane;
     const int b = bl.list[e] >> 1, side = bl.list[e] & 1;
     int dI, sI;
     if (side) { dI = d.ni + d.ng + g; sI = d.ni + d.ng - 1 - g; }
@@ -1139,7 +1205,7 @@ __global__ void __launch_bounds__(256) k_boundary(Dims d, DevBoundary bl, TS *__
     // signs: top (+,-,+,+,+,-,-,+), bottom (+,-,+,+,-,+,+,+)
     const unsigned neg = side ? 0x62u : 0x12u;   // bit v set -> negate variable v
     // (J, K) of this thread's cell, enumerated row by row over the padded plane
-    const int J = (int)(jk / d.NK), K = (int)(jk - (long long)J * d.NK);
+    const int J = (int)(jk / (unsigned)d.NK), K = (int)(jk - (unsigned)J * (unsigned)d.NK);
     TS *base = st + (long long)b * 8 * d.P;
     const TS *src = base;
     long long soff = cell_off(d, sI, J, K);
@@ -1215,46 +1281,7 @@ __global__ void __launch_bounds__(TL * TL) k_dt_tile(Dims d, DevTables t, const 
     }
 }
 
-__global__ void __launch_bounds__(256) k_dt_final(const double *__restrict__ partial, int n, double cfl,
-                                                  double *__restrict__ dtp) {
-    double mn = INFINITY;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) mn = partial[i] < mn ? partial[i] : mn;
-    for (int off = 32; off > 0; off >>= 1) {
-        double o = __shfl_down(mn, off, 64);
-        mn = o < mn ? o : mn;
-    }
-    __shared__ double red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mn;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double r = red[0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) r = red[w] < r ? red[w] : r;
-        // dt = min(1.e20, CFL*min) (3_6/ModTimeStep.f90:254-262)
-        double dt = cfl * r;
-        const double big = (double)1.0e20f;
-        dtp[0] = dt < big ? dt : big;
-    }
-}
-
-// Radial ghost planes of top/bottom blocks copied from one buffer to another.
-template <typename TS>
-__global__ void __launch_bounds__(256) k_copy_radial(Dims d, DevBoundary bl, const TS *__restrict__ src,
-                                                     TS *__restrict__ dst) {
-    const long long plane = (long long)d.NJ * d.NK;
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long per = (long long)d.ng * plane;
-    if (tid >= per * bl.n) return;
-    const int e = (int)(tid / per);
-    const long long rem = tid - (long long)e * per;
-    const int g = (int)(rem / plane);
-    const long long jk = rem - (long long)g * plane;
-    const int b = bl.list[e] >> 1, side = bl.list[e] & 1;
-    const int I = side ? d.ni + d.ng + g : g;
-    const int J = (int)(jk / d.NK), K = (int)(jk - (long long)J * d.NK);
-    const long long base = (long long)b * 8 * d.P + cell_off(d, I, J, K);
-#pragma unroll
-    for (int v = 0; v < 8; v++) dst[base + (long long)v * d.P] = src[base + (long long)v * d.P];
-}
+__global__ void __launch_bounds__(256) k_dt_final(DtFinal f) { dt_final(f.partial, f.n, f.cfl, f.dtp); }
 
 __global__ void k_to_f32(const double *__restrict__ s, float *__restrict__ d, long long n) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1592,44 +1619,51 @@ void launch_diffusion_only(const Dims &d, const DevTables &t, const double *U, d
                         (const int32_t *)nullptr, tile, wgs, (const double *)nullptr);
 }
 
+static unsigned tail_wgs(const Dims &d, const FillTail &t) {
+    if (t.bnd.n == 0) return 0;
+    const long long n = (long long)t.bnd.n * d.ng * (t.src ? (long long)d.NJ * d.NK : (long long)d.nj * d.nk);
+    return (unsigned)((n + 255) / 256);
+}
+
 static void exchange32(const Dims &d, const DevGhosts &g, const DevFill &copy, bool faces, float *state,
-                       hipStream_t s) {
+                       hipStream_t s, const FillTail &tail) {
     auto n = [&](const DevFill &f) { return faces ? f.n_face : f.n; };
     const int nw = n(g.weighted), nl = n(g.lerp), nc = n(copy);
-    const unsigned wgs = (unsigned)((nw + 255) / 256 + (nl + 255) / 256 + (nc + 255) / 256);
-    if (wgs) hipLaunchKernelGGL(k_exchange_f32, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state);
+    const unsigned wgs = (unsigned)((nw + 255) / 256 + (nl + 255) / 256 + (nc + 255) / 256) + tail_wgs(d, tail);
+    if (wgs) hipLaunchKernelGGL(k_exchange_f32, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state, tail);
 }
 
-void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s) {
-    exchange32(d, g, g.copy, false, state, s);
+void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s, const FillTail &tail) {
+    exchange32(d, g, g.copy, false, state, s, tail);
 }
 
-void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s) {
+void launch_exchange_rest(const Dims &d, const DevGhosts &g, float *state, bool faces, hipStream_t s,
+                          const FillTail &tail) {
     if (!g.pull) throw std::runtime_error("no pull table: use the full exchange");
-    exchange32(d, g, g.copy_rest, faces, state, s);
+    exchange32(d, g, g.copy_rest, faces, state, s, tail);
 }
 
-void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s) {
+void launch_exchange64(const Dims &d, const DevGhosts64 &g, double *state, double *psi, bool faces, hipStream_t s,
+                       const FillTail &tail) {
     const int n = faces ? g.n_face : g.n;
-    if (n <= 0) return;
-    const dim3 grid((unsigned)((n + 255) / 256)), wg(256);
+    const unsigned wgs = (unsigned)((n + 255) / 256) + tail_wgs(d, tail);
+    if (wgs == 0) return;
+    const dim3 grid(wgs), wg(256);
     const int32_t *all = faces ? nullptr : g.all;
-    if (psi) hipLaunchKernelGGL(k_exchange_f64<true>, grid, wg, 0, s, d, g, all, n, state, psi);
-    else hipLaunchKernelGGL(k_exchange_f64<false>, grid, wg, 0, s, d, g, all, n, state, psi);
+    if (psi) hipLaunchKernelGGL(k_exchange_f64<true>, grid, wg, 0, s, d, g, all, n, state, psi, tail);
+    else hipLaunchKernelGGL(k_exchange_f64<false>, grid, wg, 0, s, d, g, all, n, state, psi, tail);
 }
 
 template <typename TS>
-void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull) {
-    if (b.n == 0) return;
+void launch_boundary(const Dims &d, const DevBoundary &b, TS *state, hipStream_t s, const int32_t *pull, const DtFinal &dt) {
     const long long n = (long long)b.n * d.ng * d.NJ * d.NK;
-    hipLaunchKernelGGL((k_boundary<TS>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, b, state, pull);
+    const unsigned wgs = (unsigned)((n + 255) / 256) + (dt.partial ? 1u : 0u);
+    if (wgs) hipLaunchKernelGGL((k_boundary<TS>), dim3(wgs), dim3(256), 0, s, d, b, state, pull, dt);
 }
 
-template <typename TS>
-void launch_copy_radial(const Dims &d, const DevBoundary &b, const TS *src, TS *dst, hipStream_t s) {
-    if (b.n == 0) return;
-    const long long n = (long long)b.n * d.ng * d.NJ * d.NK;
-    hipLaunchKernelGGL((k_copy_radial<TS>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, b, src, dst);
+DtFinal dt_final_args(const Dims &d, const double *partial, double *dtp, double cfl, int tile, int nseg) {
+    check_tile(tile);
+    return DtFinal{partial, (int)(tiles(d, tile) * (unsigned)nseg), cfl, dtp};
 }
 
 // the partial minima are laid out as the diffusion with the same tile edge
@@ -1644,8 +1678,7 @@ void launch_dt_partial(const Dims &d, const DevTables &t, const double *U, doubl
 
 void launch_dt_final(const Dims &d, const double *partial, double *dtp, double cfl, hipStream_t s, int tile,
                      int nseg) {
-    check_tile(tile);
-    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, s, partial, (int)(tiles(d, tile) * (unsigned)nseg), cfl, dtp);
+    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, s, dt_final_args(d, partial, dtp, cfl, tile, nseg));
 }
 
 void launch_set_scalar(double *p, double v, hipStream_t s) {
@@ -2059,9 +2092,9 @@ template void launch_diffusion<double, double>(const Dims &, const DevTables &, 
 template void launch_diffusion<float, float>(const Dims &, const DevTables &, const float *, const double *, double *, float *, double *, const double *, hipStream_t, const int32_t *, int, int, const double *);
 template void launch_diffusion_only<double>(const Dims &, const DevTables &, const double *, double *, hipStream_t, int, int);
 template void launch_diffusion_only<float>(const Dims &, const DevTables &, const double *, double *, hipStream_t, int, int);
-template void launch_boundary<double>(const Dims &, const DevBoundary &, double *, hipStream_t, const int32_t *);
-template void launch_boundary<float>(const Dims &, const DevBoundary &, float *, hipStream_t, const int32_t *);
-template void launch_copy_radial<double>(const Dims &, const DevBoundary &, const double *, double *, hipStream_t);
-template void launch_copy_radial<float>(const Dims &, const DevBoundary &, const float *, float *, hipStream_t);
+template void launch_boundary<double>(const Dims &, const DevBoundary &, double *, hipStream_t, const int32_t *,
+                                      const DtFinal &);
+template void launch_boundary<float>(const Dims &, const DevBoundary &, float *, hipStream_t, const int32_t *,
+                                     const DtFinal &);
 
 }  // namespace falcon
