@@ -89,10 +89,15 @@ struct FieldT {
     int lm;
     double omega;
     __device__ __forceinline__ double operator()(long long c) const {
-        const double v = x[c];
-        if (!FIRST) return v;
+        return FIRST ? from(x[c], diag[c >> lm]) : x[c];
+    }
+    __device__ __forceinline__ double from(double v, double2 d) const { return div_by(omega * v, d.x, d.y); }
+    // the values at c and c + 1 (one phi row, so one diagonal)
+    __device__ __forceinline__ double2 pair(long long c) const {
+        const double v0 = x[c], v1 = x[c + 1];
+        if (!FIRST) return make_double2(v0, v1);
         const double2 d = diag[c >> lm];
-        return div_by(omega * v, d.x, d.y);
+        return make_double2(from(v0, d), from(v1, d));
     }
 };
 typedef FieldT<false> Field;
@@ -162,8 +167,10 @@ template <class F>
 __device__ __forceinline__ double trilinear(const HLev &L, const F &X, long long c, int wid, double f0) {
     const double wi = L.gw[3 * wid], wj = L.gw[3 * wid + 1], wk = L.gw[3 * wid + 2];
     const long long S1 = L.m, SI = (long long)L.m * L.m;
-    const double f1 = X(c + SI), f2 = X(c + S1), f3 = X(c + 1), f4 = X(c + SI + S1), f5 = X(c + S1 + 1),
-                 f6 = X(c + SI + 1), f7 = X(c + SI + S1 + 1);
+    // (the base cell is inside its block along every axis, so are its corners)
+    const double2 p10 = X.pair(c + SI), p01 = X.pair(c + S1), p11 = X.pair(c + SI + S1);
+    const double f3 = X(c + 1);
+    const double f1 = p10.x, f2 = p01.x, f4 = p11.x, f5 = p01.y, f6 = p10.y, f7 = p11.y;
     double t = f0 * (1.0 - wi) * (1.0 - wj) * (1.0 - wk);
     t = t + f1 * (wi) * (1.0 - wj) * (1.0 - wk);
     t = t + f2 * (1.0 - wi) * (wj) * (1.0 - wk);
