@@ -132,6 +132,7 @@ struct falcon_handle {
     DevBuf diffbuf;          // falcon_state_diff's reduction words
     DevBuf scanbuf;          // falcon_check_state's count and first position
     double *pinned = nullptr;      // host staging of the block read-backs (read_block), made on first use
+    hipEvent_t pinned_ev[2] = {nullptr, nullptr};
     int cur = 0;             // index of the current state buffer in U[]
     // validity of derived device data
     bool partials_valid = false;   // partial[] holds min(h/v_wave) of U[cur]
@@ -169,6 +170,8 @@ struct falcon_handle {
                          &U[0], &U[1], &F32[0], &F32[1], &S64[0], &S64[1], &S32[0], &S32[1], &dtp, &partial, &rbuf, &diffbuf, &scanbuf,
                          &psi[0], &psi[1], &psiS[0], &psiS[1], &glmG, &glmC};
         for (DevBuf *b : all) b->free();
+        for (hipEvent_t e : pinned_ev)
+            if (e) (void)hipEventDestroy(e);
         if (pinned) (void)hipHostFree(pinned);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -773,18 +776,33 @@ void refresh_u_ghosts(falcon_handle *h) {
 void check_launch() { HIPCHECK(hipGetLastError()); }
 
 // nvar variables of one block to the caller in Fortran order: transposed by the
-// GPU into a pinned buffer that the handle keeps (at most 4 MB, or one variable
-// where that is more), then copied.  Synchronises the stream.
+// GPU into one half of a pinned buffer that the handle keeps while the host
+// copies the other half out.  A half holds up to 1 MB (one variable where that
+// is more); a block of 256 KB or more goes in at least two parts.  A block of 4.5
+// MB takes 176 us instead of 250 with one part after the other, one of 512 KB 35
+// us either way.
+// Synchronises the stream.
 void read_block(falcon_handle *h, const double *src, int nvar, double *dst) {
-    const size_t P = (size_t)h->dims.P;
-    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(8, (size_t)4194304 / (P * sizeof(double))));
-    if (!h->pinned) HIPCHECK(hipHostMalloc((void **)&h->pinned, sizeof(double) * P * chunk, hipHostMallocDefault));
-    for (int v = 0; v < nvar; v += chunk) {
-        const int n = std::min(chunk, nvar - v);
-        launch_block_to_host(h->dims, src + v * P, n, h->pinned, h->stream);
+    const size_t P = (size_t)h->dims.P, var = P * sizeof(double);
+    const int half = (int)std::max<size_t>(1, std::min<size_t>(8, ((size_t)1 << 20) / var));
+    if (!h->pinned) {
+        HIPCHECK(hipHostMalloc((void **)&h->pinned, 2 * half * var, hipHostMallocDefault));
+        for (hipEvent_t &e : h->pinned_ev) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    const int part = std::min(half, nvar > 1 && nvar * var >= ((size_t)256 << 10) ? (nvar + 1) / 2 : nvar);
+    auto launch = [&](int q) {
+        const int v = q * part;
+        launch_block_to_host(h->dims, src + v * P, std::min(part, nvar - v), h->pinned + (size_t)(q & 1) * half * P, h->stream);
         check_launch();
-        HIPCHECK(hipStreamSynchronize(h->stream));
-        std::memcpy(dst + v * P, h->pinned, sizeof(double) * P * n);
+        HIPCHECK(hipEventRecord(h->pinned_ev[q & 1], h->stream));
+    };
+    const int parts = (nvar + part - 1) / part;
+    launch(0);
+    for (int q = 0; q < parts; q++) {
+        if (q + 1 < parts) launch(q + 1);
+        HIPCHECK(hipEventSynchronize(h->pinned_ev[q & 1]));
+        const int v = q * part;
+        std::memcpy(dst + v * P, h->pinned + (size_t)(q & 1) * half * P, var * std::min(part, nvar - v));
     }
 }
 
