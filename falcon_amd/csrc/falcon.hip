@@ -9,6 +9,7 @@
 #include <cstring>
 #include <filesystem>
 #include <fstream>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <random>
@@ -377,7 +378,7 @@ void upload_ghosts64(falcon_handle *h) {
     const std::vector<GhostEntry> &G = h->lay.ghosts;
     const size_t N = G.size();
     const int nb = d.nblocks, ng = d.ng;
-    const int nt = std::max(1, std::min(host_threads(), (int)(N / 65536) + 1));
+    const int nt = std::max(1, std::min(host_threads(), (int)(N / 8192) + 1));
     auto parallel = [&](auto &&f) {
         std::vector<std::thread> th;
         for (int t = 1; t < nt; t++) th.emplace_back([&, t] { f(t); });
@@ -515,9 +516,13 @@ void upload_tables(falcon_handle *h) {
         std::sort(mid, v.end(), less);
         return (int)(mid - v.begin());
     };
-    upload_ghosts64(h);
-    DevGhosts &g32 = h->gh32;
-    {
+    // the three FP32 tables are sorted by tasks beside the FP64 table
+    struct Table {
+        std::vector<int2> idx;
+        std::vector<double> w, rot;
+        int nf = 0;
+    };
+    auto weighted = std::async(std::launch::async | std::launch::deferred, [&]() -> Table {
         // a base on an axis's last cell (weight 0 there) becomes the cell before it
         // with weight 1, so that no corner is a ghost of the donor (k_exchange_f32)
         const int n3[3] = {t.ni, t.nj, t.nk};
@@ -535,44 +540,53 @@ void upload_tables(falcon_handle *h) {
             wt.push_back({make_int2((int32_t)((uint32_t)dst | (g.yy ? 0x80000000u : 0u)),
                                     (int32_t)((long long)g.donor * 8 * P + cell(g.i0, g.j0, g.k0))), (uint32_t)e});
         }
-        const int nf = by_source(wt, [](const auto &x) -> const int2 & { return x.first; });
-        std::vector<int2> idx(wt.size());
-        std::vector<double> w(3 * wt.size()), rot(2 * wt.size());
+        Table r;
+        r.nf = by_source(wt, [](const auto &x) -> const int2 & { return x.first; });
+        r.idx.resize(wt.size());
+        r.w.resize(3 * wt.size());
+        r.rot.resize(2 * wt.size());
         for (size_t q = 0; q < wt.size(); q++) {
             const GhostEntry g = inside(G[wt[q].second]);
-            idx[q] = wt[q].first;
-            w[3 * q] = g.w[0]; w[3 * q + 1] = g.w[1]; w[3 * q + 2] = g.w[2];
-            rot[2 * q] = g.rot[0]; rot[2 * q + 1] = g.rot[1];
+            r.idx[q] = wt[q].first;
+            r.w[3 * q] = g.w[0]; r.w[3 * q + 1] = g.w[1]; r.w[3 * q + 2] = g.w[2];
+            r.rot[2 * q] = g.rot[0]; r.rot[2 * q + 1] = g.rot[1];
         }
-        up(h->ghost32[0], idx.data(), sizeof(int2) * idx.size());
-        up(h->ghost32[1], w.data(), sizeof(double) * w.size());
-        up(h->ghost32[2], rot.data(), sizeof(double) * rot.size());
-        g32.weighted = {h->ghost32[0].as<int2>(), (int)idx.size(), nf};
-        g32.w = h->ghost32[1].as<double>();
-        g32.rot = h->ghost32[2].as<double>();
-    }
-    {
-        const int nf = by_source(lerp32, [](const auto &x) -> const int2 & { return x.first; });
-        std::vector<int2> idx(lerp32.size());
-        std::vector<double> w(lerp32.size());
-        for (size_t q = 0; q < lerp32.size(); q++) { idx[q] = lerp32[q].first; w[q] = lerp32[q].second; }
-        up(h->ghost_lerp32[0], idx.data(), sizeof(int2) * idx.size());
-        up(h->ghost_lerp32[1], w.data(), sizeof(double) * w.size());
-        g32.lerp = {h->ghost_lerp32[0].as<int2>(), (int)idx.size(), nf};
-        g32.lerp_w = h->ghost_lerp32[1].as<double>();
-    }
-    {
-        std::vector<int32_t> pull;
-        std::vector<int2> rest;
-        build_pull_table(h, copy32, pull, rest);
-        const int nf = by_source(rest, [](const int2 &x) -> const int2 & { return x; });
-        up(h->ghost_copy32, copy32.data(), sizeof(int2) * copy32.size());
-        up(h->ghost_rest32, rest.data(), sizeof(int2) * rest.size());
-        up(h->ghost_pull32, pull.data(), sizeof(int32_t) * pull.size());
-        g32.copy = {h->ghost_copy32.as<int2>(), (int)copy32.size(), (int)copy32.size()};
-        g32.copy_rest = {h->ghost_rest32.as<int2>(), (int)rest.size(), nf};
-        g32.pull = h->ghost_pull32.as<int32_t>();
-    }
+        return r;
+    });
+    auto lerps = std::async(std::launch::async | std::launch::deferred, [&]() -> Table {
+        Table r;
+        r.nf = by_source(lerp32, [](const auto &x) -> const int2 & { return x.first; });
+        r.idx.resize(lerp32.size());
+        r.w.resize(lerp32.size());
+        for (size_t q = 0; q < lerp32.size(); q++) { r.idx[q] = lerp32[q].first; r.w[q] = lerp32[q].second; }
+        return r;
+    });
+    std::vector<int32_t> pull;
+    auto rests = std::async(std::launch::async | std::launch::deferred, [&]() -> Table {
+        Table r;
+        build_pull_table(h, copy32, pull, r.idx);
+        r.nf = by_source(r.idx, [](const int2 &x) -> const int2 & { return x; });
+        return r;
+    });
+    upload_ghosts64(h);
+    DevGhosts &g32 = h->gh32;
+    const Table tw = weighted.get(), tl = lerps.get(), tr = rests.get();
+    up(h->ghost32[0], tw.idx.data(), sizeof(int2) * tw.idx.size());
+    up(h->ghost32[1], tw.w.data(), sizeof(double) * tw.w.size());
+    up(h->ghost32[2], tw.rot.data(), sizeof(double) * tw.rot.size());
+    g32.weighted = {h->ghost32[0].as<int2>(), (int)tw.idx.size(), tw.nf};
+    g32.w = h->ghost32[1].as<double>();
+    g32.rot = h->ghost32[2].as<double>();
+    up(h->ghost_lerp32[0], tl.idx.data(), sizeof(int2) * tl.idx.size());
+    up(h->ghost_lerp32[1], tl.w.data(), sizeof(double) * tl.w.size());
+    g32.lerp = {h->ghost_lerp32[0].as<int2>(), (int)tl.idx.size(), tl.nf};
+    g32.lerp_w = h->ghost_lerp32[1].as<double>();
+    up(h->ghost_copy32, copy32.data(), sizeof(int2) * copy32.size());
+    up(h->ghost_rest32, tr.idx.data(), sizeof(int2) * tr.idx.size());
+    up(h->ghost_pull32, pull.data(), sizeof(int32_t) * pull.size());
+    g32.copy = {h->ghost_copy32.as<int2>(), (int)copy32.size(), (int)copy32.size()};
+    g32.copy_rest = {h->ghost_rest32.as<int2>(), (int)tr.idx.size(), tr.nf};
+    g32.pull = h->ghost_pull32.as<int32_t>();
 
     std::vector<int32_t> bl;
     for (int b = 0; b < nb; b++) {

@@ -274,3 +274,17 @@ def test_batch_gradient_is_the_sum_of_its_images(n):
     for k in range(n):
         tot = tot + c.gradient(x[k:k + 1], gout[k:k + 1])
     assert np.array_equal(g, tot)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 128, 129])
+def test_forward_is_the_same_bits_in_any_number_of_segments(n):
+    """Up to 64 images are marched in 4 plane segments, up to 128 in 2, more in
+    one: every image's output equals that of the image alone."""
+    s = _shell()
+    c = Cnn(s)
+    c.params = _params(9)
+    x = np.random.default_rng(n).standard_normal((n, 16, 16, 16)).astype(np.float32)
+    print("[cnn segments]", n, flush=True)
+    out = c.forward(x)
+    for k in sorted({0, n // 2, n - 1}):
+        assert np.array_equal(out[k], c.forward(x[k:k + 1])[0])
