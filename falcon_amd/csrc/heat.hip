@@ -896,8 +896,8 @@ __global__ void __launch_bounds__(256) k_hupdate_xr(long long n, double *__restr
     block_partials<1>(v, partial, s);
 }
 
-// p = z - beta p, beta = <z,q>/gamma (dot 0 of partial); beta = 0 (no partials)
-// starts a fresh direction
+// p = z - beta p, beta = <z,q>/gamma (dot 0 of partial); no partials: p = z, a
+// fresh direction, for which the old p is not read (it may hold anything)
 __global__ void __launch_bounds__(256) k_hupdate_p(long long n, double *__restrict__ p, const double *__restrict__ z,
                                                    const double *__restrict__ partial, int nwg,
                                                    const double *__restrict__ sc, const int *__restrict__ active,
@@ -912,7 +912,7 @@ __global__ void __launch_bounds__(256) k_hupdate_p(long long n, double *__restri
         const long long c = c0 + 256 * u;
         if (c < n) {
             const long long io = s * istride + c;
-            p[io] = z[io] - be * p[io];
+            p[io] = nwg ? z[io] - be * p[io] : z[io];
         }
     }
 }
@@ -1041,8 +1041,8 @@ __global__ void __launch_bounds__(256) k_hcopy(const double *__restrict__ a, dou
 
 // ---- learned correction of the V-cycle (features: k_hmarch with OpFeat;
 // the step's dots: k_hmarch with OpApplyDot)
-// p = z + a c - beta p: the learned direction (a = the correction step);
-// beta = 0 starts a fresh direction
+// p = z + a c - beta p: the learned direction (a = the correction step); without
+// use_beta p = z + a c, a fresh direction, for which the old p is not read
 __global__ void __launch_bounds__(256) k_hupdate_p2(long long n, double *__restrict__ p, const double *__restrict__ z,
                                                     const double *__restrict__ cc, const double *__restrict__ sc,
                                                     const double *__restrict__ ablk, int nb, const int *__restrict__ active,
@@ -1052,9 +1052,9 @@ __global__ void __launch_bounds__(256) k_hupdate_p2(long long n, double *__restr
     const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= n) return;
     const double a = ablk ? ablk[(long long)s * nb + (c >> 12)] : sc[kSc * s + 4];
-    const double be = use_beta ? sc[kSc * s + 1] : 0.0;
     const long long io = s * istride + c;
-    p[io] = (z[io] + a * cc[io]) - be * p[io];
+    const double v = z[io] + a * cc[io];
+    p[io] = use_beta ? v - sc[kSc * s + 1] * p[io] : v;
 }
 
 // Per-block correction steps (16^3 blocks, S consecutive workgroups of the

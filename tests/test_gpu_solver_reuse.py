@@ -1,0 +1,62 @@
+"""One solver used again: what a solve or an operator call left behind does not
+reach the next solve."""
+import numpy as np
+import pytest
+
+from falcon_amd import Cnn, HeatSolver, Pfss, Shell, configs
+
+pytestmark = pytest.mark.gpu
+
+LAY = configs.cubic((16, 32, 96), 16)
+
+
+def _heat(mode):
+    s = Shell(LAY)
+    hs = HeatSolver(s, 1.0, 0.7, 2)
+    if mode != "plain":
+        Cnn(s, seed=3)
+        hs.attach_corrector()
+        hs.set_learned_blockstep(mode == "blockstep")
+    hs.set_dt(np.array([30.0, 100.0]) * hs.dt_explicit)
+    return hs
+
+
+@pytest.mark.parametrize("mode", ["plain", "blockstep", "systemstep"])
+@pytest.mark.parametrize("left_by", ["solve", "apply"])
+def test_heat_solve_after_non_finite_input(mode, left_by):
+    """A system that once held a NaN or an infinity solves finite data as a
+    fresh solver does, bit for bit."""
+    learned = mode != "plain"
+    T = 1e-3 * np.random.default_rng(5).standard_normal((2,) + _heat(mode).shape[1:])
+    bad = T.copy()
+    bad[0, 0, 3, 2, 1], bad[1, 1, 0, 0, 0] = np.nan, np.inf
+    hs = _heat(mode)
+    if left_by == "solve":
+        hs.set_T(bad)
+        _, rel, _ = hs.solve(1e-10, 50, use_corrector=learned)
+        assert not np.isfinite(rel).any()
+    else:
+        hs.apply(bad)
+    print("[solver reuse]", mode, left_by, flush=True)
+    hs.set_T(T)
+    it, rel, _ = hs.solve(1e-10, 200, use_corrector=learned)
+    fresh = _heat(mode)
+    fresh.set_T(T)
+    it0, rel0, _ = fresh.solve(1e-10, 200, use_corrector=learned)
+    assert (rel0 <= 1e-10).all()
+    assert np.array_equal(it, it0) and np.array_equal(rel, rel0)
+    for k in range(2):
+        assert np.array_equal(hs.get_T(k), fresh.get_T(k))
+
+
+def test_pfss_solve_after_a_non_finite_magnetogram():
+    pf, fresh = Pfss(Shell(LAY)), Pfss(Shell(LAY))
+    br = np.random.default_rng(6).standard_normal(pf.mshape)
+    bad = br.copy()
+    bad[0, 2, 3] = np.nan
+    pf.set_magnetogram(bad)
+    assert not np.isfinite(pf.solve(1e-10, 50)[1])
+    for p in (pf, fresh):
+        p.set_magnetogram(br)
+        assert p.solve(1e-10, 500)[1] <= 1e-10
+    assert np.array_equal(pf.phi(), fresh.phi()) and np.array_equal(pf.field(), fresh.field())
