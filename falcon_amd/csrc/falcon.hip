@@ -24,6 +24,7 @@
 #include "heat.hpp"
 #include "layout.hpp"
 #include "output.hpp"
+#include "threads.hpp"
 
 // Scratch of falcon_compute_dt_noalloc, in device memory the library never
 // allocates: the dt partial minima (one per tile of the diffusion's edge, at
@@ -379,12 +380,7 @@ void upload_ghosts64(falcon_handle *h) {
     const size_t N = G.size();
     const int nb = d.nblocks, ng = d.ng;
     const int nt = std::max(1, std::min(host_threads(), (int)(N / 8192) + 1));
-    auto parallel = [&](auto &&f) {
-        std::vector<std::thread> th;
-        for (int t = 1; t < nt; t++) th.emplace_back([&, t] { f(t); });
-        f(0);
-        for (auto &x : th) x.join();
-    };
+    auto parallel = [&](auto &&f) { run_shares(nt, f); };
     auto base = [&](const GhostEntry &g) -> int32_t {
         return (int32_t)((long long)g.donor * 8 * d.P + cell_off(d, g.i0 + ng - 1, g.j0 + ng - 1, g.k0 + ng - 1));
     };
@@ -1661,12 +1657,9 @@ int falcon_save_allcells(falcon_handle_t h, int istep, const char *outdir, int m
             HIPCHECK(hipMemcpyAsync(host.data(), dout.p, sizeof(double) * per * n, hipMemcpyDeviceToHost, h->stream));
             HIPCHECK(hipStreamSynchronize(h->stream));
             std::vector<std::string> text(n);
-            std::vector<std::thread> th;
-            for (int w = 0; w < std::min(nt, n); w++)
-                th.emplace_back([&, w]() {
-                    for (int q = w; q < n; q += nt) allcells_block_text(spec, host.data() + per * q, text[q]);
-                });
-            for (auto &x : th) x.join();
+            run_shares(std::min(nt, n), [&](int w) {
+                for (int q = w; q < n; q += nt) allcells_block_text(spec, host.data() + per * q, text[q]);
+            });
             for (int q = 0; q < n; q++) {
                 if (merged) {
                     put(mpath, text[q], true);

@@ -37,7 +37,6 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1525,16 +1524,16 @@ struct Prefault {
         const size_t n = std::min(8u, std::max(1u, std::thread::hardware_concurrency() / 2));
         if (bytes < (32u << 20) || n < 2) return;
         char *p = (char *)dst;
-        t.reserve(n);
         try {
+            t.reserve(n);
             for (size_t k = 0; k < n; k++) {
                 char *lo = p + bytes * k / n, *hi = p + bytes * (k + 1) / n;
                 t.emplace_back([lo, hi] {
                     for (volatile char *q = lo; q < hi; q += 4096) *q = *q;
                 });
             }
-        } catch (const std::system_error &) {
-            // no more threads: the copy faults the rest in
+        } catch (...) {
+            // no more threads (or memory for one): the copy faults the rest in
         }
     }
     void join() {

@@ -7,7 +7,8 @@
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
-#include <thread>
+
+#include "threads.hpp"
 
 namespace falcon {
 
@@ -279,11 +280,8 @@ void conv_rows(const Layout &lay, int nthreads, std::vector<double> &rows) {
                 r[3] = cp / std::sin(o2[1]);
             }
     };
-    std::vector<std::thread> th;
     const int nt = std::max(1, std::min(nthreads, nb));
-    for (int t = 0; t < nt; t++)
-        th.emplace_back([&, t]() { for (int b = t; b < nb; b += nt) work(b); });
-    for (auto &x : th) x.join();
+    run_shares(nt, [&](int t) { for (int b = t; b < nb; b += nt) work(b); });
 }
 
 void Layout::build(int nthreads) {
@@ -365,11 +363,8 @@ void Layout::build(int nthreads) {
         }
     };
 
-    std::vector<std::thread> th;
-    int nt = std::min(nthreads, nb);
-    for (int t = 0; t < nt; t++)
-        th.emplace_back([&, t]() { for (int b = t; b < nb; b += nt) work(b); });
-    for (auto &x : th) x.join();
+    const int nt = std::min(nthreads, nb);
+    run_shares(nt, [&](int t) { for (int b = t; b < nb; b += nt) work(b); });
 
     size_t total = 0;
     for (auto &v : per) total += v.size();
@@ -614,10 +609,8 @@ void build_heat_levels(const Layout &lay, const HeatParams &hp, int nthreads, st
                         L.g_src[gi] = (int32_t)src;
                     }
         };
-        std::vector<std::thread> th;
-        int nt = std::max(1, std::min(nthreads, nb));
-        for (int w = 0; w < nt; w++) th.emplace_back([&, w]() { for (int b = w; b < nb; b += nt) work(b); });
-        for (auto &x : th) x.join();
+        const int nt = std::max(1, std::min(nthreads, nb));
+        run_shares(nt, [&](int w) { for (int b = w; b < nb; b += nt) work(b); });
         for (int b = 0; b < nb; b++) {
             for (size_t e = 0; e < gwslot[b].size(); e++) L.g_wid[gwslot[b][e]] = (int32_t)(L.g_w.size() / 3 + e);
             L.g_w.insert(L.g_w.end(), gw[b].begin(), gw[b].end());
