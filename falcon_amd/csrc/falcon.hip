@@ -664,11 +664,15 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
     const int ts = h->tile_stage[h->precision], td = h->tile_diff[h->precision];
     const int ws = h->wgs_stage[h->precision], wd = h->wgs_diff[h->precision];
     // dt is formed in the launch of the state's radial boundary, the stage
-    // buffers' radial ghosts in their fills
+    // buffers' radial ghosts in their fills and the new state's in its.  Timed
+    // steps (falcon_profile_step) give each a launch of its own, so that every
+    // kind's time holds that kind alone; the values are the same.
+    const bool apart = h->prof_ev != nullptr;
     DtFinal dtf;
     if (h->fixed_dt > 0) timed(h, K_DT, [&] { launch_set_scalar(dtp, h->fixed_dt, s); });
+    else if (apart) timed(h, K_DT, [&] { launch_dt_final(d, part, dtp, cfl, s, td, march_segments(d, td, wd)); });
     else dtf = dt_final_args(d, part, dtp, cfl, td, march_segments(d, td, wd));
-    const FillTail mirror{h->bnd, nullptr};
+    const FillTail mirror = apart ? FillTail{} : FillTail{h->bnd, nullptr};
     if (h->precision == 0) {
         double *S0 = h->S64[0].as<double>(), *S1 = h->S64[1].as<double>();
         const double *in[4] = {U, S0, S1, S0};
@@ -685,7 +689,10 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         if (glm) timed(h, K_OTHER, [&] { launch_glm_speed(d, t, U, Ch, s); });
         for (int k = 1; k <= 4; k++) {
             const double div = (double)(5.0f - (float)k);
-            if (k == 1) timed(h, K_BC, [&] { launch_boundary<double>(d, h->bnd, U, s, nullptr, dtf); });
+            if (k == 1 || apart)
+                timed(h, K_BC, [&] {
+                    launch_boundary<double>(d, h->bnd, const_cast<double *>(in[k - 1]), s, nullptr, k == 1 ? dtf : DtFinal{});
+                });
             if (glm)
                 timed(h, K_OTHER,
                       [&] { launch_glm_stage(d, t, in[k - 1], Ch, pin[k - 1], P, pout[k - 1], G, dtp, div, s); });
@@ -701,7 +708,13 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
         }
         timed(h, K_DIFF, [&] { launch_diffusion<double, double>(d, t, U, U, Un, nullptr, part, dtp, s, nullptr, td, wd); });
         if (glm) timed(h, K_OTHER, [&] { launch_glm_diffusion(d, t, U, P, Pn, dtp, s); });
-        timed(h, K_XSTATE, [&] { launch_exchange64(d, h->gh64, Un, Pn, false, s, FillTail{h->bnd, U}); });
+        const FillTail radial{h->bnd, U};
+        if (apart) {
+            DevGhosts64 none = h->gh64;
+            none.n = none.n_face = 0;
+            timed(h, K_OTHER, [&] { launch_exchange64(d, none, Un, nullptr, false, s, radial); });
+        }
+        timed(h, K_XSTATE, [&] { launch_exchange64(d, h->gh64, Un, Pn, false, s, apart ? FillTail{} : radial); });
     } else {
         float *S0 = h->S32[0].as<float>(), *S1 = h->S32[1].as<float>();
         float *F = h->F32[cur].as<float>(), *Fn = h->F32[1 - cur].as<float>();
@@ -719,7 +732,10 @@ void enqueue_step(falcon_handle *h, double cfl, int cur) {
             else launch_exchange(d, h->gh32, st, s, tail);
         };
         for (int k = 1; k <= 4; k++) {
-            if (k == 1) timed(h, K_BC, [&] { launch_boundary<float>(d, h->bnd, F, s, pull, dtf); });
+            if (k == 1 || apart)
+                timed(h, K_BC, [&] {
+                    launch_boundary<float>(d, h->bnd, const_cast<float *>(in[k - 1]), s, pull, k == 1 ? dtf : DtFinal{});
+                });
             const double div = (double)(5.0f - (float)k);
             if (k < 4) {
                 // intermediate stage values are FP32 temporaries: base = FP32 copy of U^n

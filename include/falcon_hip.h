@@ -208,7 +208,10 @@ int falcon_rhs(falcon_handle_t h, double *r_out);
 int falcon_diffusion_rhs(falcon_handle_t h, double *r_out);
 /* Average kernel durations (ms, HIP events on the handle's stream) over nsteps
  * steps: out[0] dt, [1] boundary, [2] stage, [3] exchange (stage buffers),
- * [4] exchange (state), [5] diffusion, [6] whole step. */
+ * [4] exchange (state), [5] diffusion, [6] whole step.  The steps are real ones
+ * (the state advances), with each of these in launches of its own: an
+ * unprofiled step forms dt in the first boundary launch and the stage buffers'
+ * and the new state's radial ghosts in the exchanges, so it is shorter than [6]. */
 int falcon_profile_step(falcon_handle_t h, int nsteps, double cfl, double *out_ms);
 /* Bytes of device memory held by the handle. */
 int falcon_device_bytes(falcon_handle_t h, int64_t *bytes);
