@@ -520,7 +520,8 @@ void upload_tables(falcon_handle *h) {
     };
     auto weighted = std::async(std::launch::async | std::launch::deferred, [&]() -> Table {
         // a base on an axis's last cell (weight 0 there) becomes the cell before it
-        // with weight 1, so that no corner is a ghost of the donor (k_exchange_f32)
+        // with weight 1, so that no corner is a ghost of the donor (k_exchange_f32,
+        // which handles axes of one cell)
         const int n3[3] = {t.ni, t.nj, t.nk};
         auto inside = [&](GhostEntry g) -> GhostEntry {
             int32_t *base[3] = {&g.i0, &g.j0, &g.k0};

@@ -1024,7 +1024,8 @@ __device__ __forceinline__ int xcd_run(int wg, int n) {
 //   weighted: every corner is loaded (a gather that skips the zero-weight ones
 //     measures twice the time); a base on an axis's last cell, whose upper
 //     corner would be a ghost that this launch fills, is in the table as the
-//     cell before it with weight 1;
+//     cell before it with weight 1.  THIN: blocks with an axis of one cell, where
+//     there is no cell before it; the base stands in for its upper corners;
 //   lerp: same-panel entries whose theta/phi weights lie within 1e-12 of 0 or
 //     1 and whose r weight does not (neighbours across a radial block face,
 //     whose radial spacings differ): the two r corners of the weighted sum;
@@ -1035,6 +1036,7 @@ __device__ __forceinline__ int xcd_run(int wg, int n) {
 // target-list and destination order took 95 us on 1536 16^3 blocks (500 MB),
 // 71 us on 528 refined ones, 20 us on 648 8^3 ones; one launch in source order
 // 81, 59 and 13 us, its face ghosts alone 52, 42 and 9 us.
+template <bool THIN>
 __global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFill copy, int nwe, int nle, int nce,
                                                       float *__restrict__ st, FillTail tail) {
     const int nw = (nwe + 255) / 256, nl = (nle + 255) / 256, nc = (nce + 255) / 256;
@@ -1047,12 +1049,13 @@ __global__ void __launch_bounds__(256) k_exchange_f32(Dims d, DevGhosts g, DevFi
         if (e >= nwe) return;
         const int2 c = g.weighted.idx[e];
         const double wi = g.w[3 * (long long)e], wj = g.w[3 * (long long)e + 1], wk = g.w[3 * (long long)e + 2];
+        const int ci = THIN && d.ni == 1 ? 0 : SI, cj = THIN && d.nj == 1 ? 0 : SJ, ck = THIN && d.nk == 1 ? 0 : 1;
         double val[8];
 #pragma unroll
         for (int v = 0; v < 8; v++) {
             const float *F = st + c.y + (long long)v * P;
-            const double f000 = F[0], f100 = F[SI], f010 = F[SJ], f001 = F[1], f110 = F[SI + SJ], f011 = F[SJ + 1],
-                         f101 = F[SI + 1], f111 = F[SI + SJ + 1];
+            const double f000 = F[0], f100 = F[ci], f010 = F[cj], f001 = F[ck], f110 = F[ci + cj], f011 = F[cj + ck],
+                         f101 = F[ci + ck], f111 = F[ci + cj + ck];
             val[v] = trilinear8(f000, f100, f010, f001, f110, f011, f101, f111, wi, wj, wk);
         }
         if (c.x < 0) yy_rotate(val, g.rot[2 * (long long)e], g.rot[2 * (long long)e + 1]);
@@ -1630,7 +1633,10 @@ static void exchange32(const Dims &d, const DevGhosts &g, const DevFill &copy, b
     auto n = [&](const DevFill &f) { return faces ? f.n_face : f.n; };
     const int nw = n(g.weighted), nl = n(g.lerp), nc = n(copy);
     const unsigned wgs = (unsigned)((nw + 255) / 256 + (nl + 255) / 256 + (nc + 255) / 256) + tail_wgs(d, tail);
-    if (wgs) hipLaunchKernelGGL(k_exchange_f32, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state, tail);
+    if (wgs == 0) return;
+    const bool thin = d.ni == 1 || d.nj == 1 || d.nk == 1;
+    if (thin) hipLaunchKernelGGL(k_exchange_f32<true>, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state, tail);
+    else hipLaunchKernelGGL(k_exchange_f32<false>, dim3(wgs), dim3(256), 0, s, d, g, copy, nw, nl, nc, state, tail);
 }
 
 void launch_exchange(const Dims &d, const DevGhosts &g, float *state, hipStream_t s, const FillTail &tail) {
