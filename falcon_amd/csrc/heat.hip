@@ -761,6 +761,7 @@ __global__ void __launch_bounds__(256) k_hdot(long long n, const double *__restr
 // [3] feature scale of the learned correction, [4] its step along c, [5] <b,b>,
 // [6] <z,q> of the V-cycle output.
 constexpr int kSc = 8;
+constexpr long long kOwnSums = 10000000;
 enum {
     kScNone = -1,
     kScStep = 2,      // correction step <c,r'>/<c,Ac> (dots: [0]=<c,r'>, [1]=<c,Ac>), 0 unless <c,Ac> > 0
@@ -862,7 +863,13 @@ __global__ void k_hizero(int *__restrict__ a, int n) {
 // Where an update needs a scalar of dots that its predecessor left in partial
 // sums, every workgroup adds the nwg partials itself (they come from the L2; the
 // same order as k_hdot_final's): the sum's own launch took 4.6 to 5.4 us, twice an
-// iteration; solve of 6.3 M cells 8.36 -> 8.20 ms, PFSS 4.48 -> 4.44.
+// iteration; solve of 6.3 M cells 8.36 -> 8.20 ms, PFSS 4.48 -> 4.44.  What all
+// // workgroups read grows with the square of the shell, so above kOwnSums reads they
+// are summed once and the workgroups get the sum (nwg = 1), the same bits.  us per
+// iteration with own sums / summed once, by reads of a dot (workgroups x partials):
+//   16^3 blocks: 4.7 M reads 492/497, 10.6 M 742/738, 18.9 M 950/945, 75 M
+//     1873/1817, 302 M (50 M cells) 3819/3525;  8^3 blocks: 9.4 M 800/805
+// and for 2 to 64 systems of up to 4.7 M each the own sums stay ahead or level.
 // x += alpha p ; r -= alpha q with alpha = <p,r>/<p,q> (dots 1 and 0 of pin,
 // gamma = <p,q> kept for beta), and partial sums of r.r into partial
 __global__ void __launch_bounds__(256) k_hupdate_xr(long long n, double *__restrict__ x, double *__restrict__ r,
@@ -1180,6 +1187,17 @@ struct HeatSolver::Impl {
         hipLaunchKernelGGL(k_hdot_final, dim3((unsigned)nsys), dim3(256), 0, stream, part ? part : partial, (int)nwg,
                            npairs, dots, what, what2, sc, active, (double)ist(0),
                            Converge{tol, iters_dev, nactive_dev, relres_dev, posted});
+    }
+    // npairs dots that nwg workgroups left in partial, for the element kernels that
+    // add them themselves: the partials, or above kOwnSums reads their sums
+    struct Sums {
+        const double *p;
+        int n;
+    };
+    Sums sums(int npairs, unsigned nwg) {
+        if ((long long)elem_wgs() * nwg <= kOwnSums) return {partial, (int)nwg};
+        final_dots(npairs, nwg, kScNone);
+        return {dots, 1};
     }
     int pre = 2, post = 2;
     // coarsest level: Jacobi-preconditioned CG to r.z <= coarse_tol^2 (r.z)_0
@@ -1738,8 +1756,9 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
         }
         const int pre0 = recording ? I.learned_pre0 : I.pre, post0 = recording ? I.learned_post0 : I.post;
         const unsigned nwg = I.vcycle(I.r, z, pre0, post0, first ? nullptr : I.q);
-        hipLaunchKernelGGL(k_hupdate_p, I.grid_elem(), dim3(256), 0, I.stream, ni, I.p, (const double *)z,
-                           (const double *)I.partial, first ? 0 : (int)nwg, (const double *)I.sc, (const int *)I.active, ni);
+        const Impl::Sums zq = first ? Impl::Sums{I.partial, 0} : I.sums(1, nwg);
+        hipLaunchKernelGGL(k_hupdate_p, I.grid_elem(), dim3(256), 0, I.stream, ni, I.p, (const double *)z, zq.p, zq.n,
+                           (const double *)I.sc, (const int *)I.active, ni);
         if (recording) {
             I.features(z);
             record(z);
@@ -1748,9 +1767,9 @@ HeatResult HeatSolver::solve(double tol, int max_iter, int mode, HeatRecord *rec
     // one FCG iteration; the convergence test runs on the device (k_hdot_final)
     auto body = [&](bool lrn) {
         I.apply0(I.p, I.q, I.r);                         // q = A p with <p,q>, <p,r>
+        const Impl::Sums pq = I.sums(2, I.march_wgs(0));
         hipLaunchKernelGGL(k_hupdate_xr, I.grid_elem(), dim3(256), 0, I.stream, ni, I.x, I.r, (const double *)I.p,
-                           (const double *)I.q, (const double *)I.partial, (int)I.march_wgs(0), I.sc, (const int *)I.active,
-                           I.partial2, ni);
+                           (const double *)I.q, pq.p, pq.n, I.sc, (const int *)I.active, I.partial2, ni);
         I.final_dots(1, I.elem_wgs(), kScConverge, kScNone, tol, I.partial2);
         precond_direction(false, lrn);
     };
