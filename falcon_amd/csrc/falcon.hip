@@ -81,6 +81,13 @@ void scratch_setup(int dev) {
     g_scratch_ptr[dev] = (double *)p;
 }
 
+// Zeroes device memory and waits for it: hipMemset returns before it has run, and
+// the handles' streams do not wait for the null stream, on which it runs.
+void clear(void *p, size_t bytes) {
+    HIPCHECK(hipMemset(p, 0, bytes));
+    HIPCHECK(hipStreamSynchronize(nullptr));
+}
+
 int host_threads() {
     unsigned n = std::thread::hardware_concurrency();
     return (int)std::max(1u, std::min(n, 32u));
@@ -600,10 +607,10 @@ void alloc_state(falcon_handle *h) {
     for (int q = 0; q < 2; q++) {
         if (!h->U[q].p) {
             h->U[q].alloc(n * sizeof(double));
-            HIPCHECK(hipMemset(h->U[q].p, 0, n * sizeof(double)));
+            clear(h->U[q].p, n * sizeof(double));
         }
     }
-    if (!h->dtp.p) { h->dtp.alloc(sizeof(double)); HIPCHECK(hipMemset(h->dtp.p, 0, sizeof(double))); }
+    if (!h->dtp.p) { h->dtp.alloc(sizeof(double)); clear(h->dtp.p, sizeof(double)); }
     // one partial minimum per workgroup of the diffusion / k_dt_tile (tile and
     // radial segment); the larger of the two tilings
     long long np = 1;
@@ -618,15 +625,15 @@ void alloc_stage(falcon_handle *h) {
     for (int q = 0; q < 2; q++) {
         if (h->precision == 0 && !h->S64[q].p) {
             h->S64[q].alloc(n * sizeof(double));
-            HIPCHECK(hipMemset(h->S64[q].p, 0, n * sizeof(double)));
+            clear(h->S64[q].p, n * sizeof(double));
         }
         if (h->precision == 1 && !h->S32[q].p) {
             h->S32[q].alloc(n * sizeof(float));
-            HIPCHECK(hipMemset(h->S32[q].p, 0, n * sizeof(float)));
+            clear(h->S32[q].p, n * sizeof(float));
         }
         if (h->precision == 1 && !h->F32[q].p) {
             h->F32[q].alloc(n * sizeof(float));
-            HIPCHECK(hipMemset(h->F32[q].p, 0, n * sizeof(float)));
+            clear(h->F32[q].p, n * sizeof(float));
         }
     }
 }
@@ -1190,12 +1197,12 @@ int falcon_set_divb(falcon_handle_t h, int option) {
             const size_t n = (size_t)d.nblocks * d.P, ng = (size_t)d.nblocks * 3 * d.ni * d.nj * d.nk;
             for (DevBuf *b : {&h->psi[0], &h->psi[1], &h->psiS[0], &h->psiS[1]}) {
                 b->alloc(n * sizeof(double));
-                HIPCHECK(hipMemset(b->p, 0, n * sizeof(double)));
+                clear(b->p, n * sizeof(double));
             }
             h->glmG.alloc(ng * sizeof(double));
-            HIPCHECK(hipMemset(h->glmG.p, 0, ng * sizeof(double)));
+            clear(h->glmG.p, ng * sizeof(double));
             h->glmC.alloc(ng / 3 * 2 * sizeof(double));
-            HIPCHECK(hipMemset(h->glmC.p, 0, ng / 3 * 2 * sizeof(double)));
+            clear(h->glmC.p, ng / 3 * 2 * sizeof(double));
         }
         h->divb = option;
     });
@@ -1460,7 +1467,7 @@ int falcon_set_ghost_pull(falcon_handle_t h, int on) {
             // from zeros and the shadow of U is rebuilt.
             if (h->stream) HIPCHECK(hipStreamSynchronize(h->stream));
             for (DevBuf *b : {&h->S32[0], &h->S32[1], &h->F32[0], &h->F32[1]})
-                if (b->p) HIPCHECK(hipMemset(b->p, 0, b->bytes));
+                if (b->p) clear(b->p, b->bytes);
             h->shadow_valid = false;
         }
         h->ghost_pull = on != 0;

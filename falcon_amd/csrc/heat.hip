@@ -1219,8 +1219,11 @@ struct HeatSolver::Impl {
     double *dalloc(size_t n) {
         void *p_ = nullptr;
         HCHECK(hipMalloc(&p_, std::max<size_t>(n, 1) * sizeof(double)));
-        HCHECK(hipMemset(p_, 0, std::max<size_t>(n, 1) * sizeof(double)));
         allocs.push_back(p_);
+        // hipMemset returns before it has run, and the solver's stream does not
+        // wait for the null stream, on which it runs
+        HCHECK(hipMemset(p_, 0, std::max<size_t>(n, 1) * sizeof(double)));
+        HCHECK(hipStreamSynchronize(nullptr));
         return (double *)p_;
     }
     template <typename T>

@@ -76,3 +76,17 @@ def test_a_solve_leaves_its_core_to_other_threads():
     cpu = time.thread_time() - cpu
     print("[solver reuse] core", cpu / sec, flush=True)
     assert cpu < 0.5 * sec
+
+
+@pytest.mark.parametrize("edge", [4, 16])
+def test_operator_of_a_solver_without_a_time_step(edge):
+    """Before the first set_dt 1/dt is 0: the diagonals that the set-up makes are
+    those of the pure diffusion operator, in every new solver."""
+    import pyoracle
+    lay = {"ni": edge, "nj": edge, "nk": edge, "ng": 2, "r_rsun": configs.R_RANGE, "ops": [("split", (2, 4, 12))]}
+    H = pyoracle.HeatOracle(pyoracle.Oracle(lay), 1.0, 0.7)
+    s = Shell(lay)
+    x = np.random.default_rng(edge).standard_normal((1, s.nblocks, edge, edge, edge))
+    want = H.apply(float("inf"), x[0])
+    for _ in range(5):
+        assert np.array_equal(HeatSolver(s, 1.0, 0.7, 1).apply(x)[0], want)
