@@ -25,6 +25,7 @@ struct DevTables {
     const BlockMeta *meta;
     // radial (NI per block)
     const double *xi, *rinv, *r2inv, *rho0, *gp, *gq, *g_over_rho0, *xir2, *heat, *cs, *sqrt_rho0;
+    const double *rho0_up;  // rho0 times kDivUp
     // theta (NJ per block)
     const double *sint, *sinv, *cot;
 };
@@ -33,9 +34,15 @@ struct DevTables {
 // reciprocal, then Markstein's correction of x*y by its exact remainder: the
 // correctly rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990) in 3
 // operations per x, where the general division takes 11 (the same steps with
-// a rescaling of operands near the ends of the exponent range, which neither
-// the divisors here (background, metric, diagonals) nor values above 1e-290 reach).  The
-// fix-up gives zeros, infinities and NaN as the division does.
+// a rescaling of operands near the ends of the exponent range).  The fix-up gives
+// zeros, infinities and NaN as the division does.
+// The remainder is exact for |x| >= 2^-969 (2e-292); below, its rounding changes
+// the last bit of one quotient in 2^1022 |x|.  Cell lengths and matrix diagonals
+// (2^27 and more) divide their dividends as they are: a normal quotient then has
+// |x| > 2^-995.  The divisors near 1 of the FP64 stage (density, sin(theta), 5-k)
+// and their dividends are multiplied by kDivUp, which is exact for every dividend
+// below 2^970 (1e292).
+constexpr double kDivUp = 0x1p54;
 __device__ __forceinline__ double div_rcp(double b) {
     double r = __builtin_amdgcn_rcp(b);
     r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);

@@ -326,7 +326,7 @@ void build_pull_table(const falcon_handle *h, const std::vector<int2> &copy32, s
     }
 }
 
-constexpr int N_RADIAL_ROWS = 11, N_ANGULAR_ROWS = 3;
+constexpr int N_RADIAL_ROWS = 12, N_ANGULAR_ROWS = 3;
 
 // Radial rows of every block from its 1-D background, as [row][block][I]:
 // the 3_6/ModBlock.f90:255-262 products, then the per-term products of
@@ -355,6 +355,7 @@ std::vector<double> radial_rows(const falcon_handle *h) {
             row(8) = (1.0 * (heat + 0.0)) / rho0T0;
             row(9) = (1.0 / xr) * std::sqrt(g1 * p0r);
             row(10) = std::sqrt(rho0);
+            row(11) = rho0 * kDivUp;
         }
     }
     return radT;
@@ -487,6 +488,7 @@ void upload_tables(falcon_handle *h) {
     dt.meta = h->meta.as<BlockMeta>();
     dt.xi = R; dt.rinv = R + rs; dt.r2inv = R + 2 * rs; dt.rho0 = R + 3 * rs; dt.gp = R + 4 * rs; dt.gq = R + 5 * rs;
     dt.g_over_rho0 = R + 6 * rs; dt.xir2 = R + 7 * rs; dt.heat = R + 8 * rs; dt.cs = R + 9 * rs; dt.sqrt_rho0 = R + 10 * rs;
+    dt.rho0_up = R + 11 * rs;
     dt.sint = A; dt.sinv = A + as; dt.cot = A + 2 * as;
 
     const auto &G = h->lay.ghosts;

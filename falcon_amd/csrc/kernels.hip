@@ -244,16 +244,20 @@ struct Marcher {
 template <typename T, typename TW, bool RECIP, typename LDSF>
 __device__ __forceinline__ void cell_rhs(const TW (&win)[8][5], LDSF L, const T xr[5], const T rho0r[5], const T gpr[5],
                                          const T gqr[5], const T st[5], T rinv, T r2inv, T xir2, T heat, T gor,
-                                         T sinv, T cot, T cr, T ct, T cp, T irho0, T R[8]) {
+                                         T sinv, T cot, T cr, T ct, T cp, T irho0, T rho0_up, T R[8]) {
     auto W = [&](int v, int q) -> T { return (T)win[v][q]; };
     const T rho0c = rho0r[2];
-    const T yst = RECIP ? T(0) : div_rcp(st[2]);
-    auto over_rho0 = [&](T x) -> T { return RECIP ? x * irho0 : div_by(x, rho0c, irho0); };
+    // Without RECIP the divisors come times kDivUp, and so do the dividends here
+    // (div_by); irho0 is 1/rho0_up then.  The density's row is in the tables that way:
+    // formed here it took registers (406 against 392 us per launch on 1536 16^3 blocks).
+    constexpr T up = RECIP ? T(1) : T(kDivUp);
+    const T bst = st[2] * up, yst = RECIP ? T(0) : div_rcp(bst);
+    auto over_rho0 = [&](T x) -> T { return RECIP ? x * irho0 : div_by(x * up, rho0_up, irho0); };
     // d4 of f/sin(theta) along phi (sin(theta) is constant along phi)
     auto d4_over_st = [&](T f0, T f1, T f3, T f4) -> T {
         return RECIP ? d4(f0, f1, f3, f4, cp) * sinv
-                     : d4(div_by(f0, st[2], yst), div_by(f1, st[2], yst), div_by(f3, st[2], yst),
-                          div_by(f4, st[2], yst), cp);
+                     : d4(div_by(f0 * up, bst, yst), div_by(f1 * up, bst, yst), div_by(f3 * up, bst, yst),
+                          div_by(f4 * up, bst, yst), cp);
     };
     const T vr = W(1, 2), vt = W(2, 2), vp = W(3, 2);
     const T br = W(4, 2), bt = W(5, 2), bp = W(6, 2);
@@ -438,7 +442,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
         // the FP32 path's reciprocal form (cell_rhs): the stage increment
         // (dt*R)/(5-k) as a product with 1/(5-k)
         constexpr bool RECIP = LEAN;
-        const double rdiv = 1.0 / div, ydiv = div_rcp(div);
+        const double rdiv = kDivUp / div, ydiv = div_rcp(div);
 
         T win[8][5];
         T nxt[8], hn[8];
@@ -469,13 +473,15 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                 if (m.hv) lds[buf][v][m.hly][m.hlx] = hn[v];
             }
             // prefetch the next window plane and the next halo (on the last plane
-            // the clamped loads are discarded)
+            // the clamped loads are discarded; FP64 16-edge tiles leave them out, where
+            // the 8-edge ones would spill 16 registers for the branch: 50.5 against
+            // 48 us per launch on 648 8^3 blocks)
             const int In = min(I + 3, d.NI - 1), Ih = min(I + 1, d.NI - 1);
             const bool more = i + 1 < iB;
     #pragma unroll
             for (int v = 0; v < 8; v++) {
-                nxt[v] = (LEAN || (m.act && more)) ? m.col(v, In) : T(0);
-                hn[v] = (LEAN || (m.hv && more)) ? m.halo(v, Ih) : T(0);
+                nxt[v] = (LEAN || TL == 8 || (m.act && more)) ? m.col(v, In) : T(0);
+                hn[v] = (LEAN || TL == 8 || (m.hv && more)) ? m.halo(v, Ih) : T(0);
             }
             __syncthreads();
             if (m.act) {
@@ -498,7 +504,8 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
                 double R[8];
                 cell_rhs<double, T, RECIP>(win, L, xr, rho0r, gpr, gqr, st, coef(4, I), coef(5, I), coef(6, I),
                                            coef(7, I), coef(8, I), sinv, cot, cr, ct, cp,
-                                           RECIP ? coef(9, I) : div_rcp(rho0r[2]), R);
+                                           RECIP ? coef(9, I) : div_rcp(t.rho0_up[rb + I]),
+                                           RECIP ? 1.0 : t.rho0_up[rb + I], R);
                 if (MODE == 0) {
                     if constexpr (GLM && sizeof(T) == 8) {
                         // ModDivB_GLM (3_6/ModDivB.f90:27-28): R(B) = R(B) - grad(psi)
@@ -511,7 +518,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
     #pragma unroll
                     for (int v = 0; v < 8; v++) {
                         const long long q = base + (long long)v * d.P;
-                        const double inc = RECIP ? (dt * R[v]) * rdiv : div_by(dt * R[v], div, ydiv);
+                        const double inc = RECIP ? (dt * R[v]) * rdiv : div_by((dt * R[v]) * kDivUp, div, ydiv);
                         const double x = (double)(LEAN ? ub[v] : (U + q)[m.coff]) + inc;
                         (out + q)[m.coff] = (TOUT)x;
                         if (SHADOW) (shadow + q)[m.coff] = (float)x;
@@ -1514,6 +1521,7 @@ template <int TL, typename T, typename TIN, typename TOUT, typename TB>
 static void stage_tl(const Dims &d, const DevTables &t, const TIN *in, const TB *U, TOUT *out, float *shadow,
                      const double *dtp, double div, hipStream_t s, const int32_t *pull, int wgs, const double *glm) {
     const int nseg = march_segments(d, TL, wgs);
+    div *= kDivUp;
     const dim3 g = march_grid(d, TL, wgs, nseg), b(TL * TL);
     if constexpr (sizeof(T) == 8) {
         if (glm) {
