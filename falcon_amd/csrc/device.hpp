@@ -57,7 +57,6 @@ struct Dims {
     int ni, nj, nk, ng;
     int NI, NJ, NK;
     int nblocks;
-    int tiles_j, tiles_k;   // 16x16 (theta, phi) tiles per block (k_dt_tile and the 16-edge marches)
     long long P;            // cells per variable per block (NI*NJ*NK)
     // cell layout within one block variable (cell_off): main part strides
     int SJ;                 // nk
@@ -100,8 +99,6 @@ inline Dims make_dims(int ni, int nj, int nk, int ng, int nblocks) {
     d.ni = ni; d.nj = nj; d.nk = nk; d.ng = ng;
     d.NI = ni + 2 * ng; d.NJ = nj + 2 * ng; d.NK = nk + 2 * ng;
     d.nblocks = nblocks;
-    d.tiles_j = (nj + 15) / 16;
-    d.tiles_k = (nk + 15) / 16;
     d.P = (long long)d.NI * d.NJ * d.NK;
     d.SJ = nk;
     d.SI = (long long)d.NJ * nk;

@@ -756,12 +756,11 @@ __global__ void __launch_bounds__(256) k_hdot(long long n, const double *__restr
     block_partials<2>(v, partial, s);
 }
 
-// Per-system scalars on the device, kSc slots each:
-// [0] alpha = <p,r>/<p,q>, [1] beta of the learned direction, [2] gamma = <p,q>,
-// [3] feature scale of the learned correction, [4] its step along c, [5] <b,b>,
-// [6] <z,q> of the V-cycle output.
+// Per-system scalars on the device, kSc slots each: [1] beta of the learned
+// direction, [2] gamma = <p,q>, [3] feature scale of the learned correction, [4]
+// its step along c, [5] <b,b>, [6] <z,q> of the V-cycle output ([0], [7]: none).
 constexpr int kSc = 8;
-constexpr long long kOwnSums = 10000000;
+constexpr long long kOwnSums = 10000000;   // see k_hupdate_xr
 enum {
     kScNone = -1,
     kScStep = 2,      // correction step <c,r'>/<c,Ac> (dots: [0]=<c,r'>, [1]=<c,Ac>), 0 unless <c,Ac> > 0
@@ -882,10 +881,7 @@ __global__ void __launch_bounds__(256) k_hupdate_xr(long long n, double *__restr
     if (!active[s]) return;
     const double pq = sum_partials(pin + (long long)s * 3 * nwg, nwg, red[0]);
     const double a = sum_partials(pin + ((long long)s * 3 + 1) * nwg, nwg, red[1]) / pq;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc[kSc * s] = a;
-        sc[kSc * s + 2] = pq;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[kSc * s + 2] = pq;
     double v[1] = {0.0};
     const long long c0 = (long long)blockIdx.x * kElem + threadIdx.x;
 #pragma unroll 4
