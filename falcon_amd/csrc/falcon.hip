@@ -821,9 +821,11 @@ void check_launch() { HIPCHECK(hipGetLastError()); }
 void read_block(falcon_handle *h, const double *src, int nvar, double *dst) {
     const size_t P = (size_t)h->dims.P, var = P * sizeof(double);
     const int half = (int)std::max<size_t>(1, std::min<size_t>(8, ((size_t)1 << 20) / var));
+    // the buffer last: it stands for all of it, so what could not be made is tried again
     if (!h->pinned) {
+        for (hipEvent_t &e : h->pinned_ev)
+            if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         HIPCHECK(hipHostMalloc((void **)&h->pinned, 2 * half * var, hipHostMallocDefault));
-        for (hipEvent_t &e : h->pinned_ev) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     const int part = std::min(half, nvar > 1 && nvar * var >= ((size_t)256 << 10) ? (nvar + 1) / 2 : nvar);
     auto launch = [&](int q) {
