@@ -442,7 +442,7 @@ __device__ __forceinline__ void stage_body(Dims d, DevTables t, const TIN *__res
         // the FP32 path's reciprocal form (cell_rhs): the stage increment
         // (dt*R)/(5-k) as a product with 1/(5-k)
         constexpr bool RECIP = LEAN;
-        const double rdiv = kDivUp / div, ydiv = div_rcp(div);
+        const double rdiv = 1.0 / div, ydiv = div_rcp(div);
 
         T win[8][5];
         T nxt[8], hn[8];
@@ -1521,7 +1521,7 @@ template <int TL, typename T, typename TIN, typename TOUT, typename TB>
 static void stage_tl(const Dims &d, const DevTables &t, const TIN *in, const TB *U, TOUT *out, float *shadow,
                      const double *dtp, double div, hipStream_t s, const int32_t *pull, int wgs, const double *glm) {
     const int nseg = march_segments(d, TL, wgs);
-    div *= kDivUp;
+    if (sizeof(T) == 8) div *= kDivUp;   // as cell_rhs takes its divisors
     const dim3 g = march_grid(d, TL, wgs, nseg), b(TL * TL);
     if constexpr (sizeof(T) == 8) {
         if (glm) {
