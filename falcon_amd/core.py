@@ -388,6 +388,8 @@ class Shell:
         return out
 
     def profile_step(self, nsteps, cfl=0.5):
+        """Milliseconds per launch of every kind over nsteps real steps, and per
+        step; each kind runs in launches of its own, which a plain step fuses."""
         out = np.zeros(7)
         _check(self.L.falcon_profile_step(self.h, nsteps, cfl, _p(out)))
         keys = ["dt", "boundary", "stage", "exchange_stage", "exchange_state", "diffusion", "step"]

@@ -5,11 +5,13 @@
 // so a wavefront's loads along phi are contiguous.
 //
 // Stage and diffusion kernels march each block along r.  A workgroup of 256
-// lanes owns a 16x16 (theta, phi) tile of one block; lane (ty, tx) owns one
-// (j, k) column and keeps a 5-plane register window of all 8 variables for the
-// r-stencils, while the current r-plane with its 2-cell theta/phi halo is staged
-// in double-buffered LDS for the theta/phi stencils.  Corner (edge) halo cells
-// are never needed by these stencils, so they are never loaded.
+// lanes owns a 16x16 (theta, phi) tile of one block (64 lanes an 8x8 one); lane
+// (ty, tx) owns one (j, k) column and keeps a register window of all 8 variables
+// for the r-stencils (the stage 5 planes; the diffusion 3, with the radial face
+// and half slope it carries), while the current r-plane with its 2-cell theta/phi
+// halo is staged in LDS for the theta/phi stencils (the stage double-buffered).
+// Corner (edge) halo cells are never needed by these stencils, so they are never
+// loaded.
 //
 // Every arithmetic expression keeps the operand order of the reference line it
 // restates; with -ffp-contract=off the FP64 instantiation is bit-identical to
@@ -45,9 +47,9 @@ __device__ __forceinline__ int xcd_tile(int w, int n) {
 
 // the lane index of a flat 1-D launch with the workgroups in xcd_tile's order:
 // a run of consecutive lanes (the cells of one block) is served by one XCD,
-// whose L2 then holds the neighbour planes the run shares.  The scattered
-// gathers of the ghost fill measure 5-8% slower in this order than in the
-// dispatcher's round-robin, and keep the latter.
+// whose L2 then holds the neighbour planes the run shares.  (The ghost fills take
+// shorter runs of workgroups, xcd_run: one contiguous range per XCD measured
+// slower.)
 __device__ __forceinline__ long long xcd_lane() {
     return (long long)xcd_tile((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
 }
@@ -553,12 +555,12 @@ __global__ void __launch_bounds__(TL * TL) k_stage(Dims d, DevTables t, const TI
 }
 
 // The FP64 step's stage (16-edge tiles, one workgroup per tile) held to two
-// wavefronts per SIMD: left to itself the compiler gives it 256 VGPRs plus 2
-// AGPRs, one wavefront per SIMD; held to two it spills a few values (36 bytes
-// per lane) and runs in 2.9 instead of 3.9 ms on 12288 16^3 blocks (386 us on
-// 1536, 1.58 GB at 4.1 TB/s: near the memory rate of a copy, 4.7 TB/s).  The
-// other builds either fit two wavefronts already (the FP32 stages) or would
-// spill tens of registers.
+// wavefronts per SIMD: left to itself the compiler gives it one (3.9 instead of 2.9
+// ms on 12288 16^3 blocks); held to two it takes 250 VGPRs without a spill.  392 us on
+// 1536 blocks, 1.55 GB at 4.0 TB/s: bound by the latency of its loads at two
+// wavefronts per SIMD (62% of their life waiting on a dependency, the SIMD's VALU
+// 28% busy).  The other builds either fit two wavefronts already (the FP32 stages)
+// or would spill tens of registers.
 template <typename T, typename TIN, typename TOUT, typename TB, int MODE, bool SHADOW, int TL, bool PERSIST,
           bool GLM = false>
 __global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2)))
@@ -582,7 +584,8 @@ __constant__ double kParTop[8] = {1.0, -1.0, 1.0, 1.0, 1.0, -1.0, -1.0, 1.0};
 // for :96 and :130.
 // MODE 0: out = U + (0.5*dt)*R (3_6/ModAdvance.f90:104-107); `shadow` (if not
 // null) receives the same value in FP32, and the workgroup's min(h/v_wave) of the
-// new state (the next step's ModTimeStep_Dynamo input) goes to partial[tile].
+// new state (the next step's ModTimeStep_Dynamo input) goes to partial[tile], one
+// per tile and radial segment.
 // MODE 1: write R.  `in` is the stencil input (the state or its FP32 shadow).
 // FP32 path (T = float, MODE 0): U and out are the same buffer, updated in
 // place, and Uold is U^n.  The radial ghosts of the input are the mirror of
@@ -607,19 +610,19 @@ __constant__ double kParTop[8] = {1.0, -1.0, 1.0, 1.0, 1.0, -1.0, -1.0, 1.0};
 // workgroup: done by the first wavefront for all variables, as before, the
 // others waited about a fifth of the plane for it.  FP64 takes the phases in
 // two passes of four variables, so that two workgroups fit a CU's LDS.
-// Bound by vector instructions in FP64 (two thirds busy at two wavefronts per
-// SIMD) and near the memory rate in FP32 (1.5 GB at 4.2 TB/s).  Against one
+// Bound by vector instructions and the latency of a plane's chain: on either path
+// the SIMD's VALU is 60% busy at two wavefronts (FP64 1.5 GB at 3.3 TB/s, FP32
+// 1.6 GB at 4.3 TB/s).  Against one
 // pass that recomputed the slopes per face and kept a five-plane window, with
 // the general divisions and the edges on the first wavefront: FP64 706 -> 476
 // us, FP32 490 -> 360 us on 1536 16^3 blocks; 192 blocks 105 -> 83 and 91 -> 72
 // us.  FP64 held to two wavefronts per SIMD spills 28 bytes per lane; with the
 // eight variables in one pass 124 bytes (607 us).
 template <typename T, typename TIN, int MODE, int TL, bool PERSIST>
-__global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2))) k_diffusion(Dims d, DevTables t, const TIN *__restrict__ in,
-                                                   const double *U, double *out, float *__restrict__ shadow,
-                                                   double *__restrict__ partial, const double *__restrict__ dtp,
-                                                   const int32_t *__restrict__ pull, const double *__restrict__ Uold,
-                                                   int nseg) {
+__global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2)))
+k_diffusion(Dims d, DevTables t, const TIN *__restrict__ in, const double *U, double *out,
+            float *__restrict__ shadow, double *__restrict__ partial, const double *__restrict__ dtp,
+            const int32_t *__restrict__ pull, const double *__restrict__ Uold, int nseg) {
     constexpr int PL = tile_pl<TL>(), NL = TL * TL;
     constexpr bool F32 = sizeof(T) == 4;
     // FP32 path in a step: pulled ghosts, boundary faces from U^n, reciprocals
@@ -954,6 +957,13 @@ __global__ void __launch_bounds__(TL * TL) __attribute__((amdgpu_waves_per_eu(2)
 
 // ---------------------------------------------------------------- exchange
 
+// ModCommunication_SendRecvGC_new (3_6/ModCommunication.f90:678-721) as a
+// table-driven gather: trilinear in the fixed term order of ModMath.f90:283-291
+// with FP64 weights and FP64 accumulation, then the Yin-Yang rotation of v and B
+// (ModYinYang_VecConv_1D, ModYinYang.f90:59-60).  Each ghost has one donor, and
+// donors are read only at interior cells (clamped bases touch a donor ghost only
+// with an exactly-zero weight), so entries are independent.
+
 // the trilinear sum in the term order of ModMath.f90:283-291
 __device__ __forceinline__ double trilinear8(double f000, double f100, double f010, double f001, double f110,
                                              double f011, double f101, double f111, double wi, double wj, double wk) {
@@ -978,14 +988,6 @@ __device__ __forceinline__ void yy_rotate(double (&val)[8], double a, double bb)
     val[2] = v2; val[3] = v3;
 }
 
-// ModCommunication_SendRecvGC_new (3_6/ModCommunication.f90:678-721) as one
-// table-driven gather: trilinear in the fixed term order of ModMath.f90:283-291
-// with FP64 weights and FP64 accumulation, then the Yin-Yang rotation of v and B
-// (ModYinYang_VecConv_1D, ModYinYang.f90:59-60).  Each ghost has one donor, and
-// donors are read only at interior cells (clamped bases touch a donor ghost only
-// with an exactly-zero weight), so entries are independent.
-//
-//
 // The radial ghosts that go with a fill, formed by workgroups behind those of the
 // entries (they read and write other cells: interior and radial-ghost planes,
 // where no entry has its target or a loaded corner).  On their own each was a

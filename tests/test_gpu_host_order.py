@@ -13,8 +13,9 @@ def _shell(edges):
                   "ops": [("split", (1, 2, 6))]})
 
 
-# rows (I, J) around a multiple of 64, K around a multiple of 4, a block of
-# more than the staging buffer's 4 MB (8 variables of 68 x 36 x 52 cells)
+# rows (I, J) around a multiple of 64, K around a multiple of 4, a block whose
+# variables (68 x 36 x 52 cells, 1.02 MB) are so large that each half of the
+# staging buffer holds one of them
 @pytest.mark.parametrize("edges", [(4, 4, 4), (5, 7, 6), (12, 12, 13), (13, 11, 9), (64, 32, 48)])
 def test_state_and_psi_read_back(edges):
     s = _shell(edges)
