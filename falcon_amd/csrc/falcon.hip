@@ -81,12 +81,11 @@ void scratch_setup(int dev) {
     g_scratch_ptr[dev] = (double *)p;
 }
 
-// Zeroes device memory and waits for it: hipMemset returns before it has run, and
-// the handles' streams do not wait for the null stream, on which it runs.
-void clear(void *p, size_t bytes) {
-    HIPCHECK(hipMemset(p, 0, bytes));
-    HIPCHECK(hipStreamSynchronize(nullptr));
-}
+// Zeroed device memory, once wait_cleared has returned: hipMemset returns before it
+// has run, and the handles' streams do not wait for the null stream, on which it
+// runs.
+void clear(void *p, size_t bytes) { HIPCHECK(hipMemset(p, 0, bytes)); }
+void wait_cleared() { HIPCHECK(hipStreamSynchronize(nullptr)); }
 
 int host_threads() {
     unsigned n = std::thread::hardware_concurrency();
@@ -388,7 +387,7 @@ void upload_ghosts64(falcon_handle *h) {
     const size_t N = G.size();
     const int nb = d.nblocks, ng = d.ng;
     const int nt = std::max(1, std::min(host_threads(), (int)(N / 8192) + 1));
-    auto parallel = [&](auto &&f) { run_shares(nt, f); };
+    auto parallel = [&](auto &&f) { run_shares(nt, f, true); };
     auto base = [&](const GhostEntry &g) -> int32_t {
         return (int32_t)((long long)g.donor * 8 * d.P + cell_off(d, g.i0 + ng - 1, g.j0 + ng - 1, g.k0 + ng - 1));
     };
@@ -613,6 +612,7 @@ void alloc_state(falcon_handle *h) {
         }
     }
     if (!h->dtp.p) { h->dtp.alloc(sizeof(double)); clear(h->dtp.p, sizeof(double)); }
+    wait_cleared();
     // one partial minimum per workgroup of the diffusion / k_dt_tile (tile and
     // radial segment); the larger of the two tilings
     long long np = 1;
@@ -624,20 +624,22 @@ void alloc_state(falcon_handle *h) {
 
 void alloc_stage(falcon_handle *h) {
     const size_t n = (size_t)h->dims.nblocks * 8 * h->dims.P;
+    bool made = false;
+    auto make = [&](DevBuf &b, size_t bytes) {
+        if (b.p) return;
+        b.alloc(bytes);
+        clear(b.p, bytes);
+        made = true;
+    };
     for (int q = 0; q < 2; q++) {
-        if (h->precision == 0 && !h->S64[q].p) {
-            h->S64[q].alloc(n * sizeof(double));
-            clear(h->S64[q].p, n * sizeof(double));
-        }
-        if (h->precision == 1 && !h->S32[q].p) {
-            h->S32[q].alloc(n * sizeof(float));
-            clear(h->S32[q].p, n * sizeof(float));
-        }
-        if (h->precision == 1 && !h->F32[q].p) {
-            h->F32[q].alloc(n * sizeof(float));
-            clear(h->F32[q].p, n * sizeof(float));
+        if (h->precision == 0) {
+            make(h->S64[q], n * sizeof(double));
+        } else {
+            make(h->S32[q], n * sizeof(float));
+            make(h->F32[q], n * sizeof(float));
         }
     }
+    if (made) wait_cleared();
 }
 
 enum Kind { K_DT, K_BC, K_STAGE, K_XSTAGE, K_XSTATE, K_DIFF, K_OTHER, K_NKIND };
@@ -1207,6 +1209,7 @@ int falcon_set_divb(falcon_handle_t h, int option) {
             clear(h->glmG.p, ng * sizeof(double));
             h->glmC.alloc(ng / 3 * 2 * sizeof(double));
             clear(h->glmC.p, ng / 3 * 2 * sizeof(double));
+            wait_cleared();
         }
         h->divb = option;
     });
@@ -1472,6 +1475,7 @@ int falcon_set_ghost_pull(falcon_handle_t h, int on) {
             if (h->stream) HIPCHECK(hipStreamSynchronize(h->stream));
             for (DevBuf *b : {&h->S32[0], &h->S32[1], &h->F32[0], &h->F32[1]})
                 if (b->p) clear(b->p, b->bytes);
+            wait_cleared();
             h->shadow_valid = false;
         }
         h->ghost_pull = on != 0;

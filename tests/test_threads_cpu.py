@@ -28,7 +28,7 @@ extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(
 }
 using namespace falcon;
 
-static int shares(int n, int threads, int bad) {
+static int shares(int n, int threads, int bad, bool caller) {
     left = threads;
     std::vector<std::atomic<int>> done(n);
     int err = -1;
@@ -36,7 +36,7 @@ static int shares(int n, int threads, int bad) {
         run_shares(n, [&](int t) {
             done[t]++;
             if (bad >= 0 && t >= bad) throw std::runtime_error(std::to_string(t));
-        });
+        }, caller);
     } catch (const std::exception &e) {
         err = std::stoi(e.what());
     }
@@ -58,10 +58,14 @@ static std::vector<GhostEntry> ghosts(int threads) {
 int main() {
     for (int n : {0, 1, 2, 8})
         for (int threads : {0, 1, 3, 100})
-            for (int bad : {-1, 0, 1, 5}) {
-                const int e = shares(n, threads, bad);
-                if (e) { std::printf("shares n=%d threads=%d bad=%d: %d\n", n, threads, bad, e); return 1; }
-            }
+            for (int bad : {-1, 0, 1, 5})
+                for (bool caller : {false, true}) {
+                    const int e = shares(n, threads, bad, caller);
+                    if (e) {
+                        std::printf("shares n=%d threads=%d bad=%d caller=%d: %d\n", n, threads, bad, caller, e);
+                        return 1;
+                    }
+                }
     const auto a = ghosts(1 << 30);
     for (int threads : {0, 3}) {
         const auto b = ghosts(threads);
